@@ -63,6 +63,14 @@ __device__ __forceinline__ float div_by_rcp_finite(float a, float b, float rcp) 
     return __builtin_fmaf(-e, rcp, q);
 }
 
+// Two neighbouring elements of the normed row, rT(gamma * rT(res * rstd)), packed.
+template <typename T>
+__device__ __forceinline__ uint32_t normed_pair(uint32_t gamma, uint32_t res, float rstd) {
+    using P = Pack16<T>;
+    if constexpr (is_half<T>) return P::mul(gamma, P::scale_round(res, rstd));
+    else return P::pack(P::lo(gamma) * P::round(P::lo(res) * rstd), P::hi(gamma) * P::round(P::hi(res) * rstd));
+}
+
 // The codes of one chunk by plain IEEE division, for scales so small or large (or not a number) that a reciprocal
 // leaves the normal range.  Kept out of line: it is long (eight expanded divisions and clamps), it is almost never
 // taken, and inlined it sat between the kernel's last two stretches of common-path code, which a wave then reached
@@ -151,7 +159,9 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
     for (int i = 0; i < NCHUNK; ++i) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const uint32_t w = P::pack(P::lo(xv[i][j]) + P::lo(rv[i][j]), P::hi(xv[i][j]) + P::hi(rv[i][j]));
+            uint32_t w;
+            if constexpr (is_half<T>) w = P::add(xv[i][j], rv[i][j]);
+            else w = P::pack(P::lo(xv[i][j]) + P::lo(rv[i][j]), P::hi(xv[i][j]) + P::hi(rv[i][j]));
             xv[i][j] = w;  // xv now holds the residual
             if (j & 1) ss1 = P::add_squares(w, ss1);
             else ss0 = P::add_squares(w, ss0);
@@ -189,9 +199,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         for (int i = 0; i < NCHUNK; ++i) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float lo = P::lo(gv[i][j]) * P::round(P::lo(xv[i][j]) * rstd);
-                const float hi = P::hi(gv[i][j]) * P::round(P::hi(xv[i][j]) * rstd);
-                normed[i][j] = P::pack(lo, hi);
+                normed[i][j] = normed_pair<T>(gv[i][j], xv[i][j], rstd);
             }
             if (!GATED && live[i]) store_stream(out + i * nthreads + tid, normed[i]);
         }
@@ -216,19 +224,28 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         // the normed row stays in fp32 registers, every value already rounded to the 16-bit type.
         // v_max3_f32 drops NaNs where the reference's amax propagates them: they are tracked apart
         // (kPacked, the gated four-chunk form: as 16-bit pairs instead, half the registers, so that eight waves fit a
-        // SIMD with the residual kept for the gate as well; unpacked again in phase 3)
-        constexpr bool kPacked = GATED && NCHUNK == 4;
+        // SIMD with the residual kept for the gate as well; unpacked again in phase 3.  Half precision: always, its
+        // arithmetic is packed and reads either half of a dword where bfloat16 needs an instruction to unpack it;
+        // unpacked, the kernel took 410 vector instructions per wave at two chunks per lane and the four-chunk form
+        // spilled: 4000 x 5120 ran in 34.3 us where bfloat16 takes 23.7; now 24.8, and 2000 x 7168 in 17.3
+        // against 22.2)
+        constexpr bool kPacked = (GATED && NCHUNK == 4) || is_half<T>;
         float nv[kPacked ? 1 : NCHUNK][8];
         uint32_t nw[kPacked ? NCHUNK : 1][4];
         float m0 = 0.f, m1 = 0.f;
+        uint32_t half_max = 0;  // (half precision: both halves' largest magnitude, a NaN beating every number)
         bool any_nan = false;
 #pragma unroll
         for (int i = 0; i < NCHUNK; ++i) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 float lo, hi;
-                if constexpr (kPacked) {
-                    nw[i][j] = P::pack(P::lo(gv[i][j]) * P::round(P::lo(xv[i][j]) * rstd), P::hi(gv[i][j]) * P::round(P::hi(xv[i][j]) * rstd));
+                if constexpr (is_half<T>) {
+                    nw[i][j] = normed_pair<T>(gv[i][j], xv[i][j], rstd);
+                    if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) half_max = P::max_abs(half_max, nw[i][j]);
+                    continue;
+                } else if constexpr (kPacked) {
+                    nw[i][j] = normed_pair<T>(gv[i][j], xv[i][j], rstd);
                     lo = P::lo(nw[i][j]);
                     hi = P::hi(nw[i][j]);
                 } else {
@@ -248,6 +265,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         GPUK_STAMP(6);  // row normed, the lane's maximum known
         if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
             float amax[1] = {any_nan ? __builtin_nanf("") : __builtin_fmaxf(m0, m1)};
+            if constexpr (is_half<T>) amax[0] = MaxOp::apply(P::lo(half_max), P::hi(half_max));
             block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
             GPUK_STAMP(7);  // row maximum known to every wave
             // rcp_fp8_max is RN(1 / fp8_max) for the two maxima the quotient was checked for (448, 240), else 0
@@ -266,7 +284,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         // division gives for infinite and NaN numerators.
         constexpr bool kDynamic = QUANT == GPUK_QUANT_FP8_DYNAMIC;
         u32x2 *out = reinterpret_cast<u32x2 *>(norm_out) + row_base;
-        if constexpr (kPacked) {  // (or the compiler keeps phase 2's unpacked copies alive instead)
+        if constexpr (kPacked && !is_half<T>) {  // (or the compiler keeps phase 2's unpacked copies alive instead)
 #pragma unroll
             for (int i = 0; i < NCHUNK; ++i)
 #pragma unroll
@@ -285,6 +303,13 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
                 float q[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
+                    if constexpr (is_half<T> && kDynamic) {  // div_by_rcp_finite, its numerator read in place
+                        const uint32_t w = nw[i][j >> 1];
+                        const float p = (j & 1) ? P::mul_hi(w, rcp) : P::mul_lo(w, rcp);
+                        const float e = (j & 1) ? P::fma_minus_hi(p, scale, w) : P::fma_minus_lo(p, scale, w);
+                        q[j] = __builtin_fmaf(-e, rcp, p);
+                        continue;
+                    }
                     float n;
                     if constexpr (kPacked) n = (j & 1) ? P::hi(nw[i][j >> 1]) : P::lo(nw[i][j >> 1]);
                     else n = nv[i][j];

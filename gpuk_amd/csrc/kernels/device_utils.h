@@ -17,6 +17,8 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 struct BF16 {};  // tag types: the 16-bit storage format of activations
 struct FP16 {};
+template <typename T> inline constexpr bool is_half = false;
+template <> inline constexpr bool is_half<FP16> = true;
 
 // Two 16-bit floats packed in one dword <-> two fp32 values.  Packing rounds to nearest even
 // (v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32).
@@ -40,6 +42,13 @@ template <> struct Pack16<BF16> {
     static __device__ __forceinline__ float from_bits16(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
 };
 
+// Half precision has what bfloat16 lacks: packed arithmetic on both halves of a dword (v_pk_mul_f16, v_pk_add_f16) and
+// multiply-adds that read one half of a dword as an fp32 operand (v_fma_mix_f32).  Products and sums of two halves are
+// therefore computed as such: the fp32 product of two 11-bit significands is exact, and a sum rounded to fp32's 24
+// bits and then to 11 equals the sum rounded once (24 >= 2 * 11 + 2), so both are the sequence's fp32 operation
+// followed by its rounding, in half an instruction per element instead of three and a half.  Only the product with
+// an fp32 factor (scale_round) is rounded twice, and stays two instructions.
+typedef _Float16 f16pair __attribute__((ext_vector_type(2)));
 template <> struct Pack16<FP16> {
     static __device__ __forceinline__ float lo(uint32_t w) {
         return (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu));
@@ -54,17 +63,60 @@ template <> struct Pack16<FP16> {
     static __device__ __forceinline__ uint32_t pack(float a, float b) {
         asm("" : "+v"(a));
         asm("" : "+v"(b));
-        const uint32_t l = __builtin_bit_cast(uint16_t, (_Float16)a);
-        const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)b);
-        return l | (h << 16);
+        f32x2 v = {a, b};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
     }
-    static __device__ __forceinline__ float round(float a) {
-        asm("" : "+v"(a));
-        return (float)(_Float16)a;
+    // lo(w) * b and hi(w) * b in fp32, one instruction each with no unpacking: -0 is added, which changes no product,
+    // signs of zeros included
+    static __device__ __forceinline__ float mul_lo(uint32_t w, float b) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(b));
+        return r;
     }
-    static __device__ __forceinline__ float add_squares(uint32_t w, float acc) {
-        const float a = lo(w), b = hi(w);
-        return __builtin_fmaf(b, b, __builtin_fmaf(a, a, acc));
+    static __device__ __forceinline__ float mul_hi(uint32_t w, float b) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(b));
+        return r;
+    }
+    // a * b - lo(w) and a * b - hi(w) in fp32
+    static __device__ __forceinline__ float fma_minus_lo(float a, float b, uint32_t w) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(a), "v"(b), "v"(w));
+        return r;
+    }
+    static __device__ __forceinline__ float fma_minus_hi(float a, float b, uint32_t w) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(a), "v"(b), "v"(w));
+        return r;
+    }
+    static __device__ __forceinline__ float add_squares(uint32_t w, float acc) {  // lo(w)^2 first, then hi(w)^2
+        float r;
+        asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(w), "v"(acc));
+        asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(w), "v"(r));
+        return r;
+    }
+    // both halves of rT(a + b), rT(a * b), rT(a * s) for an fp32 s
+    static __device__ __forceinline__ uint32_t add(uint32_t a, uint32_t b) {
+        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16pair, a) + __builtin_bit_cast(f16pair, b));
+    }
+    static __device__ __forceinline__ uint32_t sub(uint32_t a, uint32_t b) {
+        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16pair, a) - __builtin_bit_cast(f16pair, b));
+    }
+    static __device__ __forceinline__ uint32_t mul(uint32_t a, uint32_t b) {
+        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16pair, a) * __builtin_bit_cast(f16pair, b));
+    }
+    static __device__ __forceinline__ uint32_t scale_round(uint32_t a, float s) { return pack(mul_lo(a, s), mul_hi(a, s)); }
+    // the pair (x1, x2) rotated by (c, s): (rT(rT(x1*c) - rT(x2*s)), rT(rT(x2*c) + rT(x1*s)))
+    template <bool HIGH>  // c and s are the high (low) halves of the two dwords
+    static __device__ __forceinline__ uint32_t rotate_pair(uint32_t x, uint32_t cos2, uint32_t sin2) {
+        const f16pair n = __builtin_bit_cast(f16pair, x), c = __builtin_bit_cast(f16pair, cos2), s = __builtin_bit_cast(f16pair, sin2);
+        const f16pair p = n * f16pair{c[HIGH], c[HIGH]}, q = f16pair{n[1], n[0]} * f16pair{s[HIGH], s[HIGH]};
+        return __builtin_bit_cast(uint32_t, p + f16pair{-q[0], q[1]});
+    }
+    // the larger magnitude of each half (a NaN beats every number, as in MaxOp): magnitudes order like unsigned integers
+    static __device__ __forceinline__ uint32_t max_abs(uint32_t m, uint32_t w) {
+        typedef uint16_t u16pair __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16pair, m), __builtin_bit_cast(u16pair, w & 0x7fff7fffu)));
     }
     static __device__ __forceinline__ float from_bits16(uint32_t h) {
         return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
