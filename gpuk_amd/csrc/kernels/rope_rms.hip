@@ -230,6 +230,29 @@ __device__ __forceinline__ void store_pair(void *p, const u32x4 &a, const u32x4 
         *reinterpret_cast<u32x4 *>(static_cast<char *>(p) + OFFSET) = b;
     }
 }
+// Heads of 64 elements fill one 128-byte line each, and a lane's two chunks of its head are half a line apart: accessed
+// where they are computed, every wave instruction would touch half of each of its lines, the other half following in
+// the next one.  So eight lanes move the lines of their two heads whole -- the even head's with one instruction, the odd
+// head's with the next -- and exchange chunks: a and b on entry are the lane's pieces of the even and the odd head's
+// line, on exit the two chunks of the lane's own head, and the other way round (the exchange is its own inverse; one
+// DPP move per dword and direction).  Measured, half lines / whole ones: 10024 tokens of 64 + 64 heads in place 61.8 /
+// 54.2 us (55.6 with whole stores only), 3000 tokens 20.9 / 19.8, 16384 of 28 + 4 in half precision 32.0 / 27.3;
+// two streams of 2 x (678 + 3608) tokens, 24 + 25 heads 23.7 / 22.1.  Calls that do not stream their stores (below 8 MB)
+// are bound by latency and keep the shorter code (2.14 / 2.21 us at one token), and so do those with a cache: a unit of
+// theirs is half Q and half K rows scattered over slots, and gains nothing (12.4 / 12.6 us at 4096 tokens of 32+8+8).
+__device__ __forceinline__ void exchange_lines(u32x4 &a, u32x4 &b) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int lo = (int)a[j], hi = (int)b[j];
+        a[j] = (uint32_t)__builtin_amdgcn_update_dpp(lo, hi, 0x114, 0xf, 0xa, false);  // row_shr:4 into lanes 4-7 of 8
+        b[j] = (uint32_t)__builtin_amdgcn_update_dpp(hi, lo, 0x104, 0xf, 0x5, false);  // row_shl:4 into lanes 0-3 of 8
+    }
+}
+
+__device__ __forceinline__ void store_chunk_streamed(void *p, const u32x4 &v) {  // one of store_pair's two
+    asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+}
+
 // What one wave keeps about one unit (= one group of 64/(D/16) consecutive Q/K heads of one token, plus its share
 // of the token's V row) between issuing the unit's loads and finishing it.
 struct UnitState {
@@ -255,6 +278,7 @@ struct RopeUnit {
 
     // Issues the loads of the unit that need nothing but the kernel's leading parameters (which a wave finds in its
     // registers): the activations, the unit's share of the V row, the position(s).  Nothing is waited for.
+    template <bool WHOLE>  // whole lines: see exchange_lines
     static __device__ __forceinline__ void issue_early_loads(const RopeArgs &a, uint32_t unit, int lane, UnitState &st) {
         st.t = a.upt_magic ? __umulhi(unit, a.upt_magic) : unit;
         st.u = unit - st.t * a.units_per_token;
@@ -267,11 +291,16 @@ struct RopeUnit {
         st.active = head_raw < heads_qk;
         st.head = min(head_raw, heads_qk - 1);
         st.is_q = st.head < a.hq;
-        const uint16_t *src = st.token_in + (int64_t)st.head * D;
+        const uint16_t *src_a = st.token_in + (int64_t)st.head * D + c0(sub), *src_b = src_a + HALF;
+        if constexpr (WHOLE) {
+            const int even = (int)(st.u * HPW) + (hl & ~1);
+            src_a = st.token_in + (int64_t)min(even, heads_qk - 1) * D + 8 * (lane & 7);
+            src_b = st.token_in + (int64_t)min(even + 1, heads_qk - 1) * D + 8 * (lane & 7);
+        }
         // streamed, in place too (the lines are written a moment later, but past the L2: keeping them there cost 2-17 %
         // from 512 tokens on once the stores were streamed)
-        st.xa = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + c0(sub)));
-        st.xb = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + c1(sub)));
+        st.xa = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_a));
+        st.xb = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_b));
 
         // this wave's share of the token's V row: chunk u*64 + lane (and further strides of units_per_token*64)
         if constexpr (SETKV) {
@@ -352,12 +381,13 @@ struct RopeUnit {
 
     // Norm, rotation and all stores of the unit.  GATED: no store before a.gate ticks after `entry`, the wave's entry
     // time (a template parameter: as a run-time choice the check cost the launches without a gate 2-6 %).
-    template <bool GATED>
+    template <bool GATED, bool WHOLE>
     static __device__ __forceinline__ void finish(const RopeArgs &a, int lane, UnitState &st, uint64_t entry) {
         const int sub = lane % LPH;
         const int heads_qk = a.hq + a.hk, heads_all = heads_qk + a.hv;
         const u32x4 &xa = st.xa, &xb = st.xb, &wa = st.wa, &wb = st.wb, &cosv = st.cosv, &sinv = st.sinv;
 
+        if constexpr (WHOLE) exchange_lines(st.xa, st.xb);
         u32x4 oa, ob;
         norm_rotate<T, D, NEOX>(xa, xb, wa, wb, cosv, sinv, a.eps, oa, ob);
         // batches whose waves are all resident at once: no store before the launch's reads are through (the rotated
@@ -372,7 +402,14 @@ struct RopeUnit {
         // row is still produced, its K and V rows are dropped.  The reference would write out of bounds.
         const bool slot_ok = !SETKV || st.slot >= 0;  // wave-uniform
         const int head = st.head;
-        if (st.active && (st.is_q || slot_ok)) {
+        if constexpr (WHOLE) {
+            static_assert(!SETKV, "whole lines: in place only");
+            exchange_lines(oa, ob);
+            const int even = (int)(st.u * HPW) + ((lane / LPH) & ~1);
+            uint16_t *dst = static_cast<uint16_t *>(a.qkv_out) + ((int64_t)st.t * heads_all + even) * D + 8 * (lane & 7);
+            if (even + 1 < heads_qk) store_pair<D * 2>(dst, oa, ob, true);
+            else if (even < heads_qk) store_chunk_streamed(dst, oa);
+        } else if (st.active && (st.is_q || slot_ok)) {
             if constexpr (!SETKV) {
                 uint16_t *dst = static_cast<uint16_t *>(a.qkv_out) + ((int64_t)st.t * heads_all + head) * D;
                 store_pair<HALF * 2>(dst + c0(sub), oa, ob, a.stream_rows != 0);
@@ -435,7 +472,7 @@ struct UnitKernelLead {
 };
 static_assert(sizeof(UnitKernelLead) == 56 && sizeof(UnitKernelLead) % alignof(RopeArgs) == 0, "offset of the block");
 
-template <typename T, int D, bool NEOX, int AXES, bool SETKV, bool KVFP8, bool GATED>
+template <typename T, int D, bool NEOX, int AXES, bool SETKV, bool KVFP8, bool GATED, bool WHOLE>
 __global__ void __launch_bounds__(512)
 rope_rms_kernel(const void *qkv_in, const int64_t *positions, uint32_t total_units, uint32_t units_per_token,
                 uint32_t upt_magic, int hq, int hk, uint32_t hv_and_waves, int64_t ps_token, int64_t ps_axis,
@@ -459,7 +496,7 @@ rope_rms_kernel(const void *qkv_in, const int64_t *positions, uint32_t total_uni
     GPUK_STAMPS_BEGIN();  // profiling build only
     const int lane = threadIdx.x & 63;
     UnitState st;
-    Unit::issue_early_loads(a, unit, lane, st);
+    Unit::template issue_early_loads<WHOLE>(a, unit, lane, st);
     // The rest of the arguments is fetched from the argument block only now, behind the requests above.  (Left to
     // the compiler the fetch is the kernel's first instruction, and the first vector load then waits for it: in one
     // instantiation for a register the fetch is about to overwrite, in another for the pinned weight pointers.)
@@ -503,7 +540,7 @@ rope_rms_kernel(const void *qkv_in, const int64_t *positions, uint32_t total_uni
     // moves arithmetic above later loads and the wave pays several memory round trips in a row.
     __builtin_amdgcn_sched_barrier(0);
     GPUK_STAMP_DRAINED(3);  // everything landed
-    Unit::template finish<GATED>(a, lane, st, entry);
+    Unit::template finish<GATED, WHOLE>(a, lane, st, entry);
     GPUK_STAMP(4);          // rows stored (issued)
     GPUK_STAMP_DRAINED(5);  // ... and acknowledged
     GPUK_STAMPS_WRITE(unit);
@@ -999,7 +1036,7 @@ static_assert(sizeof(TwoWayKernelLead) == 56 && sizeof(TwoWayKernelLead) % align
 // row counts are products and sums of those, not loads.  (With everything in the argument block and the per-segment
 // values picked by index, a wave went through five dependent fetches of the block before its first request.)  The
 // block (weights, tables, outputs, the division constants) is fetched behind the activations, in one batch.
-template <typename T, int D, bool NEOX>
+template <typename T, int D, bool NEOX, bool WHOLE>
 __global__ void __launch_bounds__(256)
 rope_rms_2way_kernel(const void *q0, const void *k0, const void *q1, const void *k1, uint32_t tokens0, uint32_t tokens1,
                      uint32_t heads_q, uint32_t heads_k, uint32_t stream, const TwoWayArgs rest) {
@@ -1024,9 +1061,15 @@ rope_rms_2way_kernel(const void *q0, const void *k0, const void *q1, const void 
     const uint32_t row = min(row_raw, rows - 1);  // (token, head) flattened inside the segment
 
     const int c0 = 8 * sub, c1 = HALF + 8 * sub;
-    const uint16_t *src = static_cast<const uint16_t *>(in) + ((int64_t)batch * rows + row) * D;
-    const u32x4 xa = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + c0));
-    const u32x4 xb = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + c1));
+    const uint16_t *batch_in = static_cast<const uint16_t *>(in) + (int64_t)batch * rows * D;
+    const uint32_t even = row_raw & ~1u;  // (heads of one line: the two rows whose lines the lane moves pieces of)
+    const uint16_t *src_a = batch_in + (int64_t)row * D + c0, *src_b = src_a + HALF;
+    if constexpr (WHOLE) {
+        src_a = batch_in + (int64_t)min(even, rows - 1) * D + 8 * (lane & 7);
+        src_b = batch_in + (int64_t)min(even + 1, rows - 1) * D + 8 * (lane & 7);
+    }
+    u32x4 xa = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_a));
+    u32x4 xb = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_b));
 
     typedef const __attribute__((address_space(4))) TwoWayArgs *BlockPtr;
     BlockPtr block = (BlockPtr)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() +
@@ -1041,7 +1084,6 @@ rope_rms_2way_kernel(const void *q0, const void *k0, const void *q1, const void 
                  "s"(magic_k), "s"(eps));
     const uint32_t magic = kind ? magic_k : magic_q;
     const uint32_t token = magic ? __umulhi(row, magic) : row;
-    const uint32_t head = row - token * heads;
     const uint16_t *wsrc = static_cast<const uint16_t *>(seg == 0 ? w0 : seg == 1 ? w1 : seg == 2 ? w2 : w3);
     const u32x4 wa = *reinterpret_cast<const u32x4 *>(wsrc + c0);
     const u32x4 wb = *reinterpret_cast<const u32x4 *>(wsrc + c1);
@@ -1050,12 +1092,19 @@ rope_rms_2way_kernel(const void *q0, const void *k0, const void *q1, const void 
     const u32x4 sinv = load_trig<D, NEOX>(table + HALF, sub);
     __builtin_amdgcn_sched_barrier(0);
 
+    if constexpr (WHOLE) exchange_lines(xa, xb);
     u32x4 oa, ob;
     norm_rotate<T, D, NEOX>(xa, xb, wa, wb, cosv, sinv, eps, oa, ob);
-    if (active) {
-        const int64_t out_token = (int64_t)batch * (tokens0 + tokens1) + (stream_id ? tokens0 : 0u) + token;
-        uint16_t *dst = static_cast<uint16_t *>(kind ? out_k : out_q) + (out_token * heads + head) * D;
-        store_pair<HALF * 2>(dst + c0, oa, ob, stream != 0);
+    // (the rows of a segment are contiguous in its output too)
+    const int64_t out_token = (int64_t)batch * (tokens0 + tokens1) + (stream_id ? tokens0 : 0u);
+    uint16_t *dst = static_cast<uint16_t *>(kind ? out_k : out_q) + out_token * heads * D;
+    if constexpr (WHOLE) {
+        exchange_lines(oa, ob);
+        dst += (int64_t)even * D + 8 * (lane & 7);
+        if (even + 1 < rows) store_pair<D * 2>(dst, oa, ob, true);
+        else if (even < rows) store_chunk_streamed(dst, oa);
+    } else if (active) {
+        store_pair<HALF * 2>(dst + (int64_t)row * D + c0, oa, ob, stream != 0);
     }
 }
 
@@ -1118,11 +1167,14 @@ __global__ void __launch_bounds__(256) rope_rms_2way_wide_kernel(const TwoWayArg
 template <typename T, int D>
 int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stream) {
     const dim3 grid((a.unit_end[3] + 3) / 4, batch);
-#define GPUK_LAUNCH_2WAY(NEOX)                                                                                         \
-    rope_rms_2way_kernel<T, D, NEOX><<<grid, 256, 0, stream>>>(a.in[0], a.in[1], a.in[2], a.in[3], (uint32_t)a.tokens0,  \
+#define GPUK_LAUNCH_2WAY(NEOX, WHOLE)                                                                                  \
+    rope_rms_2way_kernel<T, D, NEOX, WHOLE><<<grid, 256, 0, stream>>>(a.in[0], a.in[1], a.in[2], a.in[3], (uint32_t)a.tokens0,  \
                                                                (uint32_t)a.tokens1, a.heads[0], a.heads[1], a.stream, a)
-    if (neox) GPUK_LAUNCH_2WAY(true);
-    else GPUK_LAUNCH_2WAY(false);
+    constexpr bool kHalfLines = D == 64;  // see exchange_lines
+    if (neox && kHalfLines && a.stream) GPUK_LAUNCH_2WAY(true, kHalfLines);
+    else if (kHalfLines && a.stream) GPUK_LAUNCH_2WAY(false, kHalfLines);
+    else if (neox) GPUK_LAUNCH_2WAY(true, false);
+    else GPUK_LAUNCH_2WAY(false, false);
 #undef GPUK_LAUNCH_2WAY
     return hip_status(hipGetLastError());
 }
@@ -1299,12 +1351,15 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
         }
     }
     const uint32_t log2_waves = p.threads == 64 ? 0u : p.threads == 128 ? 1u : p.threads == 256 ? 2u : 3u;
-#define GPUK_LAUNCH_UNITS(GATED)                                                                                        \
-    rope_rms_kernel<T, D, NEOX, AXES, SETKV, KVFP8, GATED><<<p.blocks, p.threads, 0, stream>>>(                         \
+    constexpr bool kHalfLines = D == 64 && !SETKV;  // see exchange_lines
+#define GPUK_LAUNCH_UNITS(GATED, WHOLE)                                                                                 \
+    rope_rms_kernel<T, D, NEOX, AXES, SETKV, KVFP8, GATED, WHOLE><<<p.blocks, p.threads, 0, stream>>>(                         \
         a.qkv_in, a.positions, a.total_units, a.units_per_token, a.upt_magic, a.hq, a.hk,                               \
         (uint32_t)a.hv | (log2_waves << 24), a.ps_token, a.ps_axis, b)
-    if (b.gate) GPUK_LAUNCH_UNITS(true);
-    else GPUK_LAUNCH_UNITS(false);
+    if (kHalfLines && b.stream_rows && b.gate) GPUK_LAUNCH_UNITS(true, kHalfLines);
+    else if (kHalfLines && b.stream_rows) GPUK_LAUNCH_UNITS(false, kHalfLines);
+    else if (b.gate) GPUK_LAUNCH_UNITS(true, false);
+    else GPUK_LAUNCH_UNITS(false, false);
 #undef GPUK_LAUNCH_UNITS
     return hip_status(hipGetLastError());
 }
