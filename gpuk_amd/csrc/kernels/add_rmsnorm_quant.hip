@@ -39,6 +39,7 @@ __device__ __forceinline__ void store_stream(V *p, V v) { __builtin_nontemporal_
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // The scale reciprocal is usable by div_by_rcp when scale is comfortably normal.
 __device__ __forceinline__ bool scale_in_fast_range(float s) {
@@ -480,9 +481,167 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
     }
 }
 
-// fp32 and fp64 activations: the reference dispatches them through the same template
+constexpr int kF32MaxChunks = 4 * kMaxThreads;
+// fp32 rows that stay in registers (up to 4 x 1024 chunks of 4 elements): the arrangement of add_rmsnorm_quant_rows -- same
+// arguments, lane-to-chunk mapping, store gate and short exact quotients -- around plain fp32 arithmetic, where every
+// rounding to the activation type is the identity:
+//   res = x + r;  rstd = 1/sqrt(mean(res^2) + eps);  n = gamma * (res * rstd);  scale = max|n| / fp8_max;
+//   code = e4m3fn(clamp(n / scale))
+// 13 bytes per element with codes, 16 without: bound by HBM.  The first version fetched gamma behind the first reduction,
+// divided with the full expansion, stored codes 4 bytes per lane and had no store gate.  Per call, that version / this
+// one, dynamic scale: 8192 x 4096 72.0 / 68.0 us (6.05 / 6.41 TB/s), 3000 x 7168 52.6 / 47.4, 2048 x 4096 22.3 / 18.3, 1024 x
+// 7168 21.9 / 16.8, 512 x 4096 7.7 / 7.0, 256 x 7168 7.3 / 6.15, one row of 7168 4.5 / 4.1; 8192 x 4096 without codes 87.4 / 85.5.
+template <int NCHUNK, int QUANT, bool EXACT, bool GATED>
+__global__ void __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(GATED ? 8 : 4)))
+add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_per_row, int remap_end,
+                           uint32_t lanes_and_shift, uint32_t gate, const f32x4 *__restrict__ gamma, f32x4 *residual_out,
+                           void *norm_out, float *__restrict__ scale_io, float hidden_f, float rcp_hidden, int hidden_pow2,
+                           float eps, float fp8_max, float rcp_fp8_max) {
+    const int nthreads = (int)(lanes_and_shift & 0xffffu), group_shift = (int)(lanes_and_shift >> 16);
+    __shared__ float s_sum[kReduceSlots];
+    __shared__ float s_max[kReduceSlots];
+    const uint64_t entry = GATED ? __builtin_amdgcn_s_memrealtime() : 0;
+    const int tid = threadIdx.x;
+    const int num_waves = nthreads >> 6;
+    int row = blockIdx.x;
+    if (row < remap_end) {
+        const int xcd = row & 7, idx = row >> 3;
+        row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
+    }
+    const int64_t row_base = (int64_t)row * chunks_per_row;
+
+    // every load of the row ahead of the first use of any (and of the first store: residual_out may be an input)
+    f32x4 xv[NCHUNK], rv[NCHUNK], gv[NCHUNK];
+    bool live[NCHUNK];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NCHUNK; ++i) {
+        const int c = i * nthreads + tid;
+        live[i] = EXACT || c < chunks_per_row;
+        xv[i] = live[i] ? load_stream(x + row_base + c) : zero;
+        rv[i] = live[i] ? load_stream(residual_in + row_base + c) : zero;
+    }
+#pragma unroll
+    for (int i = 0; i < NCHUNK; ++i) gv[i] = live[i] ? gamma[i * nthreads + tid] : zero;
+    asm volatile("" ::"s"(hidden_f), "s"(rcp_hidden), "s"(hidden_pow2), "s"(eps), "s"(fp8_max), "s"(rcp_fp8_max));
+    float static_scale = 0.f;
+    if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) static_scale = *(const __attribute__((address_space(4))) float *)scale_io;
+
+    __builtin_amdgcn_s_setprio(1);
+    float ss0 = 0.f, ss1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NCHUNK; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float v = xv[i][j] + rv[i][j];
+            xv[i][j] = v;  // xv now holds the residual
+            if (j & 1) ss1 = __builtin_fmaf(v, v, ss1);
+            else ss0 = __builtin_fmaf(v, v, ss0);
+        }
+        if (!GATED && live[i]) store_stream(residual_out + row_base + i * nthreads + tid, xv[i]);
+    }
+    float sumsq[1] = {ss0 + ss1};
+    if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) asm volatile("" ::"s"(static_scale));
+    block_allreduce<SumOp, 1>(sumsq, s_sum, num_waves);
+    __builtin_amdgcn_s_setprio(0);
+    float mean;
+    if (hidden_pow2) mean = sumsq[0] * rcp_hidden;
+    else if (__builtin_expect(__builtin_amdgcn_ballot_w64(!in_mid_range(sumsq[0])) == 0, 1)) mean = div_by_rcp_finite(sumsq[0], hidden_f, rcp_hidden);
+    else mean = sumsq[0] / hidden_f;
+    const float rstd = rsqrt_two_roundings(mean + eps);
+
+    f32x4 nv[NCHUNK];
+    float m0 = 0.f, m1 = 0.f;
+    bool any_nan = false;
+#pragma unroll
+    for (int i = 0; i < NCHUNK; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) nv[i][j] = gv[i][j] * (xv[i][j] * rstd);
+        if constexpr (QUANT != GPUK_QUANT_NONE) {  // (max3_abs drops NaNs, the reference's amax keeps them: tracked apart)
+            m0 = max3_abs(m0, nv[i][0], nv[i][1]);
+            m1 = max3_abs(m1, nv[i][2], nv[i][3]);
+            if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC)
+                any_nan |= __builtin_isunordered(nv[i][0], nv[i][1]) || __builtin_isunordered(nv[i][2], nv[i][3]);
+        }
+    }
+    const float lane_max = __builtin_fmaxf(m0, m1);
+    uint32_t codes[NCHUNK];
+    if constexpr (QUANT != GPUK_QUANT_NONE) {
+        float scale = static_scale;
+        bool fast = scale_in_fast_range(scale) && lane_max <= 0x1p60f;  // (a static scale may meet quotients that overflow)
+        if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
+            float amax[1] = {any_nan ? __builtin_nanf("") : lane_max};
+            block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax[0]) && rcp_fp8_max != 0.f)) == 0, 1))
+                scale = div_by_rcp_finite(amax[0], fp8_max, rcp_fp8_max);
+            else
+                scale = amax[0] == 0.f ? 1.f : amax[0] / fp8_max;
+            if (tid == 0) scale_io[row] = scale;
+            fast = scale_in_fast_range(scale);
+        }
+        // Quotients below the smallest code's half come out 0 with their sign whatever the correction step loses to
+        // underflow; the others are the correctly rounded ones.  With the dynamic scale none exceeds
+        // fp8_max * (1 + 2^-23), which the converter rounds to fp8_max.
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!fast) == 0, 1)) {
+            float rcp;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(mantissa_all_ones(scale)) == 0, 1)) rcp = rcp_rn_mid_range(scale);
+            else rcp = 1.0f / scale;
+#pragma unroll
+            for (int i = 0; i < NCHUNK; ++i) {
+                float q[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) q[j] = div_by_rcp_finite(nv[i][j], scale, rcp);
+                    else q[j] = clamp_sym(div_by_rcp(nv[i][j], scale, rcp), fp8_max);
+                }
+                codes[i] = cvt4_e4m3fn(q[0], q[1], q[2], q[3]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NCHUNK; ++i) {
+                float q[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) q[j] = clamp_sym(nv[i][j] / scale, fp8_max);
+                codes[i] = cvt4_e4m3fn(q[0], q[1], q[2], q[3]);
+            }
+        }
+    }
+    if constexpr (GATED) {  // (what is stored is pinned down ahead of the wait, as in add_rmsnorm_quant_rows)
+#pragma unroll
+        for (int i = 0; i < NCHUNK; ++i) {
+            if constexpr (QUANT == GPUK_QUANT_NONE) asm volatile("" ::"v"(nv[i]));
+            else asm volatile("" ::"v"(codes[i]));
+        }
+        while (__builtin_amdgcn_s_memrealtime() < entry + gate) __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+        for (int i = 0; i < NCHUNK; ++i)
+            if (live[i]) store_stream(residual_out + row_base + i * nthreads + tid, xv[i]);
+    }
+    if constexpr (QUANT == GPUK_QUANT_NONE) {
+        f32x4 *out = reinterpret_cast<f32x4 *>(norm_out) + row_base;
+#pragma unroll
+        for (int i = 0; i < NCHUNK; ++i)
+            if (live[i]) store_stream(out + i * nthreads + tid, nv[i]);
+    } else if constexpr (NCHUNK == 1) {
+        if (live[0]) store_stream(reinterpret_cast<uint32_t *>(norm_out) + row_base + tid, codes[0]);
+    } else {
+        // 8 codes per lane and store: of two chunks, even lanes store the first one's codes of themselves and their odd
+        // neighbour, odd lanes the second one's (a row is an even number of chunks: neighbours are live together)
+        uint32_t *out = reinterpret_cast<uint32_t *>(norm_out) + row_base;
+        const bool odd = tid & 1;
+#pragma unroll
+        for (int i = 0; i < NCHUNK; i += 2) {
+            const uint32_t give = odd ? codes[i] : codes[i + 1], keep = odd ? codes[i + 1] : codes[i];
+            const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, DPP_QUAD_XOR1, 0xf, 0xf, true);
+            if (odd ? live[i + 1] : live[i])
+                store_stream(reinterpret_cast<u32x2 *>(out + (odd ? i + 1 : i) * nthreads + (tid & ~1)), odd ? u32x2{got, keep} : u32x2{keep, got});
+        }
+    }
+}
+
+// fp64 activations and longer fp32 rows: the reference dispatches both types through the same template
 // (AT_DISPATCH_FLOATING_TYPES_AND2, src/ops/all_reduce_fusion.cpp:375-378).  4 elements per chunk; a lane keeps its
-// CPL chunks of the summed row in registers (rows of up to 4 x 1024 chunks), or, with CPL = 0, sweeps a longer row
+// CPL chunks of the summed row in registers (fp64 rows of up to 4 x 1024 chunks), or, with CPL = 0, sweeps a longer row
 // three times, reading back what it stored to residual_out.  Rounding to the activation type is the identity here, so
 // the oracle's sequence is plain arithmetic in that type around an fp32 variance:
 //   res = x + r;  rstd = 1/sqrt(mean(float(res)^2) + eps) in fp32;  n = gamma * (res * F(rstd));
@@ -502,8 +661,7 @@ add_rmsnorm_quant_wide_rows(const wide4<F> *x, const wide4<F> *residual_in,  // 
     const int num_waves = blockDim.x >> 6;
     const int64_t row_base = (int64_t)blockIdx.x * chunks_per_row;
     constexpr int KEPT = CPL ? CPL : 1;
-    // streaming accesses where the row stays in registers: measured 6-12 % faster for fp32 and 12 % slower for fp64
-    constexpr bool STREAM = CPL > 0 && sizeof(F) == 4;
+    // (no streaming accesses: measured 12 % slower for fp64)
     wide4<F> kept[KEPT];  // CPL > 0: chunk tid + i * blockDim.x of the summed row (and later of the normed row)
 
     // f(i, c) for every chunk c of the row this lane owns; i is its place in kept[]
@@ -521,14 +679,8 @@ add_rmsnorm_quant_wide_rows(const wide4<F> *x, const wide4<F> *residual_in,  // 
 
     float ss = 0.f;
     for_chunks([&](int i, int c) {
-        wide4<F> res;
-        if constexpr (STREAM) {
-            res = __builtin_nontemporal_load(x + row_base + c) + __builtin_nontemporal_load(residual_in + row_base + c);
-            __builtin_nontemporal_store(res, residual_out + row_base + c);
-        } else {
-            res = x[row_base + c] + residual_in[row_base + c];
-            residual_out[row_base + c] = res;  // CPL = 0: read back below
-        }
+        const wide4<F> res = x[row_base + c] + residual_in[row_base + c];
+        residual_out[row_base + c] = res;  // CPL = 0: read back below
         kept[i] = res;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -548,10 +700,7 @@ add_rmsnorm_quant_wide_rows(const wide4<F> *x, const wide4<F> *residual_in,  // 
 
     if constexpr (QUANT == GPUK_QUANT_NONE) {
         wide4<F> *out = reinterpret_cast<wide4<F> *>(norm_out) + row_base;
-        for_chunks([&](int i, int c) {
-            if constexpr (STREAM) __builtin_nontemporal_store(normed(i, c), out + c);
-            else out[c] = normed(i, c);
-        });
+        for_chunks([&](int i, int c) { out[c] = normed(i, c); });
     } else {
         float scale;
         if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
@@ -577,10 +726,8 @@ add_rmsnorm_quant_wide_rows(const wide4<F> *x, const wide4<F> *residual_in,  // 
             else n = normed(i, c);
             const wide4<F> q = n / wide_scale;
             // clamping after the cast to fp32 equals the oracle's clamp before it: the bounds are fp32 numbers
-            const uint32_t codes = cvt4_e4m3fn(clamp_sym((float)q[0], fp8_max), clamp_sym((float)q[1], fp8_max),
-                                               clamp_sym((float)q[2], fp8_max), clamp_sym((float)q[3], fp8_max));
-            if constexpr (STREAM) __builtin_nontemporal_store(codes, out + c);
-            else out[c] = codes;
+            out[c] = cvt4_e4m3fn(clamp_sym((float)q[0], fp8_max), clamp_sym((float)q[1], fp8_max),
+                                 clamp_sym((float)q[2], fp8_max), clamp_sym((float)q[3], fp8_max));
         });
     }
 }
@@ -612,12 +759,12 @@ int64_t resident_rows(int threads, int nchunk) {
 // 768, 9.0 against 11.7 at 1024 (gate 1.0-1.1 times the read time; 10.2 with 0.9, 9.6 with 1.2), nothing gained and
 // 0.1 us lost below a quarter of a round; at 4096 elements 6.2 against 7.7 us at 1024 rows, 10.2 against 12.4 at 2048; 20-45 % slower where the
 // batch does not fit one round.
-uint32_t store_gate(int64_t tokens, int64_t hidden, int threads, int nchunk) {
+uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk) {
     if (g_gate >= 0) return (uint32_t)g_gate;
     const int64_t resident = resident_rows(threads, nchunk);
     if (tokens > resident || 4 * tokens < resident) return 0;
     // (four chunks per lane: the shape pick_shape takes to hold in one round what two chunks per lane cannot)
-    const double ticks = (nchunk >= 4 ? 1.08 : 1.05) * (double)(4 * tokens * hidden) / 70000.0;  // 70,000 bytes per tick of 10 ns
+    const double ticks = (nchunk >= 4 ? 1.08 : 1.05) * (double)(2 * tokens * row_bytes) / 70000.0;  // 70,000 bytes per tick of 10 ns
     return (uint32_t)std::min(ticks, 5000.0);
 }
 
@@ -670,6 +817,13 @@ int launches_for(int64_t tokens, int chunks_per_row) {
     return 10 * tokens >= 11 * round ? 2 : 1;
 }
 
+// log2 of the run of consecutive rows an XCD takes.  Runs of 64 rows: +1.1 % for 16 KiB rows (8192 rows), of 16-bit
+// elements (75.5 -> 74.9 us) as of fp32 (68.8 -> 68.0, 16384 rows 138.0 -> 136.4, 1500 rows 14.1 -> 13.9); neutral or 1-10 %
+// slower for every other row size tried (2, 3, 4, 8, 10, 14, 20, 28, 32 KiB) and for fewer rows, hence the narrow rule.
+int row_group_shift(int64_t tokens, int64_t row_bytes) {
+    return g_row_group_shift >= 0 ? g_row_group_shift : row_bytes == 16384 && tokens >= 1024 ? 6 : 0;
+}
+
 // Rows of the first launch: the whole batch, or of two pieces the first, a whole number of rows per compute unit (half
 // of what the batch needs, rounded down), so that neither piece pays for a partly filled last row of workgroups twice.
 int64_t first_piece(int64_t tokens, int chunks_per_row) {
@@ -715,12 +869,8 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     const float rcp_hidden = 1.0f / hf;
     const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
     const float rcp_fp8_max = (fp8_max == 448.0f || fp8_max == 240.0f) ? 1.0f / fp8_max : 0.0f;
-    const uint32_t gate = store_gate(tokens, hidden, threads, nchunk);
-    // Runs of 64 rows per XCD: measured +1.1 % for 16 KiB rows (8192 rows); neutral or 1-10 % slower for every other
-    // row size tried (2, 3, 4, 8, 10, 14, 32 KiB) and for fewer rows, hence the narrow rule.
-    const int64_t row_bytes = hidden * 2;
-    int group_shift = row_bytes == 16384 && tokens >= 1024 ? 6 : 0;
-    if (g_row_group_shift >= 0) group_shift = g_row_group_shift;
+    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk);
+    const int group_shift = row_group_shift(tokens, hidden * 2);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
     const bool exact = (int64_t)threads * nchunk == chunks;
 #define GPUK_LAUNCH_NQ_AS(N, EXACT, GATED)                                                                              \
@@ -746,12 +896,10 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     return hip_status(hipGetLastError());
 }
 
-// Lanes and kept chunks per lane of the fp32 / fp64 kernel; 0 chunks kept = rows beyond 4096 chunks, swept.  fp32, as
-// for the 16-bit kernel: two chunks per lane unless that leaves more lanes idle in the last wave (12 % ahead of one
-// chunk at 32768 x 4096); fp64: one chunk (32 bytes) per lane up to 1024 lanes (6 % ahead of two).
-void pick_wide_shape(int chunks, bool fp64, int *threads, int *cpl) {
-    const int lanes1 = round_up(chunks, 64), lanes2 = round_up((chunks + 1) / 2, 64);
-    int n = (fp64 || 2 * lanes2 > lanes1) && lanes1 <= kMaxThreads ? 1 : 2;
+// Lanes and kept chunks per lane of the fp64 kernel; 0 chunks kept = rows beyond 4096 chunks, swept (fp32 rows come here
+// for that only).  One chunk (32 bytes) per lane up to 1024 lanes (6 % ahead of two).
+void pick_wide_shape(int chunks, int *threads, int *cpl) {
+    int n = 1;
     while (n < 4 && chunks > n * kMaxThreads) n *= 2;
     if (chunks > n * kMaxThreads) {
         *cpl = 0;
@@ -762,22 +910,76 @@ void pick_wide_shape(int chunks, bool fp64, int *threads, int *cpl) {
     *threads = round_up((chunks + n - 1) / n, 64);
 }
 
+template <int QUANT>
+int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, void *residual_out, void *norm_out,
+                    float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
+    const int chunks = (int)(hidden / 4);
+    int threads, nchunk;
+    pick_shape(tokens, chunks, &threads, &nchunk);
+    const uint32_t gate = store_gate(tokens, hidden * 4, threads, nchunk);
+    const int group_shift = row_group_shift(tokens, hidden * 4);
+    const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
+    const float hf = (float)hidden;
+    const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
+    const float rcp_fp8_max = (fp8_max == 448.0f || fp8_max == 240.0f) ? 1.0f / fp8_max : 0.0f;
+    const bool exact = (int64_t)threads * nchunk == chunks;
+#define GPUK_LAUNCH_F32_AS(N, EXACT, GATED)                                                                             \
+    add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, GATED><<<dim3((unsigned)tokens), threads, 0, stream>>>(                  \
+        static_cast<const f32x4 *>(x), static_cast<const f32x4 *>(residual_in), chunks, remap_end,                       \
+        (uint32_t)threads | ((uint32_t)group_shift << 16), gate, static_cast<const f32x4 *>(gamma),                      \
+        static_cast<f32x4 *>(residual_out), norm_out, scale, hf, 1.0f / hf, hidden_pow2, eps, fp8_max, rcp_fp8_max)
+#define GPUK_LAUNCH_F32(N)                                                                                             \
+    do {                                                                                                               \
+        if (exact && gate) GPUK_LAUNCH_F32_AS(N, true, true);                                                          \
+        else if (exact) GPUK_LAUNCH_F32_AS(N, true, false);                                                            \
+        else if (gate) GPUK_LAUNCH_F32_AS(N, false, true);                                                             \
+        else GPUK_LAUNCH_F32_AS(N, false, false);                                                                      \
+    } while (0)
+    switch (nchunk) {
+        case 1: GPUK_LAUNCH_F32(1); break;
+        case 2: GPUK_LAUNCH_F32(2); break;
+        case 4: GPUK_LAUNCH_F32(4); break;
+        default: return GPUK_ERR_INTERNAL;
+    }
+#undef GPUK_LAUNCH_F32
+#undef GPUK_LAUNCH_F32_AS
+    return hip_status(hipGetLastError());
+}
+
 template <typename F, int QUANT>
 int launch_wide(const void *x, const void *residual_in, const void *gamma, void *residual_out, void *norm_out,
                 float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 4);
+    if constexpr (sizeof(F) == 4) {
+        if (chunks <= kF32MaxChunks) {  // in pieces as for 16-bit rows, see launches_for
+            const int64_t piece = first_piece(tokens, chunks);
+            for (int64_t first = 0; first < tokens; first = first ? tokens : piece) {
+                const int64_t in_bytes = first * hidden * 4, out_bytes = first * hidden * (QUANT == GPUK_QUANT_NONE ? 4 : 1);
+                const int rc = launch_f32_rows<QUANT>(static_cast<const char *>(x) + in_bytes, static_cast<const char *>(residual_in) + in_bytes,
+                                                      gamma, static_cast<char *>(residual_out) + in_bytes, static_cast<char *>(norm_out) + out_bytes,
+                                                      QUANT == GPUK_QUANT_FP8_DYNAMIC ? scale + first : scale, first ? tokens - first : piece,
+                                                      hidden, eps, fp8_max, stream);
+                if (rc != GPUK_OK) return rc;
+            }
+            return GPUK_OK;
+        }
+    }
     int threads, cpl;
-    pick_wide_shape(chunks, sizeof(F) == 8, &threads, &cpl);
+    pick_wide_shape(chunks, &threads, &cpl);
 #define GPUK_LAUNCH_WIDE(CPL)                                                                                          \
     add_rmsnorm_quant_wide_rows<F, QUANT, CPL><<<dim3((unsigned)tokens), threads, 0, stream>>>(                        \
         static_cast<const wide4<F> *>(x), static_cast<const wide4<F> *>(residual_in),                                  \
         static_cast<const wide4<F> *>(gamma), static_cast<wide4<F> *>(residual_out), norm_out, scale, chunks,          \
         (float)hidden, eps, fp8_max)
-    switch (cpl) {
-        case 1: GPUK_LAUNCH_WIDE(1); break;
-        case 2: GPUK_LAUNCH_WIDE(2); break;
-        case 4: GPUK_LAUNCH_WIDE(4); break;
-        default: GPUK_LAUNCH_WIDE(0); break;
+    if constexpr (sizeof(F) == 4) {
+        GPUK_LAUNCH_WIDE(0);
+    } else {
+        switch (cpl) {
+            case 1: GPUK_LAUNCH_WIDE(1); break;
+            case 2: GPUK_LAUNCH_WIDE(2); break;
+            case 4: GPUK_LAUNCH_WIDE(4); break;
+            default: GPUK_LAUNCH_WIDE(0); break;
+        }
     }
 #undef GPUK_LAUNCH_WIDE
     return hip_status(hipGetLastError());
@@ -849,15 +1051,14 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
     int threads, nchunk;
     pick_shape(tokens, chunks, &threads, &nchunk);
     if (nchunk == 0) return GPUK_ERR_UNSUPPORTED;  // rows that do not stay in registers
-    int group_shift = hidden * 2 == 16384 && tokens >= 1024 ? 6 : 0;
-    if (g_row_group_shift >= 0) group_shift = g_row_group_shift;
+    const int group_shift = row_group_shift(tokens, hidden * 2);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
     auto xs = static_cast<const u32x4 *>(x), rs = static_cast<const u32x4 *>(residual_in);
     auto ro = static_cast<u32x4 *>(residual_out);
     auto co = static_cast<u32x2 *>(codes);
     const dim3 grid((unsigned)tokens);
-    const uint32_t gate = store_gate(tokens, hidden, threads, nchunk);
+    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk);
     const uint32_t shape = (uint32_t)threads | ((uint32_t)group_shift << 16);
     switch (nchunk) {
         case 1: add_rmsnorm_quant_traffic_only<1><<<grid, threads, 0, s>>>(xs, rs, chunks, remap_end, shape, gate, ro, co, scale); break;
@@ -875,8 +1076,12 @@ extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidde
     if (dtype != GPUK_DTYPE_BF16 && dtype != GPUK_DTYPE_FP16 && dtype != GPUK_DTYPE_F32 && dtype != GPUK_DTYPE_F64) return GPUK_ERR_UNSUPPORTED;
     const bool wide = dtype == GPUK_DTYPE_F32 || dtype == GPUK_DTYPE_F64;
     if (hidden % 8 != 0) return GPUK_ERR_UNSUPPORTED;  // the rule of gpuk_add_rmsnorm_quant, for every dtype
-    if (wide) {  // the fp32 / fp64 kernel: 4-element chunks, 0 = rows swept three times
-        pick_wide_shape((int)(hidden / 4), dtype == GPUK_DTYPE_F64, lanes_per_row, chunks_per_lane);
+    if (dtype == GPUK_DTYPE_F32 && hidden / 4 <= kF32MaxChunks) {
+        pick_shape(first_piece(tokens, (int)(hidden / 4)), (int)(hidden / 4), lanes_per_row, chunks_per_lane);
+        return GPUK_OK;
+    }
+    if (wide) {  // longer fp32 rows and fp64: 4-element chunks, 0 = rows swept three times
+        pick_wide_shape((int)(hidden / 4), lanes_per_row, chunks_per_lane);
         return GPUK_OK;
     }
     pick_shape(first_piece(tokens, (int)(hidden / 8)), (int)(hidden / 8), lanes_per_row, chunks_per_lane);

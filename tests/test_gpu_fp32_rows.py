@@ -1,0 +1,91 @@
+"""fp32 rows of the norm kernel, which share the 16-bit kernel's arrangement: every form of a row (one, two, four chunks per
+lane; lanes filled or not), the store gate, batches run as two launches, runs of rows per XCD, and values where its short
+quotients could go wrong.
+
+No tolerance on values: each row is bit-identical to the oracle at an rstd within 3 fp32 ULPs, the freedom that the order
+of its sum of squares leaves."""
+import pytest
+import torch
+
+from gpuk_amd import workloads
+from oracle import torch_oracle as O
+from tests.util import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def canonical(t):
+    """Bit patterns, every NaN alike."""
+    t = t.cpu().contiguous()
+    if t.element_size() == 1:
+        b = t.view(torch.uint8)
+        return torch.where((b & 0x7F) == 0x7F, torch.full_like(b, 0x7F), b)
+    return torch.where(t.isnan(), torch.full_like(t.view(torch.int32), 0x7FC00000), t.view(torch.int32))
+
+
+def run(inp, quant, device, static=None, alias=False):
+    from gpuk_amd import capi
+
+    x, r, g = inp.x.to(device), inp.residual.to(device), inp.gamma.to(device)
+    res = r if alias else torch.empty_like(x)
+    tokens, hidden = x.shape
+    norm = torch.full((tokens + 1, hidden), 3.0, device=device)   # one row more than the call may write
+    norm = norm if quant == 0 else norm.to(torch.float8_e4m3fn)
+    guard = canonical(norm[-1])
+    scale = None if quant == 0 else torch.full((tokens, 1), -1.0, device=device) if quant == 1 else static.to(device)
+    capi.add_rmsnorm_quant(x, r, g, res, norm, scale, inp.eps, quant)
+    torch.cuda.synchronize()
+    assert torch.equal(canonical(norm[-1]), guard), "written behind the last row"
+    return res, norm[:-1], scale
+
+
+def check(inp, quant, got, static=None):
+    res, norm, scale = got
+    bits = canonical(norm)
+    explained = torch.zeros(inp.x.shape[0], dtype=torch.bool)
+    for off in (0, -1, 1, -2, 2, -3, 3):
+        res_ref, norm_ref, scale_ref = O.add_rmsnorm_quant_ref(inp.x, inp.residual, inp.gamma, inp.eps, quant, static_scale=static, rstd_ulp_offset=off)
+        if off == 0:
+            assert torch.equal(canonical(res), canonical(res_ref)), "residual_out"
+        same = (bits == canonical(norm_ref)).all(dim=1)
+        if quant == 1:
+            s, w = scale.cpu().flatten(), scale_ref.flatten()
+            same &= (s == w) | (s.isnan() & w.isnan())
+        explained |= same
+        if bool(explained.all()):
+            return
+    raise AssertionError(f"rows {(~explained).nonzero().flatten().tolist()[:8]} match the oracle at no rstd within 3 ULP")
+
+
+# one chunk per lane; two, filled and not, one row and gated; four, filled and not, gated (one round); two launches of half
+# the rows; more than a round, in runs of 64 rows per XCD with rows left over
+@pytest.mark.parametrize("tokens,hidden", [(3, 264), (1, 4096), (300, 4096), (900, 1032), (1100, 4096), (1300, 2568), (5, 16384),
+                                           (2400, 4096), (4200, 4096)])
+@pytest.mark.parametrize("quant", [0, 1, 3])
+def test_row_forms(device, tokens, hidden, quant):
+    print(f"case fp32 rows {tokens}x{hidden} q{quant}", flush=True)
+    inp = workloads.norm_quant_inputs(tokens, hidden, seed=tokens + hidden, res_sigma=2.0, outlier_frac=0.01, dtype=torch.float32)
+    static = torch.tensor([0.013]) if quant == 3 else None
+    check(inp, quant, run(inp, quant, device, static, alias=tokens == 1100), static)
+
+
+@pytest.mark.parametrize("quant,static", [(0, None), (1, None), (3, 0.01), (3, 1e-17), (3, 1e-30)])
+@pytest.mark.parametrize("tokens,hidden", [(16, 264), (16, 7168), (700, 4104)])
+def test_extreme_values(device, tokens, hidden, quant, static):
+    """Zero rows, NaNs, infinities, sums of squares that overflow, subnormal elements next to ordinary ones, weights so large
+    that a quotient by the static scale overflows, and scales too small for a reciprocal."""
+    print(f"case fp32 extremes {tokens}x{hidden} q{quant} {static}", flush=True)
+    inp = workloads.norm_quant_inputs(tokens, hidden, seed=hidden, res_sigma=1.0, dtype=torch.float32)
+    x, r = inp.x, inp.residual
+    x[0], r[0] = 0.0, 0.0
+    x[1, 5] = float("nan")
+    x[2, 7] = float("inf")
+    x[3] = x[3] * 1e30
+    x[4], r[4] = x[4] * 2.0 ** -75, r[4] * 2.0 ** -76      # squares underflow: rstd from eps alone
+    x[5, ::2], r[5, ::2] = x[5, ::2] * 1e-38, r[5, ::2] * 1e-39
+    x[6], r[6] = x[6] * 2.0 ** (torch.arange(hidden) % 60 - 50).float(), 0.0
+    x[7], r[7] = -x[7].abs() * 1e-20, 0.0
+    inp.gamma[::9] = inp.gamma[::9] * 1e25 if static == 1e-17 else inp.gamma[::9] * 1e-12
+    inp.gamma[4] = -inp.gamma[4]
+    s = None if static is None else torch.tensor([static])
+    check(inp, quant, run(inp, quant, device, s), s)
