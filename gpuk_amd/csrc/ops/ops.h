@@ -41,6 +41,15 @@ inline void check_status(int status, const char *op) {
 
 void allreduce_rms(int64_t fptr, Tensor &allreduce_in, Tensor &residual_in, Tensor &rms_gamma, Tensor &residual_out,
                    Tensor &norm_out, Tensor &scale_out, double eps, int64_t quant_type);
+// The same with outputs of its own: (residual_out, norm_out, scale_out), or (residual_out, norm_out) with a static scale.
+std::tuple<Tensor, Tensor, Tensor> add_rms_fused(const Tensor &allreduce_in, const Tensor &residual_in, const Tensor &rms_gamma,
+                                                 double eps, int64_t quant_type);
+std::tuple<Tensor, Tensor> add_rms_fused_static(const Tensor &allreduce_in, const Tensor &residual_in, const Tensor &rms_gamma,
+                                                double eps, const Tensor &static_scale);
+std::tuple<Tensor, Tensor, Tensor> add_rms_fused_meta(const Tensor &allreduce_in, const Tensor &residual_in,
+                                                      const Tensor &rms_gamma, double eps, int64_t quant_type);
+std::tuple<Tensor, Tensor> add_rms_fused_static_meta(const Tensor &allreduce_in, const Tensor &residual_in,
+                                                     const Tensor &rms_gamma, double eps, const Tensor &static_scale);
 void set_fp8_max(double value);
 double get_fp8_max();
 

@@ -18,6 +18,12 @@ template <auto F> struct NoOpLike;
 template <typename... A, void (*F)(A...)> struct NoOpLike<F> {
     static void call(A...) {}
 };
+
+// vmap would run a functional operator slice by slice, each slice its own rows and scales; it is refused here as it is for
+// the in-place operators, which have no batching rule either.
+void no_batching_rule(const c10::OperatorHandle &op, c10::DispatchKeySet, torch::jit::Stack *) {
+    TORCH_CHECK(false, "Batching rule not implemented for ", op.schema().operator_name());
+}
 }  // namespace
 
 TORCH_LIBRARY(gpuk, m) {
@@ -31,6 +37,21 @@ TORCH_LIBRARY(gpuk, m) {
           "Tensor(a!) residual_out, Tensor(b!) norm_out, Tensor(c!) scale_out, float eps, SymInt quant_type) -> ()");
     m.impl("allreduce_rms.mut", c10::DispatchKey::CUDA, &allreduce_rms);
     m.impl("allreduce_rms.mut", c10::DispatchKey::Meta, &NoOpLike<&allreduce_rms>::call);
+
+    // additive: the functional form behind GPUKDistEnv.allreduce_add_rms_fused.  No gradients, as with the in-place form:
+    // autograd is passed by (without that, torch marks the outputs as differentiable where an input is, and warns).
+    m.def("add_rms_fused(Tensor allreduce_in, Tensor residual_in, Tensor rms_gamma, float eps, int quant_type) -> "
+          "(Tensor residual_out, Tensor norm_out, Tensor scale_out)");
+    m.impl("add_rms_fused", c10::DispatchKey::CUDA, &add_rms_fused);
+    m.impl("add_rms_fused", c10::DispatchKey::Meta, &add_rms_fused_meta);
+    m.impl("add_rms_fused", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+    m.impl("add_rms_fused", torch::dispatch(c10::DispatchKey::FuncTorchBatched, torch::CppFunction::makeFromBoxedFunction<&no_batching_rule>()));
+    m.def("add_rms_fused.static(Tensor allreduce_in, Tensor residual_in, Tensor rms_gamma, float eps, Tensor static_scale) -> "
+          "(Tensor residual_out, Tensor norm_out)");
+    m.impl("add_rms_fused.static", c10::DispatchKey::CUDA, &add_rms_fused_static);
+    m.impl("add_rms_fused.static", c10::DispatchKey::Meta, &add_rms_fused_static_meta);
+    m.impl("add_rms_fused.static", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+    m.impl("add_rms_fused.static", torch::dispatch(c10::DispatchKey::FuncTorchBatched, torch::CppFunction::makeFromBoxedFunction<&no_batching_rule>()));
 
     // reference: src/register.cpp:42-45
     m.def("fused_rope_rms(Tensor qkv, Tensor qw, Tensor kw, Tensor cos_sin, Tensor positions, SymInt num_tokens, "
