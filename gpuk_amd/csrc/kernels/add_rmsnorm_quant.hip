@@ -64,6 +64,21 @@ __device__ __forceinline__ float div_by_rcp_finite(float a, float b, float rcp) 
     return __builtin_fmaf(-e, rcp, q);
 }
 
+// What a launch passes beside the workgroup size (lanes_and_shift, one argument register): lanes in bits 0-15, the row-run
+// shift in bits 16-23, the mask of line_pad in bits 24-31.
+__device__ __forceinline__ int lanes_of(uint32_t lanes_and_shift) { return (int)(lanes_and_shift & 0xffffu); }
+__device__ __forceinline__ int shift_of(uint32_t lanes_and_shift) { return (int)((lanes_and_shift >> 16) & 0xffu); }
+// Chunks by which a row's first one lies behind a line boundary.  The lanes of a row whose length is no multiple of a line
+// start at the boundary, not at the row (the first `pad` of them idle), so that a wave's accesses cover whole lines but
+// for the row's two ends: started at the row itself, every one of them splits its first and last line with the next wave,
+// whose streamed access fetches or writes it again.  Multiples of 16 chunks, which are whole lines of codes as well, or of 8
+// where the workgroup has no more lanes to spare: see line_mask.
+// Lanes from the row's start / from the line: 16384 rows of 9000 elements 184.1 / 168.0 us, of 2568 55.1 / 50.3, of 7176 145.4 /
+// 141.9; 8192 fp32 rows of 9000 181.5 / 165.2, of 2568 56.0 / 49.5; batches of a few hundred rows level, one row of 1032 2.20 / 2.24.
+__device__ __forceinline__ int line_pad(const void *x, int64_t row_base, uint32_t lanes_and_shift) {
+    return (int)(((uint32_t)((uintptr_t)x >> 4) + (uint32_t)row_base) & (lanes_and_shift >> 24));
+}
+
 // Two neighbouring elements of the normed row, rT(gamma * rT(res * rstd)), packed.
 template <typename T>
 __device__ __forceinline__ uint32_t normed_pair(uint32_t gamma, uint32_t res, float rstd) {
@@ -97,7 +112,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
     // the wave in scalar registers at launch (-amdgpu-kernarg-preload-count), so the loads of the row are issued
     // without a round trip for the argument block; lanes_and_shift holds the workgroup size (bits 0-15), passed so
     // that it need not be fetched from the dispatch packet either, and the row-run shift (bits 16-31).
-    const int nthreads = (int)(lanes_and_shift & 0xffffu), group_shift = (int)(lanes_and_shift >> 16);
+    const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
     using P = Pack16<T>;
     __shared__ float s_sum[kReduceSlots];
     __shared__ float s_max[kReduceSlots];
@@ -118,7 +133,9 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         const int xcd = row & 7, idx = row >> 3;
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
-    const int64_t row_base = (int64_t)row * chunks_per_row;
+    int64_t row_base = (int64_t)row * chunks_per_row;
+    const int pad = EXACT ? 0 : line_pad(x, row_base, lanes_and_shift);
+    row_base -= pad;  // where lane 0 stands: a lane's chunk c is chunk c - pad of the row
 
     // ---- phase 0: issue every load of the row before touching any of them.  The row is loaded whole before any of
     // it is stored, so residual_out may be the same buffer as residual_in or x.
@@ -127,7 +144,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
 #pragma unroll
     for (int i = 0; i < NCHUNK; ++i) {
         const int c = i * nthreads + tid;
-        live[i] = EXACT || c < chunks_per_row;
+        live[i] = EXACT || (uint32_t)(c - pad) < (uint32_t)chunks_per_row;
         if (live[i]) {
             xv[i] = load_stream(x + row_base + c);
             rv[i] = load_stream(residual_in + row_base + c);
@@ -139,7 +156,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
 #pragma unroll
     for (int i = 0; i < NCHUNK; ++i) {
         const int c = i * nthreads + tid;
-        gv[i] = live[i] ? gamma[c] : u32x4{0, 0, 0, 0};
+        gv[i] = live[i] ? (gamma - pad)[c] : u32x4{0, 0, 0, 0};
     }
     // The arguments beyond the preloaded ones are fetched here, behind the row's loads and while those are in flight:
     // left to itself the compiler fetches them where they are first used, after the first barrier, and every wave of
@@ -364,7 +381,7 @@ __global__ void __launch_bounds__(kMaxThreads)
 add_rmsnorm_quant_traffic_only(const u32x4 *x, const u32x4 *residual_in, int chunks_per_row, int remap_end,
                                uint32_t lanes_and_shift, uint32_t gate, u32x4 *residual_out, u32x2 *codes,
                                float *__restrict__ scale_out) {
-    const int nthreads = (int)(lanes_and_shift & 0xffffu), group_shift = (int)(lanes_and_shift >> 16);
+    const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
     const uint64_t entry = __builtin_amdgcn_s_memrealtime();  // the kernel's store gate, see there
     const int tid = threadIdx.x;  // arguments in the order of add_rmsnorm_quant_rows: the same ones arrive in registers
     int row = blockIdx.x;
@@ -372,13 +389,15 @@ add_rmsnorm_quant_traffic_only(const u32x4 *x, const u32x4 *residual_in, int chu
         const int xcd = row & 7, idx = row >> 3;
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
-    const int64_t row_base = (int64_t)row * chunks_per_row;
+    int64_t row_base = (int64_t)row * chunks_per_row;
+    const int pad = line_pad(x, row_base, lanes_and_shift);
+    row_base -= pad;
     u32x4 xv[NCHUNK], rv[NCHUNK];
     bool live[NCHUNK];
 #pragma unroll
     for (int i = 0; i < NCHUNK; ++i) {
         const int c = i * nthreads + tid;
-        live[i] = c < chunks_per_row;
+        live[i] = (uint32_t)(c - pad) < (uint32_t)chunks_per_row;
         xv[i] = live[i] ? load_stream(x + row_base + c) : u32x4{0, 0, 0, 0};
         rv[i] = live[i] ? load_stream(residual_in + row_base + c) : u32x4{0, 0, 0, 0};
     }
@@ -497,7 +516,7 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
                            uint32_t lanes_and_shift, uint32_t gate, const f32x4 *__restrict__ gamma, f32x4 *residual_out,
                            void *norm_out, float *__restrict__ scale_io, float hidden_f, float rcp_hidden, int hidden_pow2,
                            float eps, float fp8_max, float rcp_fp8_max) {
-    const int nthreads = (int)(lanes_and_shift & 0xffffu), group_shift = (int)(lanes_and_shift >> 16);
+    const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
     __shared__ float s_sum[kReduceSlots];
     __shared__ float s_max[kReduceSlots];
     const uint64_t entry = GATED ? __builtin_amdgcn_s_memrealtime() : 0;
@@ -508,7 +527,9 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
         const int xcd = row & 7, idx = row >> 3;
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
-    const int64_t row_base = (int64_t)row * chunks_per_row;
+    int64_t row_base = (int64_t)row * chunks_per_row;
+    const int pad = EXACT ? 0 : line_pad(x, row_base, lanes_and_shift);  // (even: lanes stay paired)
+    row_base -= pad;
 
     // every load of the row ahead of the first use of any (and of the first store: residual_out may be an input)
     f32x4 xv[NCHUNK], rv[NCHUNK], gv[NCHUNK];
@@ -517,12 +538,12 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
 #pragma unroll
     for (int i = 0; i < NCHUNK; ++i) {
         const int c = i * nthreads + tid;
-        live[i] = EXACT || c < chunks_per_row;
+        live[i] = EXACT || (uint32_t)(c - pad) < (uint32_t)chunks_per_row;
         xv[i] = live[i] ? load_stream(x + row_base + c) : zero;
         rv[i] = live[i] ? load_stream(residual_in + row_base + c) : zero;
     }
 #pragma unroll
-    for (int i = 0; i < NCHUNK; ++i) gv[i] = live[i] ? gamma[i * nthreads + tid] : zero;
+    for (int i = 0; i < NCHUNK; ++i) gv[i] = live[i] ? (gamma - pad)[i * nthreads + tid] : zero;
     asm volatile("" ::"s"(hidden_f), "s"(rcp_hidden), "s"(hidden_pow2), "s"(eps), "s"(fp8_max), "s"(rcp_fp8_max));
     float static_scale = 0.f;
     if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) static_scale = *(const __attribute__((address_space(4))) float *)scale_io;
@@ -824,6 +845,12 @@ int row_group_shift(int64_t tokens, int64_t row_bytes) {
     return g_row_group_shift >= 0 ? g_row_group_shift : row_bytes == 16384 && tokens >= 1024 ? 6 : 0;
 }
 
+// The mask of line_pad: 15 where the lanes beyond the row's last chunk allow for it, else 7, else none.
+uint32_t line_mask(int threads, int nchunk, int chunks) {
+    const int idle = threads * nchunk - chunks;
+    return idle >= 15 ? 15u : idle >= 7 ? 7u : 0u;
+}
+
 // Rows of the first launch: the whole batch, or of two pieces the first, a whole number of rows per compute unit (half
 // of what the batch needs, rounded down), so that neither piece pays for a partly filled last row of workgroups twice.
 int64_t first_piece(int64_t tokens, int chunks_per_row) {
@@ -875,7 +902,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     const bool exact = (int64_t)threads * nchunk == chunks;
 #define GPUK_LAUNCH_NQ_AS(N, EXACT, GATED)                                                                              \
     add_rmsnorm_quant_rows<T, N, QUANT, EXACT, GATED><<<grid, threads, 0, stream>>>(                                    \
-        xs, rs, chunks, remap_end, (uint32_t)threads | ((uint32_t)group_shift << 16), gate, gs, ro, norm_out, scale, hf, \
+        xs, rs, chunks, remap_end, (uint32_t)threads | ((uint32_t)group_shift << 16) | (line_mask(threads, nchunk, chunks) << 24), gate, gs, ro, norm_out, scale, hf, \
         rcp_hidden, hidden_pow2, eps, fp8_max, rcp_fp8_max)
 #define GPUK_LAUNCH_NQ(N)                                                                                              \
     do {                                                                                                               \
@@ -926,7 +953,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
 #define GPUK_LAUNCH_F32_AS(N, EXACT, GATED)                                                                             \
     add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, GATED><<<dim3((unsigned)tokens), threads, 0, stream>>>(                  \
         static_cast<const f32x4 *>(x), static_cast<const f32x4 *>(residual_in), chunks, remap_end,                       \
-        (uint32_t)threads | ((uint32_t)group_shift << 16), gate, static_cast<const f32x4 *>(gamma),                      \
+        (uint32_t)threads | ((uint32_t)group_shift << 16) | ((line_mask(threads, nchunk, chunks) & ~1u) << 24), gate, static_cast<const f32x4 *>(gamma),                      \
         static_cast<f32x4 *>(residual_out), norm_out, scale, hf, 1.0f / hf, hidden_pow2, eps, fp8_max, rcp_fp8_max)
 #define GPUK_LAUNCH_F32(N)                                                                                             \
     do {                                                                                                               \
@@ -1059,7 +1086,7 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
     auto co = static_cast<u32x2 *>(codes);
     const dim3 grid((unsigned)tokens);
     const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk);
-    const uint32_t shape = (uint32_t)threads | ((uint32_t)group_shift << 16);
+    const uint32_t shape = (uint32_t)threads | ((uint32_t)group_shift << 16) | (line_mask(threads, nchunk, chunks) << 24);
     switch (nchunk) {
         case 1: add_rmsnorm_quant_traffic_only<1><<<grid, threads, 0, s>>>(xs, rs, chunks, remap_end, shape, gate, ro, co, scale); break;
         case 2: add_rmsnorm_quant_traffic_only<2><<<grid, threads, 0, s>>>(xs, rs, chunks, remap_end, shape, gate, ro, co, scale); break;
