@@ -789,11 +789,13 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk) 
     return (uint32_t)std::min(ticks, 5000.0);
 }
 
-// Lanes per row and chunks per lane.  Measured on MI355X over rows of 1024 .. 16384 elements: two chunks per lane
-// on as many lanes as that needs (up to 1024) streams best or ties everywhere (1-6 % over one or four chunks per
-// lane), unless rounding up to whole waves would idle more lanes that way; longer rows double the chunks per lane.
-// Decode-sized batches are served best by the same shape (7168 elements, per call replayed from a graph: 3.3 us
-// against 3.5 us with one chunk per lane at one row, 5.0 against 5.6 us at 256 rows).
+// Lanes per row and chunks per lane.  Two chunks per lane on as many lanes as that needs (up to 1024) stream best or tie
+// for 1024 .. 16384 16-bit elements (1-6 % over one or four chunks per lane; 7168 elements, per call: 3.3 us against 3.5
+// with one chunk at one row, 5.0 against 5.6 at 256 rows); longer rows double the chunks per lane.  Where rounding up to
+// whole waves idles more lanes that way (an odd number of 64 chunks, or a little more than an even one), one chunk per lane
+// serves what the chip holds in one round (1032 elements: 2.2 against 2.45 us at one row, 5.65 against 6.2 at 2048), but
+// larger batches want the loads of two in flight: 12000 rows of 2560 / 3584 / 5632 / 7680 elements 37.0 / 49.6 / 76.6 /
+// 102.8 us against 39.4 / 53.5 / 86.0 / 111.7, of 3208 45.7 against 47.1; fp32 rows of 2568 66.3 against 70.9.
 void pick_shape(int64_t tokens, int chunks_per_row, int *threads, int *nchunk) {
     auto fits = [&](int n) { return (int64_t)n * kMaxThreads >= chunks_per_row; };
     int n;
@@ -810,9 +812,10 @@ void pick_shape(int64_t tokens, int chunks_per_row, int *threads, int *nchunk) {
         // 1280, 13.0 against 16.2 at 1536, 14.3 against 17.5 at 1700; 8192 elements: 12.4 against 15.5 us at 1280 rows,
         // 16.3 against 18.7 at 1700.  (That form keeps the normed row as 16-bit pairs between its last two phases:
         // with it in fp32 the kernel took 70 registers, seven waves per SIMD, 1792 rows.)
-        if (n == 2 && !g_force_threads) {
-            const int t2 = round_up((chunks_per_row + 1) / 2, 64), t4 = round_up((chunks_per_row + 3) / 4, 64);
-            if (tokens > resident_rows(t2, 2) && tokens <= resident_rows(t4, 4)) n = 4;
+        // Not where four would idle a third of the lanes (3000 rows of 2312 elements: 12.4 us against 11.7 with two).
+        if (n <= 2 && !g_force_threads && tokens > resident_rows(n == 1 ? lanes1 : lanes2, n)) {
+            const int t4 = round_up((chunks_per_row + 3) / 4, 64);
+            n = tokens > resident_rows(lanes2, 2) && tokens <= resident_rows(t4, 4) && 8 * t4 <= 3 * chunks_per_row ? 4 : 2;
         }
     }
     while (n < 8 && !fits(n)) n *= 2;
@@ -827,15 +830,25 @@ void pick_shape(int64_t tokens, int chunks_per_row, int *threads, int *nchunk) {
     *threads = t;
 }
 
+// Rows of the first of two launches: a whole number of rows per compute unit (half of what the batch needs, rounded down),
+// so that neither piece pays for a partly filled last row of workgroups twice.
+int64_t half_of(int64_t tokens) { return (tokens + kComputeUnits - 1) / kComputeUnits / 2 * kComputeUnits; }
+
 // Launches per call.  A batch of more than one round of workgroups and at most two runs as two launches of half the
 // rows, each a round of its own with the store gate: a read phase and a write phase twice over instead of two rounds
-// that mix the directions.
+// that mix the directions.  Only where the pieces' shape idles no more than an eighth of its lanes and rows start on line
+// boundaries (us, one launch / two: 4600 rows of 4096 elements 23.6 / 22.7, 8000 rows 38.5 / 38.0, 2300 of 8192 24.4 / 23.2, 4600 of
+// 3072 19.2 / 17.8; but where the pieces take four chunks on a quarter more lanes than the row fills 5500 of 3072 22.3 / 24.3,
+// 3200 of 5120 22.1 / 23.3, and 6000 rows of 1288 elements in one launch and 12000 in two 12.6 and 24.8 against 22.0 in one;
+// 2500 of 9000, which end inside lines, 30.1 / 31.8).
 int launches_for(int64_t tokens, int chunks_per_row) {
     if (g_pieces == 1 || g_force_nchunk || g_force_threads || chunks_per_row > 2 * kMaxThreads) return 1;
     const int64_t round = resident_rows(round_up((chunks_per_row + 3) / 4, 64), 4);
     if (tokens <= round || tokens > 2 * round) return 1;
     if (g_pieces == 2) return 2;
-    return 10 * tokens >= 11 * round ? 2 : 1;
+    int threads, nchunk;
+    pick_shape(tokens - half_of(tokens), chunks_per_row, &threads, &nchunk);
+    return 10 * tokens >= 11 * round && chunks_per_row % 8 == 0 && 7 * threads * nchunk <= 8 * chunks_per_row ? 2 : 1;
 }
 
 // log2 of the run of consecutive rows an XCD takes.  Runs of 64 rows: +1.1 % for 16 KiB rows (8192 rows), of 16-bit
@@ -851,11 +864,10 @@ uint32_t line_mask(int threads, int nchunk, int chunks) {
     return idle >= 15 ? 15u : idle >= 7 ? 7u : 0u;
 }
 
-// Rows of the first launch: the whole batch, or of two pieces the first, a whole number of rows per compute unit (half
-// of what the batch needs, rounded down), so that neither piece pays for a partly filled last row of workgroups twice.
+// Rows of the first launch.
 int64_t first_piece(int64_t tokens, int chunks_per_row) {
     if (launches_for(tokens, chunks_per_row) == 1) return tokens;
-    return (tokens + kComputeUnits - 1) / kComputeUnits / 2 * kComputeUnits;
+    return half_of(tokens);
 }
 
 template <typename T, int QUANT>
