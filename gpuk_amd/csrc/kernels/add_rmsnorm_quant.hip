@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "../../../include/gpuk_amd.h"
 #include "device_utils.h"
@@ -286,8 +287,8 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
             if constexpr (is_half<T>) amax[0] = MaxOp::apply(P::lo(half_max), P::hi(half_max));
             block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
             GPUK_STAMP(7);  // row maximum known to every wave
-            // rcp_fp8_max is RN(1 / fp8_max) for the two maxima the quotient was checked for (448, 240), else 0
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax[0]) && rcp_fp8_max != 0.f)) == 0, 1))
+            // rcp_fp8_max: see reciprocal_of_max
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax[0]) && rcp_fp8_max > 0.f)) == 0, 1))
                 scale = div_by_rcp_finite(amax[0], fp8_max, rcp_fp8_max);
             else
                 scale = amax[0] == 0.f ? 1.f : amax[0] / fp8_max;
@@ -297,9 +298,10 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         }
 
         // ---- phase 3: code = e4m3fn(clamp(n2 / scale)), 8 codes per chunk.  With the dynamic scale every value is
-        // finite and |n2 / scale| <= 448 * (1 + 2^-23), which the converter already rounds to 448: no clamp, and the
-        // short form of the quotient.  The static scale may meet anything: clamp, and the form that restores what a
-        // division gives for infinite and NaN numerators.
+        // finite, hence the short form of the quotient, and |n2 / scale| exceeds fp8_max by at most one ULP, which the
+        // converter rounds to the same code: no clamp.  (Maxima where it does not, see reciprocal_of_max, take the other
+        // path, which clamps.)  The static scale may meet anything: clamp, and the form that restores what a division
+        // gives for infinite and NaN numerators.
         constexpr bool kDynamic = QUANT == GPUK_QUANT_FP8_DYNAMIC;
         u32x2 *out = reinterpret_cast<u32x2 *>(norm_out) + row_base;
         if constexpr (kPacked && !is_half<T>) {  // (or the compiler keeps phase 2's unpacked copies alive instead)
@@ -310,7 +312,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         }
         // (the scale is the same in every lane; deciding by ballot tells the compiler so, and the common path is
         // laid out as straight-line code with the other one out of the way)
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!scale_in_fast_range(scale)) == 0, 1)) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(scale_in_fast_range(scale) && (!kDynamic || rcp_fp8_max >= 0.f))) == 0, 1)) {
             float rcp;
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(mantissa_all_ones(scale)) == 0, 1)) rcp = rcp_rn_mid_range(scale);
             else rcp = 1.0f / scale;
@@ -593,16 +595,16 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
         if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
             float amax[1] = {any_nan ? __builtin_nanf("") : lane_max};
             block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax[0]) && rcp_fp8_max != 0.f)) == 0, 1))
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax[0]) && rcp_fp8_max > 0.f)) == 0, 1))
                 scale = div_by_rcp_finite(amax[0], fp8_max, rcp_fp8_max);
             else
                 scale = amax[0] == 0.f ? 1.f : amax[0] / fp8_max;
             if (tid == 0) scale_io[row] = scale;
-            fast = scale_in_fast_range(scale);
+            fast = scale_in_fast_range(scale) && rcp_fp8_max >= 0.f;
         }
         // Quotients below the smallest code's half come out 0 with their sign whatever the correction step loses to
-        // underflow; the others are the correctly rounded ones.  With the dynamic scale none exceeds
-        // fp8_max * (1 + 2^-23), which the converter rounds to fp8_max.
+        // underflow; the others are the correctly rounded ones.  With the dynamic scale no clamp, as in
+        // add_rmsnorm_quant_rows.
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(!fast) == 0, 1)) {
             float rcp;
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(mantissa_all_ones(scale)) == 0, 1)) rcp = rcp_rn_mid_range(scale);
@@ -864,6 +866,20 @@ uint32_t line_mask(int threads, int nchunk, int chunks) {
     return idle >= 15 ? 15u : idle >= 7 ? 7u : 0u;
 }
 
+// What the kernels take for rcp_fp8_max: RN(1 / fp8_max) for the two maxima whose quotient was checked (448 and 240), 0 for
+// others, and -1 where fp8_max and the next float round to different codes (400: 384 and 416), so that quotients by the
+// dynamic scale, which may exceed fp8_max by that one ULP, have to be clamped.  Those calls take the kernels' dividing
+// path, which clamps (8192 x 8192 at 400: 78.4 us, 76.0 at 448; 1024 x 7168, ungated on that path: 12.5 against 8.9; one row 3.6
+// against 2.8): a clamp in the common path would add 55 to 440 instructions to every kernel for a handful of maxima.
+float reciprocal_of_max(float fp8_max) {
+    auto code = [](float v) {  // rounded to three bits of fraction, or to the spacing of the subnormal codes
+        const float step = std::ldexp(1.0f, std::max(std::ilogb(v) - 3, -9));
+        return std::nearbyint(v / step) * step;
+    };
+    if (fp8_max == 448.0f || fp8_max == 240.0f) return 1.0f / fp8_max;
+    return code(fp8_max) == code(std::nextafter(fp8_max, INFINITY)) ? 0.0f : -1.0f;
+}
+
 // Rows of the first launch.
 int64_t first_piece(int64_t tokens, int chunks_per_row) {
     if (launches_for(tokens, chunks_per_row) == 1) return tokens;
@@ -907,7 +923,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     }
     const float rcp_hidden = 1.0f / hf;
     const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
-    const float rcp_fp8_max = (fp8_max == 448.0f || fp8_max == 240.0f) ? 1.0f / fp8_max : 0.0f;
+    const float rcp_fp8_max = reciprocal_of_max(fp8_max);
     const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk);
     const int group_shift = row_group_shift(tokens, hidden * 2);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
@@ -960,7 +976,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
     const float hf = (float)hidden;
     const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
-    const float rcp_fp8_max = (fp8_max == 448.0f || fp8_max == 240.0f) ? 1.0f / fp8_max : 0.0f;
+    const float rcp_fp8_max = reciprocal_of_max(fp8_max);
     const bool exact = (int64_t)threads * nchunk == chunks;
 #define GPUK_LAUNCH_F32_AS(N, EXACT, GATED)                                                                             \
     add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, GATED><<<dim3((unsigned)tokens), threads, 0, stream>>>(                  \

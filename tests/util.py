@@ -76,6 +76,40 @@ def assert_codes_close(got, want, what: str, min_exact: float = MIN_EXACT_FRACTI
     assert exact >= min_exact, f"{what}: only {exact:.6f} of fp8 codes bit-exact (< {min_exact})"
 
 
+def canonical(t: torch.Tensor) -> torch.Tensor:
+    """Bit patterns of fp8 codes, 16-bit or 32-bit floats, every NaN alike."""
+    t = t.cpu().contiguous()
+    if t.element_size() == 1:
+        b = t.view(torch.uint8)
+        return torch.where((b & 0x7F) == 0x7F, torch.full_like(b, 0x7F), b)
+    b = t.view(torch.int16 if t.element_size() == 2 else torch.int32)
+    return torch.where(t.isnan(), torch.full_like(b, 0x7E00), b)
+
+
+def assert_norm_rows_explained(inp, quant: int, got, static=None, fp8_max: float = 448.0):
+    """(residual_out, norm_out, scale) of a norm-quant call with no tolerance on values: the residual bit for bit, each
+    row of norm_out (and its dynamic scale) bit-identical to the oracle at an rstd within 3 fp32 ULPs, the freedom that
+    the order of its sum of squares leaves."""
+    from oracle import torch_oracle as O
+
+    res, norm, scale = got
+    bits = canonical(norm)
+    explained = torch.zeros(inp.x.shape[0], dtype=torch.bool)
+    for off in (0, -1, 1, -2, 2, -3, 3):
+        res_ref, norm_ref, scale_ref = O.add_rmsnorm_quant_ref(inp.x, inp.residual, inp.gamma, inp.eps, quant, fp8_max=fp8_max,
+                                                               static_scale=static, rstd_ulp_offset=off)
+        if off == 0:
+            assert torch.equal(canonical(res), canonical(res_ref)), "residual_out"
+        same = (bits == canonical(norm_ref)).all(dim=1)
+        if quant == 1:
+            s, w = scale.cpu().flatten(), scale_ref.flatten()
+            same &= (s == w) | (s.isnan() & w.isnan())
+        explained |= same
+        if bool(explained.all()):
+            return
+    raise AssertionError(f"rows {(~explained).nonzero().flatten().tolist()[:8]} of {len(explained)} match the oracle at no rstd within 3 ULP")
+
+
 def assert_scales_close(got, want, what: str, rtol: float = SCALE_RTOL):
     got, want = got.detach().cpu().double().flatten(), want.detach().cpu().double().flatten()
     rel = ((got - want).abs() / want.abs().clamp_min(1e-30)).max().item() if got.numel() else 0.0
