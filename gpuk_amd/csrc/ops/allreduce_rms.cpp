@@ -77,6 +77,12 @@ void check_inputs(const Tensor &allreduce_in, const Tensor &residual_in) {
     TORCH_CHECK(allreduce_in.is_cuda() && residual_in.is_cuda(), "allreduce_rms: tensors must live on the GPU");
     TORCH_CHECK(allreduce_in.is_contiguous() && residual_in.is_contiguous());
 }
+// The scale is an output of this overload: the static mode would quantise by memory nobody wrote.
+void check_functional_quant_type(int64_t quant_type) {
+    TORCH_CHECK(quant_type == GPUK_QUANT_NONE || quant_type == GPUK_QUANT_FP8_DYNAMIC,
+                "add_rms_fused: quant_type must be 0 (none) or 1 (fp8, dynamic scale), got ", quant_type,
+                "; a static scale is passed to add_rms_fused.static");
+}
 // The scale is read by the kernel as it is: a copy or cast made here would be a hidden transfer inside the call, which a
 // stream capture rejects.
 void check_static_scale(const Tensor &static_scale, const Tensor &allreduce_in) {
@@ -89,6 +95,7 @@ void check_static_scale(const Tensor &static_scale, const Tensor &allreduce_in) 
 // a decode step more than its kernel takes (9.5 us per call of one 7168-element row, 7.3 in this form; the kernel 3.3).
 std::tuple<Tensor, Tensor, Tensor> add_rms_fused(const Tensor &allreduce_in, const Tensor &residual_in, const Tensor &rms_gamma,
                                                  double eps, int64_t quant_type) {
+    check_functional_quant_type(quant_type);
     check_inputs(allreduce_in, residual_in);
     const bool fp8 = quant_type != GPUK_QUANT_NONE;
     Tensor x = allreduce_in, residual = residual_in, gamma = rms_gamma;
@@ -113,6 +120,7 @@ std::tuple<Tensor, Tensor> add_rms_fused_static(const Tensor &allreduce_in, cons
 
 std::tuple<Tensor, Tensor, Tensor> add_rms_fused_meta(const Tensor &allreduce_in, const Tensor &residual_in,
                                                       const Tensor &rms_gamma, double eps, int64_t quant_type) {
+    check_functional_quant_type(quant_type);
     const bool fp8 = quant_type != GPUK_QUANT_NONE;
     const auto f32 = allreduce_in.options().dtype(at::kFloat);
     return {at::empty_like(residual_in), at::empty_like(allreduce_in, fp8 ? allreduce_in.options().dtype(at::kFloat8_e4m3fn) : allreduce_in.options()),

@@ -19,6 +19,15 @@ def test_meta_shapes(quant, dtype):
     assert (res.dtype, norm.shape, norm.dtype) == (x.dtype, x.shape, torch.float8_e4m3fn)
 
 
+@pytest.mark.parametrize("quant", [2, 3, 7, -1])
+@pytest.mark.parametrize("where", ["meta", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_modes_without_a_scale_to_return(where, quant):
+    """The scale is an output here: a static scale has its own overload, and unknown modes are refused on meta tensors too."""
+    x = torch.zeros(2, 64, dtype=torch.bfloat16, device=where)
+    with pytest.raises(RuntimeError, match="add_rms_fused.static"):
+        torch.ops.gpuk.add_rms_fused(x, x, x[0], 1e-6, quant)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["none", "dynamic", "static"])
 def test_equals_the_in_place_operator(device, mode):
