@@ -32,6 +32,7 @@ namespace {
 
 constexpr int kMaxThreads = 1024;
 constexpr int kMaxWaves = kMaxThreads / 64;
+constexpr int kMaxChunks = 8, kMaxChunksF32 = 4;  // chunks per lane the kernels of 16-bit and of fp32 rows have forms for
 
 template <typename V>
 __device__ __forceinline__ V load_stream(const V *p) { return __builtin_nontemporal_load(p); }
@@ -502,7 +503,6 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
     }
 }
 
-constexpr int kF32MaxChunks = 4 * kMaxThreads;
 // fp32 rows that stay in registers (up to 4 x 1024 chunks of 4 elements): the arrangement of add_rmsnorm_quant_rows -- same
 // arguments, lane-to-chunk mapping, store gate and short exact quotients -- around plain fp32 arithmetic, where every
 // rounding to the activation type is the identity:
@@ -798,16 +798,17 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk) 
 // serves what the chip holds in one round (1032 elements: 2.2 against 2.45 us at one row, 5.65 against 6.2 at 2048), but
 // larger batches want the loads of two in flight: 12000 rows of 2560 / 3584 / 5632 / 7680 elements 37.0 / 49.6 / 76.6 /
 // 102.8 us against 39.4 / 53.5 / 86.0 / 111.7, of 3208 45.7 against 47.1; fp32 rows of 2568 66.3 against 70.9.
-void pick_shape(int64_t tokens, int chunks_per_row, int *threads, int *nchunk) {
+// most_chunks: the largest number of chunks per lane the type's kernel has (8; fp32 rows: 4, a forced 8 becomes that).
+void pick_shape(int64_t tokens, int chunks_per_row, int most_chunks, int *threads, int *nchunk) {
     auto fits = [&](int n) { return (int64_t)n * kMaxThreads >= chunks_per_row; };
     int n;
     if (g_force_nchunk) {
-        n = g_force_nchunk;
+        n = std::min(g_force_nchunk, most_chunks);
     } else {
         // one chunk per lane only where two would leave more lanes idle after rounding up to whole waves
         const int lanes1 = round_up(chunks_per_row, 64), lanes2 = round_up((chunks_per_row + 1) / 2, 64);
         n = (2 * lanes2 > lanes1 && lanes1 <= kMaxThreads) ? 1 : 2;
-        while (n < 8 && chunks_per_row > kMaxThreads * n) n *= 2;
+        while (n < most_chunks && chunks_per_row > kMaxThreads * n) n *= 2;
         // A batch that two chunks per lane cannot hold in one round but four can (half the lanes per row, so up to
         // 2048 rows of 7168 or 8192 elements instead of 1024) takes four: one round, with the store gate, against two
         // rounds of mixed reads and writes.  7168 elements: 10.8 against 12.8 us at 1100 rows, 10.9 against 14.3 at
@@ -820,7 +821,7 @@ void pick_shape(int64_t tokens, int chunks_per_row, int *threads, int *nchunk) {
             n = tokens > resident_rows(lanes2, 2) && tokens <= resident_rows(t4, 4) && 8 * t4 <= 3 * chunks_per_row ? 4 : 2;
         }
     }
-    while (n < 8 && !fits(n)) n *= 2;
+    while (n < most_chunks && !fits(n)) n *= 2;
     if (!fits(n)) {
         *nchunk = 0;
         *threads = kMaxThreads;
@@ -849,7 +850,7 @@ int launches_for(int64_t tokens, int chunks_per_row) {
     if (tokens <= round || tokens > 2 * round) return 1;
     if (g_pieces == 2) return 2;
     int threads, nchunk;
-    pick_shape(tokens - half_of(tokens), chunks_per_row, &threads, &nchunk);
+    pick_shape(tokens - half_of(tokens), chunks_per_row, kMaxChunks, &threads, &nchunk);
     return 10 * tokens >= 11 * round && chunks_per_row % 8 == 0 && 7 * threads * nchunk <= 8 * chunks_per_row ? 2 : 1;
 }
 
@@ -910,7 +911,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
                 float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 8);
     int threads, nchunk;
-    pick_shape(tokens, chunks, &threads, &nchunk);
+    pick_shape(tokens, chunks, kMaxChunks, &threads, &nchunk);
     const dim3 grid((unsigned)tokens);
     auto xs = static_cast<const u32x4 *>(x);
     auto rs = static_cast<const u32x4 *>(residual_in);
@@ -970,7 +971,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
                     float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 4);
     int threads, nchunk;
-    pick_shape(tokens, chunks, &threads, &nchunk);
+    pick_shape(tokens, chunks, kMaxChunksF32, &threads, &nchunk);
     const uint32_t gate = store_gate(tokens, hidden * 4, threads, nchunk);
     const int group_shift = row_group_shift(tokens, hidden * 4);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
@@ -1006,7 +1007,7 @@ int launch_wide(const void *x, const void *residual_in, const void *gamma, void 
                 float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 4);
     if constexpr (sizeof(F) == 4) {
-        if (chunks <= kF32MaxChunks) {  // in pieces as for 16-bit rows, see launches_for
+        if (chunks <= kMaxChunksF32 * kMaxThreads) {  // in pieces as for 16-bit rows, see launches_for
             const int64_t piece = first_piece(tokens, chunks);
             for (int64_t first = 0; first < tokens; first = first ? tokens : piece) {
                 const int64_t in_bytes = first * hidden * 4, out_bytes = first * hidden * (QUANT == GPUK_QUANT_NONE ? 4 : 1);
@@ -1104,7 +1105,7 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
                                                    scale + piece, tokens - piece, hidden, stream);
     }
     int threads, nchunk;
-    pick_shape(tokens, chunks, &threads, &nchunk);
+    pick_shape(tokens, chunks, kMaxChunks, &threads, &nchunk);
     if (nchunk == 0) return GPUK_ERR_UNSUPPORTED;  // rows that do not stay in registers
     const int group_shift = row_group_shift(tokens, hidden * 2);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
@@ -1131,15 +1132,15 @@ extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidde
     if (dtype != GPUK_DTYPE_BF16 && dtype != GPUK_DTYPE_FP16 && dtype != GPUK_DTYPE_F32 && dtype != GPUK_DTYPE_F64) return GPUK_ERR_UNSUPPORTED;
     const bool wide = dtype == GPUK_DTYPE_F32 || dtype == GPUK_DTYPE_F64;
     if (hidden % 8 != 0) return GPUK_ERR_UNSUPPORTED;  // the rule of gpuk_add_rmsnorm_quant, for every dtype
-    if (dtype == GPUK_DTYPE_F32 && hidden / 4 <= kF32MaxChunks) {
-        pick_shape(first_piece(tokens, (int)(hidden / 4)), (int)(hidden / 4), lanes_per_row, chunks_per_lane);
+    if (dtype == GPUK_DTYPE_F32 && hidden / 4 <= kMaxChunksF32 * kMaxThreads) {
+        pick_shape(first_piece(tokens, (int)(hidden / 4)), (int)(hidden / 4), kMaxChunksF32, lanes_per_row, chunks_per_lane);
         return GPUK_OK;
     }
     if (wide) {  // longer fp32 rows and fp64: 4-element chunks, 0 = rows swept three times
         pick_wide_shape((int)(hidden / 4), lanes_per_row, chunks_per_lane);
         return GPUK_OK;
     }
-    pick_shape(first_piece(tokens, (int)(hidden / 8)), (int)(hidden / 8), lanes_per_row, chunks_per_lane);
+    pick_shape(first_piece(tokens, (int)(hidden / 8)), (int)(hidden / 8), kMaxChunks, lanes_per_row, chunks_per_lane);
     return GPUK_OK;
 }
 

@@ -218,8 +218,8 @@ int gpuk_rope_rms_launch_shape(int64_t num_tokens, int64_t num_heads_q, int64_t 
 int gpuk_increment_floats(float *data, int64_t n, void *stream);
 
 /* Launch-shape knobs for sweeps and for the tests that show the results do not depend on them; value 0 restores
- * the built-in choice.  Keys: "norm_quant_nchunk" (1/2/4/8 16-byte chunks per lane), "norm_quant_threads" (lanes
- * per row), "norm_quant_row_group_shift" (log2 of the run of consecutive rows one XCD takes; -1, not 0, restores the
+ * the built-in choice.  Keys: "norm_quant_nchunk" (1/2/4/8 16-byte chunks per lane, 8 being 4 for
+ * fp32 rows; fp64 rows ignore it, as "norm_quant_threads"), "norm_quant_threads" (lanes per row), "norm_quant_row_group_shift" (log2 of the run of consecutive rows one XCD takes; -1, not 0, restores the
  * built-in rule), "norm_quant_gate" (how long, in ticks of 10 ns after a wave's entry, the stores of the norm-quant
  * kernel are held back so that the reads of a batch the chip holds at once go first: -1 the built-in rule, 0 never),
  * "norm_quant_launches" (1: a call is always one launch; 2: two, of half the rows each, wherever the batch is more

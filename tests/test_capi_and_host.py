@@ -296,6 +296,19 @@ def test_launch_shape_report():
     assert L.gpuk_add_rmsnorm_quant_launch_shape(4, 1024, 7, C.byref(a), C.byref(b)) == 2
 
 
+def test_launch_shape_of_forced_chunks():
+    """fp32 rows have forms of one, two and four chunks per lane: a forced eight is four there, eight for 16-bit rows."""
+    from gpuk_amd import capi
+
+    capi.set_tuning("norm_quant_nchunk", 8)
+    try:
+        assert capi.add_rmsnorm_quant_launch_shape(64, 16384, torch.float32) == (1024, 4)
+        assert capi.add_rmsnorm_quant_launch_shape(64, 1024, torch.float32) == (64, 4)
+        assert capi.add_rmsnorm_quant_launch_shape(64, 16384) == (256, 8)
+    finally:
+        capi.set_tuning("norm_quant_nchunk", 0)
+
+
 def test_rope_launch_shape_report():
     """gpuk_rope_rms_launch_shape computes on the host which rope kernel a batch gets, its grid and whether the rotated
     rows are stored past the L2; no GPU is needed."""

@@ -89,3 +89,23 @@ def test_extreme_values(device, tokens, hidden, quant, static):
     inp.gamma[4] = -inp.gamma[4]
     s = None if static is None else torch.tensor([static])
     check(inp, quant, run(inp, quant, device, s), s)
+
+
+@pytest.mark.parametrize("threads,nchunk", [(0, 8), (512, 8), (1024, 8), (1024, 2), (1024, 1), (448, 4), (0, 1)])
+def test_forced_shapes(device, threads, nchunk):
+    """The tuning keys choose another launch, never another result; eight chunks per lane, which only the 16-bit kernel has,
+    become four."""
+    from gpuk_amd import capi
+
+    print(f"case fp32 forced threads={threads} nchunk={nchunk}", flush=True)
+    capi.set_tuning("norm_quant_nchunk", nchunk)
+    capi.set_tuning("norm_quant_threads", threads)
+    try:
+        for tokens, hidden in ((301, 4096), (301, 1032), (37, 16384)):
+            inp = workloads.norm_quant_inputs(tokens, hidden, seed=threads + hidden, res_sigma=2.0, outlier_frac=0.01, dtype=torch.float32)
+            for quant in (0, 1, 3):
+                static = torch.tensor([0.013]) if quant == 3 else None
+                check(inp, quant, run(inp, quant, device, static), static)
+    finally:
+        capi.set_tuning("norm_quant_nchunk", 0)
+        capi.set_tuning("norm_quant_threads", 0)
