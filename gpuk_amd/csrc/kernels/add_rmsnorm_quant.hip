@@ -797,7 +797,10 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk) 
 // whole waves idles more lanes that way (an odd number of 64 chunks, or a little more than an even one), one chunk per lane
 // serves what the chip holds in one round (1032 elements: 2.2 against 2.45 us at one row, 5.65 against 6.2 at 2048), but
 // larger batches want the loads of two in flight: 12000 rows of 2560 / 3584 / 5632 / 7680 elements 37.0 / 49.6 / 76.6 /
-// 102.8 us against 39.4 / 53.5 / 86.0 / 111.7, of 3208 45.7 against 47.1; fp32 rows of 2568 66.3 against 70.9.
+// 102.8 us against 39.4 / 53.5 / 86.0 / 111.7, of 3208 45.7 against 47.1; fp32 rows of 2568 66.3 against 70.9.  Rows that one
+// wave holds with one chunk per lane keep it, a second chunk would be dead in every lane (one / two chunks: 9000 rows of 256
+// elements 5.4 / 6.7 us, 100000 rows 34.8 / 44.6, 20000 of 512 13.5 / 14.3; above 50000 rows of exactly 512 the two-chunk form is
+// 4 % ahead in bfloat16, 150000 rows 90.4 / 86.8, level in half precision).
 // most_chunks: the largest number of chunks per lane the type's kernel has (8; fp32 rows: 4, a forced 8 becomes that).
 void pick_shape(int64_t tokens, int chunks_per_row, int most_chunks, int *threads, int *nchunk) {
     auto fits = [&](int n) { return (int64_t)n * kMaxThreads >= chunks_per_row; };
@@ -816,7 +819,7 @@ void pick_shape(int64_t tokens, int chunks_per_row, int most_chunks, int *thread
         // 16.3 against 18.7 at 1700.  (That form keeps the normed row as 16-bit pairs between its last two phases:
         // with it in fp32 the kernel took 70 registers, seven waves per SIMD, 1792 rows.)
         // Not where four would idle a third of the lanes (3000 rows of 2312 elements: 12.4 us against 11.7 with two).
-        if (n <= 2 && !g_force_threads && tokens > resident_rows(n == 1 ? lanes1 : lanes2, n)) {
+        if (n <= 2 && lanes2 < lanes1 && !g_force_threads && tokens > resident_rows(n == 1 ? lanes1 : lanes2, n)) {
             const int t4 = round_up((chunks_per_row + 3) / 4, 64);
             n = tokens > resident_rows(lanes2, 2) && tokens <= resident_rows(t4, 4) && 8 * t4 <= 3 * chunks_per_row ? 4 : 2;
         }

@@ -309,6 +309,17 @@ def test_launch_shape_of_forced_chunks():
         capi.set_tuning("norm_quant_nchunk", 0)
 
 
+def test_launch_shape_of_short_rows():
+    """Rows that one wave holds with one chunk per lane keep that shape at every batch size."""
+    from gpuk_amd import capi
+
+    for tokens in (1, 8192, 8193, 9000, 100000):
+        for hidden in (8, 128, 264, 512):
+            assert capi.add_rmsnorm_quant_launch_shape(tokens, hidden) == (64, 1), (tokens, hidden)
+        assert capi.add_rmsnorm_quant_launch_shape(tokens, 256, torch.float32) == (64, 1)
+    assert capi.add_rmsnorm_quant_launch_shape(9000, 520) == (64, 2)
+
+
 def test_rope_launch_shape_report():
     """gpuk_rope_rms_launch_shape computes on the host which rope kernel a batch gets, its grid and whether the rotated
     rows are stored past the L2; no GPU is needed."""
