@@ -791,6 +791,9 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk) 
     return (uint32_t)std::min(ticks, 5000.0);
 }
 
+enum class RowType { BF16, FP16, F32 };
+template <typename T> constexpr RowType row_type = is_half<T> ? RowType::FP16 : RowType::BF16;
+
 // Lanes per row and chunks per lane.  Two chunks per lane on as many lanes as that needs (up to 1024) stream best or tie
 // for 1024 .. 16384 16-bit elements (1-6 % over one or four chunks per lane; 7168 elements, per call: 3.3 us against 3.5
 // with one chunk at one row, 5.0 against 5.6 at 256 rows); longer rows double the chunks per lane.  Where rounding up to
@@ -801,8 +804,8 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk) 
 // wave holds with one chunk per lane keep it, a second chunk would be dead in every lane (one / two chunks: 9000 rows of 256
 // elements 5.4 / 6.7 us, 100000 rows 34.8 / 44.6, 20000 of 512 13.5 / 14.3; above 50000 rows of exactly 512 the two-chunk form is
 // 4 % ahead in bfloat16, 150000 rows 90.4 / 86.8, level in half precision).
-// most_chunks: the largest number of chunks per lane the type's kernel has (8; fp32 rows: 4, a forced 8 becomes that).
-void pick_shape(int64_t tokens, int chunks_per_row, int most_chunks, int *threads, int *nchunk) {
+void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, int *nchunk) {
+    const int most_chunks = type == RowType::F32 ? kMaxChunksF32 : kMaxChunks;  // (a forced eight becomes four there)
     auto fits = [&](int n) { return (int64_t)n * kMaxThreads >= chunks_per_row; };
     int n;
     if (g_force_nchunk) {
@@ -842,19 +845,31 @@ int64_t half_of(int64_t tokens) { return (tokens + kComputeUnits - 1) / kCompute
 
 // Launches per call.  A batch of more than one round of workgroups and at most two runs as two launches of half the
 // rows, each a round of its own with the store gate: a read phase and a write phase twice over instead of two rounds
-// that mix the directions.  Only where the pieces' shape idles no more than an eighth of its lanes and rows start on line
-// boundaries (us, one launch / two: 4600 rows of 4096 elements 23.6 / 22.7, 8000 rows 38.5 / 38.0, 2300 of 8192 24.4 / 23.2, 4600 of
-// 3072 19.2 / 17.8; but where the pieces take four chunks on a quarter more lanes than the row fills 5500 of 3072 22.3 / 24.3,
-// 3200 of 5120 22.1 / 23.3, and 6000 rows of 1288 elements in one launch and 12000 in two 12.6 and 24.8 against 22.0 in one;
-// 2500 of 9000, which end inside lines, 30.1 / 31.8).
-int launches_for(int64_t tokens, int chunks_per_row) {
+// that mix the directions.  Only where each piece does fit a round in the shape it is given, rows start on line
+// boundaries, and that shape idles few lanes: from 1.1 rounds on one in eight, or one in five of a single wave with four
+// chunks per lane; from 1.25 rounds on one in five; from 1.5 on one in four of a single wave (fp32 rows of one wave: one in
+// eight, always).  One launch / two, us:
+// bf16 4600 rows of 4096 elements 23.6 / 22.7, 8000 rows 38.5 / 38.0, 2300 of 8192 24.4 / 23.2, 4600 of 3072 19.2 / 17.8; 3200 of
+// 5120 (a sixth idle) 22.1 / 23.3 but 4608 30.4 / 28.9; 9830 of 1664 (a fifth, one wave of four chunks) 22.2 / 21.5-22.0, 11900
+// 25.9 / 24.5; 9830 of 832 (a fifth, of two chunks) 12.4 / 13.2, 14700 17.0 / 15.8; 14700 of 768 (a quarter, one wave) 16.1 / 15.3,
+// 5500 of 3072 (a quarter, two waves) 22.3 / 24.3, 11900 of 640 (three eighths) 11.7 / 12.6; fp32 14700 of 416 15.3 / 15.8.  Pieces
+// beyond a round: 5700 of 2688 21.0 / 24.6.  One chunk per lane (rows of at most 64 chunks): 11500 of 512 8.6 / 9.6, fp32 of 256
+// 7.9 / 9.5.  Rows that end inside lines: 2500 of 9000 30.1 / 31.8.
+int launches_for(int64_t tokens, int chunks_per_row, RowType type) {
     if (g_pieces == 1 || g_force_nchunk || g_force_threads || chunks_per_row > 2 * kMaxThreads) return 1;
     const int64_t round = resident_rows(round_up((chunks_per_row + 3) / 4, 64), 4);
     if (tokens <= round || tokens > 2 * round) return 1;
     if (g_pieces == 2) return 2;
+    const int64_t piece = tokens - half_of(tokens);  // (the larger one)
     int threads, nchunk;
-    pick_shape(tokens - half_of(tokens), chunks_per_row, kMaxChunks, &threads, &nchunk);
-    return 10 * tokens >= 11 * round && chunks_per_row % 8 == 0 && 7 * threads * nchunk <= 8 * chunks_per_row ? 2 : 1;
+    pick_shape(piece, chunks_per_row, type, &threads, &nchunk);
+    if (nchunk == 1 || piece > resident_rows(threads, nchunk) || chunks_per_row % 8 != 0) return 1;
+    const int places = threads * nchunk;
+    const bool one_wave = threads == 64, eighth = 8 * chunks_per_row >= 7 * places, fifth = 5 * chunks_per_row >= 4 * places;
+    if (!eighth && one_wave && type == RowType::F32) return 1;
+    if (eighth || (fifth && one_wave && nchunk == 4)) return 10 * tokens >= 11 * round ? 2 : 1;
+    if (fifth) return 4 * tokens > 5 * round ? 2 : 1;
+    return one_wave && 4 * chunks_per_row >= 3 * places && 2 * tokens >= 3 * round ? 2 : 1;
 }
 
 // log2 of the run of consecutive rows an XCD takes.  Runs of 64 rows: +1.1 % for 16 KiB rows (8192 rows), of 16-bit
@@ -885,8 +900,8 @@ float reciprocal_of_max(float fp8_max) {
 }
 
 // Rows of the first launch.
-int64_t first_piece(int64_t tokens, int chunks_per_row) {
-    if (launches_for(tokens, chunks_per_row) == 1) return tokens;
+int64_t first_piece(int64_t tokens, int chunks_per_row, RowType type) {
+    if (launches_for(tokens, chunks_per_row, type) == 1) return tokens;
     return half_of(tokens);
 }
 
@@ -897,7 +912,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
 template <typename T, int QUANT>
 int launch(const void *x, const void *residual_in, const void *gamma, void *residual_out, void *norm_out,
            float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
-    const int64_t piece = first_piece(tokens, (int)(hidden / 8));
+    const int64_t piece = first_piece(tokens, (int)(hidden / 8), row_type<T>);
     for (int64_t first = 0; first < tokens; first = first ? tokens : piece) {
         const int64_t in_bytes = first * hidden * 2, out_bytes = first * hidden * (QUANT == GPUK_QUANT_NONE ? 2 : 1);
         const int rc = launch_rows<T, QUANT>(static_cast<const char *>(x) + in_bytes, static_cast<const char *>(residual_in) + in_bytes,
@@ -914,7 +929,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
                 float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 8);
     int threads, nchunk;
-    pick_shape(tokens, chunks, kMaxChunks, &threads, &nchunk);
+    pick_shape(tokens, chunks, row_type<T>, &threads, &nchunk);
     const dim3 grid((unsigned)tokens);
     auto xs = static_cast<const u32x4 *>(x);
     auto rs = static_cast<const u32x4 *>(residual_in);
@@ -974,7 +989,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
                     float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 4);
     int threads, nchunk;
-    pick_shape(tokens, chunks, kMaxChunksF32, &threads, &nchunk);
+    pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
     const uint32_t gate = store_gate(tokens, hidden * 4, threads, nchunk);
     const int group_shift = row_group_shift(tokens, hidden * 4);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
@@ -1011,7 +1026,7 @@ int launch_wide(const void *x, const void *residual_in, const void *gamma, void 
     const int chunks = (int)(hidden / 4);
     if constexpr (sizeof(F) == 4) {
         if (chunks <= kMaxChunksF32 * kMaxThreads) {  // in pieces as for 16-bit rows, see launches_for
-            const int64_t piece = first_piece(tokens, chunks);
+            const int64_t piece = first_piece(tokens, chunks, RowType::F32);
             for (int64_t first = 0; first < tokens; first = first ? tokens : piece) {
                 const int64_t in_bytes = first * hidden * 4, out_bytes = first * hidden * (QUANT == GPUK_QUANT_NONE ? 4 : 1);
                 const int rc = launch_f32_rows<QUANT>(static_cast<const char *>(x) + in_bytes, static_cast<const char *>(residual_in) + in_bytes,
@@ -1099,7 +1114,7 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
     if (!x || !residual_in || !residual_out || !codes || !scale) return GPUK_ERR_INVALID_ARG;
     if (!aligned16(x) || !aligned16(residual_in) || !aligned16(residual_out) || !aligned8(codes)) return GPUK_ERR_MISALIGNED;
     const int chunks = (int)(hidden / 8);
-    if (const int64_t piece = first_piece(tokens, chunks); piece < tokens) {  // two launches where the op takes two
+    if (const int64_t piece = first_piece(tokens, chunks, RowType::BF16); piece < tokens) {  // two launches where the op takes two
         const int rc = gpuk_add_rmsnorm_quant_traffic_only(x, residual_in, residual_out, codes, scale, piece, hidden, stream);
         if (rc != GPUK_OK) return rc;
         const int64_t wide = piece * hidden * 2, narrow = piece * hidden;
@@ -1108,7 +1123,7 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
                                                    scale + piece, tokens - piece, hidden, stream);
     }
     int threads, nchunk;
-    pick_shape(tokens, chunks, kMaxChunks, &threads, &nchunk);
+    pick_shape(tokens, chunks, RowType::BF16, &threads, &nchunk);
     if (nchunk == 0) return GPUK_ERR_UNSUPPORTED;  // rows that do not stay in registers
     const int group_shift = row_group_shift(tokens, hidden * 2);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
@@ -1136,14 +1151,15 @@ extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidde
     const bool wide = dtype == GPUK_DTYPE_F32 || dtype == GPUK_DTYPE_F64;
     if (hidden % 8 != 0) return GPUK_ERR_UNSUPPORTED;  // the rule of gpuk_add_rmsnorm_quant, for every dtype
     if (dtype == GPUK_DTYPE_F32 && hidden / 4 <= kMaxChunksF32 * kMaxThreads) {
-        pick_shape(first_piece(tokens, (int)(hidden / 4)), (int)(hidden / 4), kMaxChunksF32, lanes_per_row, chunks_per_lane);
+        pick_shape(first_piece(tokens, (int)(hidden / 4), RowType::F32), (int)(hidden / 4), RowType::F32, lanes_per_row, chunks_per_lane);
         return GPUK_OK;
     }
     if (wide) {  // longer fp32 rows and fp64: 4-element chunks, 0 = rows swept three times
         pick_wide_shape((int)(hidden / 4), lanes_per_row, chunks_per_lane);
         return GPUK_OK;
     }
-    pick_shape(first_piece(tokens, (int)(hidden / 8)), (int)(hidden / 8), kMaxChunks, lanes_per_row, chunks_per_lane);
+    const RowType type = dtype == GPUK_DTYPE_FP16 ? RowType::FP16 : RowType::BF16;
+    pick_shape(first_piece(tokens, (int)(hidden / 8), type), (int)(hidden / 8), type, lanes_per_row, chunks_per_lane);
     return GPUK_OK;
 }
 

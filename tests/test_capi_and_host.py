@@ -320,6 +320,22 @@ def test_launch_shape_of_short_rows():
     assert capi.add_rmsnorm_quant_launch_shape(9000, 520) == (64, 2)
 
 
+def test_launch_shape_of_two_launches():
+    """Batches of one to two rounds run as two launches where the pieces idle at most a fifth of their lanes and the batch
+    is more than a quarter over the round (the report is the first piece's: four chunks per lane instead of two)."""
+    from gpuk_amd import capi
+
+    assert capi.add_rmsnorm_quant_launch_shape(3200, 5120) == (320, 2)
+    assert capi.add_rmsnorm_quant_launch_shape(3201, 5120) == (192, 4)
+    assert capi.add_rmsnorm_quant_launch_shape(5120, 5120) == (192, 4)
+    assert capi.add_rmsnorm_quant_launch_shape(5121, 5120) == (320, 2)
+    assert capi.add_rmsnorm_quant_launch_shape(4608, 5120, torch.float16) == (192, 4)
+    assert capi.add_rmsnorm_quant_launch_shape(11878, 1664) == (64, 4)
+    assert capi.add_rmsnorm_quant_launch_shape(11878, 832, torch.float32) == (128, 2)   # fp32 rows of one wave: full ones only
+    assert capi.add_rmsnorm_quant_launch_shape(12289, 1600) == (64, 4)                  # one wave: a quarter idle, from 1.5 rounds
+    assert capi.add_rmsnorm_quant_launch_shape(5800, 3072) == (192, 2)                  # ... but not two waves
+
+
 def test_rope_launch_shape_report():
     """gpuk_rope_rms_launch_shape computes on the host which rope kernel a batch gets, its grid and whether the rotated
     rows are stored past the L2; no GPU is needed."""
