@@ -824,7 +824,17 @@ void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, 
         // Not where four would idle a third of the lanes (3000 rows of 2312 elements: 12.4 us against 11.7 with two).
         if (n <= 2 && lanes2 < lanes1 && !g_force_threads && tokens > resident_rows(n == 1 ? lanes1 : lanes2, n)) {
             const int t4 = round_up((chunks_per_row + 3) / 4, 64);
-            n = tokens > resident_rows(lanes2, 2) && tokens <= resident_rows(t4, 4) && 8 * t4 <= 3 * chunks_per_row ? 4 : 2;
+            const int64_t round1 = resident_rows(lanes1, 1), round2 = resident_rows(lanes2, 2);
+            // Rows that two chunks per lane leave a third of their lanes idle for (129 to 170 chunks, on three waves or on
+            // two): one chunk between the round of the latter and three of the former (us, one chunk / two: 1160 elements
+            // 9.7 / 10.2 at 4480 rows, 10.4 / 11.2 at 5120, 14.1 / 14.6 at 7680, 18.1 / 18.1 at 10240; 1288 10.1 / 10.9, 11.0 /
+            // 11.9, 15.1 / 15.5, 19.2 / 19.5; 1032 9.5 / 9.7, 10.1 / 10.6, 13.9 / 13.8, 17.2 / 17.1), and in bfloat16, whose
+            // arithmetic is unpacked, where two idle two fifths also up to an eighth more than a round (2611 rows of 1032 6.36 /
+            // 6.81, 2816 6.7 / 7.0, but 3072 7.5 / 7.2; half precision 6.35 / 5.97 at 2611).
+            const bool thin = n == 1 && 3 * chunks_per_row < 4 * lanes2;
+            const bool one = thin && (tokens > round2 ? tokens <= 3 * round1
+                                                      : type == RowType::BF16 && 5 * chunks_per_row < 6 * lanes2 && 8 * tokens <= 9 * round1);
+            n = one ? 1 : tokens > round2 && tokens <= resident_rows(t4, 4) && 8 * t4 <= 3 * chunks_per_row ? 4 : 2;
         }
     }
     while (n < most_chunks && !fits(n)) n *= 2;

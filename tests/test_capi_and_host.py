@@ -320,6 +320,19 @@ def test_launch_shape_of_short_rows():
     assert capi.add_rmsnorm_quant_launch_shape(9000, 520) == (64, 2)
 
 
+def test_launch_shape_of_thin_rows():
+    """Rows of a little more than two waves' chunks, which two chunks per lane would leave a third of the lanes idle for:
+    one chunk per lane from two waves' round to three of three waves, and in bfloat16 just above the latter's round."""
+    from gpuk_amd import capi
+
+    shape = capi.add_rmsnorm_quant_launch_shape
+    assert [shape(t, 1032)[1] for t in (2560, 2561, 2880, 2881, 4096, 4097, 7680, 7681)] == [1, 1, 1, 2, 2, 1, 1, 2]
+    assert [shape(t, 1032, torch.float16)[1] for t in (2560, 2561, 4096, 4097, 7680, 7681)] == [1, 2, 2, 1, 1, 2]
+    assert [shape(t, 1360)[1] for t in (2560, 2561, 4097, 7680, 7681)] == [1, 2, 1, 1, 2]
+    assert [shape(t, 516 + 4, torch.float32)[1] for t in (2560, 2561, 4097, 7681)] == [1, 2, 1, 2]
+    assert [shape(t, 2056)[1] for t in (1280, 1281, 2561, 5000)] == [1, 2, 2, 2]
+
+
 def test_launch_shape_of_two_launches():
     """Batches of one to two rounds run as two launches where the pieces idle at most a fifth of their lanes and the batch
     is more than a quarter over the round (the report is the first piece's: four chunks per lane instead of two)."""
