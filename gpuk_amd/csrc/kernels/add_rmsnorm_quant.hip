@@ -66,6 +66,20 @@ __device__ __forceinline__ float div_by_rcp_finite(float a, float b, float rcp) 
     return __builtin_fmaf(-e, rcp, q);
 }
 
+// scale = amax / fp8_max, 1 for an all-zero row.  `ranged` is the scale for scale_in_fast_range to look at: 0 instead where
+// quotients by it have to be clamped (rcp_fp8_max: see reciprocal_of_max).  Set in the branch of unusual maxima, so that
+// the common one is spared the test.
+__device__ __forceinline__ float dynamic_scale(float amax, float fp8_max, float rcp_fp8_max, float *ranged) {
+    float scale;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax) && rcp_fp8_max > 0.f)) == 0, 1)) {
+        scale = *ranged = div_by_rcp_finite(amax, fp8_max, rcp_fp8_max);
+    } else {
+        scale = amax == 0.f ? 1.f : amax / fp8_max;
+        *ranged = rcp_fp8_max < 0.f ? 0.f : scale;
+    }
+    return scale;
+}
+
 // What a launch passes beside the workgroup size (lanes_and_shift, one argument register): lanes in bits 0-15, the row-run
 // shift in bits 16-23, the mask of line_pad in bits 24-31.
 __device__ __forceinline__ int lanes_of(uint32_t lanes_and_shift) { return (int)(lanes_and_shift & 0xffffu); }
@@ -284,21 +298,17 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
                 }
             }
         }
-        float scale;
+        float scale, ranged;
         GPUK_STAMP(6);  // row normed, the lane's maximum known
         if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
             float amax[1] = {any_nan ? __builtin_nanf("") : __builtin_fmaxf(m0, m1)};
             if constexpr (is_half<T>) amax[0] = MaxOp::apply(P::lo(half_max), P::hi(half_max));
             block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
             GPUK_STAMP(7);  // row maximum known to every wave
-            // rcp_fp8_max: see reciprocal_of_max
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax[0]) && rcp_fp8_max > 0.f)) == 0, 1))
-                scale = div_by_rcp_finite(amax[0], fp8_max, rcp_fp8_max);
-            else
-                scale = amax[0] == 0.f ? 1.f : amax[0] / fp8_max;
+            scale = dynamic_scale(amax[0], fp8_max, rcp_fp8_max, &ranged);
             if (tid == 0) scale_io[row] = scale;
         } else {
-            scale = static_scale;
+            scale = ranged = static_scale;
         }
 
         // ---- phase 3: code = e4m3fn(clamp(n2 / scale)), 8 codes per chunk.  With the dynamic scale every value is
@@ -316,7 +326,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         }
         // (the scale is the same in every lane; deciding by ballot tells the compiler so, and the common path is
         // laid out as straight-line code with the other one out of the way)
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(scale_in_fast_range(scale) && (!kDynamic || rcp_fp8_max >= 0.f))) == 0, 1)) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!scale_in_fast_range(ranged)) == 0, 1)) {
             float rcp;
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(mantissa_all_ones(scale)) == 0, 1)) rcp = rcp_rn_mid_range(scale);
             else rcp = 1.0f / scale;
@@ -598,12 +608,10 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
         if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
             float amax[1] = {any_nan ? __builtin_nanf("") : lane_max};
             block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax[0]) && rcp_fp8_max > 0.f)) == 0, 1))
-                scale = div_by_rcp_finite(amax[0], fp8_max, rcp_fp8_max);
-            else
-                scale = amax[0] == 0.f ? 1.f : amax[0] / fp8_max;
+            float ranged;
+            scale = dynamic_scale(amax[0], fp8_max, rcp_fp8_max, &ranged);
             if (tid == 0) scale_io[row] = scale;
-            fast = scale_in_fast_range(scale) && rcp_fp8_max >= 0.f;
+            fast = scale_in_fast_range(ranged);
         }
         // Quotients below the smallest code's half come out 0 with their sign whatever the correction step loses to
         // underflow; the others are the correctly rounded ones.  With the dynamic scale no clamp, as in
