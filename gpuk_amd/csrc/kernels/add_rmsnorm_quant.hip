@@ -15,8 +15,9 @@
 //
 // Data movement per element: 2 B x + 2 B residual in, 2 B residual out, 1 B code (7 B); the row lives
 // in registers between the three phases, so HBM sees each byte once.  Lane `t` of the workgroup owns
-// 16-byte chunk `i*blockDim + t` of the row for i < NCHUNK: every wave load/store instruction covers
-// 1 KiB (loads) or 512 B (codes) of contiguous memory.
+// 16-byte chunk `i*blockDim + t` of the row for i < NCHUNK (counted from the line boundary before the row where the row
+// starts inside a line, see line_pad): every wave load/store instruction covers 1 KiB (loads) or 512 B (codes) of
+// contiguous memory.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -64,6 +65,18 @@ __device__ __forceinline__ float div_by_rcp_finite(float a, float b, float rcp) 
     const float q = a * rcp;
     const float e = __builtin_fmaf(q, b, -a);
     return __builtin_fmaf(-e, rcp, q);
+}
+
+// 1 / sqrt(sumsq / H + eps).  The mean as an exact IEEE quotient: a multiplication when H is a power of two (exact, and
+// rounded like the quotient when the result is subnormal), elsewhere by multiply and two fused multiply-adds (exact on the
+// guarded range, see div_by_rcp); then the short square root and reciprocal.  Every wave of a row walks this dependent chain
+// before it can go on.
+__device__ __forceinline__ float row_rstd(float sumsq, float hidden_f, float rcp_hidden, int hidden_pow2, float eps) {
+    float mean;
+    if (hidden_pow2) mean = sumsq * rcp_hidden;
+    else if (__builtin_expect(__builtin_amdgcn_ballot_w64(!in_mid_range(sumsq)) == 0, 1)) mean = div_by_rcp_finite(sumsq, hidden_f, rcp_hidden);
+    else mean = sumsq / hidden_f;
+    return rsqrt_two_roundings(mean + eps);
 }
 
 // scale = amax / fp8_max, 1 for an all-zero row.  `ranged` is the scale for scale_in_fast_range to look at: 0 instead where
@@ -129,8 +142,8 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
                        float eps, float fp8_max, float rcp_fp8_max) {
     // The arguments are ordered by when a wave needs them: the first fourteen dwords (up to norm_out) are handed to
     // the wave in scalar registers at launch (-amdgpu-kernarg-preload-count), so the loads of the row are issued
-    // without a round trip for the argument block; lanes_and_shift holds the workgroup size (bits 0-15), passed so
-    // that it need not be fetched from the dispatch packet either, and the row-run shift (bits 16-31).
+    // without a round trip for the argument block; lanes_and_shift (see lanes_of) holds the workgroup size as well, so
+    // that it need not be fetched from the dispatch packet either.
     const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
     using P = Pack16<T>;
     __shared__ float s_sum[kReduceSlots];
@@ -219,15 +232,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
     GPUK_STAMP(4);  // sum of squares of the row known to every wave
 
     // ---- phase 2: n2 = rT(gamma * rT(res * rstd)); row amax for the dynamic scale.
-    // mean = sumsq / H as an exact IEEE quotient: a multiplication when H is a power of two (exact, and rounded like
-    // the quotient when the result is subnormal), a division otherwise
-    // Elsewhere the quotient by multiply and two fused multiply-adds (exact on the guarded range, see div_by_rcp) and
-    // the short square root and reciprocal: every wave of the row walks this dependent chain before it can go on.
-    float mean;
-    if (hidden_pow2) mean = sumsq[0] * rcp_hidden;
-    else if (__builtin_expect(__builtin_amdgcn_ballot_w64(!in_mid_range(sumsq[0])) == 0, 1)) mean = div_by_rcp_finite(sumsq[0], hidden_f, rcp_hidden);
-    else mean = sumsq[0] / hidden_f;
-    const float rstd = rsqrt_two_roundings(mean + eps);
+    const float rstd = row_rstd(sumsq[0], hidden_f, rcp_hidden, hidden_pow2, eps);
     GPUK_STAMP(5);  // rstd
     if constexpr (QUANT == GPUK_QUANT_NONE) {
         u32x4 *out = reinterpret_cast<u32x4 *>(norm_out) + row_base;
@@ -580,11 +585,7 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
     if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) asm volatile("" ::"s"(static_scale));
     block_allreduce<SumOp, 1>(sumsq, s_sum, num_waves);
     __builtin_amdgcn_s_setprio(0);
-    float mean;
-    if (hidden_pow2) mean = sumsq[0] * rcp_hidden;
-    else if (__builtin_expect(__builtin_amdgcn_ballot_w64(!in_mid_range(sumsq[0])) == 0, 1)) mean = div_by_rcp_finite(sumsq[0], hidden_f, rcp_hidden);
-    else mean = sumsq[0] / hidden_f;
-    const float rstd = rsqrt_two_roundings(mean + eps);
+    const float rstd = row_rstd(sumsq[0], hidden_f, rcp_hidden, hidden_pow2, eps);
 
     f32x4 nv[NCHUNK];
     float m0 = 0.f, m1 = 0.f;
