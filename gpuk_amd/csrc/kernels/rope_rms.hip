@@ -616,8 +616,14 @@ __device__ __forceinline__ void load_trig_by_axis(const uint16_t *table, int64_t
     }
 }
 
-// Norm and rotation of a token's units, in place.
-template <typename T, int D, bool NEOX, int UPT>
+// Norm and rotation of a token's units, in place.  PIN: each unit is finished before the next.  Left to itself the compiler
+// moves half precision's packed sums, the last step of the rotation, of all units behind the last one, where the rows are
+// pinned, and keeps both products of each alive until then: forms of five units spilled 32 to 84 bytes per lane, those of two
+// tokens per wave with a cache 32 to 40.  Unpinned / pinned, us: 4096 tokens of 32+8+8 heads 20.6 / 17.3, pairwise 23.0 / 18.5, with
+// an fp8 cache 19.7 / 16.3, in place 16.0 / 15.4; 8192 of 28+4+4 29.3 / 25.7, with three axes 30.4 / 25.7.  Four units without a
+// second token do not spill (4096 tokens of 28+4+4 13.0 / 13.2), with one and in place 8 to 24 bytes, which cost less than
+// the pin's order (8192 tokens 23.8 / 24.2).
+template <typename T, int D, bool NEOX, int UPT, bool PIN>
 __device__ __forceinline__ void token_rotate(u32x4 (&xa)[UPT], u32x4 (&xb)[UPT], const u32x4 &qwa, const u32x4 &qwb,
                                              const u32x4 &kwa, const u32x4 &kwb, const u32x4 &cosv, const u32x4 &sinv,
                                              float eps, int hq, int hl) {
@@ -638,6 +644,7 @@ __device__ __forceinline__ void token_rotate(u32x4 (&xa)[UPT], u32x4 (&xb)[UPT],
         u32x4 oa, ob;
         norm_rotate<T, D, NEOX>(xa[u], xb[u], wa, wb, cosv, sinv, eps, oa, ob);
         xa[u] = oa, xb[u] = ob;
+        if constexpr (PIN) asm volatile("" : "+v"(xa[u]), "+v"(xb[u]));
     }
 }
 
@@ -707,6 +714,7 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
                       int hv, uint32_t num_waves, int64_t ps_token, int64_t ps_axis, const RopeArgs rest) {
     constexpr int LPH = D / 16, HPW = 64 / LPH, HALF = D / 2;
     constexpr int VN = TWO ? 1 : 2;  // V chunks per lane: the host admits 64 chunks per token with TWO, else 128
+    constexpr bool kPin = is_half<T> && (UPT == 5 || (TWO && SETKV));
     extern __shared__ __attribute__((aligned(16))) char token_lds[];  // TWO: 4 waves x token_kernel_lds_bytes_per_wave()
     const uint64_t entry = __builtin_amdgcn_s_memrealtime();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -821,7 +829,7 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- norm and rotation of the first token, unit by unit, in place
-    token_rotate<T, D, NEOX, UPT>(xa, xb, qwa, qwb, kwa, kwb, cosv, sinv, a.eps, hq, hl);
+    token_rotate<T, D, NEOX, UPT, kPin>(xa, xb, qwa, qwb, kwa, kwb, cosv, sinv, a.eps, hq, hl);
 
     // (the rotated rows are pinned down here, ahead of the wait: nothing ties the arithmetic to the clock, and the
     // compiler otherwise moves it behind the wait, into the writing half)
@@ -843,7 +851,7 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
                 xb[u] = *reinterpret_cast<const u32x4 *>(mine + (2 * u + 1) * 1024);
             }
             if constexpr (SETKV) v[0] = *reinterpret_cast<const u32x4 *>(mine + (2 * UPT) * 1024);
-            token_rotate<T, D, NEOX, UPT>(xa, xb, qwa, qwb, kwa, kwb, cosv2, sinv2, a.eps, hq, hl);
+            token_rotate<T, D, NEOX, UPT, kPin>(xa, xb, qwa, qwb, kwa, kwb, cosv2, sinv2, a.eps, hq, hl);
             token_store<T, D, UPT, SETKV, KVFP8, VN>(a, t2, slot2, xa, xb, v, hq, hk, hv, lane);
         }
     }

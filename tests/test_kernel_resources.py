@@ -1,0 +1,52 @@
+"""The built kernels' own metadata (no GPU needed): forms that hold their data in registers must not spill any of it to
+scratch memory."""
+import os
+import re
+import struct
+
+import msgpack
+
+LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gpuk_amd", "lib", "libgpuk_amd.so")
+BUNDLE = b"__CLANG_OFFLOAD_BUNDLE__"
+
+
+def code_objects(data):
+    """The device ELF images in a host library: bundles of (offset, size, target) entries."""
+    at = data.find(BUNDLE)
+    while at >= 0:
+        pos = at + len(BUNDLE) + 8
+        for _ in range(struct.unpack_from("<Q", data, at + len(BUNDLE))[0]):
+            offset, size, name_len = struct.unpack_from("<QQQ", data, pos)
+            if b"gfx950" in data[pos + 24:pos + 24 + name_len]:
+                yield data[at + offset:at + offset + size]
+            pos += 24 + name_len
+        at = data.find(BUNDLE, at + 1)
+
+
+def kernels(elf):
+    """amdhsa.kernels of the code object's metadata note (owner "AMDGPU", type 32: msgpack)."""
+    table, = struct.unpack_from("<Q", elf, 0x28)
+    entry, count = struct.unpack_from("<HH", elf, 0x3A)
+    for i in range(count):
+        kind, = struct.unpack_from("<I", elf, table + i * entry + 4)
+        offset, size = struct.unpack_from("<QQ", elf, table + i * entry + 24)
+        end = offset + size
+        while kind == 7 and offset < end:   # SHT_NOTE
+            name_size, desc_size, note = struct.unpack_from("<III", elf, offset)
+            desc = offset + 12 + (name_size + 3) // 4 * 4
+            if note == 32:
+                yield from msgpack.unpackb(elf[desc:desc + desc_size], strict_map_key=False)["amdhsa.kernels"]
+            offset = desc + (desc_size + 3) // 4 * 4
+
+
+def test_no_scratch_where_rows_stay_in_registers():
+    found = {k[".name"]: k for elf in code_objects(open(LIB, "rb").read()) for k in kernels(elf)}
+    assert len(found) > 100
+    # (rows of 8 chunks per lane are left out: filled bf16 ones spill a dozen registers around their reductions)
+    bounded = [n for n in found if "rope_rms" in n or ("add_rmsnorm_quant" in n and "Li8E" not in n)]
+    assert sum("rope_rms_token_kernel" in n for n in bounded) >= 24
+    # (half precision in place with two tokens per wave: up to 24 bytes per lane, cheaper there than what avoids them)
+    in_place_two = re.compile(r"rope_rms_token_kernelINS_4FP16ELi128ELb[01]ELi4ELb0ELb0ELi[13]ELb1E")
+    spilled = {n: found[n][".private_segment_fixed_size"] for n in bounded}
+    spilled = {n: b for n, b in spilled.items() if b > (24 if in_place_two.search(n) else 0)}
+    assert not spilled, spilled
