@@ -530,12 +530,27 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
 // divided with the full expansion, stored codes 4 bytes per lane and had no store gate.  Per call, that version / this
 // one, dynamic scale: 8192 x 4096 72.0 / 68.0 us (6.05 / 6.41 TB/s), 3000 x 7168 52.6 / 47.4, 2048 x 4096 22.3 / 18.3, 1024 x
 // 7168 21.9 / 16.8, 512 x 4096 7.7 / 7.0, 256 x 7168 7.3 / 6.15, one row of 7168 4.5 / 4.1; 8192 x 4096 without codes 87.4 / 85.5.
-template <int NCHUNK, int QUANT, bool EXACT, bool GATED>
-__global__ void __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(GATED ? 8 : 4)))
+//
+// When the weights are asked for.  A row of them is half as many bytes as the row's own loads, and a compute unit that holds
+// few rows waits for its own: asked for at once, the weights of its first waves go ahead of the rows of its last.  So batches
+// of up to one round that do not gate their stores ask once the lane's row has landed, behind which the reduction hides
+// them, and rows of 28 KB and more, which keep a compute unit's memory path busy by themselves, once rstd is known.  Larger
+// batches have other rows to wait for and ask at once.  us, at once / landed / rstd known: 98 rows of 3320 elements without
+// codes 3.43 / 3.21 / 3.35, 32 of 5120 with 3.78 / 3.58 / 3.61, one of 2056 2.52 / 2.48 / 2.56, but 32 of 7168 4.60 / 4.16 / 4.01, of 12288
+// 5.95 / 5.89 / 5.62, 98 of 8192 without codes 5.00 / 5.39 / 4.54, of 16384 with 8.49 / 8.22 / 7.94; 4000 of 7168 without 77.7 / 79.2 /
+// 78.8; 32 of 1024, on two waves, 2.49 / 2.51 / 2.56.  (98 of 16384 without codes remain behind the sweep of each lane's chunks
+// one by one that this kernel replaced: 8.3 us, it 7.8.)  Gated rows of one chunk per lane and eight waves or more without codes,
+// the shortest computation, ask once landed as well: 400 of 2568 elements 5.1 / 4.6 us, 290 of 3840 5.5 / 4.9, but 1280 of 1032, on
+// five waves, 5.2 / 5.4.
+enum class F32Form { STREAM, GATED, LANDED, GATED_LANDED, LAST };
+template <int NCHUNK, int QUANT, bool EXACT, F32Form FORM>
+__global__ void __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(FORM == F32Form::GATED || FORM == F32Form::GATED_LANDED ? 8 : 4)))
 add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_per_row, int remap_end,
                            uint32_t lanes_and_shift, uint32_t gate, const f32x4 *__restrict__ gamma, f32x4 *residual_out,
                            void *norm_out, float *__restrict__ scale_io, float hidden_f, float rcp_hidden, int hidden_pow2,
                            float eps, float fp8_max, float rcp_fp8_max) {
+    constexpr bool GATED = FORM == F32Form::GATED || FORM == F32Form::GATED_LANDED;
+    constexpr bool LANDED = FORM == F32Form::LANDED || FORM == F32Form::GATED_LANDED;
     const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
     __shared__ float s_sum[kReduceSlots];
     __shared__ float s_max[kReduceSlots];
@@ -562,13 +577,22 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
         xv[i] = live[i] ? load_stream(x + row_base + c) : zero;
         rv[i] = live[i] ? load_stream(residual_in + row_base + c) : zero;
     }
+    auto load_weights = [&]() {
 #pragma unroll
-    for (int i = 0; i < NCHUNK; ++i) gv[i] = live[i] ? (gamma - pad)[i * nthreads + tid] : zero;
+        for (int i = 0; i < NCHUNK; ++i) gv[i] = live[i] ? (gamma - pad)[i * nthreads + tid] : zero;
+    };
+    if constexpr (FORM != F32Form::LAST && !LANDED) load_weights();
     asm volatile("" ::"s"(hidden_f), "s"(rcp_hidden), "s"(hidden_pow2), "s"(eps), "s"(fp8_max), "s"(rcp_fp8_max));
     float static_scale = 0.f;
     if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) static_scale = *(const __attribute__((address_space(4))) float *)scale_io;
 
     __builtin_amdgcn_s_setprio(1);
+    if constexpr (LANDED) {
+#pragma unroll
+        for (int i = 0; i < NCHUNK; ++i) asm volatile("" : "+v"(xv[i]), "+v"(rv[i]));
+        load_weights();
+        __builtin_amdgcn_sched_barrier(0);
+    }
     float ss0 = 0.f, ss1 = 0.f;
 #pragma unroll
     for (int i = 0; i < NCHUNK; ++i) {
@@ -586,6 +610,7 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
     block_allreduce<SumOp, 1>(sumsq, s_sum, num_waves);
     __builtin_amdgcn_s_setprio(0);
     const float rstd = row_rstd(sumsq[0], hidden_f, rcp_hidden, hidden_pow2, eps);
+    if constexpr (FORM == F32Form::LAST) load_weights();
 
     f32x4 nv[NCHUNK];
     float m0 = 0.f, m1 = 0.f;
@@ -1012,24 +1037,44 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
     const int chunks = (int)(hidden / 4);
     int threads, nchunk;
     pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
-    const uint32_t gate = store_gate(tokens, hidden * 4, threads, nchunk);
+    // (the store gate from 7.5 MB of reads on: with less to read per compute unit than a 16-bit kernel of as many lanes, and no
+    // reason to wait for the rest, 200 rows of 2056 elements without codes took 3.53 us gated and 3.28 without, 128 of 3320
+    // 3.56 and 3.37, but 300 of 3320 4.8 and 5.4, 128 of 8192 4.9 and 5.1)
+    const bool few_bytes = tokens * hidden * 8 < 7'500'000;  // (of both inputs)
+    const uint32_t gate = g_gate < 0 && few_bytes ? 0 : store_gate(tokens, hidden * 4, threads, nchunk);
+    const bool one_round = tokens <= resident_rows(threads, nchunk);
     const int group_shift = row_group_shift(tokens, hidden * 4);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
     const float hf = (float)hidden;
     const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
     const float rcp_fp8_max = reciprocal_of_max(fp8_max);
     const bool exact = (int64_t)threads * nchunk == chunks;
-#define GPUK_LAUNCH_F32_AS(N, EXACT, GATED)                                                                             \
-    add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, GATED><<<dim3((unsigned)tokens), threads, 0, stream>>>(                  \
+#define GPUK_LAUNCH_F32_AS(N, EXACT, FORM)                                                                              \
+    add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, F32Form::FORM><<<dim3((unsigned)tokens), threads, 0, stream>>>(          \
         static_cast<const f32x4 *>(x), static_cast<const f32x4 *>(residual_in), chunks, remap_end,                       \
-        (uint32_t)threads | ((uint32_t)group_shift << 16) | ((line_mask(threads, nchunk, chunks) & ~1u) << 24), gate, static_cast<const f32x4 *>(gamma),                      \
-        static_cast<f32x4 *>(residual_out), norm_out, scale, hf, 1.0f / hf, hidden_pow2, eps, fp8_max, rcp_fp8_max)
+        (uint32_t)threads | ((uint32_t)group_shift << 16) | ((line_mask(threads, nchunk, chunks) & ~1u) << 24), gate,    \
+        static_cast<const f32x4 *>(gamma), static_cast<f32x4 *>(residual_out), norm_out, scale, hf, 1.0f / hf,           \
+        hidden_pow2, eps, fp8_max, rcp_fp8_max)
+#define GPUK_LAUNCH_F32_EXACT(N, EXACT)                                                                                \
+    do {                                                                                                               \
+        if (gate) {                                                                                                    \
+            if constexpr (N == 1 && QUANT == GPUK_QUANT_NONE) {                                                        \
+                if (threads >= 512) GPUK_LAUNCH_F32_AS(N, EXACT, GATED_LANDED);                                        \
+                else GPUK_LAUNCH_F32_AS(N, EXACT, GATED);                                                              \
+            } else {                                                                                                   \
+                GPUK_LAUNCH_F32_AS(N, EXACT, GATED);                                                                   \
+            }                                                                                                          \
+        }                                                                                                              \
+        else if (!one_round || threads < 192) GPUK_LAUNCH_F32_AS(N, EXACT, STREAM);                                    \
+        else if constexpr (N == 1) GPUK_LAUNCH_F32_AS(N, EXACT, LANDED);                                               \
+        else if constexpr (N == 4) GPUK_LAUNCH_F32_AS(N, EXACT, LAST);                                                 \
+        else if (hidden < 7168) GPUK_LAUNCH_F32_AS(N, EXACT, LANDED);                                                  \
+        else GPUK_LAUNCH_F32_AS(N, EXACT, LAST);                                                                       \
+    } while (0)
 #define GPUK_LAUNCH_F32(N)                                                                                             \
     do {                                                                                                               \
-        if (exact && gate) GPUK_LAUNCH_F32_AS(N, true, true);                                                          \
-        else if (exact) GPUK_LAUNCH_F32_AS(N, true, false);                                                            \
-        else if (gate) GPUK_LAUNCH_F32_AS(N, false, true);                                                             \
-        else GPUK_LAUNCH_F32_AS(N, false, false);                                                                      \
+        if (exact) GPUK_LAUNCH_F32_EXACT(N, true);                                                                     \
+        else GPUK_LAUNCH_F32_EXACT(N, false);                                                                          \
     } while (0)
     switch (nchunk) {
         case 1: GPUK_LAUNCH_F32(1); break;
@@ -1038,6 +1083,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
         default: return GPUK_ERR_INTERNAL;
     }
 #undef GPUK_LAUNCH_F32
+#undef GPUK_LAUNCH_F32_EXACT
 #undef GPUK_LAUNCH_F32_AS
     return hip_status(hipGetLastError());
 }

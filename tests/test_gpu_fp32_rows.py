@@ -109,3 +109,15 @@ def test_forced_shapes(device, threads, nchunk):
     finally:
         capi.set_tuning("norm_quant_nchunk", 0)
         capi.set_tuning("norm_quant_threads", 0)
+
+
+# one, two and four chunks per lane, lanes filled and not: weights asked for once the row has landed (below 7168 elements), once
+# rstd is known (from there), and at once (two waves; more than a round)
+@pytest.mark.parametrize("tokens,hidden", [(5, 3320), (3, 1536), (33, 5120), (200, 2568), (6, 10240), (6, 10248), (3, 3840), (7, 3624),
+                                           (9, 8192), (9, 7176), (4, 16384), (4, 15000), (40, 1024), (700, 5640)])
+@pytest.mark.parametrize("quant", [0, 1, 3])
+def test_weight_orders(device, tokens, hidden, quant):
+    print(f"case fp32 weights {tokens}x{hidden} q{quant}", flush=True)
+    inp = workloads.norm_quant_inputs(tokens, hidden, seed=tokens + hidden, res_sigma=2.0, outlier_frac=0.01, dtype=torch.float32)
+    static = torch.tensor([0.013]) if quant == 3 else None
+    check(inp, quant, run(inp, quant, device, static, alias=tokens == 9), static)
