@@ -104,9 +104,10 @@ __device__ __forceinline__ int shift_of(uint32_t lanes_and_shift) { return (int)
 // where the workgroup has no more lanes to spare: see line_mask.
 // Lanes from the row's start / from the line: 16384 rows of 9000 elements 184.1 / 168.0 us, of 2568 55.1 / 50.3, of 7176 145.4 /
 // 141.9; 8192 fp32 rows of 9000 181.5 / 165.2, of 2568 56.0 / 49.5; batches of a few hundred rows level.
-// Rows of one chunk per lane stay at the row: the shape serves batches of a few rounds at most, which gained nothing (1024
-// rows of 3208 elements 6.27 / 6.26 us, 40000 of 264 19.4 / 19.4), and the arithmetic ahead of the first load costs one row of
-// 1032 2.09 / 2.13, of 3208 2.44 / 2.48, one fp32 row of 2056 2.20 / 2.23.  (Half precision, where the two forms are level, keeps it.)
+// Rows of one chunk per lane that do not gate their stores stay at the row: small batches, which the arithmetic ahead of the
+// first load costs more than it gains (one row of 1032 2.09 / 2.13 us, of 3208 2.44 / 2.48, one fp32 row of 2056 2.20 / 2.23; 40000
+// rows of 264 19.4 / 19.4).  Behind a gate it costs nothing (1280 fp32 rows of 1032 without codes 5.30 / 5.15).  Half precision, where
+// the two forms are level, keeps it throughout.
 __device__ __forceinline__ int line_pad(const void *x, int64_t row_base, uint32_t lanes_and_shift) {
     return (int)(((uint32_t)((uintptr_t)x >> 4) + (uint32_t)row_base) & (lanes_and_shift >> 24));
 }
@@ -166,7 +167,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
     int64_t row_base = (int64_t)row * chunks_per_row;
-    const int pad = EXACT || (NCHUNK == 1 && !is_half<T>) ? 0 : line_pad(x, row_base, lanes_and_shift);
+    const int pad = EXACT || (NCHUNK == 1 && !GATED && !is_half<T>) ? 0 : line_pad(x, row_base, lanes_and_shift);
     row_base -= pad;  // where lane 0 stands: a lane's chunk c is chunk c - pad of the row
 
     // ---- phase 0: issue every load of the row before touching any of them.  The row is loaded whole before any of
@@ -563,7 +564,7 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
     int64_t row_base = (int64_t)row * chunks_per_row;
-    const int pad = EXACT || NCHUNK == 1 ? 0 : line_pad(x, row_base, lanes_and_shift);  // (even: lanes stay paired)
+    const int pad = EXACT || (NCHUNK == 1 && !GATED) ? 0 : line_pad(x, row_base, lanes_and_shift);  // (even: lanes stay paired)
     row_base -= pad;
 
     // every load of the row ahead of the first use of any (and of the first store: residual_out may be an input)
