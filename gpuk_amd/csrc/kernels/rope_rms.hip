@@ -240,6 +240,11 @@ __device__ __forceinline__ void store_pair(void *p, const u32x4 &a, const u32x4 
 // two streams of 2 x (678 + 3608) tokens, 24 + 25 heads 23.7 / 22.1.  Calls that do not stream their stores (below 8 MB)
 // are bound by latency and keep the shorter code (2.14 / 2.21 us at one token), and so do those with a cache: a unit of
 // theirs is half Q and half K rows scattered over slots, and gains nothing (12.4 / 12.6 us at 4096 tokens of 32+8+8).
+// In bfloat16, whose waves are busier, so do streamed calls of less than 13.5 MB, of less than 18 MB where a token's last unit
+// is not full, and all those whose units are less than three quarters full (bytes read and written; us, half / whole: 28+4
+// heads 3.37 / 3.44 at 8 MB, 4.02 / 4.07 at 12, 5.26 / 4.63 at 16; 32+8, of 48 places, 4.70 / 4.92 at 16, 6.55 / 6.27 at 24; 16+2, of
+// 32, 4.1 / 4.4 at 10, 3-7 % behind up to 24 and at 60; two streams of 24+24 heads 4.26 / 4.31 at 12 MB, 6.25 / 5.43 at 20).  Half
+// precision gains 4-17 % throughout (32+8 at 8-14 MB: 1-2 % lost).
 __device__ __forceinline__ void exchange_lines(u32x4 &a, u32x4 &b) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1172,6 +1177,9 @@ __global__ void __launch_bounds__(256) rope_rms_2way_wide_kernel(const TwoWayArg
     }
 }
 
+int g_stream_rows = 0;    // output rows stored past the L2: 0 = built-in rule, 1 = never, 2 = always
+constexpr int64_t kWholeLinesFromBytes = 13'500'000, kWholeLinesFromBytesRagged = 18'000'000;  // bfloat16, see exchange_lines
+
 template <typename T, int D>
 int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stream) {
     const dim3 grid((a.unit_end[3] + 3) / 4, batch);
@@ -1179,8 +1187,10 @@ int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stre
     rope_rms_2way_kernel<T, D, NEOX, WHOLE><<<grid, 256, 0, stream>>>(a.in[0], a.in[1], a.in[2], a.in[3], (uint32_t)a.tokens0,  \
                                                                (uint32_t)a.tokens1, a.heads[0], a.heads[1], a.stream, a)
     constexpr bool kHalfLines = D == 64;  // see exchange_lines
-    if (neox && kHalfLines && a.stream) GPUK_LAUNCH_2WAY(true, kHalfLines);
-    else if (kHalfLines && a.stream) GPUK_LAUNCH_2WAY(false, kHalfLines);
+    const int64_t call_bytes = 4 * (int64_t)batch * ((int64_t)a.rows[0] + a.rows[1] + a.rows[2] + a.rows[3]) * D;
+    const bool whole = a.stream && (is_half<T> || g_stream_rows == 2 || call_bytes >= kWholeLinesFromBytes);
+    if (neox && kHalfLines && whole) GPUK_LAUNCH_2WAY(true, kHalfLines);
+    else if (kHalfLines && whole) GPUK_LAUNCH_2WAY(false, kHalfLines);
     else if (neox) GPUK_LAUNCH_2WAY(true, false);
     else GPUK_LAUNCH_2WAY(false, false);
 #undef GPUK_LAUNCH_2WAY
@@ -1216,7 +1226,6 @@ int launch_2way_head_size(const TwoWayArgs &a, int64_t D, bool neox, unsigned ba
 }
 
 int g_block_threads = 0;  // 0 = default
-int g_stream_rows = 0;    // output rows stored past the L2: 0 = built-in rule, 1 = never, 2 = always
 int g_merge_rows = 0;     // mRoPE rows merged on load where the sections allow: 0 = yes, 1 = never
 int g_token_waves = 0;    // one-wave-per-token kernel: 0 = built-in rule, 1 = never, 2 = wherever it fits, 3 = likewise, two tokens per wave where that fits
 int g_token_gate = -1;    // its gate in ticks of 10 ns; -1 = from the bytes of the call
@@ -1233,6 +1242,7 @@ constexpr int64_t kStreamFromBytes = 8'000'000;
 struct RopePlan {
     uint32_t threads, blocks;  // workgroup size and count of the launch
     bool stream;               // q_out / K rows / in-place rows stored past the L2
+    bool whole_lines;          // heads of 64 elements in place, bfloat16: lines moved whole where they are streamed (see exchange_lines)
     bool token_waves;          // the one-wave-per-token kernel
     bool two_tokens;           // ... with two tokens per wave, the second through LDS
     uint32_t token_wave_count; // its waves
@@ -1309,6 +1319,9 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool set_kv, bool kv_fp8)
                                             (kv_fp8 ? 1 : 2) * ((int64_t)a.num_tokens * a.hk * D + elems_v)
                                       : 4 * elems_qk;
     p.stream = g_stream_rows == 2 || (g_stream_rows == 0 && call_bytes >= kStreamFromBytes);
+    const int64_t heads = a.hq + a.hk, places = (int64_t)a.units_per_token * (64 / (D / 16));
+    p.whole_lines = g_stream_rows == 2 ||
+                    (4 * heads >= 3 * places && call_bytes >= (heads == places ? kWholeLinesFromBytes : kWholeLinesFromBytesRagged));
     // Workgroup size, swept over 64/128/256/512 lanes and one workgroup per token for 2-9 units per token: four
     // waves where a workgroup then holds whole tokens (its waves share the token's position and table row in the
     // CU's caches: 3-15 % ahead at 28+4 heads) and for large batches (1-3 % ahead from 4096 tokens on), single
@@ -1364,8 +1377,9 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
     rope_rms_kernel<T, D, NEOX, AXES, SETKV, KVFP8, GATED, WHOLE><<<p.blocks, p.threads, 0, stream>>>(                         \
         a.qkv_in, a.positions, a.total_units, a.units_per_token, a.upt_magic, a.hq, a.hk,                               \
         (uint32_t)a.hv | (log2_waves << 24), a.ps_token, a.ps_axis, b)
-    if (kHalfLines && b.stream_rows && b.gate) GPUK_LAUNCH_UNITS(true, kHalfLines);
-    else if (kHalfLines && b.stream_rows) GPUK_LAUNCH_UNITS(false, kHalfLines);
+    const bool whole = p.stream && (is_half<T> || p.whole_lines);
+    if (kHalfLines && whole && b.gate) GPUK_LAUNCH_UNITS(true, kHalfLines);
+    else if (kHalfLines && whole) GPUK_LAUNCH_UNITS(false, kHalfLines);
     else if (b.gate) GPUK_LAUNCH_UNITS(true, false);
     else GPUK_LAUNCH_UNITS(false, false);
 #undef GPUK_LAUNCH_UNITS
