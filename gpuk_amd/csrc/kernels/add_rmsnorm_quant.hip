@@ -820,12 +820,16 @@ int64_t resident_rows(int threads, int nchunk) {
 // 768, 9.0 against 11.7 at 1024 (gate 1.0-1.1 times the read time; 10.2 with 0.9, 9.6 with 1.2), nothing gained and
 // 0.1 us lost below a quarter of a round; at 4096 elements 6.2 against 7.7 us at 1024 rows, 10.2 against 12.4 at 2048; 20-45 % slower where the
 // batch does not fit one round.
-uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk) {
+// short_rows: rows of two chunks per lane whose computation ends well ahead of the reads of a half-filled round (half precision,
+// static scale).  From two fifths of a round to eleven twentieths they wait 1.16 times the read time: 460 rows of 8192 elements
+// 6.28 / 5.72 us, 576 of 6144 6.55 / 6.05, 576 of 5120 5.46 / 5.3, level or slower below and above (1228 of 4096 6.6 / 6.8).
+uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, bool short_rows = false) {
     if (g_gate >= 0) return (uint32_t)g_gate;
     const int64_t resident = resident_rows(threads, nchunk);
     if (tokens > resident || 4 * tokens < resident) return 0;
     // (four chunks per lane: the shape pick_shape takes to hold in one round what two chunks per lane cannot)
-    const double ticks = (nchunk >= 4 ? 1.08 : 1.05) * (double)(2 * tokens * row_bytes) / 70000.0;  // 70,000 bytes per tick of 10 ns
+    const bool half_filled = short_rows && nchunk == 2 && 5 * tokens >= 2 * resident && 20 * tokens <= 11 * resident;
+    const double ticks = (half_filled ? 1.16 : nchunk >= 4 ? 1.08 : 1.05) * (double)(2 * tokens * row_bytes) / 70000.0;  // 70,000 bytes per tick of 10 ns
     return (uint32_t)std::min(ticks, 5000.0);
 }
 
@@ -991,7 +995,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     const float rcp_hidden = 1.0f / hf;
     const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
     const float rcp_fp8_max = reciprocal_of_max(fp8_max);
-    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk);
+    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk, is_half<T> && QUANT == GPUK_QUANT_FP8_STATIC);
     const int group_shift = row_group_shift(tokens, hidden * 2);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
     const bool exact = (int64_t)threads * nchunk == chunks;
