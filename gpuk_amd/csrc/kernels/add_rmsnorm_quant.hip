@@ -906,8 +906,11 @@ int64_t half_of(int64_t tokens) { return (tokens + kComputeUnits - 1) / kCompute
 // 25.9 / 24.5; 9830 of 832 (a fifth, of two chunks) 12.4 / 13.2, 14700 17.0 / 15.8; 14700 of 768 (a quarter, one wave) 16.1 / 15.3,
 // 5500 of 3072 (a quarter, two waves) 22.3 / 24.3, 11900 of 640 (three eighths) 11.7 / 12.6; fp32 14700 of 416 15.3 / 15.8.  Pieces
 // beyond a round: 5700 of 2688 21.0 / 24.6.  One chunk per lane (rows of at most 64 chunks): 11500 of 512 8.6 / 9.6, fp32 of 256
-// 7.9 / 9.5.  Rows that end inside lines: 2500 of 9000 30.1 / 31.8.
-int launches_for(int64_t tokens, int chunks_per_row, RowType type) {
+// 7.9 / 9.5.  Rows that end inside lines: 2500 of 9000 30.1 / 31.8.  Wide fp32 rows, of which a round is few and the second
+// launch's start is a larger share: on five waves and more with codes (1331 of 7168 24.5 / 27.0, 1433 of 6144 21.4 / 24.0), six
+// without (1433 of 6144 26.0 / 27.2, but 1536 of 5120 25.3 / 23.9), four with codes where an eighth is idle (2662 of 3584 22.9 /
+// 24.4).  codes: for fp32, whether the rows are quantised.
+int launches_for(int64_t tokens, int chunks_per_row, RowType type, bool codes) {
     if (g_pieces == 1 || g_force_nchunk || g_force_threads || chunks_per_row > 2 * kMaxThreads) return 1;
     const int64_t round = resident_rows(round_up((chunks_per_row + 3) / 4, 64), 4);
     if (tokens <= round || tokens > 2 * round) return 1;
@@ -918,7 +921,9 @@ int launches_for(int64_t tokens, int chunks_per_row, RowType type) {
     if (nchunk == 1 || piece > resident_rows(threads, nchunk) || chunks_per_row % 8 != 0) return 1;
     const int places = threads * nchunk;
     const bool one_wave = threads == 64, eighth = 8 * chunks_per_row >= 7 * places, fifth = 5 * chunks_per_row >= 4 * places;
-    if (!eighth && one_wave && type == RowType::F32) return 1;
+    if (type == RowType::F32 && ((!eighth && one_wave) || threads >= (codes ? 320 : 384) ||
+                                 (codes && threads == 256 && 8 * chunks_per_row <= 7 * places)))
+        return 1;
     if (eighth || (fifth && one_wave && nchunk == 4)) return 10 * tokens >= 11 * round ? 2 : 1;
     if (fifth) return 4 * tokens > 5 * round ? 2 : 1;
     return one_wave && 4 * chunks_per_row >= 3 * places && 2 * tokens >= 3 * round ? 2 : 1;
@@ -952,8 +957,8 @@ float reciprocal_of_max(float fp8_max) {
 }
 
 // Rows of the first launch.
-int64_t first_piece(int64_t tokens, int chunks_per_row, RowType type) {
-    if (launches_for(tokens, chunks_per_row, type) == 1) return tokens;
+int64_t first_piece(int64_t tokens, int chunks_per_row, RowType type, bool codes = true) {
+    if (launches_for(tokens, chunks_per_row, type, codes) == 1) return tokens;
     return half_of(tokens);
 }
 
@@ -1099,7 +1104,7 @@ int launch_wide(const void *x, const void *residual_in, const void *gamma, void 
     const int chunks = (int)(hidden / 4);
     if constexpr (sizeof(F) == 4) {
         if (chunks <= kMaxChunksF32 * kMaxThreads) {  // in pieces as for 16-bit rows, see launches_for
-            const int64_t piece = first_piece(tokens, chunks, RowType::F32);
+            const int64_t piece = first_piece(tokens, chunks, RowType::F32, QUANT != GPUK_QUANT_NONE);
             for (int64_t first = 0; first < tokens; first = first ? tokens : piece) {
                 const int64_t in_bytes = first * hidden * 4, out_bytes = first * hidden * (QUANT == GPUK_QUANT_NONE ? 4 : 1);
                 const int rc = launch_f32_rows<QUANT>(static_cast<const char *>(x) + in_bytes, static_cast<const char *>(residual_in) + in_bytes,

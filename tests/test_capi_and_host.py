@@ -347,6 +347,11 @@ def test_launch_shape_of_two_launches():
     assert capi.add_rmsnorm_quant_launch_shape(11878, 832, torch.float32) == (128, 2)   # fp32 rows of one wave: full ones only
     assert capi.add_rmsnorm_quant_launch_shape(12289, 1600) == (64, 4)                  # one wave: a quarter idle, from 1.5 rounds
     assert capi.add_rmsnorm_quant_launch_shape(5800, 3072) == (192, 2)                  # ... but not two waves
+    # wide fp32 rows: one launch
+    assert capi.add_rmsnorm_quant_launch_shape(1400, 7168, torch.float32) == (896, 2)
+    assert capi.add_rmsnorm_quant_launch_shape(1600, 5120, torch.float32) == (640, 2)
+    assert capi.add_rmsnorm_quant_launch_shape(2700, 3584, torch.float32) == (448, 2)
+    assert capi.add_rmsnorm_quant_launch_shape(2700, 4096, torch.float32) == (256, 4)
 
 
 def test_rope_launch_shape_report():
