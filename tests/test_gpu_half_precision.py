@@ -8,22 +8,11 @@ import pytest
 import torch
 
 from gpuk_amd import workloads
-from oracle import torch_oracle as O
 from tests.test_gpu_norm_quant import run_capi
 from tests.test_gpu_rope import check_inplace, run_inplace
-from tests.util import assert_bits_equal
+from tests.util import assert_bits_equal, assert_norm_rows_explained
 
 pytestmark = pytest.mark.gpu
-
-
-def canonical(t):
-    """Bit patterns, every NaN alike."""
-    t = t.cpu().contiguous()
-    if t.element_size() == 1:
-        b = t.view(torch.uint8)
-        return torch.where((b & 0x7F) == 0x7F, torch.full_like(b, 0x7F), b)
-    b = t.view(torch.int16)
-    return torch.where(t.isnan(), torch.full_like(b, 0x7E00), b)
 
 
 # (tokens, hidden): one, two, four (gated, one round) and eight chunks per lane, rows that fill their lanes and not
@@ -41,19 +30,7 @@ def test_norm_quant_extremes(device, tokens, hidden, quant):
     x[5], r[5] = 30000.0, 30000.0                            # the largest finite row
     inp.gamma[::5] = inp.gamma[::5] * 2.0 ** -18             # subnormal products
     static = torch.tensor([0.01]) if quant == 3 else None
-    res, norm, scale = run_capi(inp, quant, device, static_scale=static)
-    got = canonical(norm)
-    explained = torch.zeros(tokens, dtype=torch.bool)
-    for off in (0, -1, 1, -2, 2, -3, 3):
-        res_ref, norm_ref, scale_ref = O.add_rmsnorm_quant_ref(x, r, inp.gamma, inp.eps, quant, static_scale=static, rstd_ulp_offset=off)
-        if off == 0:
-            assert torch.equal(canonical(res), canonical(res_ref)), "residual_out"
-        same = (got == canonical(norm_ref)).all(dim=1)
-        if quant == 1:
-            s, w = scale.cpu().flatten(), scale_ref.flatten()
-            same &= (s == w) | (s.isnan() & w.isnan())
-        explained |= same
-    assert bool(explained.all()), f"rows {(~explained).nonzero().flatten().tolist()[:8]} match the oracle at no rstd within 3 ULP"
+    assert_norm_rows_explained(inp, quant, run_capi(inp, quant, device, static_scale=static), static)
 
 
 @pytest.mark.parametrize("neox", [True, False])

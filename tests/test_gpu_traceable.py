@@ -45,6 +45,10 @@ def test_opcheck_schema_and_fake_tensor(device):
     opcheck(gpuk_amd.traceable.allreduce_rms, args, test_utils=checks)
     _, args = norm_quant_args(device, quant=1)   # the schema checker's bookkeeping has no fp8 arithmetic
     opcheck(gpuk_amd.traceable.allreduce_rms, args, test_utils=("test_faketensor",))
+    x, r, g = args[1:4]
+    for quant in (0, 1):
+        opcheck(torch.ops.gpuk.add_rms_fused.default, (x, r, g, 1e-6, quant), test_utils=checks[quant:])
+    opcheck(torch.ops.gpuk.add_rms_fused.static, (x, r, g, 1e-6, torch.full((1,), 0.02, device=device)), test_utils=checks[1:])
     inp, qkv, qw, kw, cs, pos, loc, q, kc, vc = rope_args(device)
     opcheck(gpuk_amd.traceable.fused_rope_rms, (qkv.clone(), qw, kw, cs, pos, 40, 8, 2, 2, 128, True, inp.eps),
             test_utils=checks)
@@ -75,15 +79,17 @@ def test_compiled_function_keeps_the_writes(device):
     env = gpuk_amd.GPUKDistEnv(device_id=device.index or 0)
     inp, args = norm_quant_args(device, tokens=64, hidden=2048)
     x, r, g = args[1], args[2], args[3]
+    static = torch.full((1,), 0.02, device=device)
     rinp, qkv, qw, kw, cs, pos, loc, q, kc, vc = rope_args(device)
 
     def step(x, r, g, qkv, kc, vc):
         res, codes, scale = env.allreduce_add_rms_fused(x, r, g, inp.eps, fp8_out=True)
         dequant = codes.float() * scale                       # consumer of the written tensors
+        static_codes = env.allreduce_add_rms_fused(x, r, g, inp.eps, fp8_out=True, static_scale=static)[1]
         q_out = torch.empty((40, 8, 128), dtype=torch.bfloat16, device=x.device)
         gpuk_amd.traceable.fused_rope_rms_set_kv(qkv, qw, kw, cs, pos, 40, 8, 2, 2, 128, True, rinp.eps, q_out, kc, vc,
                                                  loc, 1.0, 1.0)
-        return res, codes, scale, dequant.sum(dim=-1), q_out, kc[loc].float().sum(), vc[loc].float().sum()
+        return res, codes, scale, dequant.sum(dim=-1), static_codes, q_out, kc[loc].float().sum(), vc[loc].float().sum()
 
     kc1, vc1 = kc.clone(), vc.clone()
     eager = step(x, r, g, qkv, kc1, vc1)
@@ -91,7 +97,7 @@ def test_compiled_function_keeps_the_writes(device):
     kc2, vc2 = kc.clone(), vc.clone()
     traced = compiled_step(x, r, g, qkv, kc2, vc2)
     torch.cuda.synchronize()
-    for a, b, name in zip(eager, traced, ("res", "codes", "scale", "dequant", "q", "k sum", "v sum")):
+    for a, b, name in zip(eager, traced, ("res", "codes", "scale", "dequant", "static codes", "q", "k sum", "v sum")):
         if a.dtype == torch.float8_e4m3fn:
             assert_bits_equal(a.view(torch.uint8), b.view(torch.uint8), name)
         else:

@@ -82,8 +82,8 @@ def canonical(t: torch.Tensor) -> torch.Tensor:
     if t.element_size() == 1:
         b = t.view(torch.uint8)
         return torch.where((b & 0x7F) == 0x7F, torch.full_like(b, 0x7F), b)
-    b = t.view(torch.int16 if t.element_size() == 2 else torch.int32)
-    return torch.where(t.isnan(), torch.full_like(b, 0x7E00), b)
+    b, nan = (t.view(torch.int16), 0x7E00) if t.element_size() == 2 else (t.view(torch.int32), 0x7FC00000)
+    return torch.where(t.isnan(), torch.full_like(b, nan), b)
 
 
 def assert_norm_rows_explained(inp, quant: int, got, static=None, fp8_max: float = 448.0):
