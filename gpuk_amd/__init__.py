@@ -114,8 +114,9 @@ class GPUKDistEnv:
 
     @contextmanager
     def capture(self):
-        """Wraps a stream capture (gpuk/__init__.py:112-120).  The fused op allocates nothing and launches on the
-        current stream, so at world size 1 a captured graph needs no pointer registration afterwards."""
+        """Wraps a stream capture (gpuk/__init__.py:112-120).  The fused op launches on the current stream and takes its
+        outputs from torch's allocator, under capture from the graph's pool, so at world size 1 a captured graph needs no
+        pointer registration afterwards."""
         try:
             self._IS_CAPTURING = True
             yield

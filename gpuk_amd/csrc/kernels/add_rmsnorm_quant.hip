@@ -813,7 +813,7 @@ int64_t resident_rows(int threads, int nchunk) {
     return (int64_t)kComputeUnits * (waves_per_cu / waves);
 }
 
-// The store gate of a launch of 16-bit rows: for batches whose workgroups are all resident at once (2048 lanes per
+// The store gate of a launch: for batches whose workgroups are all resident at once (2048 lanes per
 // compute unit) the time their reads take at 7 TB/s, the rate of a read-only kernel on this part, plus a twentieth;
 // 0 (stores as soon as they are ready) for larger batches, whose later workgroups read while earlier ones write
 // whatever a wave does.  Measured per call at 7168 elements: 6.35 against 7.2 us at 512 rows, 7.6 against 9.5 at

@@ -2,7 +2,8 @@
 // call into the C ABI (include/gpuk_amd.h).  No kernels and no device code in this layer.
 //
 // Same role as the reference's src/ops/ops.h:23-65; only the operators of the two fused paths are
-// declared, plus three additive ones (fused_rope_rms_set_kv, set_fp8_max, get_fp8_max).
+// declared, plus four additive ones (add_rms_fused with its overload for a static scale, fused_rope_rms_set_kv,
+// set_fp8_max, get_fp8_max).
 #pragma once
 
 #include <ATen/ATen.h>
