@@ -906,10 +906,12 @@ int64_t half_of(int64_t tokens) { return (tokens + kComputeUnits - 1) / kCompute
 // 25.9 / 24.5; 9830 of 832 (a fifth, of two chunks) 12.4 / 13.2, 14700 17.0 / 15.8; 14700 of 768 (a quarter, one wave) 16.1 / 15.3,
 // 5500 of 3072 (a quarter, two waves) 22.3 / 24.3, 11900 of 640 (three eighths) 11.7 / 12.6; fp32 14700 of 416 15.3 / 15.8.  Pieces
 // beyond a round: 5700 of 2688 21.0 / 24.6.  One chunk per lane (rows of at most 64 chunks): 11500 of 512 8.6 / 9.6, fp32 of 256
-// 7.9 / 9.5.  Rows that end inside lines: 2500 of 9000 30.1 / 31.8.  Wide fp32 rows, of which a round is few and the second
-// launch's start is a larger share: on five waves and more with codes (1331 of 7168 24.5 / 27.0, 1433 of 6144 21.4 / 24.0), six
-// without (1433 of 6144 26.0 / 27.2, but 1536 of 5120 25.3 / 23.9), four with codes where an eighth is idle (2662 of 3584 22.9 /
-// 24.4).  codes: for fp32, whether the rows are quantised.
+// 7.9 / 9.5.  Rows that end inside lines: 2500 of 9000 30.1 / 31.8.  Wide fp32 rows, four waves and more, of which a compute unit holds
+// few, pay for a layer of workgroups (one per compute unit) that a piece does not fill: two launches where the rows fill 94 % of
+// the two pieces' layers (92 on five waves, 96 on six), without codes 90 % (88 on five).  Two / one by that share, codes: five waves 1.04 at 88 %, 1.00 at 92, 0.96 at
+// 96; six 1.06 / 1.02 / 1.00, seven 1.04 / 1.01 / 0.98, eight 1.02 / 1.01 / 0.97; four 1.03 at 90, 1.00 at 94; without codes five to seven
+// 1.00 at 88, 0.98 at 90, 0.95 at 96 (1518 of 5120 with codes, 99 %, 20.1 / 17.8, but 1331 of 7168, 87 %, 24.5 / 27.0).  codes: for
+// fp32, whether the rows are quantised.
 int launches_for(int64_t tokens, int chunks_per_row, RowType type, bool codes) {
     if (g_pieces == 1 || g_force_nchunk || g_force_threads || chunks_per_row > 2 * kMaxThreads) return 1;
     const int64_t round = resident_rows(round_up((chunks_per_row + 3) / 4, 64), 4);
@@ -921,9 +923,11 @@ int launches_for(int64_t tokens, int chunks_per_row, RowType type, bool codes) {
     if (nchunk == 1 || piece > resident_rows(threads, nchunk) || chunks_per_row % 8 != 0) return 1;
     const int places = threads * nchunk;
     const bool one_wave = threads == 64, eighth = 8 * chunks_per_row >= 7 * places, fifth = 5 * chunks_per_row >= 4 * places;
-    if (type == RowType::F32 && ((!eighth && one_wave) || threads >= (codes ? 320 : 384) ||
-                                 (codes && threads == 256 && 8 * chunks_per_row <= 7 * places)))
-        return 1;
+    if (type == RowType::F32) {
+        const int64_t layers = (tokens - piece + kComputeUnits - 1) / kComputeUnits + (piece + kComputeUnits - 1) / kComputeUnits;
+        const int percent = !codes ? (threads == 320 ? 88 : 90) : threads == 320 ? 92 : threads == 384 ? 96 : 94;
+        if ((!eighth && one_wave) || (threads >= 256 && 100 * tokens < percent * layers * kComputeUnits)) return 1;
+    }
     if (eighth || (fifth && one_wave && nchunk == 4)) return 10 * tokens >= 11 * round ? 2 : 1;
     if (fifth) return 4 * tokens > 5 * round ? 2 : 1;
     return one_wave && 4 * chunks_per_row >= 3 * places && 2 * tokens >= 3 * round ? 2 : 1;

@@ -350,7 +350,11 @@ def test_launch_shape_of_two_launches():
     # wide fp32 rows: one launch
     assert capi.add_rmsnorm_quant_launch_shape(1400, 7168, torch.float32) == (896, 2)
     assert capi.add_rmsnorm_quant_launch_shape(1600, 5120, torch.float32) == (640, 2)
-    assert capi.add_rmsnorm_quant_launch_shape(2700, 3584, torch.float32) == (448, 2)
+    assert capi.add_rmsnorm_quant_launch_shape(2600, 3584, torch.float32) == (448, 2)
+    # wide fp32 rows that fill the layers of workgroups of both launches
+    assert capi.add_rmsnorm_quant_launch_shape(1518, 5120, torch.float32) == (320, 4)
+    assert capi.add_rmsnorm_quant_launch_shape(1531, 8192, torch.float32) == (512, 4)
+    assert capi.add_rmsnorm_quant_launch_shape(2020, 7168, torch.float32) == (448, 4)
     assert capi.add_rmsnorm_quant_launch_shape(2700, 4096, torch.float32) == (256, 4)
 
 
