@@ -1045,17 +1045,30 @@ void pick_wide_shape(int chunks, int *threads, int *cpl) {
     *threads = round_up((chunks + n - 1) / n, 64);
 }
 
+// Bytes of both inputs from which on fp32 batches gate their stores: with less to read per compute unit than a 16-bit kernel of
+// as many lanes has, a small batch has no reason to hold them.  Where the two cross depends on how long a row's own chain
+// is: few waves and no codes early, many waves and two chunks per lane late.  Gated / ungated, batches of a quarter of a round to
+// one: one wave of one chunk per lane with codes 0.994 at 4 MB, 0.97 at 6; without 0.98 / 0.92 below eleven twentieths of a
+// round, above 1.02 at 6, 0.99 at 8; more waves of one chunk without codes 1.04 / 1.03 / 0.97 / 0.90 at 4 / 5 / 6 / 7, with 1.03 / 1.02 /
+// 1.01 / 0.98; two chunks with codes 1.02 / 1.00 / 0.97 at 7 / 8 / 9, without 0.95 at 7 (0.99 on nine waves); of twelve waves 1.04 / 1.01 / 1.00 at 8 / 9 / 10,
+// 1.01 / 0.97 at 8 / 9 without,
+// four chunks 1.01 / 1.00 / 0.99.
+int64_t f32_gate_from_bytes(int64_t tokens, int threads, int nchunk, bool codes) {
+    const bool one_wave = threads == 64;
+    if (nchunk == 4 || (nchunk == 2 && threads >= 768)) return codes || nchunk == 4 ? 9'200'000 : 8'800'000;
+    if (nchunk == 2) return one_wave ? (codes ? 6'500'000 : 5'000'000) : codes ? 8'000'000 : threads < 576 ? 6'500'000 : 7'200'000;
+    if (one_wave) return !codes && 20 * tokens > 11 * resident_rows(threads, nchunk) ? 7'500'000 : 4'000'000;
+    return codes ? 7'000'000 : 6'000'000;
+}
+
 template <int QUANT>
 int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, void *residual_out, void *norm_out,
                     float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 4);
     int threads, nchunk;
     pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
-    // (the store gate from 7.5 MB of reads on: with less to read per compute unit than a 16-bit kernel of as many lanes, and no
-    // reason to wait for the rest, 200 rows of 2056 elements without codes took 3.53 us gated and 3.28 without, 128 of 3320
-    // 3.56 and 3.37, but 300 of 3320 4.8 and 5.4, 128 of 8192 4.9 and 5.1)
-    const bool few_bytes = tokens * hidden * 8 < 7'500'000;  // (of both inputs)
-    const uint32_t gate = g_gate < 0 && few_bytes ? 0 : store_gate(tokens, hidden * 4, threads, nchunk);
+    const bool gated = g_gate >= 0 || tokens * hidden * 8 >= f32_gate_from_bytes(tokens, threads, nchunk, QUANT != GPUK_QUANT_NONE);
+    const uint32_t gate = gated ? store_gate(tokens, hidden * 4, threads, nchunk) : 0;
     const bool one_round = tokens <= resident_rows(threads, nchunk);
     const int group_shift = row_group_shift(tokens, hidden * 4);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
