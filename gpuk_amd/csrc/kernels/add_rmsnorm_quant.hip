@@ -539,8 +539,13 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
 // batches have other rows to wait for and ask at once.  us, at once / landed / rstd known: 98 rows of 3320 elements without
 // codes 3.43 / 3.21 / 3.35, 32 of 5120 with 3.78 / 3.58 / 3.61, one of 2056 2.52 / 2.48 / 2.56, but 32 of 7168 4.60 / 4.16 / 4.01, of 12288
 // 5.95 / 5.89 / 5.62, 98 of 8192 without codes 5.00 / 5.39 / 4.54, of 16384 with 8.49 / 8.22 / 7.94; 4000 of 7168 without 77.7 / 79.2 /
-// 78.8; 32 of 1024, on two waves, 2.49 / 2.51 / 2.56.  (98 of 16384 without codes remain behind the sweep of each lane's chunks
-// one by one that this kernel replaced: 8.3 us, it 7.8.)  Gated rows of one chunk per lane and eight waves or more without codes,
+// 78.8; 32 of 1024, on two waves, 2.49 / 2.51 / 2.56.  At once as well: two chunks per lane on four waves and less, one row per
+// compute unit (127 rows of 1504 without codes 2.51 / 2.65, with codes level), and without codes, whose short chain leaves the
+// weights' latency open, up to 32 rows of more than 6144 elements (one of 8296 3.15 / - / 3.35, of 16384 3.73 / - / 3.97, 30 of 7760 2.90 /
+// - / 3.08) and rows of two chunks per lane that do not fill their lanes, on six waves and less or up to 128 of them on nine (one of 2968
+// 1.90 / 2.01, 29 of 2424 2.31 / 2.44, 314 of 1456 2.70 / 2.82; filled rows 1-5 % the other way).
+// (98 of 16384 without codes remain behind the sweep of each lane's chunks one by one that this kernel replaced: 8.3 us, it
+// 7.8.)  Gated rows of one chunk per lane and eight waves or more without codes,
 // the shortest computation, ask once landed as well: 400 of 2568 elements 5.1 / 4.6 us, 290 of 3840 5.5 / 4.9, but 1280 of 1032, on
 // five waves, 5.2 / 5.4.
 enum class F32Form { STREAM, GATED, LANDED, GATED_LANDED, LAST };
@@ -1067,15 +1072,19 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
     const int chunks = (int)(hidden / 4);
     int threads, nchunk;
     pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
+    const bool exact = (int64_t)threads * nchunk == chunks;
     const bool gated = g_gate >= 0 || tokens * hidden * 8 >= f32_gate_from_bytes(tokens, threads, nchunk, QUANT != GPUK_QUANT_NONE);
     const uint32_t gate = gated ? store_gate(tokens, hidden * 4, threads, nchunk) : 0;
-    const bool one_round = tokens <= resident_rows(threads, nchunk);
+    // Weights at once: more than a round, or waves that wait little for each other (see add_rmsnorm_quant_f32_rows).
+    const bool few_waves = threads < 192 || (nchunk == 2 && threads <= 256 && tokens <= kComputeUnits);
+    const bool short_chain = QUANT == GPUK_QUANT_NONE && ((hidden > 6144 && tokens <= 32) ||
+                                                          (!exact && nchunk == 2 && (threads < 448 || (threads <= 576 && tokens <= 128))));
+    const bool at_once = tokens > resident_rows(threads, nchunk) || few_waves || short_chain;
     const int group_shift = row_group_shift(tokens, hidden * 4);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
     const float hf = (float)hidden;
     const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
     const float rcp_fp8_max = reciprocal_of_max(fp8_max);
-    const bool exact = (int64_t)threads * nchunk == chunks;
 #define GPUK_LAUNCH_F32_AS(N, EXACT, FORM)                                                                              \
     add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, F32Form::FORM><<<dim3((unsigned)tokens), threads, 0, stream>>>(          \
         static_cast<const f32x4 *>(x), static_cast<const f32x4 *>(residual_in), chunks, remap_end,                       \
@@ -1092,7 +1101,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
                 GPUK_LAUNCH_F32_AS(N, EXACT, GATED);                                                                   \
             }                                                                                                          \
         }                                                                                                              \
-        else if (!one_round || threads < 192) GPUK_LAUNCH_F32_AS(N, EXACT, STREAM);                                    \
+        else if (at_once) GPUK_LAUNCH_F32_AS(N, EXACT, STREAM);                                                        \
         else if constexpr (N == 1) GPUK_LAUNCH_F32_AS(N, EXACT, LANDED);                                               \
         else if constexpr (N == 4) GPUK_LAUNCH_F32_AS(N, EXACT, LAST);                                                 \
         else if (hidden < 7168) GPUK_LAUNCH_F32_AS(N, EXACT, LANDED);                                                  \

@@ -84,10 +84,11 @@ def test_forced_shapes(device, threads, nchunk):
 
 
 # one, two and four chunks per lane, lanes filled and not: weights asked for once the row has landed (below 7168 elements), once
-# rstd is known (from there), and at once (two waves; more than a round); gated rows of one chunk per lane on nine and eleven
+# rstd is known (from there), and at once (two waves; two chunks on four and one row per compute unit; without codes up to 32 long
+# rows, and rows of two chunks that do not fill their lanes; more than a round); gated rows of one chunk per lane on nine and eleven
 # waves, which without codes ask once landed as well
-@pytest.mark.parametrize("tokens,hidden", [(5, 3320), (3, 1536), (33, 5120), (200, 2568), (6, 10240), (6, 10248), (3, 3840), (7, 3624),
-                                           (9, 8192), (9, 7176), (4, 16384), (4, 15000), (40, 1024), (700, 5640), (450, 2304), (400, 2568)])
+@pytest.mark.parametrize("tokens,hidden", [(5, 3320), (3, 1536), (33, 5120), (200, 2568), (6, 10240), (6, 10248), (3, 3840), (7, 3624), (7, 2424),
+                                           (9, 8192), (9, 7176), (4, 16384), (4, 15000), (40, 1024), (700, 5640), (450, 2304), (400, 2568), (5, 4104), (300, 1536), (33, 8192), (33, 7176), (33, 16384), (33, 15000), (300, 1456)])
 @pytest.mark.parametrize("quant", [0, 1, 3])
 def test_weight_orders(device, tokens, hidden, quant):
     print(f"case fp32 weights {tokens}x{hidden} q{quant}", flush=True)
