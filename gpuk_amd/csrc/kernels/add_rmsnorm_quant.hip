@@ -875,11 +875,12 @@ void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, 
             // Rows that two chunks per lane leave a third of their lanes idle for (129 to 170 chunks, on three waves or on
             // two): one chunk between the round of the latter and three of the former (us, one chunk / two: 1160 elements
             // 9.7 / 10.2 at 4480 rows, 10.4 / 11.2 at 5120, 14.1 / 14.6 at 7680, 18.1 / 18.1 at 10240; 1288 10.1 / 10.9, 11.0 /
-            // 11.9, 15.1 / 15.5, 19.2 / 19.5; 1032 9.5 / 9.7, 10.1 / 10.6, 13.9 / 13.8, 17.2 / 17.1), and in bfloat16, whose
+            // 11.9, 15.1 / 15.5, 19.2 / 19.5; 1032 9.5 / 9.7, 10.1 / 10.6, 13.9 / 13.8, 17.2 / 17.1; not fp32 rows, without codes 4146 of
+            // 624 8.99 / 8.54, 6676 of 552 12.2 / 11.7, with codes level), and in bfloat16, whose
             // arithmetic is unpacked, where two idle two fifths also up to an eighth more than a round (2611 rows of 1032 6.36 /
             // 6.81, 2816 6.7 / 7.0, but 3072 7.5 / 7.2; half precision 6.35 / 5.97 at 2611).
             const bool thin = n == 1 && 3 * chunks_per_row < 4 * lanes2;
-            const bool one = thin && (tokens > round2 ? tokens <= 3 * round1
+            const bool one = thin && (tokens > round2 ? type != RowType::F32 && tokens <= 3 * round1
                                                       : type == RowType::BF16 && 5 * chunks_per_row < 6 * lanes2 && 8 * tokens <= 9 * round1);
             n = one ? 1 : tokens > round2 && tokens <= resident_rows(t4, 4) && 8 * t4 <= 3 * chunks_per_row ? 4 : 2;
         }

@@ -329,7 +329,7 @@ def test_launch_shape_of_thin_rows():
     assert [shape(t, 1032)[1] for t in (2560, 2561, 2880, 2881, 4096, 4097, 7680, 7681)] == [1, 1, 1, 2, 2, 1, 1, 2]
     assert [shape(t, 1032, torch.float16)[1] for t in (2560, 2561, 4096, 4097, 7680, 7681)] == [1, 2, 2, 1, 1, 2]
     assert [shape(t, 1360)[1] for t in (2560, 2561, 4097, 7680, 7681)] == [1, 2, 1, 1, 2]
-    assert [shape(t, 516 + 4, torch.float32)[1] for t in (2560, 2561, 4097, 7681)] == [1, 2, 1, 2]
+    assert [shape(t, 516 + 4, torch.float32)[1] for t in (2560, 2561, 4097, 7681)] == [1, 2, 2, 2]
     assert [shape(t, 2056)[1] for t in (1280, 1281, 2561, 5000)] == [1, 2, 2, 2]
 
 
