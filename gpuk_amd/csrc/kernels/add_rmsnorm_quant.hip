@@ -35,13 +35,11 @@ constexpr int kMaxThreads = 1024;
 constexpr int kMaxWaves = kMaxThreads / 64;
 constexpr int kMaxChunks = 8, kMaxChunksF32 = 4;  // chunks per lane the kernels of 16-bit and of fp32 rows have forms for
 
-template <typename V>
-__device__ __forceinline__ V load_stream(const V *p) { return __builtin_nontemporal_load(p); }
-template <typename V>
-__device__ __forceinline__ void store_stream(V *p, V v) { __builtin_nontemporal_store(v, p); }
+template <typename P>
+__device__ __forceinline__ auto load_stream(P p) { return __builtin_nontemporal_load(p); }
+template <typename P, typename V>
+__device__ __forceinline__ void store_stream(P p, V v) { __builtin_nontemporal_store(v, p); }
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // The scale reciprocal is usable by div_by_rcp when scale is comfortably normal.
@@ -93,6 +91,21 @@ __device__ __forceinline__ float dynamic_scale(float amax, float fp8_max, float 
     return scale;
 }
 
+// The parameters of the kernels of rows that stay in registers, ordered by when a wave needs them: the first fourteen dwords
+// are handed to the wave in scalar registers at launch (-amdgpu-kernarg-preload-count), so that the loads of the row are
+// issued without a round trip for the argument block.  They come as three vectors and a struct, not sixteen scalars: see
+// launch_kernel (one row of 7168 elements, quantised, a call of the operator 5.36 / 4.79 us).
+//   first:  x, residual_in, chunks_per_row, remap_end, lanes_and_shift, gate
+//   second: gamma, residual_out
+//   third:  norm_out
+struct RowArgs {
+    float *scale_io;
+    float hidden_f, rcp_hidden;
+    int hidden_pow2;
+    float eps, fp8_max, rcp_fp8_max;
+};
+static_assert(sizeof(u32x8) + sizeof(u32x4) + sizeof(u32x2) + sizeof(RowArgs) <= 112, "see launch_kernel");
+
 // What a launch passes beside the workgroup size (lanes_and_shift, one argument register): lanes in bits 0-15, the row-run
 // shift in bits 16-23, the mask of line_pad in bits 24-31.
 __device__ __forceinline__ int lanes_of(uint32_t lanes_and_shift) { return (int)(lanes_and_shift & 0xffffu); }
@@ -108,8 +121,8 @@ __device__ __forceinline__ int shift_of(uint32_t lanes_and_shift) { return (int)
 // first load costs more than it gains (one row of 1032 2.09 / 2.13 us, of 3208 2.44 / 2.48, one fp32 row of 2056 2.20 / 2.23; 40000
 // rows of 264 19.4 / 19.4).  Behind a gate it costs nothing (1280 fp32 rows of 1032 without codes 5.30 / 5.15).  Half precision, where
 // the two forms are level, keeps it throughout.
-__device__ __forceinline__ int line_pad(const void *x, int64_t row_base, uint32_t lanes_and_shift) {
-    return (int)(((uint32_t)((uintptr_t)x >> 4) + (uint32_t)row_base) & (lanes_and_shift >> 24));
+__device__ __forceinline__ int line_pad(uint32_t x_low, int64_t row_base, uint32_t lanes_and_shift) {
+    return (int)(((x_low >> 4) + (uint32_t)row_base) & (lanes_and_shift >> 24));
 }
 
 // Two neighbouring elements of the normed row, rT(gamma * rT(res * rstd)), packed.
@@ -137,14 +150,16 @@ __device__ __attribute__((noinline)) u32x2 codes_by_division(f32x8 n, float scal
 // what a decode-sized batch waits for: with at most one row per compute unit the run time is the row's arithmetic).
 template <typename T, int NCHUNK, int QUANT, bool EXACT, bool GATED>
 __global__ void __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(GATED && NCHUNK <= 4 ? 8 : 4)))
-add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_row, int remap_end,
-                       uint32_t lanes_and_shift, uint32_t gate, const u32x4 *__restrict__ gamma, u32x4 *residual_out,
-                       void *norm_out, float *__restrict__ scale_io, float hidden_f, float rcp_hidden, int hidden_pow2,
-                       float eps, float fp8_max, float rcp_fp8_max) {
-    // The arguments are ordered by when a wave needs them: the first fourteen dwords (up to norm_out) are handed to
-    // the wave in scalar registers at launch (-amdgpu-kernarg-preload-count), so the loads of the row are issued
-    // without a round trip for the argument block; lanes_and_shift (see lanes_of) holds the workgroup size as well, so
-    // that it need not be fetched from the dispatch packet either.
+add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third, const RowArgs rest) {
+    Global<const u32x4> *x = global_ptr<const u32x4>(first[0], first[1]), *residual_in = global_ptr<const u32x4>(first[2], first[3]);
+    const int chunks_per_row = (int)first[4], remap_end = (int)first[5];
+    const uint32_t lanes_and_shift = first[6], gate = first[7];  // (see lanes_of: the workgroup size need not be fetched from the dispatch packet)
+    Global<const u32x4> *gamma = global_ptr<const u32x4>(second[0], second[1]);
+    Global<u32x4> *residual_out = global_ptr<u32x4>(second[2], second[3]);
+    Global<char> *norm_out = global_ptr<char>(third[0], third[1]);
+    float *scale_io = rest.scale_io;
+    const float hidden_f = rest.hidden_f, rcp_hidden = rest.rcp_hidden, eps = rest.eps, fp8_max = rest.fp8_max, rcp_fp8_max = rest.rcp_fp8_max;
+    const int hidden_pow2 = rest.hidden_pow2;
     const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
     using P = Pack16<T>;
     __shared__ float s_sum[kReduceSlots];
@@ -167,7 +182,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
     int64_t row_base = (int64_t)row * chunks_per_row;
-    const int pad = EXACT || (NCHUNK == 1 && !GATED && !is_half<T>) ? 0 : line_pad(x, row_base, lanes_and_shift);
+    const int pad = EXACT || (NCHUNK == 1 && !GATED && !is_half<T>) ? 0 : line_pad(first[0], row_base, lanes_and_shift);
     row_base -= pad;  // where lane 0 stands: a lane's chunk c is chunk c - pad of the row
 
     // ---- phase 0: issue every load of the row before touching any of them.  The row is loaded whole before any of
@@ -236,7 +251,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
     const float rstd = row_rstd(sumsq[0], hidden_f, rcp_hidden, hidden_pow2, eps);
     GPUK_STAMP(5);  // rstd
     if constexpr (QUANT == GPUK_QUANT_NONE) {
-        u32x4 *out = reinterpret_cast<u32x4 *>(norm_out) + row_base;
+        auto *out = (Global<u32x4> *)norm_out + row_base;
         u32x4 normed[NCHUNK];
 #pragma unroll
         for (int i = 0; i < NCHUNK; ++i) {
@@ -323,7 +338,7 @@ add_rmsnorm_quant_rows(const u32x4 *x, const u32x4 *residual_in, int chunks_per_
         // path, which clamps.)  The static scale may meet anything: clamp, and the form that restores what a division
         // gives for infinite and NaN numerators.
         constexpr bool kDynamic = QUANT == GPUK_QUANT_FP8_DYNAMIC;
-        u32x2 *out = reinterpret_cast<u32x2 *>(norm_out) + row_base;
+        auto *out = (Global<u32x2> *)norm_out + row_base;
         if constexpr (kPacked && !is_half<T>) {  // (or the compiler keeps phase 2's unpacked copies alive instead)
 #pragma unroll
             for (int i = 0; i < NCHUNK; ++i)
@@ -412,7 +427,7 @@ add_rmsnorm_quant_traffic_only(const u32x4 *x, const u32x4 *residual_in, int chu
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
     int64_t row_base = (int64_t)row * chunks_per_row;
-    const int pad = line_pad(x, row_base, lanes_and_shift);
+    const int pad = line_pad((uint32_t)(uintptr_t)x, row_base, lanes_and_shift);
     row_base -= pad;
     u32x4 xv[NCHUNK], rv[NCHUNK];
     bool live[NCHUNK];
@@ -551,10 +566,16 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
 enum class F32Form { STREAM, GATED, LANDED, GATED_LANDED, LAST };
 template <int NCHUNK, int QUANT, bool EXACT, F32Form FORM>
 __global__ void __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(FORM == F32Form::GATED || FORM == F32Form::GATED_LANDED ? 8 : 4)))
-add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_per_row, int remap_end,
-                           uint32_t lanes_and_shift, uint32_t gate, const f32x4 *__restrict__ gamma, f32x4 *residual_out,
-                           void *norm_out, float *__restrict__ scale_io, float hidden_f, float rcp_hidden, int hidden_pow2,
-                           float eps, float fp8_max, float rcp_fp8_max) {
+add_rmsnorm_quant_f32_rows(const u32x8 first, const u32x4 second, const u32x2 third, const RowArgs rest) {
+    Global<const f32x4> *x = global_ptr<const f32x4>(first[0], first[1]), *residual_in = global_ptr<const f32x4>(first[2], first[3]);
+    const int chunks_per_row = (int)first[4], remap_end = (int)first[5];
+    const uint32_t lanes_and_shift = first[6], gate = first[7];
+    Global<const f32x4> *gamma = global_ptr<const f32x4>(second[0], second[1]);
+    Global<f32x4> *residual_out = global_ptr<f32x4>(second[2], second[3]);
+    Global<char> *norm_out = global_ptr<char>(third[0], third[1]);
+    float *scale_io = rest.scale_io;
+    const float hidden_f = rest.hidden_f, rcp_hidden = rest.rcp_hidden, eps = rest.eps, fp8_max = rest.fp8_max, rcp_fp8_max = rest.rcp_fp8_max;
+    const int hidden_pow2 = rest.hidden_pow2;
     constexpr bool GATED = FORM == F32Form::GATED || FORM == F32Form::GATED_LANDED;
     constexpr bool LANDED = FORM == F32Form::LANDED || FORM == F32Form::GATED_LANDED;
     const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
@@ -569,7 +590,7 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
         row = ((((idx >> group_shift) << 3) | xcd) << group_shift) | (idx & ((1 << group_shift) - 1));
     }
     int64_t row_base = (int64_t)row * chunks_per_row;
-    const int pad = EXACT || (NCHUNK == 1 && !GATED) ? 0 : line_pad(x, row_base, lanes_and_shift);  // (even: lanes stay paired)
+    const int pad = EXACT || (NCHUNK == 1 && !GATED) ? 0 : line_pad(first[0], row_base, lanes_and_shift);  // (even: lanes stay paired)
     row_base -= pad;
 
     // every load of the row ahead of the first use of any (and of the first store: residual_out may be an input)
@@ -684,23 +705,23 @@ add_rmsnorm_quant_f32_rows(const f32x4 *x, const f32x4 *residual_in, int chunks_
             if (live[i]) store_stream(residual_out + row_base + i * nthreads + tid, xv[i]);
     }
     if constexpr (QUANT == GPUK_QUANT_NONE) {
-        f32x4 *out = reinterpret_cast<f32x4 *>(norm_out) + row_base;
+        auto *out = (Global<f32x4> *)norm_out + row_base;
 #pragma unroll
         for (int i = 0; i < NCHUNK; ++i)
             if (live[i]) store_stream(out + i * nthreads + tid, nv[i]);
     } else if constexpr (NCHUNK == 1) {
-        if (live[0]) store_stream(reinterpret_cast<uint32_t *>(norm_out) + row_base + tid, codes[0]);
+        if (live[0]) store_stream((Global<uint32_t> *)norm_out + row_base + tid, codes[0]);
     } else {
         // 8 codes per lane and store: of two chunks, even lanes store the first one's codes of themselves and their odd
         // neighbour, odd lanes the second one's (a row is an even number of chunks: neighbours are live together)
-        uint32_t *out = reinterpret_cast<uint32_t *>(norm_out) + row_base;
+        auto *out = (Global<uint32_t> *)norm_out + row_base;
         const bool odd = tid & 1;
 #pragma unroll
         for (int i = 0; i < NCHUNK; i += 2) {
             const uint32_t give = odd ? codes[i] : codes[i + 1], keep = odd ? codes[i + 1] : codes[i];
             const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, DPP_QUAD_XOR1, 0xf, 0xf, true);
             if (odd ? live[i + 1] : live[i])
-                store_stream(reinterpret_cast<u32x2 *>(out + (odd ? i + 1 : i) * nthreads + (tid & ~1)), odd ? u32x2{got, keep} : u32x2{keep, got});
+                store_stream((Global<u32x2> *)(out + (odd ? i + 1 : i) * nthreads + (tid & ~1)), odd ? u32x2{got, keep} : u32x2{keep, got});
         }
     }
 }
@@ -991,6 +1012,24 @@ int launch(const void *x, const void *residual_in, const void *gamma, void *resi
     return GPUK_OK;
 }
 
+// What is passed to the kernels of rows that stay in registers, see RowArgs.  shape: lanes_and_shift.
+struct RowParameters {
+    u32x8 first;
+    u32x4 second;
+    u32x2 third;
+    RowArgs rest;
+};
+RowParameters row_parameters(const void *x, const void *residual_in, const void *gamma, const void *residual_out, const void *norm_out,
+                             float *scale, int64_t tokens, int chunks, uint32_t shape, uint32_t gate, int64_t hidden, float eps, float fp8_max) {
+    const int group_shift = (int)((shape >> 16) & 0xffu);
+    const uint32_t remap_end = group_shift > 0 ? (uint32_t)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0u;
+    const float hf = (float)hidden;
+    return {u32x8{low_half(x), high_half(x), low_half(residual_in), high_half(residual_in), (uint32_t)chunks, remap_end, shape, gate},
+            u32x4{low_half(gamma), high_half(gamma), low_half(residual_out), high_half(residual_out)},
+            u32x2{low_half(norm_out), high_half(norm_out)},
+            RowArgs{scale, hf, 1.0f / hf, (hidden & (hidden - 1)) == 0, eps, fp8_max, reciprocal_of_max(fp8_max)}};
+}
+
 template <typename T, int QUANT>
 int launch_rows(const void *x, const void *residual_in, const void *gamma, void *residual_out, void *norm_out,
                 float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
@@ -998,26 +1037,18 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     int threads, nchunk;
     pick_shape(tokens, chunks, row_type<T>, &threads, &nchunk);
     const dim3 grid((unsigned)tokens);
-    auto xs = static_cast<const u32x4 *>(x);
-    auto rs = static_cast<const u32x4 *>(residual_in);
-    auto gs = static_cast<const u32x4 *>(gamma);
-    auto ro = static_cast<u32x4 *>(residual_out);
-    const float hf = (float)hidden;
     if (nchunk == 0) {
-        add_rmsnorm_quant_long_rows<T, QUANT><<<grid, kMaxThreads, 0, stream>>>(xs, rs, gs, ro, norm_out, scale, chunks, hf, eps, fp8_max);
+        add_rmsnorm_quant_long_rows<T, QUANT><<<grid, kMaxThreads, 0, stream>>>(
+            static_cast<const u32x4 *>(x), static_cast<const u32x4 *>(residual_in), static_cast<const u32x4 *>(gamma),
+            static_cast<u32x4 *>(residual_out), norm_out, scale, chunks, (float)hidden, eps, fp8_max);
         return hip_status(hipGetLastError());
     }
-    const float rcp_hidden = 1.0f / hf;
-    const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
-    const float rcp_fp8_max = reciprocal_of_max(fp8_max);
     const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk, is_half<T> && QUANT == GPUK_QUANT_FP8_STATIC);
-    const int group_shift = row_group_shift(tokens, hidden * 2);
-    const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
+    const uint32_t shape = (uint32_t)threads | ((uint32_t)row_group_shift(tokens, hidden * 2) << 16) | (line_mask(threads, nchunk, chunks) << 24);
     const bool exact = (int64_t)threads * nchunk == chunks;
+    const RowParameters p = row_parameters(x, residual_in, gamma, residual_out, norm_out, scale, tokens, chunks, shape, gate, hidden, eps, fp8_max);
 #define GPUK_LAUNCH_NQ_AS(N, EXACT, GATED)                                                                              \
-    add_rmsnorm_quant_rows<T, N, QUANT, EXACT, GATED><<<grid, threads, 0, stream>>>(                                    \
-        xs, rs, chunks, remap_end, (uint32_t)threads | ((uint32_t)group_shift << 16) | (line_mask(threads, nchunk, chunks) << 24), gate, gs, ro, norm_out, scale, hf, \
-        rcp_hidden, hidden_pow2, eps, fp8_max, rcp_fp8_max)
+    return launch_kernel(add_rmsnorm_quant_rows<T, N, QUANT, EXACT, GATED>, grid, (uint32_t)threads, 0, stream, p.first, p.second, p.third, p.rest)
 #define GPUK_LAUNCH_NQ(N)                                                                                              \
     do {                                                                                                               \
         if (exact && gate) GPUK_LAUNCH_NQ_AS(N, true, true);                                                           \
@@ -1034,7 +1065,6 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     }
 #undef GPUK_LAUNCH_NQ
 #undef GPUK_LAUNCH_NQ_AS
-    return hip_status(hipGetLastError());
 }
 
 // Lanes and kept chunks per lane of the fp64 kernel; 0 chunks kept = rows beyond 4096 chunks, swept (fp32 rows come here
@@ -1081,17 +1111,11 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
     const bool short_chain = QUANT == GPUK_QUANT_NONE && ((hidden > 6144 && tokens <= 32) ||
                                                           (!exact && nchunk == 2 && (threads < 448 || (threads <= 576 && tokens <= 128))));
     const bool at_once = tokens > resident_rows(threads, nchunk) || few_waves || short_chain;
-    const int group_shift = row_group_shift(tokens, hidden * 4);
-    const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
-    const float hf = (float)hidden;
-    const int hidden_pow2 = (hidden & (hidden - 1)) == 0;
-    const float rcp_fp8_max = reciprocal_of_max(fp8_max);
+    const uint32_t shape = (uint32_t)threads | ((uint32_t)row_group_shift(tokens, hidden * 4) << 16) | ((line_mask(threads, nchunk, chunks) & ~1u) << 24);
+    const RowParameters p = row_parameters(x, residual_in, gamma, residual_out, norm_out, scale, tokens, chunks, shape, gate, hidden, eps, fp8_max);
 #define GPUK_LAUNCH_F32_AS(N, EXACT, FORM)                                                                              \
-    add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, F32Form::FORM><<<dim3((unsigned)tokens), threads, 0, stream>>>(          \
-        static_cast<const f32x4 *>(x), static_cast<const f32x4 *>(residual_in), chunks, remap_end,                       \
-        (uint32_t)threads | ((uint32_t)group_shift << 16) | ((line_mask(threads, nchunk, chunks) & ~1u) << 24), gate,    \
-        static_cast<const f32x4 *>(gamma), static_cast<f32x4 *>(residual_out), norm_out, scale, hf, 1.0f / hf,           \
-        hidden_pow2, eps, fp8_max, rcp_fp8_max)
+    return launch_kernel(add_rmsnorm_quant_f32_rows<N, QUANT, EXACT, F32Form::FORM>, dim3((unsigned)tokens), (uint32_t)threads, 0, stream, \
+                         p.first, p.second, p.third, p.rest)
 #define GPUK_LAUNCH_F32_EXACT(N, EXACT)                                                                                \
     do {                                                                                                               \
         if (gate) {                                                                                                    \
@@ -1122,7 +1146,6 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
 #undef GPUK_LAUNCH_F32
 #undef GPUK_LAUNCH_F32_EXACT
 #undef GPUK_LAUNCH_F32_AS
-    return hip_status(hipGetLastError());
 }
 
 template <typename F, int QUANT>

@@ -14,6 +14,23 @@ namespace gpuk {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+
+// What a pointer read from the argument block by hand points at, for the compiler, to which it is a generic one otherwise:
+// accesses through it are global (not flat) ones, and scalar ones where the address is the same in every lane.
+template <typename P>
+__device__ __forceinline__ P *as_global(P *p) {
+    return (P *)(__attribute__((address_space(1))) P *)p;
+}
+// A pointer that came as two dwords of a vector parameter (see launch_kernel for why parameters are vectors).
+template <typename V>
+using Global = __attribute__((address_space(1))) V;
+template <typename V>
+__device__ __forceinline__ Global<V> *global_ptr(uint32_t low, uint32_t high) {
+    return (Global<V> *)(((uint64_t)high << 32) | low);
+}
 
 struct BF16 {};  // tag types: the 16-bit storage format of activations
 struct FP16 {};

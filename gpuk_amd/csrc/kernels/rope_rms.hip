@@ -31,9 +31,6 @@ namespace gpuk {
 
 namespace {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
 constexpr float kE4M3Max = 448.0f;
 
 struct RopeArgs {
@@ -58,12 +55,6 @@ struct RopeArgs {
     uint32_t gate;         // ticks of 10 ns after a wave's entry before which it stores nothing (0 = no gate)
 };
 
-// A pointer read from the argument block by hand is a generic one to the compiler; these say what it points at, so
-// that the accesses through it are global (not flat) ones, and scalar ones where the address is the same in every lane.
-template <typename P>
-__device__ __forceinline__ P *as_global(P *p) {
-    return (P *)(__attribute__((address_space(1))) P *)p;
-}
 template <typename P>
 __device__ __forceinline__ P load_unchanging(const P *p) {  // memory no kernel of the launch writes
     return *(const __attribute__((address_space(4))) P *)p;
@@ -318,6 +309,8 @@ struct RopeUnit {
         if constexpr (AXES == 3) {
             st.p1 = load_unchanging(a.positions + a.ps_axis + (int64_t)st.t * a.ps_token);
             st.p2 = load_unchanging(a.positions + 2 * a.ps_axis + (int64_t)st.t * a.ps_token);
+        } else if constexpr (SETKV) {
+            st.slot = load_unchanging(a.kv_loc + st.t);  // (one axis: kv_loc has the place of the axis stride)
         }
     }
 
@@ -330,7 +323,7 @@ struct RopeUnit {
         const void *qw = a.qw, *kw = a.kw;
         if constexpr (AXES == 3) asm("" : "+s"(qw), "+s"(kw));
         const int sub = lane % LPH;
-        if constexpr (SETKV) st.slot = load_unchanging(a.kv_loc + st.t);
+        if constexpr (SETKV && AXES == 3) st.slot = load_unchanging(a.kv_loc + st.t);
         typedef const __attribute__((address_space(1))) u32x4 *GlobalChunk;
         const uint16_t *wsrc = static_cast<const uint16_t *>(st.is_q ? qw : kw);
         st.wa = *(GlobalChunk)(wsrc + c0(sub));
@@ -440,7 +433,7 @@ struct RopeUnit {
             // V: copied (16-bit cache) or quantised (fp8 cache), chunk by chunk
             const int v_chunks = a.hv * (D / 8), v_first = st.u * 64 + lane;
             const int stride = a.units_per_token * 64;
-            const float s = a.v_scale, rcp = 1.0f / s;
+            const float s = KVFP8 ? a.v_scale : 1.0f, rcp = 1.0f / s;
             const bool fast = scale_is_fast(s);
             u32x4 vchunk = st.vchunk;
             for (int c = v_first; slot_ok && c < v_chunks; c += stride) {
@@ -458,46 +451,67 @@ struct RopeUnit {
     }
 };
 
-// What a wave needs to ask for its activations and its position(s) comes as 14 dwords of leading scalar parameters,
+// What a wave needs to ask for its activations and its position(s) comes as 14 dwords of leading parameters,
 // which are handed to the wave in scalar registers at launch (-amdgpu-kernarg-preload-count=14): those requests
 // leave without a round trip for the argument block, which under load costs a wave of this kernel a third of its
-// life; the block (weights, table, outputs, slots) is fetched beside the position, and everything that depends on
-// either is asked for one round trip after entry.  hv_and_waves: hv in bits 0-23, log2 of the waves per workgroup above.
-// (The three-axis instantiations take 66 registers per lane, one wave short of the eight a SIMD can hold; held to 64
-// with amdgpu_waves_per_eu they fit without spilling and run 1-4 % slower: 26.9 against 26.6 us at 8192 tokens of
-// 28+4+4 heads, 51.3 against 49.1 at 16384.)
-// The leading parameters of the kernel below as the argument segment lays them out; the block follows them.
-struct UnitKernelLead {
-    const void *qkv_in;
-    const int64_t *positions;
-    uint32_t total_units, units_per_token, upt_magic;
-    int hq, hk;
-    uint32_t hv_and_waves;
-    int64_t ps_token, ps_axis;
+// life; the block (weights, table, outputs) is fetched beside the position, and everything that depends on
+// either is asked for one round trip after entry.  The leading parameters are three vectors, and the block holds what the
+// instantiation reads and nothing else: 88 to 112 bytes in all with one axis or in place, 112 to 136 (128 elements per head)
+// with three axes and a cache, because the launch of a small call costs the host by both (see launch_kernel; a call of the
+// operator for 32 tokens of 64+8+8 heads into an fp8 cache 6.00 us with 10 scalars and a block of 184 bytes, 5.50 so).
+//   first:  qkv_in, positions, total_units, upt_magic, hq, hk
+//   second: hv_and_flags, eps, ps_token
+//   third:  ps_axis with three axes, else kv_loc with a cache
+// hv_and_flags: hv in bits 0-23, log2 of the waves per workgroup in bits 24-25, stream_rows in bit 26, merge_rows in bit 27.
+// (The three-axis instantiations of 128 elements per head with a cache are held to 64 registers, eight waves per SIMD: the
+// scheduler otherwise groups the mask operations of the three-row merge and takes 66; held, they take 55 to 57.)
+constexpr size_t kUnitLeadBytes = sizeof(u32x8) + sizeof(u32x4) + sizeof(u32x2);
+template <int D, int AXES, bool SETKV, bool KVFP8, bool GATED>
+struct UnitBlock {  // the argument block, behind the leading parameters
+    static constexpr int MAP_WORDS = AXES == 3 ? (D / 2 + 31) / 32 : 0, SCALES = KVFP8 ? 2 : 0, GATE = GATED ? 1 : 0;
+    static constexpr int POINTERS = 3 + (SETKV ? 3 : 0) + (SETKV && AXES == 3 ? 1 : 0), WORDS = 2 * MAP_WORDS + SCALES + GATE;
+    const void *pointers[POINTERS];            // qw, kw, cos_sin; with a cache q_out, k_cache, v_cache; with three axes kv_loc as well
+    uint32_t words[WORDS > 0 ? WORDS : 1];     // axis1, axis2; k_scale, v_scale; gate
+
+    explicit UnitBlock(const RopeArgs &a) : pointers{}, words{} {
+        int n = 0;
+        pointers[n++] = a.qw, pointers[n++] = a.kw, pointers[n++] = a.cos_sin;
+        if constexpr (SETKV) pointers[n++] = a.q_out, pointers[n++] = a.k_cache, pointers[n++] = a.v_cache;
+        if constexpr (SETKV && AXES == 3) pointers[n++] = a.kv_loc;
+        for (int i = 0; i < MAP_WORDS; ++i) words[i] = a.axis1[i], words[MAP_WORDS + i] = a.axis2[i];
+        if constexpr (KVFP8) words[2 * MAP_WORDS] = __builtin_bit_cast(uint32_t, a.k_scale), words[2 * MAP_WORDS + 1] = __builtin_bit_cast(uint32_t, a.v_scale);
+        if constexpr (GATED) words[2 * MAP_WORDS + SCALES] = a.gate;
+    }
 };
-static_assert(sizeof(UnitKernelLead) == 56 && sizeof(UnitKernelLead) % alignof(RopeArgs) == 0, "offset of the block");
 
 template <typename T, int D, bool NEOX, int AXES, bool SETKV, bool KVFP8, bool GATED, bool WHOLE>
-__global__ void __launch_bounds__(512)
-rope_rms_kernel(const void *qkv_in, const int64_t *positions, uint32_t total_units, uint32_t units_per_token,
-                uint32_t upt_magic, int hq, int hk, uint32_t hv_and_waves, int64_t ps_token, int64_t ps_axis,
-                const RopeArgs rest) {
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(AXES == 3 && D == 128 ? 8 : 1)))
+rope_rms_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const UnitBlock<D, AXES, SETKV, KVFP8, GATED> rest) {
     using Unit = RopeUnit<T, D, NEOX, AXES, SETKV, KVFP8>;
+    using Block = UnitBlock<D, AXES, SETKV, KVFP8, GATED>;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t unit = (blockIdx.x << (hv_and_waves >> 24)) + wave;
+    const uint32_t total_units = first[4], hv_and_flags = second[0];
+    const uint32_t unit = (blockIdx.x << ((hv_and_flags >> 24) & 3u)) + wave;
     if (unit >= total_units) return;
     const uint64_t entry = GATED ? __builtin_amdgcn_s_memrealtime() : 0;
     RopeArgs a;
-    a.qkv_in = qkv_in;
-    a.positions = positions;
+    a.qkv_in = (const void *)global_ptr<const char>(first[0], first[1]);
+    a.positions = (const int64_t *)global_ptr<const int64_t>(first[2], first[3]);
     a.total_units = total_units;
-    a.units_per_token = units_per_token;
-    a.upt_magic = upt_magic;
-    a.hq = hq;
-    a.hk = hk;
-    a.hv = (int)(hv_and_waves & 0xffffffu);
-    a.ps_token = ps_token;
-    a.ps_axis = ps_axis;
+    a.upt_magic = first[5];
+    a.hq = (int)first[6];
+    a.hk = (int)first[7];
+    a.units_per_token = (uint32_t)(a.hq + a.hk + Unit::HPW - 1) / Unit::HPW;
+    a.hv = (int)(hv_and_flags & 0xffffffu);
+    a.stream_rows = (hv_and_flags >> 26) & 1u;
+    a.merge_rows = (hv_and_flags >> 27) & 1u;
+    const uint32_t eps_bits = second[1];  // (a bit cast of the vector's element itself takes the first one)
+    a.eps = __builtin_bit_cast(float, eps_bits);
+    a.ps_token = (int64_t)(((uint64_t)second[3] << 32) | second[2]);
+    const uint64_t third64 = ((uint64_t)third[1] << 32) | third[0];
+    a.ps_axis = AXES == 3 ? (int64_t)third64 : 0;
+    a.kv_loc = AXES == 3 ? nullptr : (const int64_t *)global_ptr<const int64_t>(third[0], third[1]);
+    if constexpr (!SETKV) a.qkv_out = const_cast<void *>(a.qkv_in);  // (in place)
     GPUK_STAMPS_BEGIN();  // profiling build only
     const int lane = threadIdx.x & 63;
     UnitState st;
@@ -506,35 +520,37 @@ rope_rms_kernel(const void *qkv_in, const int64_t *positions, uint32_t total_uni
     // the compiler the fetch is the kernel's first instruction, and the first vector load then waits for it: in one
     // instantiation for a register the fetch is about to overwrite, in another for the pinned weight pointers.)
     // (`rest` is read through the argument segment's own address: taking the parameter's address would have the
-    // whole block copied to the stack.  It follows the 14 leading dwords.)
-    typedef const __attribute__((address_space(4))) RopeArgs *BlockPtr;
-    BlockPtr block = (BlockPtr)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() +
-                                sizeof(UnitKernelLead));
+    // whole block copied to the stack.  It follows the leading parameters.)
+    static_assert(kUnitLeadBytes % alignof(Block) == 0, "offset of the block");
+    typedef const __attribute__((address_space(4))) Block *BlockPtr;
+    BlockPtr block = (BlockPtr)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + kUnitLeadBytes);
     asm volatile("" : "+s"(block));
-    a.kv_loc = as_global(block->kv_loc);
-    a.qkv_out = as_global(block->qkv_out);
-    a.qw = as_global(block->qw);
-    a.kw = as_global(block->kw);
-    a.cos_sin = as_global(block->cos_sin);
-    a.q_out = as_global(block->q_out);
-    a.k_cache = as_global(block->k_cache);
-    a.v_cache = as_global(block->v_cache);
-    a.eps = block->eps;
-    a.k_scale = block->k_scale;
-    a.v_scale = block->v_scale;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        a.axis1[i] = block->axis1[i];
-        a.axis2[i] = block->axis2[i];
+    a.qw = as_global(block->pointers[0]);
+    a.kw = as_global(block->pointers[1]);
+    a.cos_sin = as_global(block->pointers[2]);
+    if constexpr (SETKV) {
+        a.q_out = const_cast<void *>(as_global(block->pointers[3]));
+        a.k_cache = const_cast<void *>(as_global(block->pointers[4]));
+        a.v_cache = const_cast<void *>(as_global(block->pointers[5]));
+        if constexpr (AXES == 3) a.kv_loc = static_cast<const int64_t *>(as_global(block->pointers[6]));
     }
-    a.stream_rows = block->stream_rows;
-    a.merge_rows = block->merge_rows;
-    a.gate = block->gate;
+#pragma unroll
+    for (int i = 0; i < Block::MAP_WORDS; ++i) {
+        a.axis1[i] = block->words[i];
+        a.axis2[i] = block->words[Block::MAP_WORDS + i];
+    }
+    if constexpr (KVFP8) {
+        a.k_scale = __builtin_bit_cast(float, block->words[2 * Block::MAP_WORDS]);
+        a.v_scale = __builtin_bit_cast(float, block->words[2 * Block::MAP_WORDS + 1]);
+    }
+    if constexpr (GATED) a.gate = block->words[2 * Block::MAP_WORDS + Block::SCALES];
     // ... all of it in one go (the compiler otherwise fetches each field where it is first used, the output pointers
     // after the arithmetic, and the wave waits for the scalar cache once more before it can store)
-    asm volatile("" ::"s"(a.kv_loc), "s"(a.qkv_out), "s"(a.qw), "s"(a.kw), "s"(a.cos_sin), "s"(a.q_out), "s"(a.k_cache),
-                 "s"(a.v_cache), "s"(a.eps), "s"(a.k_scale), "s"(a.v_scale), "s"(a.stream_rows), "s"(a.merge_rows),
-                 "s"(a.gate));
+    asm volatile("" ::"s"(a.qw), "s"(a.kw), "s"(a.cos_sin));
+    if constexpr (SETKV) asm volatile("" ::"s"(a.q_out), "s"(a.k_cache), "s"(a.v_cache));
+    if constexpr (SETKV && AXES == 3) asm volatile("" ::"s"(a.kv_loc));
+    if constexpr (KVFP8) asm volatile("" ::"s"(a.k_scale), "s"(a.v_scale));
+    if constexpr (GATED) asm volatile("" ::"s"(a.gate));
     Unit::issue_late_loads(a, lane, st);
     GPUK_STAMP(1);  // activations, weights, position and slot requested
     Unit::issue_table_loads(a, lane, st);
@@ -1036,23 +1052,29 @@ struct TwoWayArgs {
     uint32_t stream;  // 1: the output rows are stored past the L2 (calls that move more than a few MB)
 };
 
-// The leading parameters of the kernel below as the argument segment lays them out; the block follows them.
-struct TwoWayKernelLead {
-    const void *q0, *k0, *q1, *k1;
-    uint32_t tokens0, tokens1, heads_q, heads_k, stream;
-    uint32_t pad_;
+// As in rope_rms_kernel, what a wave needs to find and request its activations are leading parameters that arrive in scalar
+// registers at launch; segment bounds and row counts are products and sums of those, not loads.  (With everything in the
+// argument block and the per-segment values picked by index, a wave went through five dependent fetches of the block
+// before its first request.)  The block (weights, tables, outputs, the division constants) is fetched behind the
+// activations, in one batch.  128 bytes in all (see launch_kernel; a small call of the operator 7.70 / 7.27 us with nine scalars
+// and a block of 160 bytes / so).
+//   first:  q0, k0, q1, k1      second: tokens0, tokens1, heads_q, heads_k      third: eps, stream
+struct TwoWayBlock {
+    const void *w[4], *cos_sin[2];
+    void *out[2];
+    uint32_t heads_magic[2];
 };
-static_assert(sizeof(TwoWayKernelLead) == 56 && sizeof(TwoWayKernelLead) % alignof(TwoWayArgs) == 0, "offset of the block");
+constexpr size_t kTwoWayLeadBytes = sizeof(u32x8) + sizeof(u32x4) + sizeof(u32x2);
+static_assert(kTwoWayLeadBytes % alignof(TwoWayBlock) == 0, "offset of the block");
 
-// As in rope_rms_kernel, what a wave needs to find and request its activations -- the four input pointers, the token
-// and head counts -- are leading scalar parameters that arrive in scalar registers at launch; segment bounds and
-// row counts are products and sums of those, not loads.  (With everything in the argument block and the per-segment
-// values picked by index, a wave went through five dependent fetches of the block before its first request.)  The
-// block (weights, tables, outputs, the division constants) is fetched behind the activations, in one batch.
 template <typename T, int D, bool NEOX, bool WHOLE>
 __global__ void __launch_bounds__(256)
-rope_rms_2way_kernel(const void *q0, const void *k0, const void *q1, const void *k1, uint32_t tokens0, uint32_t tokens1,
-                     uint32_t heads_q, uint32_t heads_k, uint32_t stream, const TwoWayArgs rest) {
+rope_rms_2way_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const TwoWayBlock rest) {
+    const uint32_t tokens0 = second[0], tokens1 = second[1], heads_q = second[2], heads_k = second[3];
+    const uint32_t eps_bits = third[0], stream = third[1];
+    const float eps = __builtin_bit_cast(float, eps_bits);
+    const void *q0 = (const void *)global_ptr<const char>(first[0], first[1]), *k0 = (const void *)global_ptr<const char>(first[2], first[3]);
+    const void *q1 = (const void *)global_ptr<const char>(first[4], first[5]), *k1 = (const void *)global_ptr<const char>(first[6], first[7]);
     constexpr int LPH = D / 16, HPW = 64 / LPH, HALF = D / 2;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t unit = blockIdx.x * 4 + wave;
@@ -1084,17 +1106,14 @@ rope_rms_2way_kernel(const void *q0, const void *k0, const void *q1, const void 
     u32x4 xa = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_a));
     u32x4 xb = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_b));
 
-    typedef const __attribute__((address_space(4))) TwoWayArgs *BlockPtr;
-    BlockPtr block = (BlockPtr)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() +
-                                sizeof(TwoWayKernelLead));
+    typedef const __attribute__((address_space(4))) TwoWayBlock *BlockPtr;
+    BlockPtr block = (BlockPtr)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + kTwoWayLeadBytes);
     asm volatile("" : "+s"(block));
     const void *w0 = as_global(block->w[0]), *w1 = as_global(block->w[1]), *w2 = as_global(block->w[2]), *w3 = as_global(block->w[3]);
     const void *table0 = as_global(block->cos_sin[0]), *table1 = as_global(block->cos_sin[1]);
     void *out_q = as_global(block->out[0]), *out_k = as_global(block->out[1]);
     const uint32_t magic_q = block->heads_magic[0], magic_k = block->heads_magic[1];
-    const float eps = block->eps;
-    asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(w3), "s"(table0), "s"(table1), "s"(out_q), "s"(out_k), "s"(magic_q),
-                 "s"(magic_k), "s"(eps));
+    asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(w3), "s"(table0), "s"(table1), "s"(out_q), "s"(out_k), "s"(magic_q), "s"(magic_k));
     const uint32_t magic = kind ? magic_k : magic_q;
     const uint32_t token = magic ? __umulhi(row, magic) : row;
     const uint16_t *wsrc = static_cast<const uint16_t *>(seg == 0 ? w0 : seg == 1 ? w1 : seg == 2 ? w2 : w3);
@@ -1183,9 +1202,12 @@ constexpr int64_t kWholeLinesFromBytes = 13'500'000, kWholeLinesFromBytesRagged 
 template <typename T, int D>
 int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stream) {
     const dim3 grid((a.unit_end[3] + 3) / 4, batch);
+    const u32x8 first = {low_half(a.in[0]), high_half(a.in[0]), low_half(a.in[1]), high_half(a.in[1]), low_half(a.in[2]), high_half(a.in[2]), low_half(a.in[3]), high_half(a.in[3])};
+    const u32x4 second = {(uint32_t)a.tokens0, (uint32_t)a.tokens1, a.heads[0], a.heads[1]};
+    const u32x2 third = {__builtin_bit_cast(uint32_t, a.eps), a.stream};
+    const TwoWayBlock rest = {{a.w[0], a.w[1], a.w[2], a.w[3]}, {a.cos_sin[0], a.cos_sin[1]}, {a.out[0], a.out[1]}, {a.heads_magic[0], a.heads_magic[1]}};
 #define GPUK_LAUNCH_2WAY(NEOX, WHOLE)                                                                                  \
-    rope_rms_2way_kernel<T, D, NEOX, WHOLE><<<grid, 256, 0, stream>>>(a.in[0], a.in[1], a.in[2], a.in[3], (uint32_t)a.tokens0,  \
-                                                               (uint32_t)a.tokens1, a.heads[0], a.heads[1], a.stream, a)
+    return launch_kernel(rope_rms_2way_kernel<T, D, NEOX, WHOLE>, grid, 256, 0, stream, first, second, third, rest)
     constexpr bool kHalfLines = D == 64;  // see exchange_lines
     const int64_t call_bytes = 4 * (int64_t)batch * ((int64_t)a.rows[0] + a.rows[1] + a.rows[2] + a.rows[3]) * D;
     const bool whole = a.stream && (is_half<T> || g_stream_rows == 2 || call_bytes >= kWholeLinesFromBytes);
@@ -1194,7 +1216,6 @@ int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stre
     else if (neox) GPUK_LAUNCH_2WAY(true, false);
     else GPUK_LAUNCH_2WAY(false, false);
 #undef GPUK_LAUNCH_2WAY
-    return hip_status(hipGetLastError());
 }
 
 template <typename F, int D>
@@ -1373,17 +1394,20 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
     }
     const uint32_t log2_waves = p.threads == 64 ? 0u : p.threads == 128 ? 1u : p.threads == 256 ? 2u : 3u;
     constexpr bool kHalfLines = D == 64 && !SETKV;  // see exchange_lines
+    const void *third = a.kv_loc;  // (see rope_rms_kernel)
+    if constexpr (AXES == 3) third = reinterpret_cast<const void *>((intptr_t)a.ps_axis);
+    const u32x8 lead1 = {low_half(a.qkv_in), high_half(a.qkv_in), low_half(a.positions), high_half(a.positions), a.total_units, a.upt_magic, (uint32_t)a.hq, (uint32_t)a.hk};
+    const u32x4 lead2 = {(uint32_t)a.hv | (log2_waves << 24) | (b.stream_rows << 26) | (a.merge_rows << 27), __builtin_bit_cast(uint32_t, a.eps), (uint32_t)a.ps_token, (uint32_t)((uint64_t)a.ps_token >> 32)};
+    const u32x2 lead3 = {low_half(third), high_half(third)};
 #define GPUK_LAUNCH_UNITS(GATED, WHOLE)                                                                                 \
-    rope_rms_kernel<T, D, NEOX, AXES, SETKV, KVFP8, GATED, WHOLE><<<p.blocks, p.threads, 0, stream>>>(                         \
-        a.qkv_in, a.positions, a.total_units, a.units_per_token, a.upt_magic, a.hq, a.hk,                               \
-        (uint32_t)a.hv | (log2_waves << 24), a.ps_token, a.ps_axis, b)
+    return launch_kernel(rope_rms_kernel<T, D, NEOX, AXES, SETKV, KVFP8, GATED, WHOLE>, dim3(p.blocks), p.threads, 0, stream, lead1, lead2, lead3, \
+                         UnitBlock<D, AXES, SETKV, KVFP8, GATED>(b))
     const bool whole = p.stream && (is_half<T> || p.whole_lines);
     if (kHalfLines && whole && b.gate) GPUK_LAUNCH_UNITS(true, kHalfLines);
     else if (kHalfLines && whole) GPUK_LAUNCH_UNITS(false, kHalfLines);
     else if (b.gate) GPUK_LAUNCH_UNITS(true, false);
     else GPUK_LAUNCH_UNITS(false, false);
 #undef GPUK_LAUNCH_UNITS
-    return hip_status(hipGetLastError());
 }
 
 template <typename T, int D, bool NEOX, int AXES>

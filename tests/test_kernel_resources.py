@@ -50,3 +50,21 @@ def test_no_scratch_where_rows_stay_in_registers():
     spilled = {n: found[n][".private_segment_fixed_size"] for n in bounded}
     spilled = {n: b for n, b in spilled.items() if b > (24 if in_place_two.search(n) else 0)}
     assert not spilled, spilled
+
+
+def test_small_calls_pass_few_arguments():
+    """The kernels that small calls launch take at most four parameters, and at most 112 bytes of them (128 and 136 with
+    three position axes and a cache, or two token streams): what a launch costs the host goes by both."""
+    found = {k[".name"]: k for elf in code_objects(open(LIB, "rb").read()) for k in kernels(elf)}
+    seen = 0
+    for name, k in found.items():
+        if not re.search(r"add_rmsnorm_quant_(f32_)?rowsI|rope_rms_kernelI|rope_rms_2way_kernelI", name):
+            continue
+        seen += 1
+        assert len([a for a in k[".args"] if not a[".value_kind"].startswith("hidden")]) <= 4, name
+        head = re.search(r"rope_rms_kernelINS_4[BF][FP]16ELi(64|128|256)ELb[01]ELi([13])ELb([01])ELb([01])ELb([01])E", name)
+        most = 128 if "2way" in name else 112
+        if head:   # (the gate of launches that fill half the chip comes on top)
+            most += 8 * int(head[5]) + (8 * int(head[4]) + {64: 8, 128: 16, 256: 32}[int(head[1])] if head[2] == "3" else 0)
+        assert k[".kernarg_segment_size"] <= most, (name, k[".kernarg_segment_size"])
+    assert seen > 250
