@@ -13,7 +13,9 @@ import raises.
 """
 from __future__ import annotations
 
+import importlib.util
 import os
+import types
 from contextlib import contextmanager
 from typing import Optional
 
@@ -23,25 +25,47 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(_PKG_DIR, "lib")
 KERNEL_LIB = os.path.join(LIB_DIR, "libgpuk_amd.so")   # C ABI, include/gpuk_amd.h
 TORCH_LIB = os.path.join(LIB_DIR, "libgpuk.so")        # TORCH_LIBRARY(gpuk, ...)
+DIRECT_LIB = os.path.join(LIB_DIR, "gpuk_direct.so")   # direct calls of its operators, csrc/direct_calls.cpp
 
-if not (os.path.exists(KERNEL_LIB) and os.path.exists(TORCH_LIB)):
+if not all(map(os.path.exists, (KERNEL_LIB, TORCH_LIB, DIRECT_LIB))):
     raise ImportError(
-        f"gpuk_amd: {KERNEL_LIB} / {TORCH_LIB} not built; run `python -m gpuk_amd.build` "
+        f"gpuk_amd: {KERNEL_LIB} / {TORCH_LIB} / {DIRECT_LIB} not built; run `python -m gpuk_amd.build` "
         "(hipcc cross-compiles gfx950 without a GPU). There is no fallback path.")
 
 torch.ops.load_library(TORCH_LIB)
+_spec = importlib.util.spec_from_file_location("gpuk_direct", DIRECT_LIB)
+_direct = importlib.util.module_from_spec(_spec)
+_spec.loader.exec_module(_direct)
 
-allreduce_rms = torch.ops.gpuk.allreduce_rms
-fused_rope_rms = torch.ops.gpuk.fused_rope_rms
-fused_mrope_3d_rms = torch.ops.gpuk.fused_mrope_3d_rms
-fused_mrope_3d_rms_set_kv = torch.ops.gpuk.fused_mrope_3d_rms_set_kv
-fused_rope_rms_2way = torch.ops.gpuk.fused_rope_rms_2way
-fused_rope_rms_set_kv = torch.ops.gpuk.fused_rope_rms_set_kv       # additive: 1-D positions + KV write
+
+def _called_directly(packet):
+    """`packet`, the object that torch.ops.gpuk holds, with a class of its own in which a plain call skips the
+    interpretation of the schema (csrc/direct_calls.cpp); every other call, and everything else about it, is as before."""
+    base = type(packet)
+    call = _direct.direct(packet.__name__, "", types.MethodType(base.__call__, packet))
+    packet.__class__ = type(base.__name__, (base,), {"__call__": call, "__module__": base.__module__, "__doc__": base.__doc__})
+    return packet
+
+
+allreduce_rms = _called_directly(torch.ops.gpuk.allreduce_rms)
+fused_rope_rms = _called_directly(torch.ops.gpuk.fused_rope_rms)
+fused_mrope_3d_rms = _called_directly(torch.ops.gpuk.fused_mrope_3d_rms)
+fused_mrope_3d_rms_set_kv = _called_directly(torch.ops.gpuk.fused_mrope_3d_rms_set_kv)
+fused_rope_rms_2way = _called_directly(torch.ops.gpuk.fused_rope_rms_2way)
+fused_rope_rms_set_kv = _called_directly(torch.ops.gpuk.fused_rope_rms_set_kv)       # additive: 1-D positions + KV write
 set_fp8_max = torch.ops.gpuk.set_fp8_max                           # additive
 get_fp8_max = torch.ops.gpuk.get_fp8_max                           # additive
 
 _add_rms_fused = torch.ops.gpuk.add_rms_fused.default
-_add_rms_fused_static = torch.ops.gpuk.add_rms_fused.static
+
+
+def _add_rms_fused_static(x, residual, gamma, eps, static_scale):
+    residual_out, norm_out = torch.ops.gpuk.add_rms_fused.static(x, residual, gamma, eps, static_scale)
+    return residual_out, norm_out, static_scale.reshape(1)
+
+
+_add_rms_fused_direct = _direct.direct("add_rms_fused", "", _add_rms_fused)
+_add_rms_fused_static_direct = _direct.direct("add_rms_fused", "static", _add_rms_fused_static)
 
 
 class _Traceable:
@@ -164,8 +188,10 @@ class GPUKDistEnv:
         quantisation.
         """
         self.capture_(allreduce_in)
-        if fp8_out and static_scale is not None:
-            residual_out, norm_out = _add_rms_fused_static(allreduce_in, residual_in, rms_weight, eps, static_scale)
-            return residual_out, norm_out, static_scale.reshape(1)
         # functional schema, outputs allocated in the operator: the call survives tracing
-        return _add_rms_fused(allreduce_in, residual_in, rms_weight, eps, fp8_policy_id if fp8_out else QUANT_NONE)
+        tracing = torch.compiler.is_compiling()
+        if fp8_out and static_scale is not None:
+            op = _add_rms_fused_static if tracing else _add_rms_fused_static_direct
+            return op(allreduce_in, residual_in, rms_weight, eps, static_scale)
+        op = _add_rms_fused if tracing else _add_rms_fused_direct
+        return op(allreduce_in, residual_in, rms_weight, eps, fp8_policy_id if fp8_out else QUANT_NONE)

@@ -2,6 +2,7 @@
 
   gpuk_amd/lib/libgpuk_amd.so : HIP kernels for gfx950 behind the C ABI of include/gpuk_amd.h (no torch)
   gpuk_amd/lib/libgpuk.so     : torch library `gpuk` (csrc/register.cpp + csrc/ops/*.cpp), links the former
+  gpuk_amd/lib/gpuk_direct.so : Python functions that call the operators of libgpuk.so without interpreting their schemas
   gpuk_amd/lib/libgpuk_amd_stamps.so : the first, compiled with -DGPUK_STAMPS: a profiling build whose kernels
                                 record the shader clock at named phases (`python -m gpuk_amd.stamps`); `--stamps`
                                 builds only this one
@@ -15,6 +16,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -97,6 +99,11 @@ def build_torch_library(jobs: int = 4) -> str:
     _run([HIPCC, "-shared", "-fPIC", "-o", out] + objs +
          ["-L" + LIB, "-lgpuk_amd", "-L" + torch_lib, "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
           "-Wl,-rpath,$ORIGIN", "-Wl,--no-as-needed"])
+    direct = os.path.join(LIB, "gpuk_direct.so")
+    obj = _compile(("direct_calls.cpp", os.path.join(OBJ, "torch_direct_calls.cpp.o"),
+                    ["-x", "c++"] + flags + ["-isystem", sysconfig.get_paths()["include"]]))
+    _run([HIPCC, "-shared", "-fPIC", "-o", direct, obj, "-L" + LIB, "-lgpuk", "-L" + torch_lib, "-ltorch_python", "-ltorch",
+          "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"])
     return out
 
 
