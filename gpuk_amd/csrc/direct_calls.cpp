@@ -1,9 +1,10 @@
 // Python entry points of the operators that skip the interpretation of their schemas.
 //
 // torch.ops.gpuk.<op>(...) finds the overload, matches every Python argument against the schema and boxes it, which takes
-// longer than everything else the host does for a small call but the launch: of 4.8 us for allreduce_rms of one row (nine
-// arguments) 1.2, of 5.5 us for fused_rope_rms_set_kv of 32 tokens (eighteen) 1.8; what the operator itself does
-// beside the launch is 0.2.  The functions here take the same positional arguments, unpack them by the type the operator's
+// longer than everything else the host does for a small call but the launch: us per call that way / this way 4.79 / 3.42 for
+// allreduce_rms of one row (nine arguments), 5.50 / 3.66 for fused_rope_rms_set_kv of 32 tokens (eighteen), of which the
+// launch is 2.8 and what the operator itself does beside it 0.2.  The functions here take the same positional arguments,
+// unpack them by the type the operator's
 // C++ signature names and call the operator through the dispatcher, so that profiling, dispatch modes, functorch
 // and the keys other code registers see the call as before.  Whatever is not plain -- keywords, another number of arguments, tensor
 // subclasses, symbolic or other numbers, a __torch_function__ mode, a trace being recorded -- goes to the callable that the

@@ -92,7 +92,8 @@ void check_static_scale(const Tensor &static_scale, const Tensor &allreduce_in) 
 }  // namespace
 
 // Outputs allocated here, behind one pass through the dispatcher: allocated from Python, one call each, the three cost
-// a decode step more than its kernel takes (9.5 us per call of one 7168-element row, 7.3 in this form; the kernel 3.3).
+// a decode step more than its kernel takes (9.5 us per call of one 7168-element row, 7.3 in this form, each called through
+// torch.ops; the kernel 3.3).
 std::tuple<Tensor, Tensor, Tensor> add_rms_fused(const Tensor &allreduce_in, const Tensor &residual_in, const Tensor &rms_gamma,
                                                  double eps, int64_t quant_type) {
     check_functional_quant_type(quant_type);
