@@ -54,6 +54,7 @@ struct RopeArgs {
     uint32_t merge_rows;   // mRoPE: every aligned group of 8 frequencies takes one axis: each lane loads from that axis's row
     uint32_t gate;         // ticks of 10 ns after a wave's entry before which it stores nothing (0 = no gate)
 };
+static_assert(sizeof(RopeArgs) % 8 == 0 && alignof(RopeArgs) == 8, "offset of the block behind the leading parameters");
 
 template <typename P>
 __device__ __forceinline__ P load_unchanging(const P *p) {  // memory no kernel of the launch writes
@@ -113,6 +114,54 @@ __device__ __forceinline__ uint32_t trig_bits(const uint32_t (&bitmap)[4], int s
     } else {
         const int f0 = 4 * sub, f1 = D / 4 + 4 * sub;
         return ((bitmap_word<D>(bitmap, f0) >> (f0 & 31)) & 0xfu) | (((bitmap_word<D>(bitmap, f1) >> (f1 & 31)) & 0xfu) << 4);
+    }
+}
+
+// cos and sin pieces of a lane for a token at positions (p0, p1, p2), sections in which every aligned group of 8
+// frequencies takes one axis: each lane reads its pieces from that axis's row.
+template <int D, bool NEOX>
+__device__ __forceinline__ void load_trig_by_axis(const uint16_t *table, int64_t p0, int64_t p1, int64_t p2,
+                                                  const uint32_t (&axis1)[4], const uint32_t (&axis2)[4], int sub,
+                                                  u32x4 &cosv, u32x4 &sinv) {
+    constexpr int HALF = D / 2;
+    const uint32_t b1 = trig_bits<D, NEOX>(axis1, sub), b2 = trig_bits<D, NEOX>(axis2, sub);
+    const int64_t pa = (b2 & 1u) ? p2 : ((b1 & 1u) ? p1 : p0);
+    if constexpr (NEOX) {
+        cosv = load_trig<D, NEOX>(table + pa * D, sub);
+        sinv = load_trig<D, NEOX>(table + pa * D + HALF, sub);
+    } else {
+        const int64_t pb = (b2 & 16u) ? p2 : ((b1 & 16u) ? p1 : p0);
+        const u32x2 cl = *reinterpret_cast<const u32x2 *>(table + pa * D + 4 * sub);
+        const u32x2 ch = *reinterpret_cast<const u32x2 *>(table + pb * D + D / 4 + 4 * sub);
+        const u32x2 sl = *reinterpret_cast<const u32x2 *>(table + pa * D + HALF + 4 * sub);
+        const u32x2 sh = *reinterpret_cast<const u32x2 *>(table + pb * D + HALF + D / 4 + 4 * sub);
+        cosv = u32x4{cl[0], cl[1], ch[0], ch[1]};
+        sinv = u32x4{sl[0], sl[1], sh[0], sh[1]};
+    }
+}
+// ... and for any sections: one axis, or the three rows merged
+template <int D, bool NEOX, int AXES>
+__device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t p0, int64_t p1, int64_t p2,
+                                                 const uint32_t (&axis1)[4], const uint32_t (&axis2)[4], int sub,
+                                                 u32x4 &cosv, u32x4 &sinv) {
+    constexpr int HALF = D / 2;
+    cosv = load_trig<D, NEOX>(table + p0 * D, sub);
+    sinv = load_trig<D, NEOX>(table + p0 * D + HALF, sub);
+    if constexpr (AXES == 3) {
+        if (p1 != p0 || p2 != p0) {  // wave-uniform; text tokens carry three equal positions
+            const u32x4 cos1 = load_trig<D, NEOX>(table + p1 * D, sub);
+            const u32x4 sin1 = load_trig<D, NEOX>(table + p1 * D + HALF, sub);
+            const u32x4 cos2 = load_trig<D, NEOX>(table + p2 * D, sub);
+            const u32x4 sin2 = load_trig<D, NEOX>(table + p2 * D + HALF, sub);
+            // the axis bits of the lane's 8 frequencies, in the order of the loaded values
+            const uint32_t b1 = trig_bits<D, NEOX>(axis1, sub), b2 = trig_bits<D, NEOX>(axis2, sub);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t m1 = halves_mask(b1 >> (2 * j)), m2 = halves_mask(b2 >> (2 * j));
+                cosv[j] = bitselect(m2, cos2[j], bitselect(m1, cos1[j], cosv[j]));
+                sinv[j] = bitselect(m2, sin2[j], bitselect(m1, sin1[j], sinv[j]));
+            }
+        }
     }
 }
 
@@ -334,47 +383,13 @@ struct RopeUnit {
     static __device__ __forceinline__ void issue_table_loads(const RopeArgs &a, int lane, UnitState &st) {
         const int sub = lane % LPH;
         const uint16_t *table = static_cast<const uint16_t *>(a.cos_sin);
-        const int64_t p0 = st.p0;
         if constexpr (AXES == 3) {
-            const int64_t p1 = st.p1, p2 = st.p2;
-            if (a.merge_rows && (p1 != p0 || p2 != p0)) {
-                // every aligned group of 8 frequencies takes one axis: each lane reads its pieces from that axis's row
-                const uint32_t b1 = trig_bits<D, NEOX>(a.axis1, sub), b2 = trig_bits<D, NEOX>(a.axis2, sub);
-                const int64_t pa = (b2 & 1u) ? p2 : ((b1 & 1u) ? p1 : p0);
-                if constexpr (NEOX) {
-                    st.cosv = load_trig<D, NEOX>(table + pa * D, sub);
-                    st.sinv = load_trig<D, NEOX>(table + pa * D + HALF, sub);
-                } else {
-                    const int64_t pb = (b2 & 16u) ? p2 : ((b1 & 16u) ? p1 : p0);
-                    const u32x2 cl = *reinterpret_cast<const u32x2 *>(table + pa * D + 4 * sub);
-                    const u32x2 ch = *reinterpret_cast<const u32x2 *>(table + pb * D + D / 4 + 4 * sub);
-                    const u32x2 sl = *reinterpret_cast<const u32x2 *>(table + pa * D + HALF + 4 * sub);
-                    const u32x2 sh = *reinterpret_cast<const u32x2 *>(table + pb * D + HALF + D / 4 + 4 * sub);
-                    st.cosv = u32x4{cl[0], cl[1], ch[0], ch[1]};
-                    st.sinv = u32x4{sl[0], sl[1], sh[0], sh[1]};
-                }
+            if (a.merge_rows && (st.p1 != st.p0 || st.p2 != st.p0)) {
+                load_trig_by_axis<D, NEOX>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
                 return;
             }
         }
-        st.cosv = load_trig<D, NEOX>(table + p0 * D, sub);
-        st.sinv = load_trig<D, NEOX>(table + p0 * D + HALF, sub);
-        if constexpr (AXES == 3) {
-            const int64_t p1 = st.p1, p2 = st.p2;
-            if (p1 != p0 || p2 != p0) {  // wave-uniform; text tokens carry three equal positions
-                const u32x4 cos1 = load_trig<D, NEOX>(table + p1 * D, sub);
-                const u32x4 sin1 = load_trig<D, NEOX>(table + p1 * D + HALF, sub);
-                const u32x4 cos2 = load_trig<D, NEOX>(table + p2 * D, sub);
-                const u32x4 sin2 = load_trig<D, NEOX>(table + p2 * D + HALF, sub);
-                // the axis bits of the lane's 8 frequencies, in the order of the loaded values
-                const uint32_t b1 = trig_bits<D, NEOX>(a.axis1, sub), b2 = trig_bits<D, NEOX>(a.axis2, sub);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t m1 = halves_mask(b1 >> (2 * j)), m2 = halves_mask(b2 >> (2 * j));
-                    st.cosv[j] = bitselect(m2, cos2[j], bitselect(m1, cos1[j], st.cosv[j]));
-                    st.sinv[j] = bitselect(m2, sin2[j], bitselect(m1, sin1[j], st.sinv[j]));
-                }
-            }
-        }
+        load_trig_merged<D, NEOX, AXES>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
     }
 
     // Norm, rotation and all stores of the unit.  GATED: no store before a.gate ticks after `entry`, the wave's entry
@@ -568,35 +583,26 @@ rope_rms_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const 
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// One wave per token -- or per two tokens --, for batches that the chip holds in one round (a cache write, up to
+// One wave per token, per part of a token, or per two of those, for batches that the chip holds in one round (up to
 // kTokenWaveCapacity waves).  The memory system serves reads and writes one direction at a time, and a kernel of this
-// size (tens of MB each way, 15-25 us) spends a fifth of its time paying for the mix; here the launch is arranged so
-// that there is hardly any: every wave is resident from the start and asks for everything it will read -- all UPT
-// units of its token, its token's V row, the weights, then the table row -- before it computes anything, the
-// rotated rows replace the activations in the wave's registers, and no store is issued before `gate` ticks (10 ns)
-// after the wave's entry, the time the launch's reads take at the read-only rate (the host computes it from the
-// bytes of the call).  The chip thus reads for the first half of the launch and writes for the second.
-// TWO: the wave takes a second token (the one num_waves further on), whose activations and V row travel from global
-// memory straight into the wave's 9 KB of LDS (global_load_lds_dwordx4: no register is the destination) during the
-// same read phase, and are taken into the first token's registers once that one is stored.  Registers and LDS
-// together hold 8192 tokens of up to 32 Q and K heads and 4 V heads: twice the batch, still one round.
+// size (tens of MB each way, 8-25 us) spends a fifth of its time paying for the mix; here the launch is arranged so
+// that there is hardly any: every wave is resident from the start and asks for everything it will read -- UPT units of its
+// token (an item: the whole token, or one of its `parts` parts of UPT units each), its share of the token's V row, the weights,
+// then the table row -- before it computes anything, the rotated rows replace the activations in the wave's registers, and no
+// store is issued before `gate` ticks (10 ns) after the wave's entry, the time the launch's reads take at the read-only
+// rate (the host computes it from the bytes of the call).  The chip thus reads for the first half of the launch and
+// writes for the second.  A wave holds three to five units where a wave of the kernel above holds one, so four of them per
+// SIMD hold 12288 to 20480 units where eight of those hold 8192; measured sizes in plan_rope.
+// TWO: the wave takes a second item (see there for which), whose activations and V chunks travel from global
+// memory straight into the wave's 7 or 9 KB of LDS (global_load_lds_dwordx4: no register is the destination) during the
+// same read phase, and are taken into the first item's registers once that one is stored.  Registers and LDS
+// together hold 8192 items of up to four units and 64 V chunks: twice the batch, still one round.
 // The arithmetic is norm_rotate's, as in the kernel above.
 constexpr uint32_t kTokenWaveCapacity = 4096;  // 4 waves per SIMD: the 100-odd registers a wave of this kernel takes
 // The gate: 0.97 of the time the launch's reads take at 7 TB/s, the rate of a read-only kernel on this part (4096
 // tokens of 32+8+8 heads: 15.6-15.8 us with 0.95 to 1.0 of that time, 16.0 with 0.9, 17.0 with 0.85, 16.5 with 1.05,
 // 19-20 with no gate at all; the kernel above: 18.2).
 constexpr double kGateBytesPerTick = 70000.0 / 0.97;
-
-// The leading parameters of the kernel below as the argument segment lays them out; the block follows them.
-struct TokenKernelLead {
-    const void *qkv_in;
-    const int64_t *positions;
-    uint32_t num_tokens, gate;
-    int hq, hk, hv;
-    uint32_t num_waves;
-    int64_t ps_token, ps_axis;
-};
-static_assert(sizeof(TokenKernelLead) == 56 && sizeof(TokenKernelLead) % alignof(RopeArgs) == 0, "offset of the block");
 
 // One 16-byte piece per lane from global memory into LDS at lds_byte_offset + 16 * lane; the address is the lane's
 // own.  M0 carries the LDS offset: one wait state after writing it, and it is named as clobbered so that the compiler
@@ -609,34 +615,6 @@ __device__ __forceinline__ void lds_fill16(uint32_t lds_byte_offset, const void 
 }
 #pragma clang diagnostic pop
 
-// cos and sin pieces of a lane for a token at positions (p0, p1, p2): with three axes every aligned group of 8
-// frequencies takes one axis (the host checks the sections), so each lane reads its pieces from that axis's row
-template <int D, bool NEOX, int AXES>
-__device__ __forceinline__ void load_trig_by_axis(const uint16_t *table, int64_t p0, int64_t p1, int64_t p2,
-                                                  const uint32_t (&axis1)[4], const uint32_t (&axis2)[4], int sub,
-                                                  u32x4 &cosv, u32x4 &sinv) {
-    constexpr int HALF = D / 2;
-    if constexpr (AXES == 1) {
-        cosv = load_trig<D, NEOX>(table + p0 * D, sub);
-        sinv = load_trig<D, NEOX>(table + p0 * D + HALF, sub);
-    } else {
-        const uint32_t b1 = trig_bits<D, NEOX>(axis1, sub), b2 = trig_bits<D, NEOX>(axis2, sub);
-        const int64_t pa = (b2 & 1u) ? p2 : ((b1 & 1u) ? p1 : p0);
-        if constexpr (NEOX) {
-            cosv = load_trig<D, NEOX>(table + pa * D, sub);
-            sinv = load_trig<D, NEOX>(table + pa * D + HALF, sub);
-        } else {
-            const int64_t pb = (b2 & 16u) ? p2 : ((b1 & 16u) ? p1 : p0);
-            const u32x2 cl = *reinterpret_cast<const u32x2 *>(table + pa * D + 4 * sub);
-            const u32x2 ch = *reinterpret_cast<const u32x2 *>(table + pb * D + D / 4 + 4 * sub);
-            const u32x2 sl = *reinterpret_cast<const u32x2 *>(table + pa * D + HALF + 4 * sub);
-            const u32x2 sh = *reinterpret_cast<const u32x2 *>(table + pb * D + HALF + D / 4 + 4 * sub);
-            cosv = u32x4{cl[0], cl[1], ch[0], ch[1]};
-            sinv = u32x4{sl[0], sl[1], sh[0], sh[1]};
-        }
-    }
-}
-
 // Norm and rotation of a token's units, in place.  PIN: each unit is finished before the next.  Left to itself the compiler
 // moves half precision's packed sums, the last step of the rotation, of all units behind the last one, where the rows are
 // pinned, and keeps both products of each alive until then: forms of five units spilled 32 to 84 bytes per lane, those of two
@@ -647,18 +625,18 @@ __device__ __forceinline__ void load_trig_by_axis(const uint16_t *table, int64_t
 template <typename T, int D, bool NEOX, int UPT, bool PIN>
 __device__ __forceinline__ void token_rotate(u32x4 (&xa)[UPT], u32x4 (&xb)[UPT], const u32x4 &qwa, const u32x4 &qwb,
                                              const u32x4 &kwa, const u32x4 &kwb, const u32x4 &cosv, const u32x4 &sinv,
-                                             float eps, int hq, int hl) {
+                                             float eps, int hq, int first_head, int lane_head) {
     constexpr int HPW = 64 / (D / 16);
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
-        const int h0 = u * HPW;
+        const int h0 = first_head + u * HPW;
         u32x4 wa, wb;
         if (h0 + HPW <= hq) {  // wave-uniform: a unit of Q heads, of K heads, or of both
             wa = qwa, wb = qwb;
         } else if (h0 >= hq) {
             wa = kwa, wb = kwb;
         } else {
-            const bool is_q = h0 + hl < hq;
+            const bool is_q = lane_head < hq - u * HPW;
 #pragma unroll
             for (int j = 0; j < 4; ++j) wa[j] = is_q ? qwa[j] : kwa[j], wb[j] = is_q ? qwb[j] : kwb[j];
         }
@@ -673,15 +651,15 @@ __device__ __forceinline__ void token_rotate(u32x4 (&xa)[UPT], u32x4 (&xb)[UPT],
 // the rotated Q and K heads back where they came from.
 template <typename T, int D, int UPT, bool SETKV, bool KVFP8, int VN>
 __device__ __forceinline__ void token_store(const RopeArgs &a, uint32_t t, int64_t slot, const u32x4 (&xa)[UPT],
-                                            const u32x4 (&xb)[UPT], const u32x4 (&v)[VN], int hq, int hk, int hv, int lane) {
+                                            const u32x4 (&xb)[UPT], const u32x4 (&v)[VN], int hq, int hk, int hv, int lane, int part,
+                                            int lane_head) {
     constexpr int LPH = D / 16, HPW = 64 / LPH, HALF = D / 2;
-    const int sub = lane % LPH, hl = lane / LPH, heads_qk = hq + hk, v_chunks = hv * (D / 8);
+    const int sub = lane % LPH, heads_qk = hq + hk, v_chunks = hv * (D / 8);
     if constexpr (!SETKV) {
 #pragma unroll
         for (int u = 0; u < UPT; ++u) {
-            const int head = u * HPW + hl;
-            if (head < heads_qk) {
-                uint16_t *dst = static_cast<uint16_t *>(a.qkv_out) + ((int64_t)t * (heads_qk + hv) + head) * D + 8 * sub;
+            if (lane_head < heads_qk - u * HPW) {
+                uint16_t *dst = static_cast<uint16_t *>(a.qkv_out) + ((int64_t)t * (heads_qk + hv) + lane_head + u * HPW) * D + 8 * sub;
                 store_pair<HALF * 2>(dst, xa[u], xb[u], true);
             }
         }
@@ -690,11 +668,11 @@ __device__ __forceinline__ void token_store(const RopeArgs &a, uint32_t t, int64
     const bool slot_ok = slot >= 0;  // a negative slot: no place in the cache, the K and V rows are dropped
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
-        const int head = u * HPW + hl;
-        if (head < hq) {
+        const int head = lane_head + u * HPW;
+        if (lane_head < hq - u * HPW) {
             uint16_t *dst = static_cast<uint16_t *>(a.q_out) + ((int64_t)t * hq + head) * D + 8 * sub;
             store_pair<HALF * 2>(dst, xa[u], xb[u], true);
-        } else if (head < heads_qk && slot_ok) {
+        } else if (lane_head < heads_qk - u * HPW && slot_ok) {
             const int64_t at = (slot * hk + (head - hq)) * D + 8 * sub;
             if constexpr (KVFP8) {
                 uint8_t *dst = static_cast<uint8_t *>(a.k_cache) + at;
@@ -713,7 +691,7 @@ __device__ __forceinline__ void token_store(const RopeArgs &a, uint32_t t, int64
     }
 #pragma unroll
     for (int j = 0; j < VN; ++j) {
-        const int c = lane + 64 * j;
+        const int c = lane + 64 * (part * VN + j);
         if (slot_ok && c < v_chunks) {
             const int64_t off = slot * hv * D + 8 * (int64_t)c;
             if constexpr (KVFP8) {
@@ -727,40 +705,52 @@ __device__ __forceinline__ void token_store(const RopeArgs &a, uint32_t t, int64
     }
 }
 
+// Item -> token: item / parts is (item * ceil(2^18 / parts)) >> 18 for every item the host admits (up to 8192) and up to 31 parts.
+constexpr int kPartsShift = 18, kMaxParts = 31;
+constexpr int token_kernel_v_chunks(int upt, bool two) { return two ? 1 : upt == 3 ? 3 : 2; }  // per lane and part
 constexpr int token_kernel_lds_bytes_per_wave(int upt, bool set_kv) { return (2 * upt + (set_kv ? 1 : 0)) * 1024; }  // TWO: a token's units and 64 V chunks
 
-template <typename T, int D, bool NEOX, int UPT, bool SETKV, bool KVFP8, int AXES, bool TWO>
+// PARTS: tokens may be split (as run-time values the parts cost whole tokens 0.3 to 1 %: 28+4+4 heads 18.66 / 18.82 us at 6144 tokens).
+// AXES: 1; 3 with sections in which every aligned group of 8 frequencies takes one axis (no branch around the table loads);
+// kMergedAxes with any others.
+constexpr int kMergedAxes = 4;
+template <typename T, int D, bool NEOX, int UPT, bool SETKV, bool KVFP8, int AXES, bool TWO, bool PARTS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
-rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num_tokens, uint32_t gate, int hq, int hk,
-                      int hv, uint32_t num_waves, int64_t ps_token, int64_t ps_axis, const RopeArgs rest) {
+rope_rms_token_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const RopeArgs rest) {
     constexpr int LPH = D / 16, HPW = 64 / LPH, HALF = D / 2;
-    constexpr int VN = TWO ? 1 : 2;  // V chunks per lane: the host admits 64 chunks per token with TWO, else 128
-    constexpr bool kPin = is_half<T> && (UPT == 5 || (TWO && SETKV));
+    constexpr int VN = token_kernel_v_chunks(UPT, TWO);
+    constexpr bool kPin = is_half<T> && (UPT == 5 || (TWO && (SETKV || PARTS)));
     extern __shared__ __attribute__((aligned(16))) char token_lds[];  // TWO: 4 waves x token_kernel_lds_bytes_per_wave()
     const uint64_t entry = __builtin_amdgcn_s_memrealtime();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t w = blockIdx.x * 4 + wave;
+    const uint32_t num_items = first[4], parts_magic = first[5], num_waves = second[1];  // (parts_magic: see kPartsShift)
+    const int hq = (int)first[6], hk = (int)first[7], hv = (int)(second[0] & 0xffffffu), parts = PARTS ? (int)(second[0] >> 24) : 1;
+    const void *qkv_in = (const void *)global_ptr<const char>(first[0], first[1]);
+    const int64_t *positions = (const int64_t *)global_ptr<const int64_t>(first[2], first[3]);
+    const int64_t ps_token = (int64_t)(((uint64_t)second[3] << 32) | second[2]), ps_axis = (int64_t)(((uint64_t)third[1] << 32) | third[0]);
     if (w >= num_waves) return;
-    // The wave's token(s).  TWO: the tokens beyond num_waves (a multiple of 1024 wherever there are any: a whole
-    // number of waves on every SIMD) ride as second tokens, dealt out evenly over the compute units -- workgroup g runs
-    // on compute unit g mod 256 while the launch is one round, so the waves of a compute unit are w = 4 (cu + 256 l) + i,
-    // ranked l, i here, and the first extra / 256 of each rank order take one (the remainder: one more on the first units).
-    // (Any other num_waves: wave w takes token w + num_waves as well, where there is one.)
-    const uint32_t t = w;
-    uint32_t t2 = num_tokens;
+    // The wave's item(s); an item is one of the `parts` parts of a token.  TWO: the items beyond num_waves (a multiple of 1024
+    // wherever there are any: a whole number of waves on every SIMD) ride as second items, dealt out evenly over the compute
+    // units -- workgroup g runs on compute unit g mod 256 while the launch is one round, so the waves of a compute unit are
+    // w = 4 (cu + 256 l) + i, ranked l, i here, and the first extra / 256 of each rank order take one (the remainder: one more
+    // on the first units).  (Any other num_waves: wave w takes item w + num_waves as well, where there is one.)
+    uint32_t item2 = num_items;
     if constexpr (TWO) {
         if (num_waves & 1023u) {
-            t2 = w + num_waves;
+            item2 = w + num_waves;
         } else {
-            const uint32_t extra = num_tokens - num_waves, each = extra >> 8, more = extra & 255u;
+            const uint32_t extra = num_items - num_waves, each = extra >> 8, more = extra & 255u;
             const uint32_t cu = (w >> 2) & 255u, layer = w >> 10, rank = (layer << 2) | (w & 3u);
             // (in wave order as far as whole layers of 1024 waves go -- neighbouring workgroups then take neighbouring
             // tokens, 1 % at 8192 tokens -- then the waves of the part layer, then the remainder)
-            if (rank < each) t2 = num_waves + (layer < (each >> 2) ? w : (layer << 10) + cu * (each & 3u) + (w & 3u));
-            else if (rank == each && cu < more) t2 = num_waves + (each << 8) + cu;
+            if (rank < each) item2 = num_waves + (layer < (each >> 2) ? w : (layer << 10) + cu * (each & 3u) + (w & 3u));
+            else if (rank == each && cu < more) item2 = num_waves + (each << 8) + cu;
         }
     }
-    const bool second = TWO && t2 < num_tokens;  // wave-uniform
+    const bool second_item = TWO && item2 < num_items;  // wave-uniform
+    const uint32_t t = PARTS ? (w * parts_magic) >> kPartsShift : w, t2 = PARTS ? (item2 * parts_magic) >> kPartsShift : item2;
+    const int part = PARTS ? (int)(w - t * (uint32_t)parts) : 0, part2 = PARTS ? (int)(item2 - t2 * (uint32_t)parts) : 0;
     const int lane = threadIdx.x & 63, sub = lane % LPH, hl = lane / LPH;
     const int heads_qk = hq + hk, heads_all = heads_qk + hv, v_chunks = hv * (D / 8);
     const uint16_t *token_in = static_cast<const uint16_t *>(qkv_in) + (int64_t)t * heads_all * D;
@@ -769,7 +759,7 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
     u32x4 xa[UPT], xb[UPT], v[VN];
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
-        const int head = min(u * HPW + hl, heads_qk - 1);  // lanes past the last head re-read it
+        const int head = min((part * UPT + u) * HPW + hl, heads_qk - 1);  // lanes past the last head re-read it
         const uint16_t *src = token_in + (int64_t)head * D;
         xa[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + 8 * sub));
         xb[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + HALF + 8 * sub));
@@ -777,24 +767,24 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
     if constexpr (SETKV) {
 #pragma unroll
         for (int j = 0; j < VN; ++j) {
-            const int c = min(lane + 64 * j, v_chunks - 1);
+            const int c = min(lane + 64 * (part * VN + j), v_chunks - 1);
             v[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(token_in + (int64_t)heads_qk * D + 8 * c));
         }
     }
     uint32_t lds_base = 0;
     if constexpr (TWO) {
         lds_base = (uint32_t)(uintptr_t)token_lds + wave * (uint32_t)token_kernel_lds_bytes_per_wave(UPT, SETKV);
-        if (second) {
+        if (second_item) {
             const uint16_t *token2_in = static_cast<const uint16_t *>(qkv_in) + (int64_t)t2 * heads_all * D;
 #pragma unroll
             for (int u = 0; u < UPT; ++u) {
-                const int head = min(u * HPW + hl, heads_qk - 1);
+                const int head = min((part2 * UPT + u) * HPW + hl, heads_qk - 1);
                 const uint16_t *src = token2_in + (int64_t)head * D;
                 lds_fill16(lds_base + (2 * u) * 1024u, src + 8 * sub);
                 lds_fill16(lds_base + (2 * u + 1) * 1024u, src + HALF + 8 * sub);
             }
             if constexpr (SETKV) {
-                const int c = min(lane, v_chunks - 1);
+                const int c = min(lane + 64 * part2, v_chunks - 1);
                 lds_fill16(lds_base + (2 * UPT) * 1024u, token2_in + (int64_t)heads_qk * D + 8 * c);
             }
         }
@@ -802,24 +792,25 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
     // (positions: read as memory that no kernel of the launch writes, scalar loads whatever else the kernel contains)
     int64_t p[3] = {0, 0, 0}, p2[3] = {0, 0, 0};
 #pragma unroll
-    for (int ax = 0; ax < AXES; ++ax) {
+    for (int ax = 0; ax < (AXES == 1 ? 1 : 3); ++ax) {
         p[ax] = load_unchanging(positions + ax * ps_axis + (int64_t)t * ps_token);
-        if (second) p2[ax] = load_unchanging(positions + ax * ps_axis + (int64_t)t2 * ps_token);
+        if (second_item) p2[ax] = load_unchanging(positions + ax * ps_axis + (int64_t)t2 * ps_token);
     }
     // the rest of the arguments, fetched from the argument block behind the requests above (see rope_rms_kernel)
     typedef const __attribute__((address_space(4))) RopeArgs *BlockPtr;
     BlockPtr block = (BlockPtr)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() +
-                                sizeof(TokenKernelLead));
+                                kUnitLeadBytes);
     asm volatile("" : "+s"(block));
     RopeArgs a;
     a.qw = as_global(block->qw);
     a.kw = as_global(block->kw);
     a.cos_sin = as_global(block->cos_sin);
     a.eps = block->eps;
+    a.gate = block->gate;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        a.axis1[i] = AXES == 3 ? block->axis1[i] : 0u;
-        a.axis2[i] = AXES == 3 ? block->axis2[i] : 0u;
+        a.axis1[i] = AXES != 1 ? block->axis1[i] : 0u;
+        a.axis2[i] = AXES != 1 ? block->axis2[i] : 0u;
     }
     int64_t slot = 0, slot2 = 0;
     if constexpr (SETKV) {
@@ -830,27 +821,31 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
         a.k_scale = block->k_scale;
         a.v_scale = block->v_scale;
         asm volatile("" ::"s"(a.kv_loc), "s"(a.qw), "s"(a.kw), "s"(a.cos_sin), "s"(a.q_out), "s"(a.k_cache), "s"(a.v_cache),
-                     "s"(a.eps), "s"(a.k_scale), "s"(a.v_scale));
+                     "s"(a.eps), "s"(a.gate), "s"(a.k_scale), "s"(a.v_scale));
         slot = load_unchanging(a.kv_loc + t);
-        slot2 = second ? load_unchanging(a.kv_loc + t2) : -1;
+        slot2 = second_item ? load_unchanging(a.kv_loc + t2) : -1;
     } else {
         a.qkv_out = as_global(block->qkv_out);
-        asm volatile("" ::"s"(a.qw), "s"(a.kw), "s"(a.cos_sin), "s"(a.qkv_out), "s"(a.eps));
+        asm volatile("" ::"s"(a.qw), "s"(a.kw), "s"(a.cos_sin), "s"(a.qkv_out), "s"(a.eps), "s"(a.gate));
     }
     const uint16_t *qw = static_cast<const uint16_t *>(a.qw), *kw = static_cast<const uint16_t *>(a.kw);
     const u32x4 qwa = *reinterpret_cast<const u32x4 *>(qw + 8 * sub), qwb = *reinterpret_cast<const u32x4 *>(qw + HALF + 8 * sub);
     const u32x4 kwa = *reinterpret_cast<const u32x4 *>(kw + 8 * sub), kwb = *reinterpret_cast<const u32x4 *>(kw + HALF + 8 * sub);
     const uint16_t *table = static_cast<const uint16_t *>(a.cos_sin);
     u32x4 cosv, sinv, cosv2 = {0, 0, 0, 0}, sinv2 = {0, 0, 0, 0};
-    load_trig_by_axis<D, NEOX, AXES>(table, p[0], p[1], p[2], a.axis1, a.axis2, sub, cosv, sinv);
-    if (second) load_trig_by_axis<D, NEOX, AXES>(table, p2[0], p2[1], p2[2], a.axis1, a.axis2, sub, cosv2, sinv2);
+    auto load_table = [&](const int64_t (&q)[3], u32x4 &c, u32x4 &sn) {
+        if constexpr (AXES == 3) load_trig_by_axis<D, NEOX>(table, q[0], q[1], q[2], a.axis1, a.axis2, sub, c, sn);
+        else load_trig_merged<D, NEOX, AXES == 1 ? 1 : 3>(table, q[0], q[1], q[2], a.axis1, a.axis2, sub, c, sn);
+    };
+    load_table(p, cosv, sinv);
+    if (second_item) load_table(p2, cosv2, sinv2);
     // (the slots are asked for here and not where the rows are stored)
     if constexpr (SETKV)
         asm volatile("" ::"s"((uint32_t)slot), "s"((uint32_t)(slot >> 32)), "s"((uint32_t)slot2), "s"((uint32_t)(slot2 >> 32)));
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- norm and rotation of the first token, unit by unit, in place
-    token_rotate<T, D, NEOX, UPT, kPin>(xa, xb, qwa, qwb, kwa, kwb, cosv, sinv, a.eps, hq, hl);
+    token_rotate<T, D, NEOX, UPT, kPin>(xa, xb, qwa, qwb, kwa, kwb, cosv, sinv, a.eps, hq, part * UPT * HPW, part * UPT * HPW + hl);
 
     // (the rotated rows are pinned down here, ahead of the wait: nothing ties the arithmetic to the clock, and the
     // compiler otherwise moves it behind the wait, into the writing half)
@@ -858,13 +853,13 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
     for (int u = 0; u < UPT; ++u) asm volatile("" ::"v"(xa[u]), "v"(xb[u]));
 
     // ---- the writing half of the launch
-    while (__builtin_amdgcn_s_memrealtime() < entry + gate) __builtin_amdgcn_s_sleep(1);
+    while (__builtin_amdgcn_s_memrealtime() < entry + a.gate) __builtin_amdgcn_s_sleep(1);
     // (the transfers into LDS are not loads the compiler knows of; they landed long ago, and with nothing else of
     // the wave outstanding at this point the wait that says so to the hardware costs nothing)
     if constexpr (TWO) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    token_store<T, D, UPT, SETKV, KVFP8, VN>(a, t, slot, xa, xb, v, hq, hk, hv, lane);
+    token_store<T, D, UPT, SETKV, KVFP8, VN>(a, t, slot, xa, xb, v, hq, hk, hv, lane, part, part * UPT * HPW + hl);
     if constexpr (TWO) {
-        if (second) {  // the second token takes the registers of the first
+        if (second_item) {  // the second token takes the registers of the first
             const char *mine = token_lds + wave * token_kernel_lds_bytes_per_wave(UPT, SETKV) + lane * 16;
 #pragma unroll
             for (int u = 0; u < UPT; ++u) {
@@ -872,8 +867,8 @@ rope_rms_token_kernel(const void *qkv_in, const int64_t *positions, uint32_t num
                 xb[u] = *reinterpret_cast<const u32x4 *>(mine + (2 * u + 1) * 1024);
             }
             if constexpr (SETKV) v[0] = *reinterpret_cast<const u32x4 *>(mine + (2 * UPT) * 1024);
-            token_rotate<T, D, NEOX, UPT, kPin>(xa, xb, qwa, qwb, kwa, kwb, cosv2, sinv2, a.eps, hq, hl);
-            token_store<T, D, UPT, SETKV, KVFP8, VN>(a, t2, slot2, xa, xb, v, hq, hk, hv, lane);
+            token_rotate<T, D, NEOX, UPT, kPin>(xa, xb, qwa, qwb, kwa, kwb, cosv2, sinv2, a.eps, hq, part2 * UPT * HPW, part2 * UPT * HPW + hl);
+            token_store<T, D, UPT, SETKV, KVFP8, VN>(a, t2, slot2, xa, xb, v, hq, hk, hv, lane, part2, part2 * UPT * HPW + hl);
         }
     }
 }
@@ -1248,7 +1243,7 @@ int launch_2way_head_size(const TwoWayArgs &a, int64_t D, bool neox, unsigned ba
 
 int g_block_threads = 0;  // 0 = default
 int g_merge_rows = 0;     // mRoPE rows merged on load where the sections allow: 0 = yes, 1 = never
-int g_token_waves = 0;    // one-wave-per-token kernel: 0 = built-in rule, 1 = never, 2 = wherever it fits, 3 = likewise, two tokens per wave where that fits
+int g_token_waves = 0;    // one-wave-per-token kernel: 0 = built-in rule, 1 = never, 2 = wherever it fits, 3 = likewise, two items per wave where that fits
 int g_token_gate = -1;    // its gate in ticks of 10 ns; -1 = from the bytes of the call
 int g_unit_gate = -1;     // gate of the kernel with one wave per unit: -1 = built-in rule, 0 = none, > 0 = ticks
 constexpr uint32_t kResidentUnits = 8192;  // waves of the one-wave-per-unit kernel the chip holds at once (8 per SIMD)
@@ -1267,50 +1262,107 @@ struct RopePlan {
     bool token_waves;          // the one-wave-per-token kernel
     bool two_tokens;           // ... with two tokens per wave, the second through LDS
     uint32_t token_wave_count; // its waves
+    uint32_t token_units, token_parts;  // units per wave, and waves that share a token
     uint32_t gate;             // its gate: ticks of 10 ns before which no wave stores
     uint32_t unit_gate;        // the same for the kernel with one wave per unit (0 = none)
 };
 
-RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool set_kv, bool kv_fp8) {
+// How the one-wave-per-token kernel takes a call: the units of a token in `parts` parts of `units` each, one part (an item)
+// per wave or two.
+struct TokenShape {
+    int units, parts;  // 0: it does not take it
+    int64_t items;
+};
+
+// Up to five units (40 Q and K heads of 128 elements, 20 of 256) are one part; more are split so that at most an eighth of the
+// lanes idle, with the fewest idle units and then the fewest parts.  One item per wave: 4096 waves, four on every SIMD, and the
+// V chunks they hold in registers; two: twice as many items of three or four units, 64 V chunks each in LDS.
+// An fp8 cache, whose conversions lengthen the wave, only in the shapes where that was ahead: heads of 128 elements, four or
+// five units, one axis.  In place, where a token's waves have no V row and no scatter to share, up to three parts (64+64
+// heads of 128, four parts of four, 800 tokens 10.7 us / 10.9 here; of 256, eight parts, 778 tokens 18.6 / 19.3).  Heads of 64
+// elements stay with the kernel above: ahead where the items fill whole layers of 1024 waves, behind between them (3072 /
+// 3563 tokens of 64+8+8 heads 14.5 / 12.6 and 16.4 / 17.3 us).
+TokenShape token_shape(const RopeArgs &a, int D, int axes, bool set_kv, bool kv_fp8, bool two) {
+    TokenShape best{0, 0, 0};
+    const int upt = (int)a.units_per_token;
+    if ((D != 128 && D != 256) || upt < 3 || (set_kv && a.hv == 0)) return best;
+    if (kv_fp8 && (D != 128 || axes != 1 || upt < 4 || upt > 5 || two)) return best;
+    int best_idle = 0;
+    for (int units = two ? 4 : 5; units >= 3; --units) {
+        const int parts = (upt + units - 1) / units, idle = parts * units - upt;
+        const int64_t items = (int64_t)a.num_tokens * parts;
+        if (7 * idle > upt || parts > (set_kv ? kMaxParts : 3) || items > (two ? 2 : 1) * (int64_t)kTokenWaveCapacity) continue;
+        if (set_kv && (int64_t)a.hv * (D / 8) > (int64_t)64 * token_kernel_v_chunks(units, two) * parts) continue;
+        if (best.units && idle >= best_idle) continue;
+        best = {units, parts, items};
+        best_idle = idle;
+    }
+    return best;
+}
+
+RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, bool kv_fp8, bool half) {
     RopePlan p{};
-    // One wave per token (or per two) where the whole batch is resident at once and large enough for its traffic to
-    // matter: head size 128, 4 or 5 units (25-40 Q and K heads) and at most 128 chunks of V per token, a cache; with
-    // three position axes only where every aligned group of 8 frequencies takes one axis, and not with an fp8 cache.
     const int64_t read_bytes = 2 * (int64_t)a.num_tokens * (a.hq + a.hk + (set_kv ? a.hv : 0)) * D;
-    const bool shape = D == 128 && a.units_per_token >= 4 && a.units_per_token <= 5 &&
-                       (!set_kv || (a.hv * (D / 8) <= 128 && a.hv > 0)) && (axes == 1 || (axes == 3 && a.merge_rows && !kv_fp8));
-    const bool one = shape && a.num_tokens <= kTokenWaveCapacity;
-    // Two tokens per wave, the second through LDS (4 units and 64 V chunks per token: 9 KB of the 160 KB of a compute
-    // unit for each of its 16 waves), for up to twice that many tokens.
-    const bool two_shape = shape && a.units_per_token == 4 && (!set_kv || a.hv * (D / 8) <= 64) && !kv_fp8 &&
-                           a.num_tokens <= 2 * kTokenWaveCapacity;
-    const bool two = two_shape && (g_token_waves == 3 || !one);
+    const int64_t heads = a.hq + a.hk, places = (int64_t)a.units_per_token * (64 / (D / 16));
+    // One wave per part of a token (or per two) where the whole batch is resident at once and large enough for its traffic
+    // to matter.
+    const TokenShape one_item = token_shape(a, D, axes, set_kv, kv_fp8, false), two_items = token_shape(a, D, axes, set_kv, kv_fp8, true);
+    const bool two = two_items.units && (g_token_waves == 3 || !one_item.units);
+    const TokenShape shape = two ? two_items : one_item;
     // ... and clearly too large for the kernel above to hold all of its waves at once (from 10240 units, five quarters
     // of what it holds; below that the kernel above, gated, is ahead or level: 8.3 against 9.7 us at 1536 tokens of
     // 32+8+8 heads, 9.1 against 9.5 at 2100 tokens of 28+4+4; from there on this one is: 32+8+8 heads 10.3 against
     // 11.1 us at 2048 tokens, 13.6 against 14.8 at 3000, 16.6 against 17.3 at 3700, 16.2 against 18.2 at 4096; 28+4+4
-    // heads with three axes 10.0 against 11.7 us at 3000 tokens, 12.2 against 14.5 at 4096).
-    // With two tokens per wave from there to twice that many tokens: 4096 waves, four on every SIMD, one token each and
-    // the others dealt out evenly.  The SIMD with the most tokens sets the time (the rotation arithmetic of its waves
-    // is two thirds of the launch), so the time goes up in steps of 1024 tokens where the kernel above is linear; this
+    // heads with three axes 10.0 against 11.7 us at 3000 tokens, 12.2 against 14.5 at 4096, interleaved sections 10.0 against
+    // 11.6 at 2621, 12.7 against 16.2 at 4096; heads of 256 elements, 28+4+4, two parts of four, from 11264: 10.2 against 12.4 at
+    // 1536 tokens, 12.5 against 15.5 at 2048; 64+8+8, two of five, 14.2 against 16.0 at 2048).  With three units per wave from 9216 units:
+    // 40+8+8 heads, two parts, 8.5 against 9.7 us at 1536 tokens, 10.2 against 12.2 at 2048; 16+2+2 7.9 against 8.9 at 3072, 9.4
+    // against 10.6 at 4096; 12+12+12 10.3 against 12.7, 12.8 against 15.5.
+    // With two items per wave from there to twice that many items: 4096 waves, four on every SIMD, one item each and
+    // the others dealt out evenly.  The SIMD with the most items sets the time (the rotation arithmetic of its waves
+    // is two thirds of the launch), so the time goes up in steps of 1024 items where the kernel above is linear; this
     // one is ahead or level everywhere (graph replays, 28+4+4 heads, one axis / three: 16.1 / 16.4 against 17.2 / 17.5 us
     // at 4800 tokens, 18.2 / 18.5 against 18.4 / 18.8 at 5200, 19.1 / 19.6 against 21.1 / 21.5 at 6144, 21.7 / 21.7 against
-    // 23.5 / 23.7 at 7000, 24.2 / 24.4 against 24.7 / 25.3 at 7500, 25.3 / 25.3 against 26.8 / 27.3 at 8192; level below
-    // 4608 tokens, where the kernel above stays).  Half as many waves with two tokens each were behind that: 20.0 at 6144 tokens.
+    // 23.5 / 23.7 at 7000, 24.2 / 24.4 against 24.7 / 25.3 at 7500, 25.3 / 25.3 against 26.8 / 27.3 at 8192, interleaved 19.7
+    // against 22.5 at 6144, 26.0 against 28.5 at 8192; 40+8+8, two parts of three, 12.1 against 13.2 at 2304, 19.9 against 21.5 at
+    // 4096; 28+4+4 heads of 256, two of four, 18.4 against 20.8 at 3000, 25.4 against 27.1 at 4096; level below
+    // 4608 items, where the kernel above stays).  Half as many waves with two items each were behind that: 20.0 at 6144 tokens.
     // (in place, with no V row and no scatter, the kernel above holds out a little longer: 9.0 against 9.5 us at 2048
     // tokens of 32+8 heads, then 11.9 against 11.2 at 3000, 15.4 against 13.7 at 4096; 28+4 heads with three axes 10.7
     // against 9.5 at 3000 tokens, 13.2 against 11.5 at 4096, 18.4 against 17.4 at 6144 and 23.2 against 21.6 at 8192 with
-    // two tokens per wave)
-    const bool large = a.total_units >= (set_kv ? kResidentUnits + kResidentUnits / 4 : kResidentUnits + 2 * kResidentUnits / 5);
+    // two items per wave; 40+8, parts of three, 8.3 against 7.9 at 1536, 10.4 against 9.4 at 2048, 11.2 against 11.4 at 2304 and
+    // 13.9 against 13.5 at 3000 with two items per wave)
+    // Half precision, whose arithmetic is packed, from seven eighths of the other kernel's round where nearly all lanes have a
+    // head and two waves are left per SIMD: 40+8+8 heads 6.6 against 7.0 us at 1228 tokens, 6.8 against 7.5 at 1365, 9.6 against
+    // 11.7 at 2048 (32+8+8, parts of five, 7.4 against 7.1 at 1471; 48+8+8, an idle unit, 7.2 against 6.8 at 1056).
+    const bool full = 8 * heads >= 7 * places, no_idle_unit = shape.units * shape.parts == (int)a.units_per_token;
+    const int64_t from_units = half && full && no_idle_unit && shape.units <= 4 && shape.items >= 2048 ? 7 * kResidentUnits / 8
+                               : shape.units == 3 ? 9 * kResidentUnits / 8
+                               : !set_kv ? 7 * kResidentUnits / 5 : shape.parts == 1 ? 5 * kResidentUnits / 4 : 11 * kResidentUnits / 8;
     // (with an fp8 cache the conversions lengthen the wave and the gate hardly matters; one token per wave is still
     // ahead once the batch is large: 28+4+4 heads 10.8 against 11.9 us at 3000 tokens, 13.3 against 14.2 at 4096; 32+8+8
     // heads 16.8 against 17.6 at 4096, level at 3000, behind at 2560)
-    const bool large_fp8 = a.total_units >= (a.units_per_token == 4 ? kResidentUnits + kResidentUnits / 4 : 7 * kResidentUnits / 4);
-    const bool extra_enough = a.num_tokens >= kTokenWaveCapacity + kTokenWaveCapacity / 8;  // (level or 1 % behind below: 15.4 against 15.2 us at 4100 tokens)
-    const bool by_rule = g_token_waves == 0 && (two ? extra_enough : (kv_fp8 ? large_fp8 : large));
-    p.token_waves = (one || two) && (g_token_waves >= 2 || by_rule);
+    const int64_t from_units_fp8 = a.units_per_token == 4 ? 5 * kResidentUnits / 4 : 7 * kResidentUnits / 4;
+    // (two items per wave: level or 1 % behind below, 15.4 against 15.2 us at 4100 tokens)
+    bool large = two ? shape.items >= kTokenWaveCapacity + kTokenWaveCapacity / 8 : a.total_units >= (kv_fp8 ? from_units_fp8 : from_units);
+    // Where the margin is thin it does not cover every fill of the last layer of waves.  Beyond whole tokens of four or five
+    // units of 128-element heads that read one table row, these stay with the kernel above (us, that one / this one).  In place:
+    // pairwise rotation (28+4 heads of 256 in half precision 10.4 / 11.2 at 1611 tokens, 40+8 17.1 / 17.7 at 3802), parts of five or with
+    // idle units (64+8 heads 10.4 / 10.7 at 1370 tokens, 48+8 10.3 / 10.7 at 1739), a layer that has just begun (64+8 heads 11.5 / 12.6 at 1618
+    // tokens, 3236 items) and two items per wave in bfloat16 (40+8 16.7 / 16.7 at 3749) or with idle lanes (16+2 in half precision 13.8 / 15.3 at 8186).
+    // With a cache: a layer that has just begun where lanes or units idle (16+2+2 in half precision 7.6 / 8.2 at 3148), two items per wave
+    // where lanes idle in bfloat16 but for merged table rows (16+2+2 16.1 / 16.6 at 7544).  Pairwise with a cache: the latter in every type, seven layers and
+    // more (20+4+4 in half precision 21.0 / 21.5 at 7797), a layer that has just begun, and bfloat16 with three V chunks per lane (12+12+12 14.3 / 14.9 at 3592).
+    if (!(D == 128 && shape.parts == 1 && shape.units >= 4 && (axes == 1 || a.merge_rows))) {
+        const int64_t last = shape.items > 3072 ? shape.items % 1024 : 0;  // items of the last layer, 0: it is full
+        if (!set_kv) large = large && neox && shape.units < 5 && no_idle_unit && (two ? half && full : last == 0 || last >= 256);
+        else if (neox) large = large && (!two || full || half || (axes == 3 && !a.merge_rows)) && ((full && no_idle_unit) || last == 0 || last >= 256);
+        else large = large && (!two || (full && shape.items <= 7168)) && (last == 0 || last >= 384) && (half || a.hv * (D / 8) <= 128 * shape.parts);
+    }
+    const bool by_rule = g_token_waves == 0 && large;
+    p.token_waves = shape.units && (g_token_waves >= 2 || by_rule);
     p.two_tokens = p.token_waves && two;
-    // (with two tokens per wave the full read time: 24.4 us at 8192 tokens of 28+4+4 heads with three axes, against 25.4
+    // (with two items per wave the full read time: 24.4 us at 8192 tokens of 28+4+4 heads with three axes, against 25.4
     // with 0.95 of it, 24.8 with 1.05, 27.2 with 0.9 -- opening early, into the last reads, costs more than waiting)
     const double gate = g_token_gate >= 0 ? (double)g_token_gate : (double)read_bytes / (two ? 70000.0 : kGateBytesPerTick);
     p.gate = (uint32_t)std::min(gate, 5000.0);
@@ -1340,7 +1392,6 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool set_kv, bool kv_fp8)
                                             (kv_fp8 ? 1 : 2) * ((int64_t)a.num_tokens * a.hk * D + elems_v)
                                       : 4 * elems_qk;
     p.stream = g_stream_rows == 2 || (g_stream_rows == 0 && call_bytes >= kStreamFromBytes);
-    const int64_t heads = a.hq + a.hk, places = (int64_t)a.units_per_token * (64 / (D / 16));
     p.whole_lines = g_stream_rows == 2 ||
                     (4 * heads >= 3 * places && call_bytes >= (heads == places ? kWholeLinesFromBytes : kWholeLinesFromBytesRagged));
     // Workgroup size, swept over 64/128/256/512 lanes and one workgroup per token for 2-9 units per token: four
@@ -1353,9 +1404,11 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool set_kv, bool kv_fp8)
     p.blocks = (a.total_units + units_per_block - 1) / units_per_block;
     if (p.token_waves) {
         p.threads = 256;
-        // (two tokens per wave: every SIMD's four waves take one token each and the rest are dealt out over them; a
-        // batch that two tokens per wave are forced onto although one would do is halved instead)
-        p.token_wave_count = !p.two_tokens ? a.num_tokens : a.num_tokens > kTokenWaveCapacity ? kTokenWaveCapacity : (a.num_tokens + 1) / 2;
+        // (two items per wave: every SIMD's four waves take one item each and the rest are dealt out over them; a
+        // batch that two items per wave are forced onto although one would do is halved instead)
+        p.token_units = (uint32_t)shape.units;
+        p.token_parts = (uint32_t)shape.parts;
+        p.token_wave_count = (uint32_t)(!p.two_tokens ? shape.items : shape.items > kTokenWaveCapacity ? kTokenWaveCapacity : (shape.items + 1) / 2);
         p.blocks = (p.token_wave_count + 3) / 4;
         p.stream = true;
     }
@@ -1364,32 +1417,47 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool set_kv, bool kv_fp8)
 
 template <typename T, int D, bool NEOX, int AXES, bool SETKV, bool KVFP8>
 int launch_one(const RopeArgs &a, hipStream_t stream) {
-    const RopePlan p = plan_rope(a, D, AXES, SETKV, KVFP8);
+    const RopePlan p = plan_rope(a, D, AXES, NEOX, SETKV, KVFP8, is_half<T>);
     RopeArgs b = a;
     b.stream_rows = p.stream ? 1u : 0u;
     b.gate = p.unit_gate;
-    if constexpr (D == 128 && (AXES == 1 || !KVFP8)) {
+    if constexpr (D != 64 && (!KVFP8 || (D == 128 && AXES == 1))) {  // (see token_shape)
         if (p.token_waves) {
+            b.gate = p.gate;
+            const uint32_t items = a.num_tokens * p.token_parts;
+            const uint32_t magic = ((1u << kPartsShift) + p.token_parts - 1) / p.token_parts;
+            const u32x8 first = {low_half(a.qkv_in), high_half(a.qkv_in), low_half(a.positions), high_half(a.positions), items, magic, (uint32_t)a.hq, (uint32_t)a.hk};
+            const u32x4 second = {(uint32_t)a.hv | (p.token_parts << 24), p.token_wave_count, (uint32_t)a.ps_token, (uint32_t)((uint64_t)a.ps_token >> 32)};
+            const u32x2 third = {(uint32_t)a.ps_axis, (uint32_t)((uint64_t)a.ps_axis >> 32)};
 #define GPUK_LAUNCH_TOKEN(UPT, TWO)                                                                                    \
-    rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES, TWO>                                                    \
-        <<<p.blocks, 256, TWO ? 4 * token_kernel_lds_bytes_per_wave(UPT, SETKV) : 0, stream>>>(                        \
-            a.qkv_in, a.positions, a.num_tokens, p.gate, a.hq, a.hk, a.hv, p.token_wave_count, a.ps_token, a.ps_axis, b)
+    do {                                                                                                               \
+        constexpr uint32_t lds = TWO ? 4 * token_kernel_lds_bytes_per_wave(UPT, SETKV) : 0;                            \
+        constexpr bool whole = D == 128 && UPT >= 4, parts_too = !KVFP8;                                               \
+        if (AXES == 3 && !a.merge_rows)                                                                                \
+            return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES == 3 ? kMergedAxes : 1, TWO, parts_too>, \
+                                 dim3(p.blocks), 256, lds, stream, first, second, third, b);                           \
+        if (whole && p.token_parts == 1)                                                                               \
+            return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES, TWO, !whole>, dim3(p.blocks), 256, lds, \
+                                 stream, first, second, third, b);                                                     \
+        return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES, TWO, parts_too>, dim3(p.blocks), 256, lds, \
+                             stream, first, second, third, b);                                                         \
+    } while (0)
             if (p.two_tokens) {
                 if constexpr (!KVFP8) {
-                    if (a.units_per_token != 4) return GPUK_ERR_INTERNAL;
-                    GPUK_LAUNCH_TOKEN(4, true);
-                } else {
+                    if (p.token_units == 4) GPUK_LAUNCH_TOKEN(4, true);
+                    if (p.token_units == 3) GPUK_LAUNCH_TOKEN(3, true);
+                }
+                return GPUK_ERR_INTERNAL;
+            }
+            switch (p.token_units) {
+                case 3:
+                    if constexpr (!KVFP8) GPUK_LAUNCH_TOKEN(3, false);
                     return GPUK_ERR_INTERNAL;
-                }
-            } else {
-                switch (a.units_per_token) {
-                    case 4: GPUK_LAUNCH_TOKEN(4, false); break;
-                    case 5: GPUK_LAUNCH_TOKEN(5, false); break;
-                    default: return GPUK_ERR_INTERNAL;
-                }
+                case 4: GPUK_LAUNCH_TOKEN(4, false); break;
+                case 5: GPUK_LAUNCH_TOKEN(5, false); break;
+                default: return GPUK_ERR_INTERNAL;
             }
 #undef GPUK_LAUNCH_TOKEN
-            return hip_status(hipGetLastError());
         }
     }
     const uint32_t log2_waves = p.threads == 64 ? 0u : p.threads == 128 ? 1u : p.threads == 256 ? 2u : 3u;
@@ -1587,7 +1655,7 @@ int rope_launch_shape(int64_t T, int64_t hq, int64_t hk, int64_t hv, int64_t D, 
         *streamed = 1;  // the fp32 / fp64 kernel always stores its rotated rows past the L2
         return GPUK_OK;
     }
-    const RopePlan p = plan_rope(a, (int)D, n_axes, set_kv, set_kv && kv_dtype == GPUK_KV_E4M3FN);
+    const RopePlan p = plan_rope(a, (int)D, n_axes, true, set_kv, set_kv && kv_dtype == GPUK_KV_E4M3FN, dtype == GPUK_DTYPE_FP16);
     *workgroups = (int)p.blocks;
     *lanes = (int)p.threads;
     *streamed = p.stream ? 1 : 0;
