@@ -278,13 +278,18 @@ __device__ __forceinline__ void store_pair(void *p, const u32x4 &a, const u32x4 
 // DPP move per dword and direction).  Measured, half lines / whole ones: 10024 tokens of 64 + 64 heads in place 61.8 /
 // 54.2 us (55.6 with whole stores only), 3000 tokens 20.9 / 19.8, 16384 of 28 + 4 in half precision 32.0 / 27.3;
 // two streams of 2 x (678 + 3608) tokens, 24 + 25 heads 23.7 / 22.1.  Calls that do not stream their stores (below 8 MB)
-// are bound by latency and keep the shorter code (2.14 / 2.21 us at one token), and so do those with a cache: a unit of
-// theirs is half Q and half K rows scattered over slots, and gains nothing (12.4 / 12.6 us at 4096 tokens of 32+8+8).
-// In bfloat16, whose waves are busier, so do streamed calls of less than 13.5 MB, of less than 18 MB where a token's last unit
+// are bound by latency and keep the shorter code (2.14 / 2.21 us at one token).
+// In bfloat16, whose waves are busier, so do streamed calls in place of less than 13.5 MB, of less than 18 MB where a token's last unit
 // is not full, and all those whose units are less than three quarters full (bytes read and written; us, half / whole: 28+4
 // heads 3.37 / 3.44 at 8 MB, 4.02 / 4.07 at 12, 5.26 / 4.63 at 16; 32+8, of 48 places, 4.70 / 4.92 at 16, 6.55 / 6.27 at 24; 16+2, of
 // 32, 4.1 / 4.4 at 10, 3-7 % behind up to 24 and at 60; two streams of 24+24 heads 4.26 / 4.31 at 12 MB, 6.25 / 5.43 at 20).  Half
 // precision gains 4-17 % throughout (32+8 at 8-14 MB: 1-2 % lost).
+// With a 16-bit cache: half precision from a third of a round of waves on (28+4+4 3.54 / 3.65 at 907 tokens, 4.6 / 4.2 at 1500; 64+8+8 6.9 / 6.3 at 1500, 17.9 / 15.4 at 4000, 62.3 / 53.1 at 16000,
+// 32+8+8 11.6 / 10.6 and 38.3 / 33.5); bfloat16 beyond one round of waves where units are four fifths full (64+8+8 18.0 / 16.7 and 61.2 / 54.5, 40+8+8 13.4 /
+// 12.9 and 43.3 / 38.5, 32+8+8 12.1 / 11.8 and 37.6 / 34.3, but 5.4 / 6.1 at 1500), beyond three where they are three quarters full
+// (12+12+12 18.2 / 18.3 at 9000 tokens, 29.0 / 27.0 at 16000; 16+2+2, of 32 places, 19.2 / 20.8).  An fp8 cache, whose conversions then run
+// on both chunks of every lane, gains 4-6 % with few K heads and loses as much with others (64+8+8 34.8 / 32.8 at 9000 tokens, 32+8+8
+// 36.5 / 37.4 at 16000): not done.
 __device__ __forceinline__ void exchange_lines(u32x4 &a, u32x4 &b) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -416,12 +421,21 @@ struct RopeUnit {
         const bool slot_ok = !SETKV || st.slot >= 0;  // wave-uniform
         const int head = st.head;
         if constexpr (WHOLE) {
-            static_assert(!SETKV, "whole lines: in place only");
             exchange_lines(oa, ob);
-            const int even = (int)(st.u * HPW) + ((lane / LPH) & ~1);
-            uint16_t *dst = static_cast<uint16_t *>(a.qkv_out) + ((int64_t)st.t * heads_all + even) * D + 8 * (lane & 7);
-            if (even + 1 < heads_qk) store_pair<D * 2>(dst, oa, ob, true);
-            else if (even < heads_qk) store_chunk_streamed(dst, oa);
+            const int even = (int)(st.u * HPW) + ((lane / LPH) & ~1), piece = 8 * (lane & 7);
+            if constexpr (!SETKV) {
+                uint16_t *dst = static_cast<uint16_t *>(a.qkv_out) + ((int64_t)st.t * heads_all + even) * D + piece;
+                if (even + 1 < heads_qk) store_pair<D * 2>(dst, oa, ob, true);
+                else if (even < heads_qk) store_chunk_streamed(dst, oa);
+            } else {
+                static_assert(!KVFP8, "whole lines: not with an fp8 cache");
+                auto store_piece = [&](int h, const u32x4 &o) {
+                    if (h < a.hq) store_chunk_streamed(static_cast<uint16_t *>(a.q_out) + ((int64_t)st.t * a.hq + h) * D + piece, o);
+                    else if (h < heads_qk && slot_ok) store_chunk_streamed(static_cast<uint16_t *>(a.k_cache) + (st.slot * a.hk + (h - a.hq)) * D + piece, o);
+                };
+                store_piece(even, oa);
+                store_piece(even + 1, ob);
+            }
         } else if (st.active && (st.is_q || slot_ok)) {
             if constexpr (!SETKV) {
                 uint16_t *dst = static_cast<uint16_t *>(a.qkv_out) + ((int64_t)st.t * heads_all + head) * D;
@@ -1258,7 +1272,7 @@ constexpr int64_t kStreamFromBytes = 8'000'000;
 struct RopePlan {
     uint32_t threads, blocks;  // workgroup size and count of the launch
     bool stream;               // q_out / K rows / in-place rows stored past the L2
-    bool whole_lines;          // heads of 64 elements in place, bfloat16: lines moved whole where they are streamed (see exchange_lines)
+    bool whole_lines;          // heads of 64 elements: lines moved whole where they are streamed (see exchange_lines)
     bool token_waves;          // the one-wave-per-token kernel
     bool two_tokens;           // ... with two tokens per wave, the second through LDS
     uint32_t token_wave_count; // its waves
@@ -1392,8 +1406,10 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
                                             (kv_fp8 ? 1 : 2) * ((int64_t)a.num_tokens * a.hk * D + elems_v)
                                       : 4 * elems_qk;
     p.stream = g_stream_rows == 2 || (g_stream_rows == 0 && call_bytes >= kStreamFromBytes);
-    p.whole_lines = g_stream_rows == 2 ||
-                    (4 * heads >= 3 * places && call_bytes >= (heads == places ? kWholeLinesFromBytes : kWholeLinesFromBytesRagged));
+    if (g_stream_rows == 2) p.whole_lines = true;
+    else if (half) p.whole_lines = !set_kv || 3 * a.total_units >= kResidentUnits;
+    else if (!set_kv) p.whole_lines = 4 * heads >= 3 * places && call_bytes >= (heads == places ? kWholeLinesFromBytes : kWholeLinesFromBytesRagged);
+    else p.whole_lines = (5 * heads >= 4 * places && a.total_units > kResidentUnits) || (4 * heads >= 3 * places && a.total_units > 3 * kResidentUnits);
     // Workgroup size, swept over 64/128/256/512 lanes and one workgroup per token for 2-9 units per token: four
     // waves where a workgroup then holds whole tokens (its waves share the token's position and table row in the
     // CU's caches: 3-15 % ahead at 28+4 heads) and for large batches (1-3 % ahead from 4096 tokens on), single
@@ -1461,7 +1477,7 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
         }
     }
     const uint32_t log2_waves = p.threads == 64 ? 0u : p.threads == 128 ? 1u : p.threads == 256 ? 2u : 3u;
-    constexpr bool kHalfLines = D == 64 && !SETKV;  // see exchange_lines
+    constexpr bool kHalfLines = D == 64 && !KVFP8;  // see exchange_lines
     const void *third = a.kv_loc;  // (see rope_rms_kernel)
     if constexpr (AXES == 3) third = reinterpret_cast<const void *>((intptr_t)a.ps_axis);
     const u32x8 lead1 = {low_half(a.qkv_in), high_half(a.qkv_in), low_half(a.positions), high_half(a.positions), a.total_units, a.upt_magic, (uint32_t)a.hq, (uint32_t)a.hk};
@@ -1470,7 +1486,7 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
 #define GPUK_LAUNCH_UNITS(GATED, WHOLE)                                                                                 \
     return launch_kernel(rope_rms_kernel<T, D, NEOX, AXES, SETKV, KVFP8, GATED, WHOLE>, dim3(p.blocks), p.threads, 0, stream, lead1, lead2, lead3, \
                          UnitBlock<D, AXES, SETKV, KVFP8, GATED>(b))
-    const bool whole = p.stream && (is_half<T> || p.whole_lines);
+    const bool whole = p.stream && p.whole_lines;
     if (kHalfLines && whole && b.gate) GPUK_LAUNCH_UNITS(true, kHalfLines);
     else if (kHalfLines && whole) GPUK_LAUNCH_UNITS(false, kHalfLines);
     else if (b.gate) GPUK_LAUNCH_UNITS(true, false);
