@@ -489,7 +489,7 @@ struct RopeUnit {
 // with three axes and a cache, because the launch of a small call costs the host by both (see launch_kernel; a call of the
 // operator for 32 tokens of 64+8+8 heads into an fp8 cache 6.00 us with 10 scalars and a block of 184 bytes, 5.50 so).
 //   first:  qkv_in, positions, total_units, upt_magic, hq, hk
-//   second: hv_and_flags, eps, ps_token
+//   second: hv_and_flags, units_per_token with one axis and no fp8 cache (where the block has room for eps), else eps, ps_token
 //   third:  ps_axis with three axes, else kv_loc with a cache
 // hv_and_flags: hv in bits 0-23, log2 of the waves per workgroup in bits 24-25, stream_rows in bit 26, merge_rows in bit 27.
 // (The three-axis instantiations of 128 elements per head with a cache are held to 64 registers, eight waves per SIMD: the
@@ -497,10 +497,11 @@ struct RopeUnit {
 constexpr size_t kUnitLeadBytes = sizeof(u32x8) + sizeof(u32x4) + sizeof(u32x2);
 template <int D, int AXES, bool SETKV, bool KVFP8, bool GATED>
 struct UnitBlock {  // the argument block, behind the leading parameters
-    static constexpr int MAP_WORDS = AXES == 3 ? (D / 2 + 31) / 32 : 0, SCALES = KVFP8 ? 2 : 0, GATE = GATED ? 1 : 0;
+    static constexpr bool HAS_EPS = AXES == 1 && !KVFP8;
+    static constexpr int MAP_WORDS = AXES == 3 ? (D / 2 + 31) / 32 : 0, SCALES = KVFP8 ? 2 : HAS_EPS ? 1 : 0, GATE = GATED ? 1 : 0;
     static constexpr int POINTERS = 3 + (SETKV ? 3 : 0) + (SETKV && AXES == 3 ? 1 : 0), WORDS = 2 * MAP_WORDS + SCALES + GATE;
     const void *pointers[POINTERS];            // qw, kw, cos_sin; with a cache q_out, k_cache, v_cache; with three axes kv_loc as well
-    uint32_t words[WORDS > 0 ? WORDS : 1];     // axis1, axis2; k_scale, v_scale; gate
+    uint32_t words[WORDS > 0 ? WORDS : 1];     // axis1, axis2; k_scale, v_scale, or eps; gate
 
     explicit UnitBlock(const RopeArgs &a) : pointers{}, words{} {
         int n = 0;
@@ -509,6 +510,7 @@ struct UnitBlock {  // the argument block, behind the leading parameters
         if constexpr (SETKV && AXES == 3) pointers[n++] = a.kv_loc;
         for (int i = 0; i < MAP_WORDS; ++i) words[i] = a.axis1[i], words[MAP_WORDS + i] = a.axis2[i];
         if constexpr (KVFP8) words[2 * MAP_WORDS] = __builtin_bit_cast(uint32_t, a.k_scale), words[2 * MAP_WORDS + 1] = __builtin_bit_cast(uint32_t, a.v_scale);
+        if constexpr (HAS_EPS) words[0] = __builtin_bit_cast(uint32_t, a.eps);
         if constexpr (GATED) words[2 * MAP_WORDS + SCALES] = a.gate;
     }
 };
@@ -530,12 +532,12 @@ rope_rms_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const 
     a.upt_magic = first[5];
     a.hq = (int)first[6];
     a.hk = (int)first[7];
-    a.units_per_token = (uint32_t)(a.hq + a.hk + Unit::HPW - 1) / Unit::HPW;
+    a.units_per_token = Block::HAS_EPS ? second[1] : (uint32_t)(a.hq + a.hk + Unit::HPW - 1) / Unit::HPW;
     a.hv = (int)(hv_and_flags & 0xffffffu);
     a.stream_rows = (hv_and_flags >> 26) & 1u;
     a.merge_rows = (hv_and_flags >> 27) & 1u;
-    const uint32_t eps_bits = second[1];  // (a bit cast of the vector's element itself takes the first one)
-    a.eps = __builtin_bit_cast(float, eps_bits);
+    const uint32_t second1 = second[1];  // (a bit cast of the vector's element itself takes the first one)
+    if constexpr (!Block::HAS_EPS) a.eps = __builtin_bit_cast(float, second1);
     a.ps_token = (int64_t)(((uint64_t)second[3] << 32) | second[2]);
     const uint64_t third64 = ((uint64_t)third[1] << 32) | third[0];
     a.ps_axis = AXES == 3 ? (int64_t)third64 : 0;
@@ -572,10 +574,11 @@ rope_rms_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const 
         a.k_scale = __builtin_bit_cast(float, block->words[2 * Block::MAP_WORDS]);
         a.v_scale = __builtin_bit_cast(float, block->words[2 * Block::MAP_WORDS + 1]);
     }
+    if constexpr (Block::HAS_EPS) a.eps = __builtin_bit_cast(float, block->words[0]);
     if constexpr (GATED) a.gate = block->words[2 * Block::MAP_WORDS + Block::SCALES];
     // ... all of it in one go (the compiler otherwise fetches each field where it is first used, the output pointers
     // after the arithmetic, and the wave waits for the scalar cache once more before it can store)
-    asm volatile("" ::"s"(a.qw), "s"(a.kw), "s"(a.cos_sin));
+    asm volatile("" ::"s"(a.qw), "s"(a.kw), "s"(a.cos_sin), "s"(a.eps));
     if constexpr (SETKV) asm volatile("" ::"s"(a.q_out), "s"(a.k_cache), "s"(a.v_cache));
     if constexpr (SETKV && AXES == 3) asm volatile("" ::"s"(a.kv_loc));
     if constexpr (KVFP8) asm volatile("" ::"s"(a.k_scale), "s"(a.v_scale));
@@ -1481,7 +1484,8 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
     const void *third = a.kv_loc;  // (see rope_rms_kernel)
     if constexpr (AXES == 3) third = reinterpret_cast<const void *>((intptr_t)a.ps_axis);
     const u32x8 lead1 = {low_half(a.qkv_in), high_half(a.qkv_in), low_half(a.positions), high_half(a.positions), a.total_units, a.upt_magic, (uint32_t)a.hq, (uint32_t)a.hk};
-    const u32x4 lead2 = {(uint32_t)a.hv | (log2_waves << 24) | (b.stream_rows << 26) | (a.merge_rows << 27), __builtin_bit_cast(uint32_t, a.eps), (uint32_t)a.ps_token, (uint32_t)((uint64_t)a.ps_token >> 32)};
+    const u32x4 lead2 = {(uint32_t)a.hv | (log2_waves << 24) | (b.stream_rows << 26) | (a.merge_rows << 27),
+                         UnitBlock<D, AXES, SETKV, KVFP8, false>::HAS_EPS ? a.units_per_token : __builtin_bit_cast(uint32_t, a.eps), (uint32_t)a.ps_token, (uint32_t)((uint64_t)a.ps_token >> 32)};
     const u32x2 lead3 = {low_half(third), high_half(third)};
 #define GPUK_LAUNCH_UNITS(GATED, WHOLE)                                                                                 \
     return launch_kernel(rope_rms_kernel<T, D, NEOX, AXES, SETKV, KVFP8, GATED, WHOLE>, dim3(p.blocks), p.threads, 0, stream, lead1, lead2, lead3, \
