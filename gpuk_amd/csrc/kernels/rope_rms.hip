@@ -1070,7 +1070,7 @@ struct TwoWayArgs {
 // before its first request.)  The block (weights, tables, outputs, the division constants) is fetched behind the
 // activations, in one batch.  128 bytes in all (see launch_kernel; a small call of the operator 7.70 / 7.27 us with nine scalars
 // and a block of 160 bytes / so).
-//   first:  q0, k0, q1, k1      second: tokens0, tokens1, heads_q, heads_k      third: eps, stream
+//   first:  q0, k0, q1, k1      second: tokens0, tokens1, heads_q, heads_k      third: eps, stream (bit 0) and gate (above)
 struct TwoWayBlock {
     const void *w[4], *cos_sin[2];
     void *out[2];
@@ -1079,12 +1079,13 @@ struct TwoWayBlock {
 constexpr size_t kTwoWayLeadBytes = sizeof(u32x8) + sizeof(u32x4) + sizeof(u32x2);
 static_assert(kTwoWayLeadBytes % alignof(TwoWayBlock) == 0, "offset of the block");
 
-template <typename T, int D, bool NEOX, bool WHOLE>
+template <typename T, int D, bool NEOX, bool WHOLE, bool GATED>
 __global__ void __launch_bounds__(256)
 rope_rms_2way_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const TwoWayBlock rest) {
     const uint32_t tokens0 = second[0], tokens1 = second[1], heads_q = second[2], heads_k = second[3];
-    const uint32_t eps_bits = third[0], stream = third[1];
+    const uint32_t eps_bits = third[0], stream = third[1] & 1u, gate = third[1] >> 1;
     const float eps = __builtin_bit_cast(float, eps_bits);
+    const uint64_t entry = GATED ? __builtin_amdgcn_s_memrealtime() : 0;
     const void *q0 = (const void *)global_ptr<const char>(first[0], first[1]), *k0 = (const void *)global_ptr<const char>(first[2], first[3]);
     const void *q1 = (const void *)global_ptr<const char>(first[4], first[5]), *k1 = (const void *)global_ptr<const char>(first[6], first[7]);
     constexpr int LPH = D / 16, HPW = 64 / LPH, HALF = D / 2;
@@ -1139,6 +1140,10 @@ rope_rms_2way_kernel(const u32x8 first, const u32x4 second, const u32x2 third, c
     if constexpr (WHOLE) exchange_lines(xa, xb);
     u32x4 oa, ob;
     norm_rotate<T, D, NEOX>(xa, xb, wa, wb, cosv, sinv, eps, oa, ob);
+    if constexpr (GATED) {  // (all waves resident at once: no store before the launch's reads are through, as in RopeUnit::finish)
+        asm volatile("" ::"v"(oa), "v"(ob));
+        while (__builtin_amdgcn_s_memrealtime() < entry + gate) __builtin_amdgcn_s_sleep(1);
+    }
     // (the rows of a segment are contiguous in its output too)
     const int64_t out_token = (int64_t)batch * (tokens0 + tokens1) + (stream_id ? tokens0 : 0u);
     uint16_t *dst = static_cast<uint16_t *>(kind ? out_k : out_q) + out_token * heads * D;
@@ -1208,20 +1213,36 @@ __global__ void __launch_bounds__(256) rope_rms_2way_wide_kernel(const TwoWayArg
     }
 }
 
+int g_unit_gate = -1;     // gate of the kernels with one wave per unit: -1 = built-in rule, 0 = none, > 0 = ticks
+constexpr uint32_t kResidentUnits = 8192;  // waves of those kernels the chip holds at once (8 per SIMD)
 int g_stream_rows = 0;    // output rows stored past the L2: 0 = built-in rule, 1 = never, 2 = always
 constexpr int64_t kWholeLinesFromBytes = 13'500'000, kWholeLinesFromBytesRagged = 18'000'000;  // bfloat16, see exchange_lines
 
 template <typename T, int D>
 int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stream) {
     const dim3 grid((a.unit_end[3] + 3) / 4, batch);
+    const int64_t rows = (int64_t)batch * ((int64_t)a.rows[0] + a.rows[1] + a.rows[2] + a.rows[3]), waves = (int64_t)batch * a.unit_end[3];
+    // The store gate (see RopeUnit::finish) where the waves are all resident at once: 1.1 times the read time at 7 TB/s, 1.25 with
+    // pairwise rotation, whose two table pieces per chunk lengthen the loading.  Half precision from three eighths of a round on (us, ungated /
+    // gated: 4.74 / 4.13 at 3820 waves, 5.08 / 4.42 at 4476, 6.99 / 6.2 at 7075, 7.24 / 6.1 at 7730; pairwise 6.56 / 5.8 at 6304, 7.38 / 6.6 at 7638; level at 2694);
+    // bfloat16, whose arithmetic takes longer than the reads of a full round, from a half to 27/32 of it (4.58 / 4.72 at 3950, 5.18 / 4.94 at 4962, 5.55 / 5.0 at 5072, 6.30 / 6.0 at 6080;
+    // 7.76 / 7.9 at 7938; pairwise from 15/32, 6.16 / 5.5 at 5201), and not heads of 64 rotated by halves (5.58 / 5.68 at 4582, 7.79 / 8.0 at 7356).
+    uint32_t gate = 0;
+    const bool gated = is_half<T> ? 8 * waves >= 3 * kResidentUnits && waves <= kResidentUnits
+                                  : 32 * waves >= (neox ? 16 : 15) * kResidentUnits && 32 * waves <= 27 * kResidentUnits && (D != 64 || !neox);
+    if (g_unit_gate > 0) gate = (uint32_t)g_unit_gate;
+    else if (g_unit_gate < 0 && gated) gate = (uint32_t)((neox ? 1.1 : 1.25) * (double)(2 * rows * D) / 70000.0);
     const u32x8 first = {low_half(a.in[0]), high_half(a.in[0]), low_half(a.in[1]), high_half(a.in[1]), low_half(a.in[2]), high_half(a.in[2]), low_half(a.in[3]), high_half(a.in[3])};
     const u32x4 second = {(uint32_t)a.tokens0, (uint32_t)a.tokens1, a.heads[0], a.heads[1]};
-    const u32x2 third = {__builtin_bit_cast(uint32_t, a.eps), a.stream};
+    const u32x2 third = {__builtin_bit_cast(uint32_t, a.eps), a.stream | (gate << 1)};
     const TwoWayBlock rest = {{a.w[0], a.w[1], a.w[2], a.w[3]}, {a.cos_sin[0], a.cos_sin[1]}, {a.out[0], a.out[1]}, {a.heads_magic[0], a.heads_magic[1]}};
 #define GPUK_LAUNCH_2WAY(NEOX, WHOLE)                                                                                  \
-    return launch_kernel(rope_rms_2way_kernel<T, D, NEOX, WHOLE>, grid, 256, 0, stream, first, second, third, rest)
+    do {                                                                                                               \
+        if (gate) return launch_kernel(rope_rms_2way_kernel<T, D, NEOX, WHOLE, true>, grid, 256, 0, stream, first, second, third, rest); \
+        return launch_kernel(rope_rms_2way_kernel<T, D, NEOX, WHOLE, false>, grid, 256, 0, stream, first, second, third, rest); \
+    } while (0)
     constexpr bool kHalfLines = D == 64;  // see exchange_lines
-    const int64_t call_bytes = 4 * (int64_t)batch * ((int64_t)a.rows[0] + a.rows[1] + a.rows[2] + a.rows[3]) * D;
+    const int64_t call_bytes = 4 * rows * D;
     const bool whole = a.stream && (is_half<T> || g_stream_rows == 2 || call_bytes >= kWholeLinesFromBytes);
     if (neox && kHalfLines && whole) GPUK_LAUNCH_2WAY(true, kHalfLines);
     else if (kHalfLines && whole) GPUK_LAUNCH_2WAY(false, kHalfLines);
@@ -1262,8 +1283,6 @@ int g_block_threads = 0;  // 0 = default
 int g_merge_rows = 0;     // mRoPE rows merged on load where the sections allow: 0 = yes, 1 = never
 int g_token_waves = 0;    // one-wave-per-token kernel: 0 = built-in rule, 1 = never, 2 = wherever it fits, 3 = likewise, two items per wave where that fits
 int g_token_gate = -1;    // its gate in ticks of 10 ns; -1 = from the bytes of the call
-int g_unit_gate = -1;     // gate of the kernel with one wave per unit: -1 = built-in rule, 0 = none, > 0 = ticks
-constexpr uint32_t kResidentUnits = 8192;  // waves of the one-wave-per-unit kernel the chip holds at once (8 per SIMD)
 
 // Streaming stores, measured on MI355X (32/8/8, 28/4/4 and 64/8/8 heads, head sizes 64-256, random slots): q_out /
 // K rows / in-place rows written past the L2 are ahead from about 10 MB per call on (64+8 heads, fp8 cache: 5.9

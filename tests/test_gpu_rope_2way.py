@@ -85,3 +85,31 @@ def test_fp16_and_rejections(device):
     with pytest.raises(RuntimeError):   # non-contiguous input (reference: TORCH_CHECK fused_rope.cpp:175)
         gpuk.fused_rope_rms_2way(d(c["q0"]).transpose(1, 2), d(c["k0"]), d(c["q1"]), d(c["k1"]), *[d(w) for w in c["w"]],
                                  d(c["cs0"]), d(c["cs1"]), B, T0, T1, Hq, Hk, D, False, 1e-6)
+
+
+@pytest.mark.parametrize("B,T0,T1,Hq,Hk,D", [(1, 1, 0, 1, 1, 256), (2, 7, 2, 16, 17, 64), (3, 5, 33, 7, 3, 128), (1, 200, 333, 24, 25, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_store_gate_changes_no_bits(device, B, T0, T1, Hq, Hk, D, dtype):
+    """Launches whose waves are all resident at once hold their stores back until the launch's reads are through: no gate, the
+    shortest and 4 us give the same bits, the row behind each output included."""
+    from gpuk_amd import capi
+
+    for il in (False, True):
+        c = make(B, T0, T1, Hq, Hk, D, seed=T0 + 10 * Hq, dtype=dtype)
+        d = lambda t: t.to(device)
+        got = []
+        try:
+            for gate in (0, 1, 400):
+                capi.set_tuning("rope_unit_gate", gate)
+                out = [torch.full((B * (T0 + T1) + 1, h, D), 7.0, dtype=dtype, device=device) for h in (Hq, Hk)]
+                capi.rope_rms_2way(d(c["q0"]), d(c["k0"]), d(c["q1"]), d(c["k1"]), *[d(w) for w in c["w"]], d(c["cs0"]),
+                                   d(c["cs1"]), B, T0, T1, Hq, Hk, D, il, 1e-6, *out)
+                torch.cuda.synchronize()
+                got.append([o.cpu().view(torch.int16) for o in out])
+        finally:
+            capi.set_tuning("rope_unit_gate", -1)
+        for other in got[1:]:
+            assert all(torch.equal(a, b) for a, b in zip(got[0], other)), (il, "the gate changes bits")
+        ref = O.rope_rms_2way_ref(c["q0"], c["k0"], c["q1"], c["k1"], *c["w"], c["cs0"], c["cs1"], B, T0, T1, Hq, Hk, D, il, 1e-6)
+        for out, want in zip(got[0], ref):
+            assert_rotated_close(out[:-1].view(dtype).reshape(want.shape), want, f"gated two streams il={il}")
