@@ -55,6 +55,11 @@ extern "C" int gpuk_set_tuning(const char *key, int value) {
         gpuk::set_rope_tuning(1, value);
         return GPUK_OK;
     }
+    if (strcmp(key, "rope_2way_units") == 0) {  // 0 = built-in rule, 1, 2
+        if (value < 0 || value > 2) return GPUK_ERR_INVALID_ARG;
+        gpuk::set_rope_tuning(7, value);
+        return GPUK_OK;
+    }
     if (strcmp(key, "rope_token_gate") == 0) {  // ticks of 10 ns; -1 = from the bytes of the call
         if (value < -1 || value > 5000) return GPUK_ERR_INVALID_ARG;
         gpuk::set_rope_tuning(2, value);

@@ -1157,6 +1157,104 @@ rope_rms_2way_kernel(const u32x8 first, const u32x4 second, const u32x2 third, c
     }
 }
 
+// The same for batches of one to two rounds of that: a wave takes two groups of heads, one after the other in their segment, which
+// share their weights, so that a round holds 16384 groups (half precision, eight waves per SIMD) or 14336 (bfloat16, whose unpacked
+// arithmetic spills three registers at eight: seven), and holds its stores until the launch's reads are through.  NeoX-style
+// rotation only, sizes measured in launch_2way.  (A kernel of its own: with the number of groups as a template parameter the allocator gave
+// the kernel above 46 registers for 35 and 2 x (678 + 3608) tokens took 35.4 us for 35.3.)
+constexpr int kTwoUnitWaves[2] = {7, 8};  // per SIMD: bfloat16, half precision
+template <typename T, int D, bool WHOLE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kTwoUnitWaves[is_half<T>])))
+rope_rms_2way_pairs_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const TwoWayBlock rest) {
+    const uint32_t tokens0 = second[0], tokens1 = second[1], heads_q = second[2], heads_k = second[3];
+    const uint32_t eps_bits = third[0], stream = third[1] & 1u, gate = third[1] >> 1;
+    const float eps = __builtin_bit_cast(float, eps_bits);
+    const uint64_t entry = __builtin_amdgcn_s_memrealtime();
+    const void *q0 = (const void *)global_ptr<const char>(first[0], first[1]), *k0 = (const void *)global_ptr<const char>(first[2], first[3]);
+    const void *q1 = (const void *)global_ptr<const char>(first[4], first[5]), *k1 = (const void *)global_ptr<const char>(first[6], first[7]);
+    constexpr int LPH = D / 16, HPW = 64 / LPH, HALF = D / 2, UNITS = 2, RPW = HPW * UNITS;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t unit = blockIdx.x * 4 + wave;
+    const uint32_t rows0 = tokens0 * heads_q, rows1 = tokens0 * heads_k, rows2 = tokens1 * heads_q, rows3 = tokens1 * heads_k;
+    const uint32_t end0 = (rows0 + RPW - 1) / RPW, end1 = end0 + (rows1 + RPW - 1) / RPW, end2 = end1 + (rows2 + RPW - 1) / RPW,
+                   end3 = end2 + (rows3 + RPW - 1) / RPW;
+    if (unit >= end3) return;
+    const int seg = (unit >= end0) + (unit >= end1) + (unit >= end2);  // wave-uniform
+    const uint32_t unit_in_seg = unit - (seg == 0 ? 0u : seg == 1 ? end0 : seg == 2 ? end1 : end2);
+    const int kind = seg & 1, stream_id = seg >> 1;  // q|k, stream 0|1
+    const uint32_t heads = kind ? heads_k : heads_q;
+    const uint32_t rows = seg == 0 ? rows0 : seg == 1 ? rows1 : seg == 2 ? rows2 : rows3;
+    const void *in = seg == 0 ? q0 : seg == 1 ? k0 : seg == 2 ? q1 : k1;
+    const int batch = blockIdx.y;
+
+    const int lane = threadIdx.x & 63, sub = lane % LPH, hl = lane / LPH;
+    const int c0 = 8 * sub, c1 = HALF + 8 * sub;
+    const uint16_t *batch_in = static_cast<const uint16_t *>(in) + (int64_t)batch * rows * D;
+    u32x4 xa[UNITS], xb[UNITS];
+    uint32_t row[UNITS], row_raw[UNITS], even[UNITS];  // (token, head) flattened inside the segment; row_raw may lie behind it
+#pragma unroll
+    for (int k = 0; k < UNITS; ++k) {
+        row_raw[k] = unit_in_seg * RPW + k * HPW + hl;
+        row[k] = min(row_raw[k], rows - 1);
+        even[k] = row_raw[k] & ~1u;  // (heads of one line: the two rows whose lines the lane moves pieces of)
+        const uint16_t *src_a = batch_in + (int64_t)row[k] * D + c0, *src_b = src_a + HALF;
+        if constexpr (WHOLE) {
+            src_a = batch_in + (int64_t)min(even[k], rows - 1) * D + 8 * (lane & 7);
+            src_b = batch_in + (int64_t)min(even[k] + 1, rows - 1) * D + 8 * (lane & 7);
+        }
+        xa[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_a));
+        xb[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src_b));
+    }
+
+    typedef const __attribute__((address_space(4))) TwoWayBlock *BlockPtr;
+    BlockPtr block = (BlockPtr)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + kTwoWayLeadBytes);
+    asm volatile("" : "+s"(block));
+    const void *w0 = as_global(block->w[0]), *w1 = as_global(block->w[1]), *w2 = as_global(block->w[2]), *w3 = as_global(block->w[3]);
+    const void *table0 = as_global(block->cos_sin[0]), *table1 = as_global(block->cos_sin[1]);
+    void *out_q = as_global(block->out[0]), *out_k = as_global(block->out[1]);
+    const uint32_t magic_q = block->heads_magic[0], magic_k = block->heads_magic[1];
+    asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(w3), "s"(table0), "s"(table1), "s"(out_q), "s"(out_k), "s"(magic_q), "s"(magic_k));
+    const uint32_t magic = kind ? magic_k : magic_q;
+    uint32_t token[UNITS];
+#pragma unroll
+    for (int k = 0; k < UNITS; ++k) token[k] = magic ? __umulhi(row[k], magic) : row[k];
+    const uint16_t *wsrc = static_cast<const uint16_t *>(seg == 0 ? w0 : seg == 1 ? w1 : seg == 2 ? w2 : w3);
+    const u32x4 wa = *reinterpret_cast<const u32x4 *>(wsrc + c0);
+    const u32x4 wb = *reinterpret_cast<const u32x4 *>(wsrc + c1);
+    u32x4 cosv[UNITS], sinv[UNITS];
+#pragma unroll
+    for (int k = 0; k < UNITS; ++k) {
+        const uint16_t *table = static_cast<const uint16_t *>(stream_id ? table1 : table0) + (int64_t)token[k] * D;
+        cosv[k] = load_trig<D, true>(table, sub);
+        sinv[k] = load_trig<D, true>(table + HALF, sub);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+#pragma unroll
+    for (int k = 0; k < UNITS; ++k) {  // (in place: the rotated rows take the registers of the activations, one group finished before the next)
+        if constexpr (WHOLE) exchange_lines(xa[k], xb[k]);
+        u32x4 oa, ob;
+        norm_rotate<T, D, true>(xa[k], xb[k], wa, wb, cosv[k], sinv[k], eps, oa, ob);
+        xa[k] = oa, xb[k] = ob;
+        asm volatile("" : "+v"(xa[k]), "+v"(xb[k]));
+    }
+    while (__builtin_amdgcn_s_memrealtime() < entry + gate) __builtin_amdgcn_s_sleep(1);
+    // (the rows of a segment are contiguous in its output too)
+    const int64_t out_token = (int64_t)batch * (tokens0 + tokens1) + (stream_id ? tokens0 : 0u);
+    uint16_t *out = static_cast<uint16_t *>(kind ? out_k : out_q) + out_token * heads * D;
+#pragma unroll
+    for (int k = 0; k < UNITS; ++k) {
+        if constexpr (WHOLE) {
+            exchange_lines(xa[k], xb[k]);
+            uint16_t *dst = out + (int64_t)even[k] * D + 8 * (lane & 7);
+            if (even[k] + 1 < rows) store_pair<D * 2>(dst, xa[k], xb[k], true);
+            else if (even[k] < rows) store_chunk_streamed(dst, xa[k]);
+        } else if (row_raw[k] < rows) {
+            store_pair<HALF * 2>(out + (int64_t)row[k] * D + c0, xa[k], xb[k], stream != 0);
+        }
+    }
+}
+
 // fp32 / fp64 form of the two-stream op (the reference dispatches float and double here too:
 // src/ops/fused_rope.cpp:197-200): one wave per (token, head) row of a segment, lane l owns rotation pairs l, l+64, ...;
 // plain arithmetic in the activation type F around an fp32 variance, every product rounded before the add.  The host
@@ -1215,12 +1313,13 @@ __global__ void __launch_bounds__(256) rope_rms_2way_wide_kernel(const TwoWayArg
 
 int g_unit_gate = -1;     // gate of the kernels with one wave per unit: -1 = built-in rule, 0 = none, > 0 = ticks
 constexpr uint32_t kResidentUnits = 8192;  // waves of those kernels the chip holds at once (8 per SIMD)
+int g_two_way_units = 0;  // units per wave of the two-stream kernel: 0 = built-in rule, 1 or 2
 int g_stream_rows = 0;    // output rows stored past the L2: 0 = built-in rule, 1 = never, 2 = always
 constexpr int64_t kWholeLinesFromBytes = 13'500'000, kWholeLinesFromBytesRagged = 18'000'000;  // bfloat16, see exchange_lines
 
 template <typename T, int D>
 int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stream) {
-    const dim3 grid((a.unit_end[3] + 3) / 4, batch);
+    constexpr int HPW = 64 / (D / 16);
     const int64_t rows = (int64_t)batch * ((int64_t)a.rows[0] + a.rows[1] + a.rows[2] + a.rows[3]), waves = (int64_t)batch * a.unit_end[3];
     // The store gate (see RopeUnit::finish) where the waves are all resident at once: 1.1 times the read time at 7 TB/s, 1.25 with
     // pairwise rotation, whose two table pieces per chunk lengthen the loading.  Half precision from three eighths of a round on (us, ungated /
@@ -1232,12 +1331,23 @@ int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stre
                                   : 32 * waves >= (neox ? 16 : 15) * kResidentUnits && 32 * waves <= 27 * kResidentUnits && (D != 64 || !neox);
     if (g_unit_gate > 0) gate = (uint32_t)g_unit_gate;
     else if (g_unit_gate < 0 && gated) gate = (uint32_t)((neox ? 1.1 : 1.25) * (double)(2 * rows * D) / 70000.0);
+    // Two units per wave where a round holds the batch so and not with one, gate 1.03 times the read time.  Rotated by halves only: pairwise it is level
+    // to 10 % behind (us, one unit / two: 9.39 / 8.1 at 11081 waves, 10.32 / 8.8 at 12366 and 12.47 / 10.8 at 16070 in half precision, 8.86 / 7.8 at
+    // 9740, 10.48 / 8.9 at 12024, 11.50 / 10.1 at 13752 in bfloat16; 6.68 / 7.0 at 7198; pairwise 10.06 / 10.5 at 11915, 11.86 / 12.7 at 14450).
+    int64_t pairs = 0;
+    for (int seg = 0; seg < 4; ++seg) pairs += ((int64_t)a.rows[seg] + 2 * HPW - 1) / (2 * HPW);
+    const bool fits = (int64_t)batch * pairs <= 1024 * kTwoUnitWaves[is_half<T>];
+    const bool two_units = neox && (g_two_way_units == 2 || (g_two_way_units == 0 && g_unit_gate < 0 && waves > kResidentUnits && fits));
+    if (two_units && g_unit_gate < 0) gate = (uint32_t)std::min(1.03 * (double)(2 * rows * D) / 70000.0, 5000.0);
+    const dim3 grid((unsigned)(((two_units ? pairs : a.unit_end[3]) + 3) / 4), batch);
     const u32x8 first = {low_half(a.in[0]), high_half(a.in[0]), low_half(a.in[1]), high_half(a.in[1]), low_half(a.in[2]), high_half(a.in[2]), low_half(a.in[3]), high_half(a.in[3])};
     const u32x4 second = {(uint32_t)a.tokens0, (uint32_t)a.tokens1, a.heads[0], a.heads[1]};
     const u32x2 third = {__builtin_bit_cast(uint32_t, a.eps), a.stream | (gate << 1)};
     const TwoWayBlock rest = {{a.w[0], a.w[1], a.w[2], a.w[3]}, {a.cos_sin[0], a.cos_sin[1]}, {a.out[0], a.out[1]}, {a.heads_magic[0], a.heads_magic[1]}};
 #define GPUK_LAUNCH_2WAY(NEOX, WHOLE)                                                                                  \
     do {                                                                                                               \
+        if constexpr (NEOX)                                                                                            \
+            if (two_units) return launch_kernel(rope_rms_2way_pairs_kernel<T, D, WHOLE>, grid, 256, 0, stream, first, second, third, rest); \
         if (gate) return launch_kernel(rope_rms_2way_kernel<T, D, NEOX, WHOLE, true>, grid, 256, 0, stream, first, second, third, rest); \
         return launch_kernel(rope_rms_2way_kernel<T, D, NEOX, WHOLE, false>, grid, 256, 0, stream, first, second, third, rest); \
     } while (0)
@@ -1711,6 +1821,7 @@ void set_rope_tuning(int key, int value) {
     if (key == 2) g_token_gate = value;
     if (key == 3) g_stream_rows = value;
     if (key == 4) g_merge_rows = value;
+    if (key == 7) g_two_way_units = value;
 }
 
 }  // namespace gpuk

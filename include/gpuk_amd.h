@@ -229,7 +229,8 @@ int gpuk_increment_floats(float *data, int64_t n, void *stream);
  * the rope kernels stored past the L2: 1 never, 2 always), "rope_merge_rows" (1: never let the lanes of an mRoPE
  * token load their cos/sin pieces straight from the row of their axis), "rope_token_waves" (the kernel in which one
  * wave takes a token or a part of one: 1 never, 2 wherever the shape fits it, 3 likewise with two of them per wave where that fits), "rope_token_gate" and "rope_unit_gate" (the
- * store gate of the two rope kernels, in ticks as above: -1 the built-in rule, 0 never).  The results do not depend
+ * store gate of the two rope kernels, the latter of the two-stream kernel as well, in ticks as above: -1 the built-in rule, 0
+ * never), "rope_2way_units" (1 or 2 groups of heads per wave of the two-stream kernel, 2 with rotation by halves only).  The results do not depend
  * on any of them.  Unknown keys or values return GPUK_ERR_INVALID_ARG.  The settings are process-global plain
  * variables read at launch: set them from one thread while no other thread is launching.  Not part of the
  * reference. */

@@ -89,9 +89,10 @@ def test_fp16_and_rejections(device):
 
 @pytest.mark.parametrize("B,T0,T1,Hq,Hk,D", [(1, 1, 0, 1, 1, 256), (2, 7, 2, 16, 17, 64), (3, 5, 33, 7, 3, 128), (1, 200, 333, 24, 25, 128)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_store_gate_changes_no_bits(device, B, T0, T1, Hq, Hk, D, dtype):
-    """Launches whose waves are all resident at once hold their stores back until the launch's reads are through: no gate, the
-    shortest and 4 us give the same bits, the row behind each output included."""
+def test_store_gate_and_units_per_wave_change_no_bits(device, B, T0, T1, Hq, Hk, D, dtype):
+    """Launches whose waves are all resident at once hold their stores back until the launch's reads are through, and a wave may
+    take two groups of heads: no gate, the shortest and 4 us, one group and two (segments of an odd number of groups, of part of
+    one, and of none among them) give the same bits, the row behind each output included."""
     from gpuk_amd import capi
 
     for il in (False, True):
@@ -99,8 +100,9 @@ def test_store_gate_changes_no_bits(device, B, T0, T1, Hq, Hk, D, dtype):
         d = lambda t: t.to(device)
         got = []
         try:
-            for gate in (0, 1, 400):
+            for units, gate in ((1, 0), (1, 1), (1, 400), (2, 0), (2, 400)):
                 capi.set_tuning("rope_unit_gate", gate)
+                capi.set_tuning("rope_2way_units", units)
                 out = [torch.full((B * (T0 + T1) + 1, h, D), 7.0, dtype=dtype, device=device) for h in (Hq, Hk)]
                 capi.rope_rms_2way(d(c["q0"]), d(c["k0"]), d(c["q1"]), d(c["k1"]), *[d(w) for w in c["w"]], d(c["cs0"]),
                                    d(c["cs1"]), B, T0, T1, Hq, Hk, D, il, 1e-6, *out)
@@ -108,8 +110,29 @@ def test_store_gate_changes_no_bits(device, B, T0, T1, Hq, Hk, D, dtype):
                 got.append([o.cpu().view(torch.int16) for o in out])
         finally:
             capi.set_tuning("rope_unit_gate", -1)
+            capi.set_tuning("rope_2way_units", 0)
         for other in got[1:]:
-            assert all(torch.equal(a, b) for a, b in zip(got[0], other)), (il, "the gate changes bits")
+            assert all(torch.equal(a, b) for a, b in zip(got[0], other)), (il, "gate or units change bits")
         ref = O.rope_rms_2way_ref(c["q0"], c["k0"], c["q1"], c["k1"], *c["w"], c["cs0"], c["cs1"], B, T0, T1, Hq, Hk, D, il, 1e-6)
         for out, want in zip(got[0], ref):
             assert_rotated_close(out[:-1].view(dtype).reshape(want.shape), want, f"gated two streams il={il}")
+
+
+@pytest.mark.parametrize("T1", [1365, 1366, 2388, 2389, 2729, 2731])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_two_units_per_wave_by_rule(device, T1, dtype):
+    """Around the sizes where a wave begins and ends to take two groups of heads (8192 groups; 14336 in bfloat16, 16384 in half
+    precision): the same bits as with one group per wave."""
+    from gpuk_amd import capi
+
+    B, T0, Hq, Hk, D = 1, 1, 24, 24, 128
+    c = make(B, T0, T1, Hq, Hk, D, seed=T1, dtype=dtype)
+    got = [run_op(c, B, T0, T1, Hq, Hk, D, False, device)]
+    try:
+        capi.set_tuning("rope_2way_units", 1)
+        capi.set_tuning("rope_unit_gate", 0)
+        got.append(run_op(c, B, T0, T1, Hq, Hk, D, False, device))
+    finally:
+        capi.set_tuning("rope_2way_units", 0)
+        capi.set_tuning("rope_unit_gate", -1)
+    assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(*got))
