@@ -56,15 +56,6 @@ __device__ __forceinline__ float max3_abs(float m, float a, float b) {
     return r;
 }
 
-// a / b for finite a and b > 0 comfortably normal, given rcp = RN(1/b): the correctly rounded quotient by one
-// multiply and two fused multiply-adds (Markstein), arranged so that a = -0 gives -0: with e = q*b - a the last step
-// fma(-e, rcp, q) adds two negative zeros, where the usual fma(a - q*b, rcp, q) adds +0 and -0.
-__device__ __forceinline__ float div_by_rcp_finite(float a, float b, float rcp) {
-    const float q = a * rcp;
-    const float e = __builtin_fmaf(q, b, -a);
-    return __builtin_fmaf(-e, rcp, q);
-}
-
 // 1 / sqrt(sumsq / H + eps).  The mean as an exact IEEE quotient: a multiplication when H is a power of two (exact, and
 // rounded like the quotient when the result is subnormal), elsewhere by multiply and two fused multiply-adds (exact on the
 // guarded range, see div_by_rcp); then the short square root and reciprocal.  Every wave of a row walks this dependent chain

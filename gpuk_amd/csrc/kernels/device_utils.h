@@ -255,6 +255,15 @@ __device__ __forceinline__ float div_by_rcp(float a, float b, float rcp) {
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(e, rcp, q), b, a);
 }
 
+// a / b for finite a and b > 0 comfortably normal, given rcp = RN(1/b): the correctly rounded quotient by one
+// multiply and two fused multiply-adds (Markstein), arranged so that a = -0 gives -0: with e = q*b - a the last step
+// fma(-e, rcp, q) adds two negative zeros, where the usual fma(a - q*b, rcp, q) adds +0 and -0.
+__device__ __forceinline__ float div_by_rcp_finite(float a, float b, float rcp) {
+    const float q = a * rcp;
+    const float e = __builtin_fmaf(q, b, -a);
+    return __builtin_fmaf(-e, rcp, q);
+}
+
 // ---- Correctly rounded square root and reciprocal by short sequences.  The compiler's expansions of sqrtf() and of
 // 1.0f / x are correct for every operand and pay for it with rescaling and fix-up steps (about 20 and 11 dependent
 // instructions); on operands in the middle of the exponent range those steps do nothing.  These start from
