@@ -169,7 +169,8 @@ __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t 
 // Then, with bf16 and where no value of the wave comes near what has to be clamped (nor is infinite or a NaN), the quotients are the
 // short ones for finite numerators and the rounded pairs are converted as they are: what the many fp8 rows of a call without shared
 // KV heads wait for.  In us without / with, bf16: 900 tokens of 64+64+64 heads of 128 elements 18.5 / 17.05, of 64 elements (919
-// tokens) 11.2 / 10.5, 3000 of 32+32+32 26.95 / 24.8, 32 of 64+8+8 3.00 / 2.90, long calls with few KV heads level.  fp16 keeps the
+// tokens) 11.2 / 10.5, 3000 of 32+32+32 26.95 / 24.8, 32 of 64+8+8 3.00 / 2.90, long calls with few KV heads level; with a scale a thousand times too small, so that every wave
+// clamps, 3000 tokens of 32+32+32 27.8 / 28.6.  fp16 keeps the
 // general form: its own short one was 3 % faster at 2000 tokens of 32+32+32 heads (16.5 / 16.0) and 3 % slower at 4000 (27.95 / 28.7).
 template <typename T, bool FAST>
 __device__ __forceinline__ u32x2 quantize_chunk(const u32x4 &v, float scale, float rcp) {

@@ -387,8 +387,8 @@ def test_token_kernel_three_axes_and_two_tokens_per_wave(device, case, gate):
 
 def test_token_kernel_leaves_other_sections_to_the_other_kernel(device):
     """Sections that do not split at multiples of 8 frequencies, or the interleaved map, cannot take their cos/sin
-    pieces from one row per lane: even when the one-wave-per-token kernel is asked for, such calls run the other one
-    (and meet the oracle)."""
+    pieces from one row per lane: when the one-wave-per-token kernel is asked for, such calls run its form that merges the
+    three rows first (once the other kernel), and meet the oracle."""
     from gpuk_amd import capi
 
     capi.set_tuning("rope_token_waves", 3)
