@@ -830,6 +830,9 @@ int64_t resident_rows(int threads, int nchunk) {
     return (int64_t)kComputeUnits * (waves_per_cu / waves);
 }
 
+enum class RowType { BF16, FP16, F32 };
+template <typename T> constexpr RowType row_type = is_half<T> ? RowType::FP16 : RowType::BF16;
+
 // The store gate of a launch: for batches whose workgroups are all resident at once (2048 lanes per
 // compute unit) the time their reads take at 7 TB/s, the rate of a read-only kernel on this part, plus a twentieth;
 // 0 (stores as soon as they are ready) for larger batches, whose later workgroups read while earlier ones write
@@ -837,21 +840,29 @@ int64_t resident_rows(int threads, int nchunk) {
 // 768, 9.0 against 11.7 at 1024 (gate 1.0-1.1 times the read time; 10.2 with 0.9, 9.6 with 1.2), nothing gained and
 // 0.1 us lost below a quarter of a round; at 4096 elements 6.2 against 7.7 us at 1024 rows, 10.2 against 12.4 at 2048; 20-45 % slower where the
 // batch does not fit one round.
+// A compute unit reads no faster than its share of that rate by much, so a layer of rows (one per compute unit) that has just begun
+// takes nearly the time of a full one where rows are wide and a compute unit holds few: the gate is at least 0.93 of the time of whole layers for 16-bit
+// rows of four chunks per lane, else 0.86 with codes and 0.82 without (those store more, the rows' own gate / this one, us: bf16, four chunks, 522 rows
+// of 16384 14.7 / 12.0, 614 15.1 / 12.9, 775 18.4 / 16.2, 780 of 10240 12.3 / 10.8, 1030 of 12288 17.6 / 15.8, 1044 of 8192 11.3 / 10.8; two chunks, fp16
+// 559 of 8192 7.45 / 6.8, 377 of 16384 8.9 / 8.3, 300 of 8192 without codes 5.5 / 5.0; fp32 387 of 7168 8.1 / 7.4, 340 of 8192 8.9 / 7.6, 368
+// of 13184 14.5 / 12.1, without codes 318 of 5120 6.4 / 5.7; narrow rows and nearly full layers level.  More than that share holds back nearly full ones:
+// fp32 without codes 592 of 4096 7.1 / 7.3 with 0.9, 7.5 with 0.94).
 // short_rows: rows of two chunks per lane whose computation ends well ahead of the reads of a half-filled round (half precision,
 // static scale).  From two fifths of a round to eleven twentieths they wait 1.16 times the read time: 460 rows of 8192 elements
 // 6.28 / 5.72 us, 576 of 6144 6.55 / 6.05, 576 of 5120 5.46 / 5.3, level or slower below and above (1228 of 4096 6.6 / 6.8).
-uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, bool short_rows = false) {
+uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, RowType type, int quant) {
     if (g_gate >= 0) return (uint32_t)g_gate;
     const int64_t resident = resident_rows(threads, nchunk);
     if (tokens > resident || 4 * tokens < resident) return 0;
     // (four chunks per lane: the shape pick_shape takes to hold in one round what two chunks per lane cannot)
+    const bool short_rows = type == RowType::FP16 && quant == GPUK_QUANT_FP8_STATIC;
     const bool half_filled = short_rows && nchunk == 2 && 5 * tokens >= 2 * resident && 20 * tokens <= 11 * resident;
-    const double ticks = (half_filled ? 1.16 : nchunk >= 4 ? 1.08 : 1.05) * (double)(2 * tokens * row_bytes) / 70000.0;  // 70,000 bytes per tick of 10 ns
+    const double rows = (half_filled ? 1.16 : nchunk >= 4 ? 1.08 : 1.05) * (double)tokens;
+    const double share = nchunk == 4 && type != RowType::F32 ? 0.93 : quant != GPUK_QUANT_NONE ? 0.86 : 0.82;
+    const double layers = share * (double)((tokens + kComputeUnits - 1) / kComputeUnits * kComputeUnits);
+    const double ticks = 2 * std::max(rows, layers) * (double)row_bytes / 70000.0;  // 70,000 bytes per tick of 10 ns
     return (uint32_t)std::min(ticks, 5000.0);
 }
-
-enum class RowType { BF16, FP16, F32 };
-template <typename T> constexpr RowType row_type = is_half<T> ? RowType::FP16 : RowType::BF16;
 
 // Lanes per row and chunks per lane.  Two chunks per lane on as many lanes as that needs (up to 1024) stream best or tie
 // for 1024 .. 16384 16-bit elements (1-6 % over one or four chunks per lane; 7168 elements, per call: 3.3 us against 3.5
@@ -1034,7 +1045,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
             static_cast<u32x4 *>(residual_out), norm_out, scale, chunks, (float)hidden, eps, fp8_max);
         return hip_status(hipGetLastError());
     }
-    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk, is_half<T> && QUANT == GPUK_QUANT_FP8_STATIC);
+    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk, row_type<T>, QUANT);
     const uint32_t shape = (uint32_t)threads | ((uint32_t)row_group_shift(tokens, hidden * 2) << 16) | (line_mask(threads, nchunk, chunks) << 24);
     const bool exact = (int64_t)threads * nchunk == chunks;
     const RowParameters p = row_parameters(x, residual_in, gamma, residual_out, norm_out, scale, tokens, chunks, shape, gate, hidden, eps, fp8_max);
@@ -1096,7 +1107,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
     pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
     const bool exact = (int64_t)threads * nchunk == chunks;
     const bool gated = g_gate >= 0 || tokens * hidden * 8 >= f32_gate_from_bytes(tokens, threads, nchunk, QUANT != GPUK_QUANT_NONE);
-    const uint32_t gate = gated ? store_gate(tokens, hidden * 4, threads, nchunk) : 0;
+    const uint32_t gate = gated ? store_gate(tokens, hidden * 4, threads, nchunk, RowType::F32, QUANT) : 0;
     // Weights at once: more than a round, or waves that wait little for each other (see add_rmsnorm_quant_f32_rows).
     const bool few_waves = threads < 192 || (nchunk == 2 && threads <= 256 && tokens <= kComputeUnits);
     const bool short_chain = QUANT == GPUK_QUANT_NONE && ((hidden > 6144 && tokens <= 32) ||
@@ -1251,7 +1262,7 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
     auto ro = static_cast<u32x4 *>(residual_out);
     auto co = static_cast<u32x2 *>(codes);
     const dim3 grid((unsigned)tokens);
-    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk);
+    const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk, RowType::BF16, GPUK_QUANT_FP8_DYNAMIC);
     const uint32_t shape = (uint32_t)threads | ((uint32_t)group_shift << 16) | (line_mask(threads, nchunk, chunks) << 24);
     switch (nchunk) {
         case 1: add_rmsnorm_quant_traffic_only<1><<<grid, threads, 0, s>>>(xs, rs, chunks, remap_end, shape, gate, ro, co, scale); break;

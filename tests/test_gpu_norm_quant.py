@@ -220,6 +220,29 @@ def test_store_gate_changes_no_bits(device, gate):
         capi.set_tuning("norm_quant_gate", -1)
 
 
+@pytest.mark.parametrize("tokens,hidden,dtype", [(257, 8192, torch.bfloat16), (513, 16384, torch.bfloat16),
+                                                 (780, 10240, torch.float16), (559, 8192, torch.float16),
+                                                 (257, 16384, torch.float32), (513, 4096, torch.float32)])
+def test_layer_that_has_just_begun(device, tokens, hidden, dtype):
+    """Batches whose last layer of rows, one per compute unit, has just begun hold their stores back for most of the time a
+    full layer's reads take: the same bits as without a gate, in every quant mode."""
+    from gpuk_amd import capi
+
+    print(f"case layer begun {tokens}x{hidden} {dtype}", flush=True)
+    inp = workloads.norm_quant_inputs(tokens, hidden, seed=tokens, res_sigma=2.0, outlier_frac=0.01, dtype=dtype)
+    for quant in (0, 1, 3):
+        st = torch.tensor([0.05]) if quant == 3 else None
+        got = run_capi(inp, quant, device, static_scale=st)
+        capi.set_tuning("norm_quant_gate", 0)
+        try:
+            plain = run_capi(inp, quant, device, static_scale=st)
+        finally:
+            capi.set_tuning("norm_quant_gate", -1)
+        for a, b in zip(got, plain):
+            if torch.is_tensor(a):
+                assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
 @pytest.mark.parametrize("tokens,hidden,dtype", [(1025, 7168, torch.bfloat16), (1700, 7168, torch.bfloat16),
                                                  (2048, 8192, torch.bfloat16), (2049, 8192, torch.bfloat16),
                                                  (3000, 4096, torch.bfloat16), (1700, 5120, torch.bfloat16),
