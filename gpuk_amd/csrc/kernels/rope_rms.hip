@@ -139,8 +139,13 @@ __device__ __forceinline__ void load_trig_by_axis(const uint16_t *table, int64_t
         sinv = u32x4{sl[0], sl[1], sh[0], sh[1]};
     }
 }
-// ... and for any sections: one axis, or the three rows merged
-template <int D, bool NEOX, int AXES>
+// ... and for any sections: one axis, or the three rows merged.  FEWER_REGISTERS: the masks of one axis before those of the
+// other; left to itself the scheduler works out all sixteen halves side by side, and the kernel with one wave per unit then takes
+// 66 registers for 59 with a cache, one wave short of the eight per SIMD that its store gate counts on.  Held to 64 by an attribute
+// instead it takes 55 to 57, but spreads the table loads between their uses.  us, 66 / 55 to 57 / 59: 805 tokens of 64+8+8
+// heads, gated, 9.02 / 7.48 / 7.12; 3134 of 24+8+8 14.4 / 15.4 / 14.2; 9000 of 16+2+2 19.6 / 21.2 / 19.5; 16384 of 28+4+4 50.0 /
+// 53.0 / 50.1; heads of 256 elements, 28+4+4, 900 tokens, gated, 9.07 / - / 7.22.
+template <int D, bool NEOX, int AXES, bool FEWER_REGISTERS>
 __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t p0, int64_t p1, int64_t p2,
                                                  const uint32_t (&axis1)[4], const uint32_t (&axis2)[4], int sub,
                                                  u32x4 &cosv, u32x4 &sinv) {
@@ -155,11 +160,17 @@ __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t 
             const u32x4 sin2 = load_trig<D, NEOX>(table + p2 * D + HALF, sub);
             // the axis bits of the lane's 8 frequencies, in the order of the loaded values
             const uint32_t b1 = trig_bits<D, NEOX>(axis1, sub), b2 = trig_bits<D, NEOX>(axis2, sub);
+            uint32_t m1[4], m2[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) m1[j] = halves_mask(b1 >> (2 * j));
+            if constexpr (FEWER_REGISTERS) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) m2[j] = halves_mask(b2 >> (2 * j));
+            if constexpr (FEWER_REGISTERS) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const uint32_t m1 = halves_mask(b1 >> (2 * j)), m2 = halves_mask(b2 >> (2 * j));
-                cosv[j] = bitselect(m2, cos2[j], bitselect(m1, cos1[j], cosv[j]));
-                sinv[j] = bitselect(m2, sin2[j], bitselect(m1, sin1[j], sinv[j]));
+                cosv[j] = bitselect(m2[j], cos2[j], bitselect(m1[j], cos1[j], cosv[j]));
+                sinv[j] = bitselect(m2[j], sin2[j], bitselect(m1[j], sin1[j], sinv[j]));
             }
         }
     }
@@ -423,7 +434,7 @@ struct RopeUnit {
                 return;
             }
         }
-        load_trig_merged<D, NEOX, AXES>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
+        load_trig_merged<D, NEOX, AXES, true>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
     }
 
     // Norm, rotation and all stores of the unit.  GATED: no store before a.gate ticks after `entry`, the wave's entry
@@ -521,8 +532,6 @@ struct RopeUnit {
 //   second: hv_and_flags, units_per_token with one axis and no fp8 cache (where the block has room for eps), else eps, ps_token
 //   third:  ps_axis with three axes, else kv_loc with a cache
 // hv_and_flags: hv in bits 0-23, log2 of the waves per workgroup in bits 24-25, stream_rows in bit 26, merge_rows in bit 27.
-// (The three-axis instantiations of 128 elements per head with a cache are held to 64 registers, eight waves per SIMD: the
-// scheduler otherwise groups the mask operations of the three-row merge and takes 66; held, they take 55 to 57.)
 constexpr size_t kUnitLeadBytes = sizeof(u32x8) + sizeof(u32x4) + sizeof(u32x2);
 template <int D, int AXES, bool SETKV, bool KVFP8, bool GATED>
 struct UnitBlock {  // the argument block, behind the leading parameters
@@ -545,7 +554,7 @@ struct UnitBlock {  // the argument block, behind the leading parameters
 };
 
 template <typename T, int D, bool NEOX, int AXES, bool SETKV, bool KVFP8, bool GATED, bool WHOLE>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(AXES == 3 && D == 128 ? 8 : 1)))
+__global__ void __launch_bounds__(512)
 rope_rms_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const UnitBlock<D, AXES, SETKV, KVFP8, GATED> rest) {
     using Unit = RopeUnit<T, D, NEOX, AXES, SETKV, KVFP8>;
     using Block = UnitBlock<D, AXES, SETKV, KVFP8, GATED>;
@@ -881,7 +890,7 @@ rope_rms_token_kernel(const u32x8 first, const u32x4 second, const u32x2 third, 
     u32x4 cosv, sinv, cosv2 = {0, 0, 0, 0}, sinv2 = {0, 0, 0, 0};
     auto load_table = [&](const int64_t (&q)[3], u32x4 &c, u32x4 &sn) {
         if constexpr (AXES == 3) load_trig_by_axis<D, NEOX>(table, q[0], q[1], q[2], a.axis1, a.axis2, sub, c, sn);
-        else load_trig_merged<D, NEOX, AXES == 1 ? 1 : 3>(table, q[0], q[1], q[2], a.axis1, a.axis2, sub, c, sn);
+        else load_trig_merged<D, NEOX, AXES == 1 ? 1 : 3, false>(table, q[0], q[1], q[2], a.axis1, a.axis2, sub, c, sn);
     };
     load_table(p, cosv, sinv);
     if (second_item) load_table(p2, cosv2, sinv2);

@@ -52,6 +52,14 @@ def test_no_scratch_where_rows_stay_in_registers():
     assert not spilled, spilled
 
 
+def test_gated_waves_are_all_resident():
+    """The store gate of the rope kernel with one wave per group of heads counts on eight waves per SIMD (512 registers per lane)."""
+    found = {k[".name"]: k[".vgpr_count"] for elf in code_objects(open(LIB, "rb").read()) for k in kernels(elf)}
+    units = {n: v for n, v in found.items() if "rope_rms_kernelI" in n}
+    assert len(units) >= 100
+    assert not {n: v for n, v in units.items() if v > 64}
+
+
 def test_small_calls_pass_few_arguments():
     """The kernels that small calls launch take at most four parameters, and at most 112 bytes of them (128 and 136 with
     three position axes and a cache, or two token streams): what a launch costs the host goes by both."""
