@@ -144,7 +144,8 @@ __device__ __forceinline__ void load_trig_by_axis(const uint16_t *table, int64_t
 // 66 registers for 59 with a cache, one wave short of the eight per SIMD that its store gate counts on.  Held to 64 by an attribute
 // instead it takes 55 to 57, but spreads the table loads between their uses.  us, 66 / 55 to 57 / 59: 805 tokens of 64+8+8
 // heads, gated, 9.02 / 7.48 / 7.12; 3134 of 24+8+8 14.4 / 15.4 / 14.2; 9000 of 16+2+2 19.6 / 21.2 / 19.5; 16384 of 28+4+4 50.0 /
-// 53.0 / 50.1; heads of 256 elements, 28+4+4, 900 tokens, gated, 9.07 / - / 7.22.
+// 53.0 / 50.1; heads of 256 elements, 28+4+4, 900 tokens, gated, 9.07 / - / 7.22.  Ungated ones of 256 are level on average, and
+// 6 % ahead to 9 % behind by size (24+8+8 11.5 / - / 12.3 at 1150 tokens, 32+8+8 9.8 / - / 9.2 at 830): those keep 66.
 template <int D, bool NEOX, int AXES, bool FEWER_REGISTERS>
 __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t p0, int64_t p1, int64_t p2,
                                                  const uint32_t (&axis1)[4], const uint32_t (&axis2)[4], int sub,
@@ -425,6 +426,7 @@ struct RopeUnit {
     }
 
     // The cos/sin loads, whose addresses wait for the positions.
+    template <bool GATED>
     static __device__ __forceinline__ void issue_table_loads(const RopeArgs &a, int lane, UnitState &st) {
         const int sub = lane % LPH;
         const uint16_t *table = static_cast<const uint16_t *>(a.cos_sin);
@@ -434,7 +436,7 @@ struct RopeUnit {
                 return;
             }
         }
-        load_trig_merged<D, NEOX, AXES, true>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
+        load_trig_merged<D, NEOX, AXES, GATED || D != 256>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
     }
 
     // Norm, rotation and all stores of the unit.  GATED: no store before a.gate ticks after `entry`, the wave's entry
@@ -623,7 +625,7 @@ rope_rms_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const 
     if constexpr (GATED) asm volatile("" ::"s"(a.gate));
     Unit::issue_late_loads(a, lane, st);
     GPUK_STAMP(1);  // activations, weights, position and slot requested
-    Unit::issue_table_loads(a, lane, st);
+    Unit::template issue_table_loads<GATED>(a, lane, st);
     // (the slot is asked for here and not where the rows are stored, for the same reason)
     if constexpr (SETKV) asm volatile("" ::"s"((uint32_t)st.slot), "s"((uint32_t)(st.slot >> 32)));
     GPUK_STAMP(2);  // position known, cos/sin requested
