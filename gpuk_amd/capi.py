@@ -16,7 +16,7 @@ _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "lib
 EXPORTS = ("gpuk_status_string", "gpuk_abi_version", "gpuk_add_rmsnorm_quant", "gpuk_rope_rms",
            "gpuk_rope_rms_set_kv", "gpuk_rope_rms_2way", "gpuk_copy_bytes", "gpuk_increment_floats", "gpuk_set_tuning",
            "gpuk_add_rmsnorm_quant_traffic_only", "gpuk_add_rmsnorm_quant_launch_shape",
-           "gpuk_rope_rms_launch_shape", "gpuk_read_bytes", "gpuk_fill_bytes", "gpuk_empty_grid")
+           "gpuk_add_rmsnorm_quant_store_gate", "gpuk_rope_rms_launch_shape", "gpuk_read_bytes", "gpuk_fill_bytes", "gpuk_empty_grid")
 
 DTYPE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2, torch.float64: 3}
 QUANT_NONE, QUANT_FP8_DYNAMIC, QUANT_FP8_E4M3FNUZ, QUANT_FP8_STATIC = 0, 1, 2, 3
@@ -67,6 +67,8 @@ def lib():
         L.gpuk_add_rmsnorm_quant_traffic_only.argtypes = [C.c_void_p] * 5 + [C.c_int64, C.c_int64, C.c_void_p]
         L.gpuk_add_rmsnorm_quant_launch_shape.restype = C.c_int
         L.gpuk_add_rmsnorm_quant_launch_shape.argtypes = [C.c_int64, C.c_int64, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]
+        L.gpuk_add_rmsnorm_quant_store_gate.restype = C.c_int
+        L.gpuk_add_rmsnorm_quant_store_gate.argtypes = [C.c_int64, C.c_int64, C.c_int, C.c_int, C.POINTER(C.c_int)]
         L.gpuk_rope_rms_launch_shape.restype = C.c_int
         L.gpuk_rope_rms_launch_shape.argtypes = [C.c_int64] * 5 + [C.c_int] * 4 + [C.POINTER(C.c_int)] * 4
         L.gpuk_copy_bytes.restype = C.c_int
@@ -122,6 +124,15 @@ def add_rmsnorm_quant_launch_shape(tokens: int, hidden: int, dtype=torch.bfloat1
     if rc:
         raise GpukError(rc, "gpuk_add_rmsnorm_quant_launch_shape")
     return lanes.value, chunks.value
+
+
+def add_rmsnorm_quant_store_gate(tokens: int, hidden: int, dtype=torch.bfloat16, quant: int = QUANT_FP8_DYNAMIC) -> int:
+    """Ticks of 10 ns for which the waves of that launch hold their stores back, 0 where they do not."""
+    ticks = C.c_int(0)
+    rc = lib().gpuk_add_rmsnorm_quant_store_gate(tokens, hidden, DTYPE[dtype], quant, C.byref(ticks))
+    if rc:
+        raise GpukError(rc, "gpuk_add_rmsnorm_quant_store_gate")
+    return ticks.value
 
 
 def rope_rms_launch_shape(num_tokens: int, num_heads_q: int, num_heads_k: int, num_heads_v: int, head_size: int,

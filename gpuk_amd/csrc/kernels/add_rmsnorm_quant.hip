@@ -846,7 +846,9 @@ template <typename T> constexpr RowType row_type = is_half<T> ? RowType::FP16 : 
 // of 16384 14.7 / 12.0, 614 15.1 / 12.9, 775 18.4 / 16.2, 780 of 10240 12.3 / 10.8, 1030 of 12288 17.6 / 15.8, 1044 of 8192 11.3 / 10.8; two chunks, fp16
 // 559 of 8192 7.45 / 6.8, 377 of 16384 8.9 / 8.3, 300 of 8192 without codes 5.5 / 5.0; fp32 387 of 7168 8.1 / 7.4, 340 of 8192 8.9 / 7.6, 368
 // of 13184 14.5 / 12.1, without codes 318 of 5120 6.4 / 5.7; narrow rows and nearly full layers level.  More than that share holds back nearly full ones:
-// fp32 without codes 592 of 4096 7.1 / 7.3 with 0.9, 7.5 with 0.94).
+// fp32 without codes 592 of 4096 7.1 / 7.3 with 0.9, 7.5 with 0.94).  Only behind a full layer: in the first one a compute unit has
+// one row or none, and the row's own share of the time is all there is to wait for (bf16 without codes, 32768 elements, 128 rows
+// 7.95 / 8.39, 160 8.71 / 8.99, 200 10.1 / 10.3; level up to 16384 elements and at 65536).
 // short_rows: rows of two chunks per lane whose computation ends well ahead of the reads of a half-filled round (half precision,
 // static scale).  From two fifths of a round to eleven twentieths they wait 1.16 times the read time: 460 rows of 8192 elements
 // 6.28 / 5.72 us, 576 of 6144 6.55 / 6.05, 576 of 5120 5.46 / 5.3, level or slower below and above (1228 of 4096 6.6 / 6.8).
@@ -859,7 +861,7 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, 
     const bool half_filled = short_rows && nchunk == 2 && 5 * tokens >= 2 * resident && 20 * tokens <= 11 * resident;
     const double rows = (half_filled ? 1.16 : nchunk >= 4 ? 1.08 : 1.05) * (double)tokens;
     const double share = nchunk == 4 && type != RowType::F32 ? 0.93 : quant != GPUK_QUANT_NONE ? 0.86 : 0.82;
-    const double layers = share * (double)((tokens + kComputeUnits - 1) / kComputeUnits * kComputeUnits);
+    const double layers = tokens > kComputeUnits ? share * (double)((tokens + kComputeUnits - 1) / kComputeUnits * kComputeUnits) : 0.0;
     const double ticks = 2 * std::max(rows, layers) * (double)row_bytes / 70000.0;  // 70,000 bytes per tick of 10 ns
     return (uint32_t)std::min(ticks, 5000.0);
 }
@@ -1099,6 +1101,11 @@ int64_t f32_gate_from_bytes(int64_t tokens, int threads, int nchunk, bool codes)
     return codes ? 7'000'000 : 6'000'000;
 }
 
+uint32_t f32_store_gate(int64_t tokens, int64_t hidden, int threads, int nchunk, int quant) {
+    const bool gated = g_gate >= 0 || tokens * hidden * 8 >= f32_gate_from_bytes(tokens, threads, nchunk, quant != GPUK_QUANT_NONE);
+    return gated ? store_gate(tokens, hidden * 4, threads, nchunk, RowType::F32, quant) : 0;
+}
+
 template <int QUANT>
 int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, void *residual_out, void *norm_out,
                     float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
@@ -1106,8 +1113,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
     int threads, nchunk;
     pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
     const bool exact = (int64_t)threads * nchunk == chunks;
-    const bool gated = g_gate >= 0 || tokens * hidden * 8 >= f32_gate_from_bytes(tokens, threads, nchunk, QUANT != GPUK_QUANT_NONE);
-    const uint32_t gate = gated ? store_gate(tokens, hidden * 4, threads, nchunk, RowType::F32, QUANT) : 0;
+    const uint32_t gate = f32_store_gate(tokens, hidden, threads, nchunk, QUANT);
     // Weights at once: more than a round, or waves that wait little for each other (see add_rmsnorm_quant_f32_rows).
     const bool few_waves = threads < 192 || (nchunk == 2 && threads <= 256 && tokens <= kComputeUnits);
     const bool short_chain = QUANT == GPUK_QUANT_NONE && ((hidden > 6144 && tokens <= 32) ||
@@ -1290,6 +1296,30 @@ extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidde
     }
     const RowType type = dtype == GPUK_DTYPE_FP16 ? RowType::FP16 : RowType::BF16;
     pick_shape(first_piece(tokens, (int)(hidden / 8), type), (int)(hidden / 8), type, lanes_per_row, chunks_per_lane);
+    return GPUK_OK;
+}
+
+extern "C" int gpuk_add_rmsnorm_quant_store_gate(int64_t tokens, int64_t hidden, int dtype, int quant_mode, int *ticks) {
+    using namespace gpuk;
+    if (tokens <= 0 || hidden <= 0 || !ticks) return GPUK_ERR_INVALID_ARG;
+    if (hidden % 8 != 0) return GPUK_ERR_UNSUPPORTED;
+    if (quant_mode != GPUK_QUANT_NONE && quant_mode != GPUK_QUANT_FP8_DYNAMIC && quant_mode != GPUK_QUANT_FP8_STATIC) return GPUK_ERR_UNSUPPORTED;
+    int threads, nchunk;
+    *ticks = 0;
+    if (dtype == GPUK_DTYPE_F64) return GPUK_OK;  // (no gate in the kernels of fp64 and of swept rows)
+    if (dtype == GPUK_DTYPE_F32) {
+        const int chunks = (int)(hidden / 4);
+        if (chunks > kMaxChunksF32 * kMaxThreads) return GPUK_OK;
+        tokens = first_piece(tokens, chunks, RowType::F32, quant_mode != GPUK_QUANT_NONE);
+        pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
+        *ticks = (int)f32_store_gate(tokens, hidden, threads, nchunk, quant_mode);
+        return GPUK_OK;
+    }
+    if (dtype != GPUK_DTYPE_BF16 && dtype != GPUK_DTYPE_FP16) return GPUK_ERR_UNSUPPORTED;
+    const RowType type = dtype == GPUK_DTYPE_FP16 ? RowType::FP16 : RowType::BF16;
+    tokens = first_piece(tokens, (int)(hidden / 8), type);
+    pick_shape(tokens, (int)(hidden / 8), type, &threads, &nchunk);
+    if (nchunk) *ticks = (int)store_gate(tokens, hidden * 2, threads, nchunk, type, quant_mode);
     return GPUK_OK;
 }
 

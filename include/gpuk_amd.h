@@ -198,6 +198,12 @@ int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidden, int dtyp
                                         int *chunks_per_lane);
 
 /*
+ * How long the waves of that launch hold their stores back, in ticks of 10 ns after each wave's entry; 0 where they do not (see
+ * "norm_quant_gate" below).  For reports.  Not part of the reference.
+ */
+int gpuk_add_rmsnorm_quant_store_gate(int64_t tokens, int64_t hidden, int dtype, int quant_mode, int *ticks);
+
+/*
  * The launch gpuk_rope_rms_set_kv (set_kv != 0) or gpuk_rope_rms (set_kv == 0) makes for a batch: the grid as
  * workgroups x lanes per workgroup; *streamed = 1 when the rotated rows are stored past the L2; *token_waves = 1 for
  * the kernel in which a wave of 64 lanes takes a whole token or one of several parts of it (batches the chip holds in

@@ -296,6 +296,35 @@ def test_launch_shape_report():
     assert L.gpuk_add_rmsnorm_quant_launch_shape(4, 1024, 7, C.byref(a), C.byref(b)) == 2
 
 
+def test_store_gate_report():
+    """gpuk_add_rmsnorm_quant_store_gate: a layer of rows, one per compute unit, that has just begun counts for most of a full one,
+    but only behind a full one; up to 256 rows wait for their own share of the reads (no GPU needed)."""
+    import ctypes as C
+    from gpuk_amd import capi
+
+    ticks = lambda rows, row_bytes: int(2 * rows * row_bytes / 70000.0)
+    gate, f32 = capi.add_rmsnorm_quant_store_gate, torch.float32
+    for tokens, hidden, rows in ((128, 16384, 1.05), (256, 16384, 1.05), (128, 32768, 1.08), (200, 32768, 1.08), (256, 32768, 1.08), (64, 65536, 1.08), (256, 65536, 1.08)):
+        for quant in (0, 1, 3):
+            assert gate(tokens, hidden, torch.bfloat16, quant) == ticks(rows * tokens, 2 * hidden), (tokens, hidden, quant)
+    assert gate(200, 12288, f32, 0) == ticks(1.08 * 200, 4 * 12288)
+    # behind a full layer: 0.93 of whole layers for 16-bit rows of four chunks per lane, else 0.86 with codes and 0.82 without
+    assert gate(257, 8192) == ticks(0.86 * 512, 16384) and gate(257, 8192, quant=0) == ticks(0.82 * 512, 16384)
+    assert gate(513, 16384) == ticks(0.93 * 768, 32768) and gate(257, 32768) == ticks(0.93 * 512, 65536)
+    assert gate(340, 8192, f32) == ticks(0.86 * 512, 32768) and gate(318, 5120, f32, 0) == ticks(0.82 * 512, 20480)
+    # ... unless the rows themselves are more than that
+    assert gate(512, 8192) == ticks(1.05 * 512, 16384) and gate(500, 32768) == ticks(1.08 * 500, 65536)
+    # no gate: less than a quarter of a round, more than one, small fp32 batches, fp64, swept rows
+    for args in ((1, 8192), (127, 16384), (8192, 8192), (64, 4096, f32), (512, 4096, torch.float64), (300, 16392, f32), (4, 65600 * 2)):
+        assert gate(*args) == 0, args
+    out = C.c_int(0)
+    assert capi.lib().gpuk_add_rmsnorm_quant_store_gate(0, 1024, 0, 1, C.byref(out)) == 1
+    assert capi.lib().gpuk_add_rmsnorm_quant_store_gate(4, 1024, 0, 1, None) == 1
+    assert capi.lib().gpuk_add_rmsnorm_quant_store_gate(4, 1028, 0, 1, C.byref(out)) == 2
+    assert capi.lib().gpuk_add_rmsnorm_quant_store_gate(4, 1024, 0, 2, C.byref(out)) == 2
+    assert capi.lib().gpuk_add_rmsnorm_quant_store_gate(4, 1024, 7, 1, C.byref(out)) == 2
+
+
 def test_launch_shape_of_forced_chunks():
     """fp32 rows have forms of one, two and four chunks per lane: a forced eight is four there, eight for 16-bit rows."""
     from gpuk_amd import capi
