@@ -40,10 +40,13 @@ _spec.loader.exec_module(_direct)
 
 def _called_directly(packet):
     """`packet`, the object that torch.ops.gpuk holds, with a class of its own in which a plain call skips the
-    interpretation of the schema (csrc/direct_calls.cpp); every other call, and everything else about it, is as before."""
-    base = type(packet)
-    call = _direct.direct(packet.__name__, "", types.MethodType(base.__call__, packet))
-    packet.__class__ = type(base.__name__, (base,), {"__call__": call, "__module__": base.__module__, "__doc__": base.__doc__})
+    interpretation of the schema (csrc/direct_calls.cpp); every other call, and everything else about it, is as before.
+    (The general call is torch's own and not that of the class the packet has: that one is this function's where the module
+    is executed once more.)"""
+    base = torch._ops.OpOverloadPacket
+    general = types.MethodType(base.__call__, packet)
+    packet.__class__ = type(base.__name__, (base,), {"__call__": _direct.direct(packet.__name__, "", general),
+                                                     "__module__": base.__module__, "__doc__": base.__doc__})
     return packet
 
 

@@ -40,6 +40,18 @@ def test_the_packet_stays_what_it_was(name):
     assert packet.default._schema.name == f"gpuk::{name}"
 
 
+@pytest.mark.parametrize("name", NAMES)
+def test_wrapped_once_more(name):
+    """As where the module is executed again: keyword calls must still reach the packet's own call, with its own arguments."""
+    packet = getattr(gpuk, name)
+    expect = outcome(general(packet), **{"eps": 1e-6})
+    assert gpuk._called_directly(packet) is packet
+    assert outcome(packet, **{"eps": 1e-6}) == expect
+    if name == "fused_rope_rms_2way":
+        args = two_way()
+        assert outcome(packet, *args[:17], eps=1e-6) == outcome(packet, *args) == outcome(general(packet), *args)
+
+
 @pytest.mark.parametrize("change", [
     {}, {10: 1.5}, {10: True}, {16: 1}, {17: 0}, {0: None}, {11: 2 ** 70}, {"cut": 17}, {"add": 3}, {"device": "cpu"},
     {"requires_grad": True}, {0: torch.nn.Parameter(torch.zeros(B, T0, H, D, device="meta"))}])
