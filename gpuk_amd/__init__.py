@@ -14,6 +14,7 @@ import raises.
 from __future__ import annotations
 
 import importlib.util
+import inspect
 import os
 import types
 from contextlib import contextmanager
@@ -45,7 +46,7 @@ def _called_directly(packet):
     is executed once more.)"""
     base = torch._ops.OpOverloadPacket
     general = types.MethodType(base.__call__, packet)
-    packet.__class__ = type(base.__name__, (base,), {"__call__": _direct.direct(packet.__name__, "", general),
+    packet.__class__ = type(base.__name__, (base,), {"__call__": _direct.direct(packet.__name__, "", general), "__signature__": inspect.signature(general),
                                                      "__module__": base.__module__, "__doc__": base.__doc__})
     return packet
 

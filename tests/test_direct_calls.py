@@ -1,5 +1,6 @@
 """The operators' names in the package call past the interpretation of the schema where the arguments are plain: what they
 return, raise and let others see is what the general call of the same packet gives (no GPU needed: meta tensors)."""
+import inspect
 import types
 
 import pytest
@@ -38,6 +39,7 @@ def test_the_packet_stays_what_it_was(name):
     assert packet is getattr(torch.ops.gpuk, name)
     assert isinstance(packet, torch._ops.OpOverloadPacket) and str(packet) == f"gpuk.{name}"
     assert packet.default._schema.name == f"gpuk::{name}"
+    assert inspect.signature(packet) == inspect.signature(general(packet))
 
 
 @pytest.mark.parametrize("name", NAMES)
