@@ -4,11 +4,10 @@
 // longer than everything else the host does for a small call but the launch: us per call that way / this way 4.79 / 3.42 for
 // allreduce_rms of one row (nine arguments), 5.50 / 3.66 for fused_rope_rms_set_kv of 32 tokens (eighteen), of which the
 // launch is 2.8 and what the operator itself does beside it 0.2.  The functions here take the same positional arguments,
-// unpack them by the type the operator's
-// C++ signature names and call the operator through the dispatcher, so that profiling, dispatch modes, functorch
-// and the keys other code registers see the call as before.  Whatever is not plain -- keywords, another number of arguments, tensor
-// subclasses, symbolic or other numbers, a __torch_function__ mode, a trace being recorded -- goes to the callable that the
-// function was made with, which is the packet's own.
+// unpack them by the type the operator's C++ signature names and call the operator through the dispatcher, so that
+// profiling, dispatch modes, functorch and the keys other code registers see the call as before.  Whatever is not plain --
+// keywords, another number of arguments, tensor subclasses, symbolic or other numbers, a __torch_function__ mode, a trace
+// being recorded -- goes to the callable that the function was made with, which is the packet's own.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -97,6 +96,9 @@ PyObject *as_tuple(std::tuple<R...> &result, std::index_sequence<I...>) {
     return tuple;
 }
 
+template <auto F, auto G>
+constexpr bool same_function = std::is_same_v<std::integral_constant<decltype(F), F>, std::integral_constant<decltype(G), G>>;
+
 template <auto F> struct Call;
 template <typename R, typename... A, R (*F)(A...)>
 struct Call<F> {
@@ -118,8 +120,8 @@ struct Call<F> {
         } else {
             auto result = [&] {
                 pybind11::gil_scoped_release no_gil;
-                if constexpr (std::is_same_v<R, std::tuple<at::Tensor, at::Tensor>> && sizeof...(A) == 5) {
-                    // (add_rms_fused.static: the scale comes back as a third output, in the shape the callers of
+                if constexpr (same_function<F, &gpuk_ops::add_rms_fused_static>) {
+                    // (the scale comes back as a third output, in the shape the callers of
                     // GPUKDistEnv.allreduce_add_rms_fused expect; reshaped from Python it cost as much as an allocation)
                     auto [residual_out, norm_out] = handle->call(std::get<I>(args).pass()...);
                     return std::make_tuple(std::move(residual_out), std::move(norm_out), std::get<4>(args).value.reshape({1}));

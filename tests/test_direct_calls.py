@@ -54,6 +54,110 @@ def test_wrapped_once_more(name):
         assert outcome(packet, *args[:17], eps=1e-6) == outcome(packet, *args) == outcome(general(packet), *args)
 
 
+def arguments(name, device="meta", dtype=torch.bfloat16):
+    """Plain arguments of every function that calls an operator directly."""
+    new = lambda *shape, dt=dtype: torch.zeros(shape, dtype=dt, device=device)
+    tokens, hq, hk, hv = 5, 4, 2, 2
+    if name == "allreduce_rms":
+        return 0, new(tokens, 64), new(tokens, 64), new(64), new(tokens, 64), new(tokens, 64), new(tokens, 1, dt=torch.float32), 1e-6, 0
+    if name == "add_rms_fused":
+        return new(tokens, 64), new(tokens, 64), new(64), 1e-6, 1
+    if name == "add_rms_fused.static":
+        return new(tokens, 64), new(tokens, 64), new(64), 1e-6, new(1, dt=torch.float32)
+    if name == "fused_rope_rms_2way":
+        return two_way(device, dtype)
+    axes = (3,) if "mrope" in name else ()
+    args = (new(tokens, hq + hk + hv, D), new(D), new(D), new(16, D), new(*axes, tokens, dt=torch.int64), tokens, hq, hk, hv, D, True)
+    args += ([8, 12, 12], False, 1e-6) if axes else (1e-6,)
+    if "set_kv" in name:
+        args += (new(tokens, hq, D), new(32, hk, D), new(32, hv, D), new(tokens, dt=torch.int64), 0.5, 0.25)
+    return args
+
+
+def both(name):
+    """(direct function, general one) of an entry of the table in csrc/direct_calls.cpp."""
+    if name == "add_rms_fused":
+        return gpuk._add_rms_fused_direct, gpuk._add_rms_fused
+    if name == "add_rms_fused.static":
+        return gpuk._add_rms_fused_static_direct, gpuk._add_rms_fused_static
+    return getattr(gpuk, name), general(getattr(gpuk, name))
+
+
+ENTRIES = NAMES + ["add_rms_fused", "add_rms_fused.static"]
+
+
+class recorded:
+    """Kernels of the CPU key for the length of a test, which note what reached the operator."""
+
+    def __enter__(self):
+        self.lib, self.calls = torch.library.Library("gpuk", "IMPL"), []
+        for name in ENTRIES:
+            def kernel(*args, name=name):
+                self.calls.append((name, [(a.shape, a.dtype, a.data_ptr()) if torch.is_tensor(a) else (type(a), a) for a in args]))
+                if "add_rms_fused" in name:
+                    out = torch.ones_like(args[1]), torch.full_like(args[0], 2)
+                    return out if "static" in name else (*out, torch.full((1,), 3.0))
+                return (args[0] + 1, args[1] + 2) if "2way" in name else None
+            self.lib.impl(name, kernel, "CPU")
+        return self.calls
+
+    def __exit__(self, *_):
+        self.lib._destroy()
+
+
+@pytest.mark.parametrize("name", ENTRIES)
+def test_every_function_hands_on_its_arguments(name):
+    direct, packet = both(name)
+    args = arguments(name, "cpu")
+    values = [7 + i if type(a) is int else 0.25 + i if type(a) is float else a for i, a in enumerate(args)]   # (each to be told apart)
+    with recorded() as calls:
+        out, expect = direct(*values), packet(*values)
+        assert len(calls) == 2 and calls[0] == calls[1] and calls[0][0] == name
+        assert [type(a) for a in values] == [a[0] if isinstance(a[0], type) else torch.Tensor for a in calls[0][1]]
+    if expect is None:
+        assert out is None
+    else:
+        assert type(out) is type(expect) and len(out) == len(expect) and all(torch.equal(a, b) for a, b in zip(out, expect))
+
+
+@pytest.mark.parametrize("name", ENTRIES)
+def test_every_function_raises_what_the_general_call_raises(name):
+    direct, packet = both(name)
+    meta, cpu = arguments(name), arguments(name, "cpu")
+    assert outcome(direct, *meta) == outcome(packet, *meta)
+    with recorded() as calls:
+        for at, a in enumerate(cpu):
+            for other in (None, "x", 1.5, 3, True, 2 ** 70, torch.tensor(2), [1, 2, 3], (1, 2, 3), [1, 2.0, 3], [1, True, 3], [1, 2 ** 70, 3], []):
+                if name.endswith("static") and at == 4 and torch.is_tensor(other):
+                    other = other.float()
+                args = (*cpu[:at], other, *cpu[at + 1:])
+                assert outcome(direct, *args) == outcome(packet, *args), (at, other)
+        for args in (cpu[:-1], (*cpu, 1), ()):
+            got, expect = outcome(direct, *args), outcome(packet, *args)
+            assert got[0] == expect[0] and (got == expect or "static" in name), args   # (the message names a Python function there)
+        # what arrived, arrived the same either way
+        assert len(calls) % 2 == 0 and all(a == b for a, b in zip(calls[::2], calls[1::2]))
+
+
+@pytest.mark.parametrize("sections", [[8, 12, 12], (8, 12, 12), torch.Size([8, 12, 12]), [], [1, 2], [2 ** 62, -1, 0]])
+@pytest.mark.parametrize("name", ["fused_mrope_3d_rms", "fused_mrope_3d_rms_set_kv"])
+def test_sections(name, sections):
+    direct, packet = both(name)
+    args = [sections if type(a) is list else a for a in arguments(name, "cpu")]
+    with recorded() as calls:
+        direct(*args), packet(*args)
+        assert calls[0] == calls[1] and (list, list(sections)) in calls[0][1]
+
+
+@pytest.mark.parametrize("shape", [(), (1,), (1, 1)])
+def test_the_static_scale_is_the_third_output(shape):
+    args = (*arguments("add_rms_fused.static", "cpu")[:4], torch.full(shape, 0.5))
+    with recorded():
+        for f in both("add_rms_fused.static"):
+            out = f(*args)
+            assert len(out) == 3 and out[2].shape == (1,) and out[2].data_ptr() == args[4].data_ptr()
+
+
 @pytest.mark.parametrize("change", [
     {}, {10: 1.5}, {10: True}, {16: 1}, {17: 0}, {0: None}, {11: 2 ** 70}, {"cut": 17}, {"add": 3}, {"device": "cpu"},
     {"requires_grad": True}, {0: torch.nn.Parameter(torch.zeros(B, T0, H, D, device="meta"))}])
@@ -91,21 +195,23 @@ def test_modes_see_the_call():
 
     class Functions(TorchFunctionMode):
         def __torch_function__(self, func, types, args=(), kwargs=None):
-            seen.append(func)
+            seen.append(str(func))
             return func(*args, **(kwargs or {}))
 
     class Dispatch(TorchDispatchMode):
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
-            seen.append(func)
+            seen.append(str(func))
             return func(*args, **(kwargs or {}))
 
     for mode in (Functions, Dispatch):
+        records = []
         for f in (packet, general(packet)):
             seen.clear()
             with mode():
                 f(*args)
-            assert [str(s) for s in seen if "gpuk" in str(s)] == ["gpuk.fused_rope_rms_2way.default"] or mode is Functions, (mode, seen)
-            assert any("fused_rope_rms_2way" in str(s) for s in seen), (mode, seen)
+            records.append(list(seen))
+        assert records[0] == records[1] and any("fused_rope_rms_2way" in s for s in records[0]), (mode, records)
+    assert records[0][0] == "gpuk.fused_rope_rms_2way.default"
     with FakeTensorMode():
         out = packet(*two_way("cuda"))
     assert out[0].device.type == "cuda" and out[0].shape == (B, T0 + T1, H, D)
