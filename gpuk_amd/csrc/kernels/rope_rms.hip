@@ -1496,6 +1496,11 @@ TokenShape token_shape(const RopeArgs &a, int D, int axes, bool set_kv, bool kv_
     return best;
 }
 
+// Whole tokens of four or five units of 128-element heads that read one table row gain most and are taken in every form; the others
+// in place only where token_form_in_place (behind in some part of their range, see plan_rope, and not compiled).
+constexpr bool token_form_in_place(bool neox, bool half, int units, bool two) { return neox && units < 5 && (half || !two); }
+bool whole_token(const RopeArgs &a, int D, int axes, int units, int parts) { return D == 128 && parts == 1 && units >= 4 && (axes == 1 || a.merge_rows); }
+
 RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, bool kv_fp8, bool half) {
     RopePlan p{};
     const int64_t read_bytes = 2 * (int64_t)a.num_tokens * (a.hq + a.hk + (set_kv ? a.hv : 0)) * D;
@@ -1549,14 +1554,15 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // With a cache: a layer that has just begun where lanes or units idle (16+2+2 in half precision 7.6 / 8.2 at 3148), two items per wave
     // where lanes idle in bfloat16 but for merged table rows (16+2+2 16.1 / 16.6 at 7544).  Pairwise with a cache: the latter in every type, seven layers and
     // more (20+4+4 in half precision 21.0 / 21.5 at 7797), a layer that has just begun, and bfloat16 with three V chunks per lane (12+12+12 14.3 / 14.9 at 3592).
-    if (!(D == 128 && shape.parts == 1 && shape.units >= 4 && (axes == 1 || a.merge_rows))) {
+    if (!whole_token(a, D, axes, shape.units, shape.parts)) {
         const int64_t last = shape.items > 3072 ? shape.items % 1024 : 0;  // items of the last layer, 0: it is full
-        if (!set_kv) large = large && neox && shape.units < 5 && no_idle_unit && (two ? half && full : last == 0 || last >= 256);
+        if (!set_kv) large = large && no_idle_unit && (two ? full : last == 0 || last >= 256);  // (and see token_form_in_place)
         else if (neox) large = large && (!two || full || half || (axes == 3 && !a.merge_rows)) && ((full && no_idle_unit) || last == 0 || last >= 256);
         else large = large && (!two || (full && shape.items <= 7168)) && (last == 0 || last >= 384) && (half || a.hv * (D / 8) <= 128 * shape.parts);
     }
     const bool by_rule = g_token_waves == 0 && large;
-    p.token_waves = shape.units && (g_token_waves >= 2 || by_rule);
+    const bool has_form = set_kv || whole_token(a, D, axes, shape.units, shape.parts) || token_form_in_place(neox, half, shape.units, two);
+    p.token_waves = shape.units && has_form && (g_token_waves >= 2 || by_rule);
     p.two_tokens = p.token_waves && two;
     // (with two items per wave the full read time: 24.4 us at 8192 tokens of 28+4+4 heads with three axes, against 25.4
     // with 0.95 of it, 24.8 with 1.05, 27.2 with 0.9 -- opening early, into the last reads, costs more than waiting)
@@ -1630,15 +1636,19 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
 #define GPUK_LAUNCH_TOKEN(UPT, TWO)                                                                                    \
     do {                                                                                                               \
         constexpr uint32_t lds = TWO ? 4 * token_kernel_lds_bytes_per_wave(UPT, SETKV) : 0;                            \
-        constexpr bool whole = D == 128 && UPT >= 4, parts_too = !KVFP8;                                               \
-        if (AXES == 3 && !a.merge_rows)                                                                                \
-            return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES == 3 ? kMergedAxes : 1, TWO, parts_too>, \
-                                 dim3(p.blocks), 256, lds, stream, first, second, third, b);                           \
-        if (whole && p.token_parts == 1)                                                                               \
-            return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES, TWO, !whole>, dim3(p.blocks), 256, lds, \
-                                 stream, first, second, third, b);                                                     \
-        return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES, TWO, parts_too>, dim3(p.blocks), 256, lds, \
-                             stream, first, second, third, b);                                                         \
+        if constexpr (D == 128 && UPT >= 4)                                                                            \
+            if (whole_token(a, D, AXES, UPT, (int)p.token_parts))                                                      \
+                return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES, TWO, false>, dim3(p.blocks), 256, lds, stream, first, \
+                                     second, third, b);                                                                \
+        if constexpr (!KVFP8 && (SETKV || token_form_in_place(NEOX, is_half<T>, UPT, TWO))) {                           \
+            if constexpr (AXES == 3)                                                                                   \
+                if (!a.merge_rows)                                                                                     \
+                    return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, kMergedAxes, TWO, true>, dim3(p.blocks), 256, lds, \
+                                         stream, first, second, third, b);                                             \
+            return launch_kernel(rope_rms_token_kernel<T, D, NEOX, UPT, SETKV, KVFP8, AXES, TWO, true>, dim3(p.blocks), 256, lds, stream, first, \
+                                 second, third, b);                                                                    \
+        }                                                                                                              \
+        return GPUK_ERR_INTERNAL;                                                                                      \
     } while (0)
             if (p.two_tokens) {
                 if constexpr (!KVFP8) {
@@ -1648,11 +1658,9 @@ int launch_one(const RopeArgs &a, hipStream_t stream) {
                 return GPUK_ERR_INTERNAL;
             }
             switch (p.token_units) {
-                case 3:
-                    if constexpr (!KVFP8) GPUK_LAUNCH_TOKEN(3, false);
-                    return GPUK_ERR_INTERNAL;
-                case 4: GPUK_LAUNCH_TOKEN(4, false); break;
-                case 5: GPUK_LAUNCH_TOKEN(5, false); break;
+                case 3: GPUK_LAUNCH_TOKEN(3, false);
+                case 4: GPUK_LAUNCH_TOKEN(4, false);
+                case 5: GPUK_LAUNCH_TOKEN(5, false);
                 default: return GPUK_ERR_INTERNAL;
             }
 #undef GPUK_LAUNCH_TOKEN

@@ -33,6 +33,11 @@ CASES = [
 ]
 
 
+# (in place there are no forms of five units but for whole tokens of one table row, nor of two items in bfloat16, nor, which the query
+# does not know, with pairwise rotation or merged table rows of those)
+IN_PLACE = {7: 0, 8: 0, 14: 0, 16: 0, 19: 0}
+
+
 @pytest.mark.parametrize("case", range(len(CASES)))
 @pytest.mark.parametrize("gate", [-1, 600])
 def test_tokens_in_parts(device, case, gate):
@@ -54,7 +59,7 @@ def test_tokens_in_parts(device, case, gate):
         capi.set_tuning("rope_token_waves", 3 if two else 2)
         capi.set_tuning("rope_token_gate", gate)
         assert capi.rope_rms_launch_shape(tokens, *heads, D, axes, inp.qkv.dtype, True, False)[3] == (2 if two else 1), "the case must reach the kernel under test"
-        assert capi.rope_rms_launch_shape(tokens, *heads, D, axes, inp.qkv.dtype, False, False)[3] == (2 if two else 1)
+        assert capi.rope_rms_launch_shape(tokens, *heads, D, axes, inp.qkv.dtype, False, False)[3] == IN_PLACE.get(case, 2 if two else 1)
         got, got_inplace = run_set_kv(inp, device), run_inplace(inp, device)
     finally:
         capi.set_tuning("rope_token_waves", 0)

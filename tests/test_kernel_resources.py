@@ -60,6 +60,16 @@ def test_gated_waves_are_all_resident():
     assert not {n: v for n, v in gated.items() if v > 64}
 
 
+def test_every_token_form_is_one_that_a_call_can_reach():
+    """The rope kernel with one wave per token, in place: beyond whole tokens only rotation by halves and three or four units, two
+    items per wave in half precision only."""
+    names = [k[".name"] for elf in code_objects(open(LIB, "rb").read()) for k in kernels(elf) if "rope_rms_token_kernelI" in k[".name"]]
+    forms = [re.search(r"INS_4(\w{4})ELi(\d+)ELb(\d)ELi(\d)ELb(\d)ELb(\d)ELi(\d)ELb(\d)ELb(\d)E", n).groups() for n in names]
+    assert len(forms) == len(set(forms)) >= 200
+    for dtype, _, neox, units, set_kv, _, _, two, parts in forms:
+        assert set_kv == "1" or parts == "0" or (neox == "1" and units != "5" and (two == "0" or dtype == "FP16"))
+
+
 def test_small_calls_pass_few_arguments():
     """The kernels that small calls launch take at most four parameters, and at most 112 bytes of them (128 and 136 with
     three position axes and a cache, or two token streams): what a launch costs the host goes by both."""
