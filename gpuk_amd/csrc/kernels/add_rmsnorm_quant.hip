@@ -540,20 +540,20 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
 //
 // When the weights are asked for.  A row of them is half as many bytes as the row's own loads, and a compute unit that holds
 // few rows waits for its own: asked for at once, the weights of its first waves go ahead of the rows of its last.  So batches
-// of up to one round that do not gate their stores ask once the lane's row has landed, behind which the reduction hides
-// them, and rows of 28 KB and more, which keep a compute unit's memory path busy by themselves, once rstd is known.  Larger
-// batches have other rows to wait for and ask at once.  us, at once / landed / rstd known: 98 rows of 3320 elements without
-// codes 3.43 / 3.21 / 3.35, 32 of 5120 with 3.78 / 3.58 / 3.61, one of 2056 2.52 / 2.48 / 2.56, but 32 of 7168 4.60 / 4.16 / 4.01, of 12288
-// 5.95 / 5.89 / 5.62, 98 of 8192 without codes 5.00 / 5.39 / 4.54, of 16384 with 8.49 / 8.22 / 7.94; 4000 of 7168 without 77.7 / 79.2 /
-// 78.8; 32 of 1024, on two waves, 2.49 / 2.51 / 2.56.  At once as well: two chunks per lane on four waves and less, one row per
-// compute unit (127 rows of 1504 without codes 2.51 / 2.65, with codes level), and without codes, whose short chain leaves the
-// weights' latency open, up to 32 rows of more than 6144 elements (one of 8296 3.15 / - / 3.35, of 16384 3.73 / - / 3.97, 30 of 7760 2.90 /
-// - / 3.08) and rows of two chunks per lane that do not fill their lanes, on six waves and less or up to 128 of them on nine (one of 2968
-// 1.90 / 2.01, 29 of 2424 2.31 / 2.44, 314 of 1456 2.70 / 2.82; filled rows 1-5 % the other way).
+// of up to one round that do not gate their stores ask once the lane's row has landed, behind which the reduction hides them,
+// and rows of 28 KB and more, which keep a compute unit's memory path busy by themselves, once rstd is known.  Larger batches
+// have other rows to wait for and ask at once.  us, at once / landed / rstd known: 98 rows of 3320 elements without codes 3.43
+// / 3.21 / 3.35, 32 of 5120 with 3.78 / 3.58 / 3.61, one of 2056 2.52 / 2.48 / 2.56, but 32 of 7168 4.60 / 4.16 / 4.01, of
+// 12288 5.95 / 5.89 / 5.62, 98 of 8192 without codes 5.00 / 5.39 / 4.54, of 16384 with 8.49 / 8.22 / 7.94; 4000 of 7168 without
+// 77.7 / 79.2 / 78.8; 32 of 1024, on two waves, 2.49 / 2.51 / 2.56.  At once as well: two chunks per lane on four waves and
+// less, one row per compute unit (127 rows of 1504 without codes 2.51 / 2.65, with codes level), and without codes, whose short
+// chain leaves the weights' latency open, up to 32 rows of more than 6144 elements (one of 8296 3.15 / - / 3.35, of 16384 3.73
+// / - / 3.97, 30 of 7760 2.90 / - / 3.08) and rows of two chunks per lane that do not fill their lanes, on six waves and less
+// or up to 128 of them on nine (one of 2968 1.90 / 2.01, 29 of 2424 2.31 / 2.44, 314 of 1456 2.70 / 2.82; filled rows 1-5 % the
+// other way).
 // (98 of 16384 without codes remain behind the sweep of each lane's chunks one by one that this kernel replaced: 8.3 us, it
-// 7.8.)  Gated rows of one chunk per lane and eight waves or more without codes,
-// the shortest computation, ask once landed as well: 400 of 2568 elements 5.1 / 4.6 us, 290 of 3840 5.5 / 4.9, but 1280 of 1032, on
-// five waves, 5.2 / 5.4.
+// 7.8.)  Gated rows of one chunk per lane and eight waves or more without codes, the shortest computation, ask once landed as
+// well: 400 of 2568 elements 5.1 / 4.6 us, 290 of 3840 5.5 / 4.9, but 1280 of 1032, on five waves, 5.2 / 5.4.
 enum class F32Form { STREAM, GATED, LANDED, GATED_LANDED, LAST };
 template <int NCHUNK, int QUANT, bool EXACT, F32Form FORM>
 __global__ void __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(FORM == F32Form::GATED || FORM == F32Form::GATED_LANDED ? 8 : 4)))
@@ -833,25 +833,26 @@ int64_t resident_rows(int threads, int nchunk) {
 enum class RowType { BF16, FP16, F32 };
 template <typename T> constexpr RowType row_type = is_half<T> ? RowType::FP16 : RowType::BF16;
 
-// The store gate of a launch: for batches whose workgroups are all resident at once (2048 lanes per
-// compute unit) the time their reads take at 7 TB/s, the rate of a read-only kernel on this part, plus a twentieth;
-// 0 (stores as soon as they are ready) for larger batches, whose later workgroups read while earlier ones write
-// whatever a wave does.  Measured per call at 7168 elements: 6.35 against 7.2 us at 512 rows, 7.6 against 9.5 at
-// 768, 9.0 against 11.7 at 1024 (gate 1.0-1.1 times the read time; 10.2 with 0.9, 9.6 with 1.2), nothing gained and
-// 0.1 us lost below a quarter of a round; at 4096 elements 6.2 against 7.7 us at 1024 rows, 10.2 against 12.4 at 2048; 20-45 % slower where the
-// batch does not fit one round.
-// A compute unit reads no faster than its share of that rate by much, so a layer of rows (one per compute unit) that has just begun
-// takes nearly the time of a full one where rows are wide and a compute unit holds few: the gate is at least 0.93 of the time of whole layers for 16-bit
-// rows of four chunks per lane, else 0.86 with codes and 0.82 without (those store more, the rows' own gate / this one, us: bf16, four chunks, 522 rows
-// of 16384 14.7 / 12.0, 614 15.1 / 12.9, 775 18.4 / 16.2, 780 of 10240 12.3 / 10.8, 1030 of 12288 17.6 / 15.8, 1044 of 8192 11.3 / 10.8; two chunks, fp16
-// 559 of 8192 7.45 / 6.8, 377 of 16384 8.9 / 8.3, 300 of 8192 without codes 5.5 / 5.0; fp32 387 of 7168 8.1 / 7.4, 340 of 8192 8.9 / 7.6, 368
-// of 13184 14.5 / 12.1, without codes 318 of 5120 6.4 / 5.7; narrow rows and nearly full layers level.  More than that share holds back nearly full ones:
-// fp32 without codes 592 of 4096 7.1 / 7.3 with 0.9, 7.5 with 0.94).  Only behind a full layer: in the first one a compute unit has
-// one row or none, and the row's own share of the time is all there is to wait for (bf16 without codes, 32768 elements, 128 rows
-// 7.95 / 8.39, 160 8.71 / 8.99, 200 10.1 / 10.3; level up to 16384 elements and at 65536).
-// short_rows: rows of two chunks per lane whose computation ends well ahead of the reads of a half-filled round (half precision,
-// static scale).  From two fifths of a round to eleven twentieths they wait 1.16 times the read time: 460 rows of 8192 elements
-// 6.28 / 5.72 us, 576 of 6144 6.55 / 6.05, 576 of 5120 5.46 / 5.3, level or slower below and above (1228 of 4096 6.6 / 6.8).
+// The store gate of a launch: for batches whose workgroups are all resident at once (2048 lanes per compute unit) the time
+// their reads take at 7 TB/s, the rate of a read-only kernel on this part, plus a twentieth; 0 (stores as soon as they are
+// ready) for larger batches, whose later workgroups read while earlier ones write whatever a wave does.  Measured per call at
+// 7168 elements: 6.35 against 7.2 us at 512 rows, 7.6 against 9.5 at 768, 9.0 against 11.7 at 1024 (gate 1.0-1.1 times the read
+// time; 10.2 with 0.9, 9.6 with 1.2), nothing gained and 0.1 us lost below a quarter of a round; at 4096 elements 6.2 against
+// 7.7 us at 1024 rows, 10.2 against 12.4 at 2048; 20-45 % slower where the batch does not fit one round.
+// A compute unit reads no faster than its share of that rate by much, so a layer of rows (one per compute unit) that has just
+// begun takes nearly the time of a full one where rows are wide and a compute unit holds few: the gate is at least 0.93 of the
+// time of whole layers for 16-bit rows of four chunks per lane, else 0.86 with codes and 0.82 without (those store more, the
+// rows' own gate / this one, us: bf16, four chunks, 522 rows of 16384 14.7 / 12.0, 614 15.1 / 12.9, 775 18.4 / 16.2, 780 of
+// 10240 12.3 / 10.8, 1030 of 12288 17.6 / 15.8, 1044 of 8192 11.3 / 10.8; two chunks, fp16 559 of 8192 7.45 / 6.8, 377 of 16384
+// 8.9 / 8.3, 300 of 8192 without codes 5.5 / 5.0; fp32 387 of 7168 8.1 / 7.4, 340 of 8192 8.9 / 7.6, 368 of 13184 14.5 / 12.1,
+// without codes 318 of 5120 6.4 / 5.7; narrow rows and nearly full layers level.  More than that share holds back nearly full
+// ones: fp32 without codes 592 of 4096 7.1 / 7.3 with 0.9, 7.5 with 0.94).  Only behind a full layer: in the first one a
+// compute unit has one row or none, and the row's own share of the time is all there is to wait for (bf16 without codes, 32768
+// elements, 128 rows 7.95 / 8.39, 160 8.71 / 8.99, 200 10.1 / 10.3; level up to 16384 elements and at 65536).
+// short_rows: rows of two chunks per lane whose computation ends well ahead of the reads of a half-filled round (half
+// precision, static scale).  From two fifths of a round to eleven twentieths they wait 1.16 times the read time: 460 rows of
+// 8192 elements 6.28 / 5.72 us, 576 of 6144 6.55 / 6.05, 576 of 5120 5.46 / 5.3, level or slower below and above (1228 of 4096
+// 6.6 / 6.8).
 uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, RowType type, int quant) {
     if (g_gate >= 0) return (uint32_t)g_gate;
     const int64_t resident = resident_rows(threads, nchunk);
@@ -898,12 +899,12 @@ void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, 
             const int t4 = round_up((chunks_per_row + 3) / 4, 64);
             const int64_t round1 = resident_rows(lanes1, 1), round2 = resident_rows(lanes2, 2);
             // Rows that two chunks per lane leave a third of their lanes idle for (129 to 170 chunks, on three waves or on
-            // two): one chunk between the round of the latter and three of the former (us, one chunk / two: 1160 elements
-            // 9.7 / 10.2 at 4480 rows, 10.4 / 11.2 at 5120, 14.1 / 14.6 at 7680, 18.1 / 18.1 at 10240; 1288 10.1 / 10.9, 11.0 /
-            // 11.9, 15.1 / 15.5, 19.2 / 19.5; 1032 9.5 / 9.7, 10.1 / 10.6, 13.9 / 13.8, 17.2 / 17.1; not fp32 rows, without codes 4146 of
-            // 624 8.99 / 8.54, 6676 of 552 12.2 / 11.7, with codes level), and in bfloat16, whose
-            // arithmetic is unpacked, where two idle two fifths also up to an eighth more than a round (2611 rows of 1032 6.36 /
-            // 6.81, 2816 6.7 / 7.0, but 3072 7.5 / 7.2; half precision 6.35 / 5.97 at 2611).
+            // two): one chunk between the round of the latter and three of the former (us, one chunk / two: 1160 elements 9.7 /
+            // 10.2 at 4480 rows, 10.4 / 11.2 at 5120, 14.1 / 14.6 at 7680, 18.1 / 18.1 at 10240; 1288 10.1 / 10.9, 11.0 / 11.9,
+            // 15.1 / 15.5, 19.2 / 19.5; 1032 9.5 / 9.7, 10.1 / 10.6, 13.9 / 13.8, 17.2 / 17.1; not fp32 rows, without codes
+            // 4146 of 624 8.99 / 8.54, 6676 of 552 12.2 / 11.7, with codes level), and in bfloat16, whose arithmetic is
+            // unpacked, where two idle two fifths also up to an eighth more than a round (2611 rows of 1032 6.36 / 6.81, 2816
+            // 6.7 / 7.0, but 3072 7.5 / 7.2; half precision 6.35 / 5.97 at 2611).
             const bool thin = n == 1 && 3 * chunks_per_row < 4 * lanes2;
             const bool one = thin && (tokens > round2 ? type != RowType::F32 && tokens <= 3 * round1
                                                       : type == RowType::BF16 && 5 * chunks_per_row < 6 * lanes2 && 8 * tokens <= 9 * round1);
@@ -926,23 +927,24 @@ void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, 
 // so that neither piece pays for a partly filled last row of workgroups twice.
 int64_t half_of(int64_t tokens) { return (tokens + kComputeUnits - 1) / kComputeUnits / 2 * kComputeUnits; }
 
-// Launches per call.  A batch of more than one round of workgroups and at most two runs as two launches of half the
-// rows, each a round of its own with the store gate: a read phase and a write phase twice over instead of two rounds
-// that mix the directions.  Only where each piece does fit a round in the shape it is given, rows start on line
-// boundaries, and that shape idles few lanes: from 1.1 rounds on one in eight, or one in five of a single wave with four
-// chunks per lane; from 1.25 rounds on one in five; from 1.5 on one in four of a single wave (fp32 rows of one wave: one in
-// eight, always).  One launch / two, us:
-// bf16 4600 rows of 4096 elements 23.6 / 22.7, 8000 rows 38.5 / 38.0, 2300 of 8192 24.4 / 23.2, 4600 of 3072 19.2 / 17.8; 3200 of
-// 5120 (a sixth idle) 22.1 / 23.3 but 4608 30.4 / 28.9; 9830 of 1664 (a fifth, one wave of four chunks) 22.2 / 21.5-22.0, 11900
-// 25.9 / 24.5; 9830 of 832 (a fifth, of two chunks) 12.4 / 13.2, 14700 17.0 / 15.8; 14700 of 768 (a quarter, one wave) 16.1 / 15.3,
-// 5500 of 3072 (a quarter, two waves) 22.3 / 24.3, 11900 of 640 (three eighths) 11.7 / 12.6; fp32 14700 of 416 15.3 / 15.8.  Pieces
-// beyond a round: 5700 of 2688 21.0 / 24.6.  One chunk per lane (rows of at most 64 chunks): 11500 of 512 8.6 / 9.6, fp32 of 256
-// 7.9 / 9.5.  Rows that end inside lines: 2500 of 9000 30.1 / 31.8.  Wide fp32 rows, four waves and more, of which a compute unit holds
-// few, pay for a layer of workgroups (one per compute unit) that a piece does not fill: two launches where the rows fill 94 % of
-// the two pieces' layers (92 on five waves, 96 on six), without codes 90 % (88 on five).  Two / one by that share, codes: five waves 1.04 at 88 %, 1.00 at 92, 0.96 at
-// 96; six 1.06 / 1.02 / 1.00, seven 1.04 / 1.01 / 0.98, eight 1.02 / 1.01 / 0.97; four 1.03 at 90, 1.00 at 94; without codes five to seven
-// 1.00 at 88, 0.98 at 90, 0.95 at 96 (1518 of 5120 with codes, 99 %, 20.1 / 17.8, but 1331 of 7168, 87 %, 24.5 / 27.0).  codes: for
-// fp32, whether the rows are quantised.
+// Launches per call.  A batch of more than one round of workgroups and at most two runs as two launches of half the rows, each
+// a round of its own with the store gate: a read phase and a write phase twice over instead of two rounds that mix the
+// directions.  Only where each piece does fit a round in the shape it is given, rows start on line boundaries, and that shape
+// idles few lanes: from 1.1 rounds on one in eight, or one in five of a single wave with four chunks per lane; from 1.25 rounds
+// on one in five; from 1.5 on one in four of a single wave (fp32 rows of one wave: one in eight, always).  One launch / two,
+// us:
+// bf16 4600 rows of 4096 elements 23.6 / 22.7, 8000 rows 38.5 / 38.0, 2300 of 8192 24.4 / 23.2, 4600 of 3072 19.2 / 17.8; 3200
+// of 5120 (a sixth idle) 22.1 / 23.3 but 4608 30.4 / 28.9; 9830 of 1664 (a fifth, one wave of four chunks) 22.2 / 21.5-22.0,
+// 11900 25.9 / 24.5; 9830 of 832 (a fifth, of two chunks) 12.4 / 13.2, 14700 17.0 / 15.8; 14700 of 768 (a quarter, one wave)
+// 16.1 / 15.3, 5500 of 3072 (a quarter, two waves) 22.3 / 24.3, 11900 of 640 (three eighths) 11.7 / 12.6; fp32 14700 of 416
+// 15.3 / 15.8.  Pieces beyond a round: 5700 of 2688 21.0 / 24.6.  One chunk per lane (rows of at most 64 chunks): 11500 of 512
+// 8.6 / 9.6, fp32 of 256 7.9 / 9.5.  Rows that end inside lines: 2500 of 9000 30.1 / 31.8.  Wide fp32 rows, four waves and
+// more, of which a compute unit holds few, pay for a layer of workgroups (one per compute unit) that a piece does not fill: two
+// launches where the rows fill 94 % of the two pieces' layers (92 on five waves, 96 on six), without codes 90 % (88 on five).
+// Two / one by that share, codes: five waves 1.04 at 88 %, 1.00 at 92, 0.96 at 96; six 1.06 / 1.02 / 1.00, seven 1.04 / 1.01 /
+// 0.98, eight 1.02 / 1.01 / 0.97; four 1.03 at 90, 1.00 at 94; without codes five to seven 1.00 at 88, 0.98 at 90, 0.95 at 96
+// (1518 of 5120 with codes, 99 %, 20.1 / 17.8, but 1331 of 7168, 87 %, 24.5 / 27.0).  codes: for fp32, whether the rows are
+// quantised.
 int launches_for(int64_t tokens, int chunks_per_row, RowType type, bool codes) {
     if (g_pieces == 1 || g_force_nchunk || g_force_threads || chunks_per_row > 2 * kMaxThreads) return 1;
     const int64_t round = resident_rows(round_up((chunks_per_row + 3) / 4, 64), 4);
@@ -1086,13 +1088,12 @@ void pick_wide_shape(int chunks, int *threads, int *cpl) {
 }
 
 // Bytes of both inputs from which on fp32 batches gate their stores: with less to read per compute unit than a 16-bit kernel of
-// as many lanes has, a small batch has no reason to hold them.  Where the two cross depends on how long a row's own chain
-// is: few waves and no codes early, many waves and two chunks per lane late.  Gated / ungated, batches of a quarter of a round to
+// as many lanes has, a small batch has no reason to hold them.  Where the two cross depends on how long a row's own chain is:
+// few waves and no codes early, many waves and two chunks per lane late.  Gated / ungated, batches of a quarter of a round to
 // one: one wave of one chunk per lane with codes 0.994 at 4 MB, 0.97 at 6; without 0.98 / 0.92 below eleven twentieths of a
-// round, above 1.02 at 6, 0.99 at 8; more waves of one chunk without codes 1.04 / 1.03 / 0.97 / 0.90 at 4 / 5 / 6 / 7, with 1.03 / 1.02 /
-// 1.01 / 0.98; two chunks with codes 1.02 / 1.00 / 0.97 at 7 / 8 / 9, without 0.95 at 7 (0.99 on nine waves); of twelve waves 1.04 / 1.01 / 1.00 at 8 / 9 / 10,
-// 1.01 / 0.97 at 8 / 9 without,
-// four chunks 1.01 / 1.00 / 0.99.
+// round, above 1.02 at 6, 0.99 at 8; more waves of one chunk without codes 1.04 / 1.03 / 0.97 / 0.90 at 4 / 5 / 6 / 7, with
+// 1.03 / 1.02 / 1.01 / 0.98; two chunks with codes 1.02 / 1.00 / 0.97 at 7 / 8 / 9, without 0.95 at 7 (0.99 on nine waves); of
+// twelve waves 1.04 / 1.01 / 1.00 at 8 / 9 / 10, 1.01 / 0.97 at 8 / 9 without, four chunks 1.01 / 1.00 / 0.99.
 int64_t f32_gate_from_bytes(int64_t tokens, int threads, int nchunk, bool codes) {
     const bool one_wave = threads == 64;
     if (nchunk == 4 || (nchunk == 2 && threads >= 768)) return codes || nchunk == 4 ? 9'200'000 : 8'800'000;

@@ -179,14 +179,14 @@ __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t 
 
 // 8 codes = e4m3fn(clamp(rT(v / scale))) for one chunk; `rcp` is RN(1/scale) and is used when FAST.
 // Then, with bf16 and where no value of the wave is infinite, a NaN or beyond 2^60 scales, the quotients are the short ones for
-// finite numerators and the rounded pairs are converted as they are, clamped first (as whole numbers, in pairs) where some value of
-// the wave comes near what has to be: what the many fp8 rows of a call without shared KV heads wait for.  In us, general form for
-// all / this, bf16: 900 tokens of 64+64+64 heads of 128 elements 18.4 / 17.1, of 64 elements (919 tokens) 11.4 / 10.8, 3000 of
-// 32+32+32 27.1 / 24.8, 32 of 64+8+8 2.99 / 2.92, long calls with few KV heads level; with a scale a thousand times too small, so
-// that every wave clamps, 3000 tokens of 32+32+32 27.7 / 25.3, 900 of 64+64+64 19.1 / 17.1.  (Taking those to the general form as
-// well spares the others the choice, half a percent of the first calls, and costs 28.6 and 19.6; with infinities in every wave, which
-// do go there, 27.0 / 27.8.)  fp16 keeps the general form: its own short one was 3 % faster at 2000 tokens of 32+32+32 heads (16.5 / 16.0)
-// and 3 % slower at 4000 (27.95 / 28.7).
+// finite numerators and the rounded pairs are converted as they are, clamped first (as whole numbers, in pairs) where some
+// value of the wave comes near what has to be: what the many fp8 rows of a call without shared KV heads wait for.  In us,
+// general form for all / this, bf16: 900 tokens of 64+64+64 heads of 128 elements 18.4 / 17.1, of 64 elements (919 tokens) 11.4
+// / 10.8, 3000 of 32+32+32 27.1 / 24.8, 32 of 64+8+8 2.99 / 2.92, long calls with few KV heads level; with a scale a thousand
+// times too small, so that every wave clamps, 3000 tokens of 32+32+32 27.7 / 25.3, 900 of 64+64+64 19.1 / 17.1.  (Taking those
+// to the general form as well spares the others the choice, half a percent of the first calls, and costs 28.6 and 19.6; with
+// infinities in every wave, which do go there, 27.0 / 27.8.)  fp16 keeps the general form: its own short one was 3 % faster at
+// 2000 tokens of 32+32+32 heads (16.5 / 16.0) and 3 % slower at 4000 (27.95 / 28.7).
 template <typename T, bool FAST>
 __device__ __forceinline__ u32x2 quantize_chunk(const u32x4 &v, float scale, float rcp) {
     using P = Pack16<T>;
@@ -321,26 +321,27 @@ __device__ __forceinline__ void store_pair(void *p, const u32x4 &a, const u32x4 
         *reinterpret_cast<u32x4 *>(static_cast<char *>(p) + OFFSET) = b;
     }
 }
-// Heads of 64 elements fill one 128-byte line each, and a lane's two chunks of its head are half a line apart: accessed
-// where they are computed, every wave instruction would touch half of each of its lines, the other half following in
-// the next one.  So eight lanes move the lines of their two heads whole -- the even head's with one instruction, the odd
-// head's with the next -- and exchange chunks: a and b on entry are the lane's pieces of the even and the odd head's
-// line, on exit the two chunks of the lane's own head, and the other way round (the exchange is its own inverse; one
-// DPP move per dword and direction).  Measured, half lines / whole ones: 10024 tokens of 64 + 64 heads in place 61.8 /
-// 54.2 us (55.6 with whole stores only), 3000 tokens 20.9 / 19.8, 16384 of 28 + 4 in half precision 32.0 / 27.3;
-// two streams of 2 x (678 + 3608) tokens, 24 + 25 heads 23.7 / 22.1.  Calls that do not stream their stores (below 8 MB)
-// are bound by latency and keep the shorter code (2.14 / 2.21 us at one token).
-// In bfloat16, whose waves are busier, so do streamed calls in place of less than 13.5 MB, of less than 18 MB where a token's last unit
-// is not full, and all those whose units are less than three quarters full (bytes read and written; us, half / whole: 28+4
-// heads 3.37 / 3.44 at 8 MB, 4.02 / 4.07 at 12, 5.26 / 4.63 at 16; 32+8, of 48 places, 4.70 / 4.92 at 16, 6.55 / 6.27 at 24; 16+2, of
-// 32, 4.1 / 4.4 at 10, 3-7 % behind up to 24 and at 60; two streams of 24+24 heads 4.26 / 4.31 at 12 MB, 6.25 / 5.43 at 20).  Half
-// precision gains 4-17 % throughout (32+8 at 8-14 MB: 1-2 % lost).
-// With a 16-bit cache: half precision from a third of a round of waves on (28+4+4 3.54 / 3.65 at 907 tokens, 4.6 / 4.2 at 1500; 64+8+8 6.9 / 6.3 at 1500, 17.9 / 15.4 at 4000, 62.3 / 53.1 at 16000,
-// 32+8+8 11.6 / 10.6 and 38.3 / 33.5); bfloat16 beyond one round of waves where units are four fifths full (64+8+8 18.0 / 16.7 and 61.2 / 54.5, 40+8+8 13.4 /
-// 12.9 and 43.3 / 38.5, 32+8+8 12.1 / 11.8 and 37.6 / 34.3, but 5.4 / 6.1 at 1500), beyond three where they are three quarters full
-// (12+12+12 18.2 / 18.3 at 9000 tokens, 29.0 / 27.0 at 16000; 16+2+2, of 32 places, 19.2 / 20.8).  An fp8 cache, whose conversions then run
-// on both chunks of every lane, gains 4-6 % with few K heads and loses as much with others (64+8+8 34.8 / 32.8 at 9000 tokens, 32+8+8
-// 36.5 / 37.4 at 16000): not done.
+// Heads of 64 elements fill one 128-byte line each, and a lane's two chunks of its head are half a line apart: accessed where
+// they are computed, every wave instruction would touch half of each of its lines, the other half following in the next one.
+// So eight lanes move the lines of their two heads whole -- the even head's with one instruction, the odd head's with the next
+// -- and exchange chunks: a and b on entry are the lane's pieces of the even and the odd head's line, on exit the two chunks of
+// the lane's own head, and the other way round (the exchange is its own inverse; one DPP move per dword and direction).
+// Measured, half lines / whole ones: 10024 tokens of 64 + 64 heads in place 61.8 / 54.2 us (55.6 with whole stores only), 3000
+// tokens 20.9 / 19.8, 16384 of 28 + 4 in half precision 32.0 / 27.3; two streams of 2 x (678 + 3608) tokens, 24 + 25 heads 23.7
+// / 22.1.  Calls that do not stream their stores (below 8 MB) are bound by latency and keep the shorter code (2.14 / 2.21 us at
+// one token).
+// In bfloat16, whose waves are busier, so do streamed calls in place of less than 13.5 MB, of less than 18 MB where a token's
+// last unit is not full, and all those whose units are less than three quarters full (bytes read and written; us, half / whole:
+// 28+4 heads 3.37 / 3.44 at 8 MB, 4.02 / 4.07 at 12, 5.26 / 4.63 at 16; 32+8, of 48 places, 4.70 / 4.92 at 16, 6.55 / 6.27 at
+// 24; 16+2, of 32, 4.1 / 4.4 at 10, 3-7 % behind up to 24 and at 60; two streams of 24+24 heads 4.26 / 4.31 at 12 MB, 6.25 /
+// 5.43 at 20).  Half precision gains 4-17 % throughout (32+8 at 8-14 MB: 1-2 % lost).
+// With a 16-bit cache: half precision from a third of a round of waves on (28+4+4 3.54 / 3.65 at 907 tokens, 4.6 / 4.2 at 1500;
+// 64+8+8 6.9 / 6.3 at 1500, 17.9 / 15.4 at 4000, 62.3 / 53.1 at 16000, 32+8+8 11.6 / 10.6 and 38.3 / 33.5); bfloat16 beyond one
+// round of waves where units are four fifths full (64+8+8 18.0 / 16.7 and 61.2 / 54.5, 40+8+8 13.4 / 12.9 and 43.3 / 38.5,
+// 32+8+8 12.1 / 11.8 and 37.6 / 34.3, but 5.4 / 6.1 at 1500), beyond three where they are three quarters full (12+12+12 18.2 /
+// 18.3 at 9000 tokens, 29.0 / 27.0 at 16000; 16+2+2, of 32 places, 19.2 / 20.8).  An fp8 cache, whose conversions then run on
+// both chunks of every lane, gains 4-6 % with few K heads and loses as much with others (64+8+8 34.8 / 32.8 at 9000 tokens,
+// 32+8+8 36.5 / 37.4 at 16000): not done.
 __device__ __forceinline__ void exchange_lines(u32x4 &a, u32x4 &b) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -777,7 +778,8 @@ constexpr int kPartsShift = 18, kMaxParts = 31;
 constexpr int token_kernel_v_chunks(int upt, bool two) { return two ? 1 : upt == 3 ? 3 : 2; }  // per lane and part
 constexpr int token_kernel_lds_bytes_per_wave(int upt, bool set_kv) { return (2 * upt + (set_kv ? 1 : 0)) * 1024; }  // TWO: a token's units and 64 V chunks
 
-// PARTS: tokens may be split (as run-time values the parts cost whole tokens 0.3 to 1 %: 28+4+4 heads 18.66 / 18.82 us at 6144 tokens).
+// PARTS: tokens may be split (as run-time values the parts cost whole tokens 0.3 to 1 %: 28+4+4 heads 18.66 / 18.82 us at 6144
+// tokens).
 // AXES: 1; 3 with sections in which every aligned group of 8 frequencies takes one axis (no branch around the table loads);
 // kMergedAxes with any others.
 constexpr int kMergedAxes = 4;
@@ -1207,11 +1209,12 @@ rope_rms_2way_kernel(const u32x8 first, const u32x4 second, const u32x2 third, c
     }
 }
 
-// The same for batches of one to two rounds of that: a wave takes two groups of heads, one after the other in their segment, which
-// share their weights, so that a round holds 16384 groups (half precision, eight waves per SIMD) or 14336 (bfloat16, whose unpacked
-// arithmetic spills three registers at eight: seven), and holds its stores until the launch's reads are through.  NeoX-style
-// rotation only, sizes measured in launch_2way.  (A kernel of its own: with the number of groups as a template parameter the allocator gave
-// the kernel above 46 registers for 35 and 2 x (678 + 3608) tokens took 35.4 us for 35.3.)
+// The same for batches of one to two rounds of that: a wave takes two groups of heads, one after the other in their segment,
+// which share their weights, so that a round holds 16384 groups (half precision, eight waves per SIMD) or 14336 (bfloat16,
+// whose unpacked arithmetic spills three registers at eight: seven), and holds its stores until the launch's reads are
+// through.  NeoX-style rotation only, sizes measured in launch_2way.  (A kernel of its own: with the number of groups as a
+// template parameter the allocator gave the kernel above 46 registers for 35 and 2 x (678 + 3608) tokens took 35.4 us for
+// 35.3.)
 constexpr int kTwoUnitWaves[2] = {7, 8};  // per SIMD: bfloat16, half precision
 template <typename T, int D, bool WHOLE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kTwoUnitWaves[is_half<T>])))
@@ -1371,19 +1374,22 @@ template <typename T, int D>
 int launch_2way(const TwoWayArgs &a, bool neox, unsigned batch, hipStream_t stream) {
     constexpr int HPW = 64 / (D / 16);
     const int64_t rows = (int64_t)batch * ((int64_t)a.rows[0] + a.rows[1] + a.rows[2] + a.rows[3]), waves = (int64_t)batch * a.unit_end[3];
-    // The store gate (see RopeUnit::finish) where the waves are all resident at once: 1.1 times the read time at 7 TB/s, 1.25 with
-    // pairwise rotation, whose two table pieces per chunk lengthen the loading.  Half precision from three eighths of a round on (us, ungated /
-    // gated: 4.74 / 4.13 at 3820 waves, 5.08 / 4.42 at 4476, 6.99 / 6.2 at 7075, 7.24 / 6.1 at 7730; pairwise 6.56 / 5.8 at 6304, 7.38 / 6.6 at 7638; level at 2694);
-    // bfloat16, whose arithmetic takes longer than the reads of a full round, from a half to 27/32 of it (4.58 / 4.72 at 3950, 5.18 / 4.94 at 4962, 5.55 / 5.0 at 5072, 6.30 / 6.0 at 6080;
-    // 7.76 / 7.9 at 7938; pairwise from 15/32, 6.16 / 5.5 at 5201), and not heads of 64 rotated by halves (5.58 / 5.68 at 4582, 7.79 / 8.0 at 7356).
+    // The store gate (see RopeUnit::finish) where the waves are all resident at once: 1.1 times the read time at 7 TB/s, 1.25
+    // with pairwise rotation, whose two table pieces per chunk lengthen the loading.  Half precision from three eighths of a
+    // round on (us, ungated / gated: 4.74 / 4.13 at 3820 waves, 5.08 / 4.42 at 4476, 6.99 / 6.2 at 7075, 7.24 / 6.1 at 7730;
+    // pairwise 6.56 / 5.8 at 6304, 7.38 / 6.6 at 7638; level at 2694); bfloat16, whose arithmetic takes longer than the reads
+    // of a full round, from a half to 27/32 of it (4.58 / 4.72 at 3950, 5.18 / 4.94 at 4962, 5.55 / 5.0 at 5072, 6.30 / 6.0 at
+    // 6080; 7.76 / 7.9 at 7938; pairwise from 15/32, 6.16 / 5.5 at 5201), and not heads of 64 rotated by halves (5.58 / 5.68 at
+    // 4582, 7.79 / 8.0 at 7356).
     uint32_t gate = 0;
     const bool gated = is_half<T> ? 8 * waves >= 3 * kResidentUnits && waves <= kResidentUnits
                                   : 32 * waves >= (neox ? 16 : 15) * kResidentUnits && 32 * waves <= 27 * kResidentUnits && (D != 64 || !neox);
     if (g_unit_gate > 0) gate = (uint32_t)g_unit_gate;
     else if (g_unit_gate < 0 && gated) gate = (uint32_t)((neox ? 1.1 : 1.25) * (double)(2 * rows * D) / 70000.0);
-    // Two units per wave where a round holds the batch so and not with one, gate 1.03 times the read time.  Rotated by halves only: pairwise it is level
-    // to 10 % behind (us, one unit / two: 9.39 / 8.1 at 11081 waves, 10.32 / 8.8 at 12366 and 12.47 / 10.8 at 16070 in half precision, 8.86 / 7.8 at
-    // 9740, 10.48 / 8.9 at 12024, 11.50 / 10.1 at 13752 in bfloat16; 6.68 / 7.0 at 7198; pairwise 10.06 / 10.5 at 11915, 11.86 / 12.7 at 14450).
+    // Two units per wave where a round holds the batch so and not with one, gate 1.03 times the read time.  Rotated by halves
+    // only: pairwise it is level to 10 % behind (us, one unit / two: 9.39 / 8.1 at 11081 waves, 10.32 / 8.8 at 12366 and 12.47
+    // / 10.8 at 16070 in half precision, 8.86 / 7.8 at 9740, 10.48 / 8.9 at 12024, 11.50 / 10.1 at 13752 in bfloat16; 6.68 /
+    // 7.0 at 7198; pairwise 10.06 / 10.5 at 11915, 11.86 / 12.7 at 14450).
     int64_t pairs = 0;
     for (int seg = 0; seg < 4; ++seg) pairs += ((int64_t)a.rows[seg] + 2 * HPW - 1) / (2 * HPW);
     const bool fits = (int64_t)batch * pairs <= 1024 * kTwoUnitWaves[is_half<T>];
@@ -1510,32 +1516,32 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     const TokenShape one_item = token_shape(a, D, axes, set_kv, kv_fp8, false), two_items = token_shape(a, D, axes, set_kv, kv_fp8, true);
     const bool two = two_items.units && (g_token_waves == 3 || !one_item.units);
     const TokenShape shape = two ? two_items : one_item;
-    // ... and clearly too large for the kernel above to hold all of its waves at once (from 10240 units, five quarters
-    // of what it holds; below that the kernel above, gated, is ahead or level: 8.3 against 9.7 us at 1536 tokens of
-    // 32+8+8 heads, 9.1 against 9.5 at 2100 tokens of 28+4+4; from there on this one is: 32+8+8 heads 10.3 against
-    // 11.1 us at 2048 tokens, 13.6 against 14.8 at 3000, 16.6 against 17.3 at 3700, 16.2 against 18.2 at 4096; 28+4+4
-    // heads with three axes 10.0 against 11.7 us at 3000 tokens, 12.2 against 14.5 at 4096, interleaved sections 10.0 against
-    // 11.6 at 2621, 12.7 against 16.2 at 4096; heads of 256 elements, 28+4+4, two parts of four, from 11264: 10.2 against 12.4 at
-    // 1536 tokens, 12.5 against 15.5 at 2048; 64+8+8, two of five, 14.2 against 16.0 at 2048).  With three units per wave from 9216 units:
-    // 40+8+8 heads, two parts, 8.5 against 9.7 us at 1536 tokens, 10.2 against 12.2 at 2048; 16+2+2 7.9 against 8.9 at 3072, 9.4
-    // against 10.6 at 4096; 12+12+12 10.3 against 12.7, 12.8 against 15.5.
-    // With two items per wave from there to twice that many items: 4096 waves, four on every SIMD, one item each and
-    // the others dealt out evenly.  The SIMD with the most items sets the time (the rotation arithmetic of its waves
-    // is two thirds of the launch), so the time goes up in steps of 1024 items where the kernel above is linear; this
-    // one is ahead or level everywhere (graph replays, 28+4+4 heads, one axis / three: 16.1 / 16.4 against 17.2 / 17.5 us
-    // at 4800 tokens, 18.2 / 18.5 against 18.4 / 18.8 at 5200, 19.1 / 19.6 against 21.1 / 21.5 at 6144, 21.7 / 21.7 against
-    // 23.5 / 23.7 at 7000, 24.2 / 24.4 against 24.7 / 25.3 at 7500, 25.3 / 25.3 against 26.8 / 27.3 at 8192, interleaved 19.7
-    // against 22.5 at 6144, 26.0 against 28.5 at 8192; 40+8+8, two parts of three, 12.1 against 13.2 at 2304, 19.9 against 21.5 at
-    // 4096; 28+4+4 heads of 256, two of four, 18.4 against 20.8 at 3000, 25.4 against 27.1 at 4096; level below
-    // 4608 items, where the kernel above stays).  Half as many waves with two items each were behind that: 20.0 at 6144 tokens.
-    // (in place, with no V row and no scatter, the kernel above holds out a little longer: 9.0 against 9.5 us at 2048
-    // tokens of 32+8 heads, then 11.9 against 11.2 at 3000, 15.4 against 13.7 at 4096; 28+4 heads with three axes 10.7
-    // against 9.5 at 3000 tokens, 13.2 against 11.5 at 4096, 18.4 against 17.4 at 6144 and 23.2 against 21.6 at 8192 with
-    // two items per wave; 40+8, parts of three, 8.3 against 7.9 at 1536, 10.4 against 9.4 at 2048, 11.2 against 11.4 at 2304 and
-    // 13.9 against 13.5 at 3000 with two items per wave)
+    // ... and clearly too large for the kernel above to hold all of its waves at once (from 10240 units, five quarters of what
+    // it holds; below that the kernel above, gated, is ahead or level: 8.3 against 9.7 us at 1536 tokens of 32+8+8 heads, 9.1
+    // against 9.5 at 2100 tokens of 28+4+4; from there on this one is: 32+8+8 heads 10.3 against 11.1 us at 2048 tokens, 13.6
+    // against 14.8 at 3000, 16.6 against 17.3 at 3700, 16.2 against 18.2 at 4096; 28+4+4 heads with three axes 10.0 against
+    // 11.7 us at 3000 tokens, 12.2 against 14.5 at 4096, interleaved sections 10.0 against 11.6 at 2621, 12.7 against 16.2 at
+    // 4096; heads of 256 elements, 28+4+4, two parts of four, from 11264: 10.2 against 12.4 at 1536 tokens, 12.5 against 15.5
+    // at 2048; 64+8+8, two of five, 14.2 against 16.0 at 2048).  With three units per wave from 9216 units: 40+8+8 heads, two
+    // parts, 8.5 against 9.7 us at 1536 tokens, 10.2 against 12.2 at 2048; 16+2+2 7.9 against 8.9 at 3072, 9.4 against 10.6 at
+    // 4096; 12+12+12 10.3 against 12.7, 12.8 against 15.5.
+    // With two items per wave from there to twice that many items: 4096 waves, four on every SIMD, one item each and the others
+    // dealt out evenly.  The SIMD with the most items sets the time (the rotation arithmetic of its waves is two thirds of the
+    // launch), so the time goes up in steps of 1024 items where the kernel above is linear; this one is ahead or level
+    // everywhere (graph replays, 28+4+4 heads, one axis / three: 16.1 / 16.4 against 17.2 / 17.5 us at 4800 tokens, 18.2 / 18.5
+    // against 18.4 / 18.8 at 5200, 19.1 / 19.6 against 21.1 / 21.5 at 6144, 21.7 / 21.7 against 23.5 / 23.7 at 7000, 24.2 /
+    // 24.4 against 24.7 / 25.3 at 7500, 25.3 / 25.3 against 26.8 / 27.3 at 8192, interleaved 19.7 against 22.5 at 6144, 26.0
+    // against 28.5 at 8192; 40+8+8, two parts of three, 12.1 against 13.2 at 2304, 19.9 against 21.5 at 4096; 28+4+4 heads of
+    // 256, two of four, 18.4 against 20.8 at 3000, 25.4 against 27.1 at 4096; level below 4608 items, where the kernel above
+    // stays).  Half as many waves with two items each were behind that: 20.0 at 6144 tokens.
+    // (in place, with no V row and no scatter, the kernel above holds out a little longer: 9.0 against 9.5 us at 2048 tokens of
+    // 32+8 heads, then 11.9 against 11.2 at 3000, 15.4 against 13.7 at 4096; 28+4 heads with three axes 10.7 against 9.5 at
+    // 3000 tokens, 13.2 against 11.5 at 4096, 18.4 against 17.4 at 6144 and 23.2 against 21.6 at 8192 with two items per wave;
+    // 40+8, parts of three, 8.3 against 7.9 at 1536, 10.4 against 9.4 at 2048, 11.2 against 11.4 at 2304 and 13.9 against 13.5
+    // at 3000 with two items per wave)
     // Half precision, whose arithmetic is packed, from seven eighths of the other kernel's round where nearly all lanes have a
-    // head and two waves are left per SIMD: 40+8+8 heads 6.6 against 7.0 us at 1228 tokens, 6.8 against 7.5 at 1365, 9.6 against
-    // 11.7 at 2048 (32+8+8, parts of five, 7.4 against 7.1 at 1471; 48+8+8, an idle unit, 7.2 against 6.8 at 1056).
+    // head and two waves are left per SIMD: 40+8+8 heads 6.6 against 7.0 us at 1228 tokens, 6.8 against 7.5 at 1365, 9.6
+    // against 11.7 at 2048 (32+8+8, parts of five, 7.4 against 7.1 at 1471; 48+8+8, an idle unit, 7.2 against 6.8 at 1056).
     const bool full = 8 * heads >= 7 * places, no_idle_unit = shape.units * shape.parts == (int)a.units_per_token;
     const int64_t from_units = half && full && no_idle_unit && shape.units <= 4 && shape.items >= 2048 ? 7 * kResidentUnits / 8
                                : shape.units == 3 ? 9 * kResidentUnits / 8
@@ -1547,13 +1553,15 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // (two items per wave: level or 1 % behind below, 15.4 against 15.2 us at 4100 tokens)
     bool large = two ? shape.items >= kTokenWaveCapacity + kTokenWaveCapacity / 8 : a.total_units >= (kv_fp8 ? from_units_fp8 : from_units);
     // Where the margin is thin it does not cover every fill of the last layer of waves.  Beyond whole tokens of four or five
-    // units of 128-element heads that read one table row, these stay with the kernel above (us, that one / this one).  In place:
-    // pairwise rotation (28+4 heads of 256 in half precision 10.4 / 11.2 at 1611 tokens, 40+8 17.1 / 17.7 at 3802), parts of five or with
-    // idle units (64+8 heads 10.4 / 10.7 at 1370 tokens, 48+8 10.3 / 10.7 at 1739), a layer that has just begun (64+8 heads 11.5 / 12.6 at 1618
-    // tokens, 3236 items) and two items per wave in bfloat16 (40+8 16.7 / 16.7 at 3749) or with idle lanes (16+2 in half precision 13.8 / 15.3 at 8186).
-    // With a cache: a layer that has just begun where lanes or units idle (16+2+2 in half precision 7.6 / 8.2 at 3148), two items per wave
-    // where lanes idle in bfloat16 but for merged table rows (16+2+2 16.1 / 16.6 at 7544).  Pairwise with a cache: the latter in every type, seven layers and
-    // more (20+4+4 in half precision 21.0 / 21.5 at 7797), a layer that has just begun, and bfloat16 with three V chunks per lane (12+12+12 14.3 / 14.9 at 3592).
+    // units of 128-element heads that read one table row, these stay with the kernel above (us, that one / this one).  In
+    // place: pairwise rotation (28+4 heads of 256 in half precision 10.4 / 11.2 at 1611 tokens, 40+8 17.1 / 17.7 at 3802),
+    // parts of five or with idle units (64+8 heads 10.4 / 10.7 at 1370 tokens, 48+8 10.3 / 10.7 at 1739), a layer that has just
+    // begun (64+8 heads 11.5 / 12.6 at 1618 tokens, 3236 items) and two items per wave in bfloat16 (40+8 16.7 / 16.7 at 3749)
+    // or with idle lanes (16+2 in half precision 13.8 / 15.3 at 8186). With a cache: a layer that has just begun where lanes or
+    // units idle (16+2+2 in half precision 7.6 / 8.2 at 3148), two items per wave where lanes idle in bfloat16 but for merged
+    // table rows (16+2+2 16.1 / 16.6 at 7544).  Pairwise with a cache: the latter in every type, seven layers and more (20+4+4
+    // in half precision 21.0 / 21.5 at 7797), a layer that has just begun, and bfloat16 with three V chunks per lane (12+12+12
+    // 14.3 / 14.9 at 3592).
     if (!whole_token(a, D, axes, shape.units, shape.parts)) {
         const int64_t last = shape.items > 3072 ? shape.items % 1024 : 0;  // items of the last layer, 0: it is full
         if (!set_kv) large = large && no_idle_unit && (two ? full : last == 0 || last >= 256);  // (and see token_form_in_place)
