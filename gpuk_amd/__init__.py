@@ -30,7 +30,7 @@ DIRECT_LIB = os.path.join(LIB_DIR, "gpuk_direct.so")   # direct calls of its ope
 
 if not all(map(os.path.exists, (KERNEL_LIB, TORCH_LIB, DIRECT_LIB))):
     raise ImportError(
-        f"gpuk_amd: {KERNEL_LIB} / {TORCH_LIB} / {DIRECT_LIB} not built; run `python -m gpuk_amd.build` "
+        f"gpuk_amd: {KERNEL_LIB} / {TORCH_LIB} / {DIRECT_LIB} not built; run `python gpuk_amd/build.py` "
         "(hipcc cross-compiles gfx950 without a GPU). There is no fallback path.")
 
 torch.ops.load_library(TORCH_LIB)

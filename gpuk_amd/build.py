@@ -1,4 +1,4 @@
-"""In-tree build of the shared libraries (run as `python -m gpuk_amd.build`).
+"""In-tree build of the shared libraries (run as `python gpuk_amd/build.py`).
 
   gpuk_amd/lib/libgpuk_amd.so : HIP kernels for gfx950 behind the C ABI of include/gpuk_amd.h (no torch)
   gpuk_amd/lib/libgpuk.so     : torch library `gpuk` (csrc/register.cpp + csrc/ops/*.cpp), links the former

@@ -42,7 +42,7 @@ def lib():
     global _lib
     if _lib is None:
         if not os.path.exists(_LIB_PATH):
-            raise ImportError(f"{_LIB_PATH} not built; run `python -m gpuk_amd.build`")
+            raise ImportError(f"{_LIB_PATH} not built; run `python gpuk_amd/build.py`")
         L = C.CDLL(_LIB_PATH)
         L.gpuk_status_string.restype = C.c_char_p
         L.gpuk_status_string.argtypes = [C.c_int]

@@ -1,5 +1,5 @@
 """Where the time goes inside a wave: reads the phase stamps of the profiling build (libgpuk_amd_stamps.so, built by
-`python -m gpuk_amd.build --stamps`), in which every wave of the kernels records the shader clock at named points, the
+`python gpuk_amd/build.py --stamps`), in which every wave of the kernels records the shader clock at named points, the
 100 MHz wall clock at its entry and exit, and its place on the chip.
 
     python -m gpuk_amd.stamps norm_quant [--tokens 1 128 512] [--hidden 7168]
@@ -53,7 +53,7 @@ ROPE_UNIT_PHASES = [
 
 def bind():
     if not os.path.exists(STAMPS_LIB):
-        raise SystemExit(f"{STAMPS_LIB} not built; run `python -m gpuk_amd.build --stamps`")
+        raise SystemExit(f"{STAMPS_LIB} not built; run `python gpuk_amd/build.py --stamps`")
     capi.use_library(STAMPS_LIB)
     L = capi.lib()
     for name in ("gpuk_stamps_set_norm_quant", "gpuk_stamps_set_rope"):

@@ -190,6 +190,22 @@ def test_dist_env_rejects_multi_gpu_groups(monkeypatch):
         gpuk.GPUKDistEnv(device_id=0)
 
 
+def test_build_command_needs_nothing_built(tmp_path):
+    """Where the libraries are missing, importing the package names a command that gets as far as the compiler."""
+    import shutil
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    shutil.copytree(os.path.join(root, "gpuk_amd"), tmp_path / "gpuk_amd", ignore=shutil.ignore_patterns("lib", "build", "__pycache__"))
+    run = lambda *args: subprocess.run([sys.executable, *args], cwd=tmp_path, capture_output=True, text=True, env={**os.environ, "HIPCC": "/bin/false"})
+    missing = run("-c", "import gpuk_amd")
+    command = re.search(r"not built; run `python (.*?)`", missing.stderr)
+    assert missing.returncode != 0 and command
+    started = run(*command[1].split())
+    assert started.returncode != 0 and "command failed: /bin/false" in started.stderr
+
+
 def test_bench_refuses_more_than_one_gpu():
     import subprocess
     import sys
