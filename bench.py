@@ -432,8 +432,8 @@ def main():
                                                  "algorithmic_bytes": nb4}
         del ins2, out2, qkv4
 
-        # decode shapes: per call, eager (host launch overhead included) and replayed from a HIP graph of 20 calls on
-        # 20 distinct buffer sets (GPU-side cost)
+        # decode shapes, by the public names: per call, eager (what a call costs the host included) and replayed from a HIP
+        # graph of 20 calls on 20 distinct buffer sets (GPU-side cost)
         decode = {}
         NG = 20
         for t in workloads.DECODE_TOKENS_WIDE:
@@ -445,7 +445,7 @@ def main():
 
             def nq_call(i=0):
                 x, r_, ro, codes, sc = nq[i % NG]
-                capi.add_rmsnorm_quant(x, r_, g_, ro, codes, sc, d.eps, 1)
+                gpuk.allreduce_rms(0, x, r_, g_, ro, codes, sc, d.eps, 1)
 
             r = workloads.config5_rope(t)
             k0, v0 = r.new_cache()
@@ -456,8 +456,8 @@ def main():
 
             def rope_call(i=0):
                 qkv, q_out = rp[i % NG]
-                capi.rope_rms_set_kv(qkv, qw, kw, cs, pos, t, r.num_heads_q, r.num_heads_k, r.num_heads_v, r.head_size,
-                                     r.is_neox, r.eps, q_out, kc, vc, loc, r.k_scale, r.v_scale)
+                gpuk.fused_rope_rms_set_kv(qkv, qw, kw, cs, pos, t, r.num_heads_q, r.num_heads_k, r.num_heads_v, r.head_size,
+                                           r.is_neox, r.eps, q_out, kc, vc, loc, r.k_scale, r.v_scale)
 
             def nq_skeleton_call(i=0):
                 x, r_, ro, codes, sc = nq[i % NG]
@@ -482,7 +482,7 @@ def main():
 
         def c1_call(i=0):
             x, r_, ro, codes = c1_bufs[i % NG]
-            capi.add_rmsnorm_quant(x, r_, c1_g, ro, codes, c1_scale, c1.eps, 3)
+            gpuk.allreduce_rms(0, x, r_, c1_g, ro, codes, c1_scale, c1.eps, 3)
 
         extras["static_quant_T128_H4096_us_per_call"] = {"graph": round(graph_time_us(c1_call, NG), 2),
                                                          "eager": round(event_time_ms(c1_call, 200) * 1e3, 2),
