@@ -1562,6 +1562,9 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // table rows (16+2+2 16.1 / 16.6 at 7544).  Pairwise with a cache: the latter in every type, seven layers and more (20+4+4
     // in half precision 21.0 / 21.5 at 7797), a layer that has just begun, and bfloat16 with three V chunks per lane (12+12+12
     // 14.3 / 14.9 at 3592).
+    // (Over calls drawn afterwards that only one of those with a cache keeps here, the token kernel's time over this one's: two
+    // items per wave with idle lanes 0.81 to 1.03, on average 0.93, pairwise and 0.90 to 1.05, 0.96, in bfloat16 rotated by
+    // halves, a layer that has just begun 0.86 to 1.11, 0.97; the other three level, 0.88 to 1.06.)
     if (!whole_token(a, D, axes, shape.units, shape.parts)) {
         const int64_t last = shape.items > 3072 ? shape.items % 1024 : 0;  // items of the last layer, 0: it is full
         if (!set_kv) large = large && no_idle_unit && (two ? full : last == 0 || last >= 256);  // (and see token_form_in_place)
