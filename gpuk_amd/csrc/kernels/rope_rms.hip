@@ -178,15 +178,15 @@ __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t 
 }
 
 // 8 codes = e4m3fn(clamp(rT(v / scale))) for one chunk; `rcp` is RN(1/scale) and is used when FAST.
-// Then, with bf16 and where no value of the wave is infinite, a NaN or beyond 2^60 scales, the quotients are the short ones for
-// finite numerators and the rounded pairs are converted as they are, clamped first (as whole numbers, in pairs) where some
-// value of the wave comes near what has to be: what the many fp8 rows of a call without shared KV heads wait for.  In us,
-// general form for all / this, bf16: 900 tokens of 64+64+64 heads of 128 elements 18.4 / 17.1, of 64 elements (919 tokens) 11.4
-// / 10.8, 3000 of 32+32+32 27.1 / 24.8, 32 of 64+8+8 2.99 / 2.92, long calls with few KV heads level; with a scale a thousand
-// times too small, so that every wave clamps, 3000 tokens of 32+32+32 27.7 / 25.3, 900 of 64+64+64 19.1 / 17.1.  (Taking those
-// to the general form as well spares the others the choice, half a percent of the first calls, and costs 28.6 and 19.6; with
-// infinities in every wave, which do go there, 27.0 / 27.8.)  fp16 keeps the general form: its own short one was 3 % faster at
-// 2000 tokens of 32+32+32 heads (16.5 / 16.0) and 3 % slower at 4000 (27.95 / 28.7).
+// Then, with bf16 and where no value of the wave comes near what has to be clamped (nor is infinite or a NaN), the quotients
+// are the short ones for finite numerators and the rounded pairs are converted as they are: what the many fp8 rows of a call
+// without shared KV heads wait for.  In us without / with, bf16: 900 tokens of 64+64+64 heads of 128 elements 18.4 / 17.0, of
+// 64 elements (919 tokens) 11.4 / 10.7, 3000 of 32+32+32 27.1 / 24.8, 32 of 64+8+8 2.99 / 2.90, long calls with few KV heads
+// level; with a scale a thousand times too small, so that every wave clamps, 3000 tokens of 32+32+32 27.7 / 28.6.  Short
+// quotients for those too, the rounded pairs clamped as whole numbers, take 25.3 there, but the choice costs the calls that
+// clamp nothing more than it may: decode batches 0.5 to 4 % (8 tokens of 32+32+32 2.93 / 3.03, 64 of 64+8+8 2.75 / 2.81, with
+// the clamped form on a branch of its own 3.00 and 2.80): not done.  fp16 keeps the general form: its own short one was 3 %
+// faster at 2000 tokens of 32+32+32 heads (16.5 / 16.0) and 3 % slower at 4000 (27.95 / 28.7).
 template <typename T, bool FAST>
 __device__ __forceinline__ u32x2 quantize_chunk(const u32x4 &v, float scale, float rcp) {
     using P = Pack16<T>;
@@ -198,24 +198,17 @@ __device__ __forceinline__ u32x2 quantize_chunk(const u32x4 &v, float scale, flo
         u16x2 most = __builtin_bit_cast(u16x2, v[0] & 0x7fff7fffu);
 #pragma unroll
         for (int j = 1; j < 4; ++j) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, v[j] & 0x7fff7fffu));
-        const uint32_t both = __builtin_bit_cast(uint32_t, most), largest = __builtin_elementwise_max(both << 16, both);
-        const bool clamps = __builtin_amdgcn_ballot_w64(largest > __builtin_bit_cast(uint32_t, 440.0f * scale)) != 0;
-        if (__builtin_expect(!clamps || __builtin_amdgcn_ballot_w64(largest > __builtin_bit_cast(uint32_t, 0x1p60f * scale)) == 0, 1)) {
-            uint32_t w[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) w[j] = P::pack(div_by_rcp_finite(P::lo(v[j]), scale, rcp), div_by_rcp_finite(P::hi(v[j]), scale, rcp));
-            if (__builtin_expect(clamps, 0)) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const u16x2 magnitude = __builtin_elementwise_min(__builtin_bit_cast(u16x2, w[j] & 0x7fff7fffu), u16x2{0x43e0, 0x43e0});  // 448
-                    w[j] = bitselect(0x7fff7fffu, __builtin_bit_cast(uint32_t, magnitude), w[j]);
-                }
-            }
+        const uint32_t both = __builtin_bit_cast(uint32_t, most);
+        const bool clamps = __builtin_elementwise_max(both << 16, both) > __builtin_bit_cast(uint32_t, 440.0f * scale);
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(clamps) == 0, 1)) {
             u32x2 codes;
 #pragma unroll
             for (int j = 0; j < 4; j += 2) {
-                const i16x2 low = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(i16x2{0, 0}, __builtin_bit_cast(bf16x2_t, w[j]), 1.0f, false);
-                codes[j / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(low, __builtin_bit_cast(bf16x2_t, w[j + 1]), 1.0f, true));
+                const auto pair = [&](uint32_t w) {
+                    return __builtin_bit_cast(bf16x2_t, P::pack(div_by_rcp_finite(P::lo(w), scale, rcp), div_by_rcp_finite(P::hi(w), scale, rcp)));
+                };
+                const i16x2 low = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(i16x2{0, 0}, pair(v[j]), 1.0f, false);
+                codes[j / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(low, pair(v[j + 1]), 1.0f, true));
             }
             return codes;
         }

@@ -60,7 +60,7 @@ def test_every_form_of_the_conversion(device, scale):
     largest = float((unclamped.float().abs().max() / s))
     assert 432.0 < largest <= 440.0                       # up to the threshold, and rounding up to the top code
     check(unclamped, scale, torch.bfloat16, device)
-    finite, finite_top = magnitudes(float(2.0 ** 60 * s))  # short quotients of any size, clamped
+    finite, finite_top = magnitudes(float(2.0 ** 60 * s))  # quotients of any size, clamped
     check(finite, scale, torch.bfloat16, device)
     # passes of values below the threshold but for one, in every lane's first or last place in turn
     bits = unclamped.reshape(-1).view(torch.int16).to(torch.int32)[:PASS] & 0xffff
