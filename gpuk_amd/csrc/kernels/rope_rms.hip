@@ -146,6 +146,12 @@ __device__ __forceinline__ void load_trig_by_axis(const uint16_t *table, int64_t
 // heads, gated, 9.02 / 7.48 / 7.12; 3134 of 24+8+8 14.4 / 15.4 / 14.2; 9000 of 16+2+2 19.6 / 21.2 / 19.5; 16384 of 28+4+4 50.0 /
 // 53.0 / 50.1; heads of 256 elements, 28+4+4, 900 tokens, gated, 9.07 / - / 7.22.  Ungated ones of 256 are level on average, and
 // 6 % ahead to 9 % behind by size (24+8+8 11.5 / - / 12.3 at 1150 tokens, 32+8+8 9.8 / - / 9.2 at 830): those keep 66.
+// kHeldTo64: gated forms of 128 elements with a cache, but for bf16 rotated by halves, are held by the attribute, or they lose
+// where the round is nearly full (28+4+4 heads, interleaved sections, 1925 tokens, us, 55 to 57 / 59: pairwise bf16 8.6 / 9.4,
+// fp16 8.5 / 9.2, fp8 cache 8.9 / 9.7 and 8.4 / 9.3; by halves fp16 7.15 / 7.46, but bf16 7.5 / 7.4 and 6.3 / 6.0 for 655
+// tokens of 64+8+8; pairwise calls of 655 tokens gain up to 8 % with 59, which the fuller ones would pay for).
+template <typename T, int D, bool NEOX, int AXES, bool SETKV, bool GATED>
+constexpr bool kHeldTo64 = AXES == 3 && D == 128 && SETKV && GATED && (!NEOX || is_half<T>);
 template <int D, bool NEOX, int AXES, bool FEWER_REGISTERS>
 __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t p0, int64_t p1, int64_t p2,
                                                  const uint32_t (&axis1)[4], const uint32_t (&axis2)[4], int sub,
@@ -440,7 +446,7 @@ struct RopeUnit {
                 return;
             }
         }
-        load_trig_merged<D, NEOX, AXES, GATED || D != 256>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
+        load_trig_merged<D, NEOX, AXES, (GATED || D != 256) && !kHeldTo64<T, D, NEOX, AXES, SETKV, GATED>>(table, st.p0, st.p1, st.p2, a.axis1, a.axis2, sub, st.cosv, st.sinv);
     }
 
     // Norm, rotation and all stores of the unit.  GATED: no store before a.gate ticks after `entry`, the wave's entry
@@ -560,7 +566,7 @@ struct UnitBlock {  // the argument block, behind the leading parameters
 };
 
 template <typename T, int D, bool NEOX, int AXES, bool SETKV, bool KVFP8, bool GATED, bool WHOLE>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kHeldTo64<T, D, NEOX, AXES, SETKV, GATED> ? 8 : 1)))
 rope_rms_kernel(const u32x8 first, const u32x4 second, const u32x2 third, const UnitBlock<D, AXES, SETKV, KVFP8, GATED> rest) {
     using Unit = RopeUnit<T, D, NEOX, AXES, SETKV, KVFP8>;
     using Block = UnitBlock<D, AXES, SETKV, KVFP8, GATED>;
