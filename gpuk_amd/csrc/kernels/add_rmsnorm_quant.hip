@@ -32,7 +32,6 @@ namespace gpuk {
 namespace {
 
 constexpr int kMaxThreads = 1024;
-constexpr int kMaxWaves = kMaxThreads / 64;
 constexpr int kMaxChunks = 8, kMaxChunksF32 = 4;  // chunks per lane the kernels of 16-bit and of fp32 rows have forms for
 
 template <typename P>
@@ -47,38 +46,38 @@ __device__ __forceinline__ bool scale_in_fast_range(float s) {
     return s >= 0x1p-60f && s <= 0x1p60f;
 }
 
-// max(m, |a|, |b|) in one instruction.  Written in assembly: the inputs come out of integer-typed conversions and
-// the compiler turns fabs() of such a value into a separate v_and instead of a source modifier.  NaNs are dropped
-// (callers track them apart).
-__device__ __forceinline__ float max3_abs(float m, float a, float b) {
+// max(m, |a|, |b|) in one instruction, a NaN beating every number.  Written in assembly: the inputs come out of
+// integer-typed conversions and the compiler turns fabs() of such a value into a separate v_and instead of a source modifier.
+__device__ __forceinline__ float maximum3_abs(float m, float a, float b) {
     float r;
-    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
+    asm("v_maximum3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
     return r;
 }
 
-// 1 / sqrt(sumsq / H + eps).  The mean as an exact IEEE quotient: a multiplication when H is a power of two (exact, and
-// rounded like the quotient when the result is subnormal), elsewhere by multiply and two fused multiply-adds (exact on the
-// guarded range, see div_by_rcp); then the short square root and reciprocal.  Every wave of a row walks this dependent chain
-// before it can go on.
-__device__ __forceinline__ float row_rstd(float sumsq, float hidden_f, float rcp_hidden, int hidden_pow2, float eps) {
-    float mean;
-    if (hidden_pow2) mean = sumsq * rcp_hidden;
-    else if (__builtin_expect(__builtin_amdgcn_ballot_w64(!in_mid_range(sumsq)) == 0, 1)) mean = div_by_rcp_finite(sumsq, hidden_f, rcp_hidden);
-    else mean = sumsq / hidden_f;
-    return rsqrt_two_roundings(mean + eps);
+// 1 / sqrt(sumsq / H + eps).  The mean as an exact IEEE quotient by multiply and two fused multiply-adds (exact on the guarded
+// range, see div_by_rcp), then the short square root and reciprocal.  Every wave of a row walks this dependent chain before it
+// can go on: one test behind it, and what any of the three is not made for takes the general operations.  A sum in the middle
+// of the exponent range leaves the mean in [2^-91, 2^60) and, with an eps in [0, 2^60], the other two in theirs; sum_range is
+// 0 for any other eps, so that no sum passes.
+constexpr uint32_t kSumsFrom = 0x21800000u, kSumRange = 0x3c000000u;  // [2^-60, 2^60), see in_mid_range
+__device__ __forceinline__ float row_rstd(float sumsq, float hidden_f, float rcp_hidden, float eps, uint32_t sum_range) {
+    const float root = sqrt_rn_mid_range(div_by_rcp_finite(sumsq, hidden_f, rcp_hidden) + eps);
+    const bool usual = __builtin_bit_cast(uint32_t, sumsq) - kSumsFrom < sum_range && !mantissa_all_ones(root);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!usual) == 0, 1)) return rcp_rn_mid_range(root);
+    return 1.0f / sqrtf(sumsq / hidden_f + eps);
 }
 
-// scale = amax / fp8_max, 1 for an all-zero row.  `ranged` is the scale for scale_in_fast_range to look at: 0 instead where
-// quotients by it have to be clamped (rcp_fp8_max: see reciprocal_of_max).  Set in the branch of unusual maxima, so that
-// the common one is spared the test.
-__device__ __forceinline__ float dynamic_scale(float amax, float fp8_max, float rcp_fp8_max, float *ranged) {
-    float scale;
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(in_mid_range(amax) && rcp_fp8_max > 0.f)) == 0, 1)) {
-        scale = *ranged = div_by_rcp_finite(amax, fp8_max, rcp_fp8_max);
-    } else {
-        scale = amax == 0.f ? 1.f : amax / fp8_max;
-        *ranged = rcp_fp8_max < 0.f ? 0.f : scale;
+// scale = amax / fp8_max, 1 for an all-zero row; *fast: quotients by it take the short form.  rcp_fp8_max: see
+// reciprocal_of_max.  One test decides for the common maxima, whose scales are then in the fast range and never have a
+// significand of ones.
+__device__ __forceinline__ float dynamic_scale(float amax, float fp8_max, float rcp_fp8_max, bool *fast) {
+    const bool usual = __builtin_bit_cast(uint32_t, amax) - 0x26800000u < 0x37000000u && rcp_fp8_max > 0.f;  // amax in [2^-50, 2^60)
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!usual) == 0, 1)) {
+        *fast = true;
+        return div_by_rcp_finite(amax, fp8_max, rcp_fp8_max);
     }
+    const float scale = amax == 0.f ? 1.f : amax / fp8_max;
+    *fast = __builtin_amdgcn_ballot_w64(!(scale_in_fast_range(scale) && !mantissa_all_ones(scale) && rcp_fp8_max >= 0.f)) == 0;
     return scale;
 }
 
@@ -91,9 +90,9 @@ __device__ __forceinline__ float dynamic_scale(float amax, float fp8_max, float 
 //   third:  norm_out
 struct RowArgs {
     float *scale_io;
-    float hidden_f, rcp_hidden;
-    int hidden_pow2;
-    float eps, fp8_max, rcp_fp8_max;
+    float hidden_f, rcp_hidden, eps;
+    uint32_t sum_range;  // see row_rstd
+    float fp8_max, rcp_fp8_max;
 };
 static_assert(sizeof(u32x8) + sizeof(u32x4) + sizeof(u32x2) + sizeof(RowArgs) <= 112, "see launch_kernel");
 
@@ -150,7 +149,6 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
     Global<char> *norm_out = global_ptr<char>(third[0], third[1]);
     float *scale_io = rest.scale_io;
     const float hidden_f = rest.hidden_f, rcp_hidden = rest.rcp_hidden, eps = rest.eps, fp8_max = rest.fp8_max, rcp_fp8_max = rest.rcp_fp8_max;
-    const int hidden_pow2 = rest.hidden_pow2;
     const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
     using P = Pack16<T>;
     __shared__ float s_sum[kReduceSlots];
@@ -200,7 +198,9 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
     // The arguments beyond the preloaded ones are fetched here, behind the row's loads and while those are in flight:
     // left to itself the compiler fetches them where they are first used, after the first barrier, and every wave of
     // the row then waits there for the scalar cache (0.1-0.15 us of a decode-sized call).
-    asm volatile("" ::"s"(hidden_f), "s"(rcp_hidden), "s"(hidden_pow2), "s"(eps), "s"(fp8_max), "s"(rcp_fp8_max));
+    asm volatile("" ::"s"(hidden_f), "s"(rcp_hidden), "s"(eps), "s"(rest.sum_range));
+    if constexpr (QUANT != GPUK_QUANT_NONE) asm volatile("" ::"s"(fp8_max));
+    if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) asm volatile("" ::"s"(rcp_fp8_max), "s"(scale_io));
     // ... and so is the static scale, which the kernel only reads (asked for here, needed in phase 3: fetched where it
     // is first used it put a round trip through the scalar cache between the last two phases)
     float static_scale = 0.f;
@@ -231,15 +231,44 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
 #pragma unroll
             for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(xv[i][j]));
     }
-    float sumsq[1] = {ss0 + ss1};
     if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) asm volatile("" ::"s"(static_scale));  // (it has arrived by now)
     GPUK_STAMP(3);  // residual stored, the lane's squares summed
-    block_allreduce<SumOp, 1>(sumsq, s_sum, num_waves);
+    // kUnpacked: the row and the weights are unpacked behind the wave's own part of the reduction, while it has the others to wait
+    // for, and not in phase 2, where all waves of the row (two on most SIMDs of the only compute unit that a decode row has) issue
+    // at once: one row of 16384 elements 4.11 / 4.02 us, 32 of 4096 2.89 / 2.85.  Without codes, whose only chain behind the
+    // reduction is a store, it costs as much as it gains (256 rows of 4096 3.10 / 3.16), and four chunks per lane have no registers
+    // for it.
+    constexpr bool kUnpacked = !is_half<T> && NCHUNK <= 2 && QUANT != GPUK_QUANT_NONE;
+    float res[kUnpacked ? NCHUNK : 1][8], weight[kUnpacked ? NCHUNK : 1][8];
+    SplitReciprocal rcp{};  // of the scale; `fast`: quotients take the short form
+    bool fast = false;
+    const float sumsq = block_allreduce<SumOp>(ss0 + ss1, s_sum, num_waves, [&] {
+        if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) {
+            fast = __builtin_amdgcn_ballot_w64(!(scale_in_fast_range(static_scale) && !mantissa_all_ones(static_scale))) == 0;
+            rcp = split_reciprocal(static_scale);
+            asm volatile("" : "+v"(rcp.hi), "+v"(rcp.lo));
+        }
+        if constexpr (kUnpacked) {
+#pragma unroll
+            for (int i = 0; i < NCHUNK; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    res[i][2 * j] = P::lo(xv[i][j]), res[i][2 * j + 1] = P::hi(xv[i][j]);
+                    weight[i][2 * j] = P::lo(gv[i][j]), weight[i][2 * j + 1] = P::hi(gv[i][j]);
+                    asm volatile("" : "+v"(res[i][2 * j]), "+v"(res[i][2 * j + 1]), "+v"(weight[i][2 * j]), "+v"(weight[i][2 * j + 1]));
+                }
+        }
+    });
+    // element e of the normed chunk i, rT(gamma * rT(res * rstd)), ahead of the last rounding
+    const auto unrounded = [&](int i, int e, float rstd) {
+        if constexpr (kUnpacked) return weight[i][e] * P::round(res[i][e] * rstd);
+        else return 0.f;
+    };
     __builtin_amdgcn_s_setprio(0);
     GPUK_STAMP(4);  // sum of squares of the row known to every wave
 
     // ---- phase 2: n2 = rT(gamma * rT(res * rstd)); row amax for the dynamic scale.
-    const float rstd = row_rstd(sumsq[0], hidden_f, rcp_hidden, hidden_pow2, eps);
+    const float rstd = row_rstd(sumsq, hidden_f, rcp_hidden, eps, rest.sum_range);
     GPUK_STAMP(5);  // rstd
     if constexpr (QUANT == GPUK_QUANT_NONE) {
         auto *out = (Global<u32x4> *)norm_out + row_base;
@@ -271,7 +300,7 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
         return;
     } else {
         // the normed row stays in fp32 registers, every value already rounded to the 16-bit type.
-        // v_max3_f32 drops NaNs where the reference's amax propagates them: they are tracked apart
+        // (v_maximum3_f32 keeps a NaN, as the reference's amax does; tracked apart from v_max3_f32 it took a comparison per pair)
         // (kPacked, the gated four-chunk form: as 16-bit pairs instead, half the registers, so that eight waves fit a
         // SIMD with the residual kept for the gate as well; unpacked again in phase 3.  Half precision: always, its
         // arithmetic is packed and reads either half of a dword where bfloat16 needs an instruction to unpack it;
@@ -283,7 +312,6 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
         uint32_t nw[kPacked ? NCHUNK : 1][4];
         float m0 = 0.f, m1 = 0.f;
         uint32_t half_max = 0;  // (half precision: both halves' largest magnitude, a NaN beating every number)
-        bool any_nan = false;
 #pragma unroll
         for (int i = 0; i < NCHUNK; ++i) {
 #pragma unroll
@@ -298,36 +326,41 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
                     lo = P::lo(nw[i][j]);
                     hi = P::hi(nw[i][j]);
                 } else {
-                    lo = P::round(P::lo(gv[i][j]) * P::round(P::lo(xv[i][j]) * rstd));
-                    hi = P::round(P::hi(gv[i][j]) * P::round(P::hi(xv[i][j]) * rstd));
+                    if constexpr (kUnpacked) {
+                        lo = P::round(unrounded(i, 2 * j, rstd));
+                        hi = P::round(unrounded(i, 2 * j + 1, rstd));
+                    } else {
+                        lo = P::round(P::lo(gv[i][j]) * P::round(P::lo(xv[i][j]) * rstd));
+                        hi = P::round(P::hi(gv[i][j]) * P::round(P::hi(xv[i][j]) * rstd));
+                    }
                     nv[i][2 * j] = lo;
                     nv[i][2 * j + 1] = hi;
                 }
                 if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
-                    if (j & 1) m1 = max3_abs(m1, lo, hi);
-                    else m0 = max3_abs(m0, lo, hi);
-                    any_nan |= __builtin_isunordered(lo, hi);
+                    if (j & 1) m1 = maximum3_abs(m1, lo, hi);
+                    else m0 = maximum3_abs(m0, lo, hi);
                 }
             }
         }
-        float scale, ranged;
+        float scale = static_scale;
         GPUK_STAMP(6);  // row normed, the lane's maximum known
         if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
-            float amax[1] = {any_nan ? __builtin_nanf("") : __builtin_fmaxf(m0, m1)};
-            if constexpr (is_half<T>) amax[0] = MaxOp::apply(P::lo(half_max), P::hi(half_max));
-            block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
+            float amax = MaxOp::apply(m0, m1);
+            if constexpr (is_half<T>) amax = MaxOp::apply(P::lo(half_max), P::hi(half_max));
+            amax = block_allreduce<MaxOp>(amax, s_max, num_waves);
             GPUK_STAMP(7);  // row maximum known to every wave
-            scale = dynamic_scale(amax[0], fp8_max, rcp_fp8_max, &ranged);
+            scale = dynamic_scale(amax, fp8_max, rcp_fp8_max, &fast);
             if (tid == 0) scale_io[row] = scale;
-        } else {
-            scale = ranged = static_scale;
+            rcp = split_reciprocal(scale);
         }
 
-        // ---- phase 3: code = e4m3fn(clamp(n2 / scale)), 8 codes per chunk.  With the dynamic scale every value is
-        // finite, hence the short form of the quotient, and |n2 / scale| exceeds fp8_max by at most one ULP, which the
-        // converter rounds to the same code: no clamp.  (Maxima where it does not, see reciprocal_of_max, take the other
-        // path, which clamps.)  The static scale may meet anything: clamp, and the form that restores what a division
-        // gives for infinite and NaN numerators.
+        // ---- phase 3: code = e4m3fn(clamp(n2 / scale)), 8 codes per chunk.  The quotient is the short one with the same
+        // code (see SplitReciprocal; one row of 7168 elements, dynamic, 2.95 / 2.85 us with the correctly rounded quotient / this
+        // one, 512 rows 5.85 / 5.74; with a static scale, whose reciprocal is taken while the wave waits at the first barrier,
+        // 128 rows of 4096 3.24 / 3.13).  With the dynamic scale every value is finite and |n2 / scale| exceeds fp8_max by at
+        // most one ULP, which the converter rounds to the same code: no clamp.  (Maxima where it does not, see
+        // reciprocal_of_max, take the other path, which clamps.)  The static scale may meet anything: clamp; infinite and NaN
+        // numerators come through the short quotient as through a division.
         constexpr bool kDynamic = QUANT == GPUK_QUANT_FP8_DYNAMIC;
         auto *out = (Global<u32x2> *)norm_out + row_base;
         if constexpr (kPacked && !is_half<T>) {  // (or the compiler keeps phase 2's unpacked copies alive instead)
@@ -338,10 +371,7 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
         }
         // (the scale is the same in every lane; deciding by ballot tells the compiler so, and the common path is
         // laid out as straight-line code with the other one out of the way)
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!scale_in_fast_range(ranged)) == 0, 1)) {
-            float rcp;
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(mantissa_all_ones(scale)) == 0, 1)) rcp = rcp_rn_mid_range(scale);
-            else rcp = 1.0f / scale;
+        if (__builtin_expect(fast, 1)) {
             GPUK_STAMP(8);  // scale and its reciprocal
             u32x2 codes[NCHUNK];
 #pragma unroll
@@ -349,17 +379,15 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
                 float q[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    if constexpr (is_half<T> && kDynamic) {  // div_by_rcp_finite, its numerator read in place
+                    if constexpr (is_half<T>) {  // (the numerator read in place)
                         const uint32_t w = nw[i][j >> 1];
-                        const float p = (j & 1) ? P::mul_hi(w, rcp) : P::mul_lo(w, rcp);
-                        const float e = (j & 1) ? P::fma_minus_hi(p, scale, w) : P::fma_minus_lo(p, scale, w);
-                        q[j] = __builtin_fmaf(-e, rcp, p);
+                        q[j] = (j & 1) ? P::fma_hi(w, rcp.hi, P::mul_hi(w, rcp.lo)) : P::fma_lo(w, rcp.hi, P::mul_lo(w, rcp.lo));
                         continue;
                     }
                     float n;
                     if constexpr (kPacked) n = (j & 1) ? P::hi(nw[i][j >> 1]) : P::lo(nw[i][j >> 1]);
                     else n = nv[i][j];
-                    q[j] = kDynamic ? div_by_rcp_finite(n, scale, rcp) : div_by_rcp(n, scale, rcp);
+                    q[j] = __builtin_fmaf(n, rcp.hi, n * rcp.lo);
                 }
                 if constexpr (!kDynamic) clamp8_sym(q, fp8_max);
                 codes[i] = u32x2{cvt4_e4m3fn(q[0], q[1], q[2], q[3]), cvt4_e4m3fn(q[4], q[5], q[6], q[7])};
@@ -477,9 +505,8 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
         }
         residual_out[row_base + c] = xv;
     }
-    float sumsq[1] = {ss};
-    block_allreduce<SumOp, 1>(sumsq, s_sum, num_waves);
-    const float rstd = 1.0f / sqrtf(sumsq[0] / hidden_f + eps);
+    const float sumsq = block_allreduce<SumOp>(ss, s_sum, num_waves);
+    const float rstd = 1.0f / sqrtf(sumsq / hidden_f + eps);
 
     auto normed = [&](int c) {
         u32x4 v = residual_out[row_base + c];  // written by this lane above
@@ -507,9 +534,8 @@ add_rmsnorm_quant_long_rows(const u32x4 *x, const u32x4 *residual_in,  // either
                     amax = MaxOp::apply(amax, __builtin_fabsf(P::hi(v[j])));
                 }
             }
-            float am[1] = {amax};
-            block_allreduce<MaxOp, 1>(am, s_max, num_waves);
-            scale = am[0] == 0.f ? 1.f : am[0] / fp8_max;
+            amax = block_allreduce<MaxOp>(amax, s_max, num_waves);
+            scale = amax == 0.f ? 1.f : amax / fp8_max;
             if (tid == 0) scale_io[blockIdx.x] = scale;
         } else {
             scale = scale_io[0];
@@ -566,7 +592,6 @@ add_rmsnorm_quant_f32_rows(const u32x8 first, const u32x4 second, const u32x2 th
     Global<char> *norm_out = global_ptr<char>(third[0], third[1]);
     float *scale_io = rest.scale_io;
     const float hidden_f = rest.hidden_f, rcp_hidden = rest.rcp_hidden, eps = rest.eps, fp8_max = rest.fp8_max, rcp_fp8_max = rest.rcp_fp8_max;
-    const int hidden_pow2 = rest.hidden_pow2;
     constexpr bool GATED = FORM == F32Form::GATED || FORM == F32Form::GATED_LANDED;
     constexpr bool LANDED = FORM == F32Form::LANDED || FORM == F32Form::GATED_LANDED;
     const int nthreads = lanes_of(lanes_and_shift), group_shift = shift_of(lanes_and_shift);
@@ -600,7 +625,9 @@ add_rmsnorm_quant_f32_rows(const u32x8 first, const u32x4 second, const u32x2 th
         for (int i = 0; i < NCHUNK; ++i) gv[i] = live[i] ? (gamma - pad)[i * nthreads + tid] : zero;
     };
     if constexpr (FORM != F32Form::LAST && !LANDED) load_weights();
-    asm volatile("" ::"s"(hidden_f), "s"(rcp_hidden), "s"(hidden_pow2), "s"(eps), "s"(fp8_max), "s"(rcp_fp8_max));
+    asm volatile("" ::"s"(hidden_f), "s"(rcp_hidden), "s"(eps), "s"(rest.sum_range));
+    if constexpr (QUANT != GPUK_QUANT_NONE) asm volatile("" ::"s"(fp8_max));
+    if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) asm volatile("" ::"s"(rcp_fp8_max), "s"(scale_io));
     float static_scale = 0.f;
     if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) static_scale = *(const __attribute__((address_space(4))) float *)scale_io;
 
@@ -623,44 +650,39 @@ add_rmsnorm_quant_f32_rows(const u32x8 first, const u32x4 second, const u32x2 th
         }
         if (!GATED && live[i]) store_stream(residual_out + row_base + i * nthreads + tid, xv[i]);
     }
-    float sumsq[1] = {ss0 + ss1};
     if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) asm volatile("" ::"s"(static_scale));
-    block_allreduce<SumOp, 1>(sumsq, s_sum, num_waves);
+    const float sumsq = block_allreduce<SumOp>(ss0 + ss1, s_sum, num_waves);
     __builtin_amdgcn_s_setprio(0);
-    const float rstd = row_rstd(sumsq[0], hidden_f, rcp_hidden, hidden_pow2, eps);
+    const float rstd = row_rstd(sumsq, hidden_f, rcp_hidden, eps, rest.sum_range);
     if constexpr (FORM == F32Form::LAST) load_weights();
 
     f32x4 nv[NCHUNK];
     float m0 = 0.f, m1 = 0.f;
-    bool any_nan = false;
 #pragma unroll
     for (int i = 0; i < NCHUNK; ++i) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) nv[i][j] = gv[i][j] * (xv[i][j] * rstd);
-        if constexpr (QUANT != GPUK_QUANT_NONE) {  // (max3_abs drops NaNs, the reference's amax keeps them: tracked apart)
-            m0 = max3_abs(m0, nv[i][0], nv[i][1]);
-            m1 = max3_abs(m1, nv[i][2], nv[i][3]);
-            if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC)
-                any_nan |= __builtin_isunordered(nv[i][0], nv[i][1]) || __builtin_isunordered(nv[i][2], nv[i][3]);
+        if constexpr (QUANT != GPUK_QUANT_NONE) {
+            m0 = maximum3_abs(m0, nv[i][0], nv[i][1]);
+            m1 = maximum3_abs(m1, nv[i][2], nv[i][3]);
         }
     }
-    const float lane_max = __builtin_fmaxf(m0, m1);
+    const float lane_max = MaxOp::apply(m0, m1);
     uint32_t codes[NCHUNK];
     if constexpr (QUANT != GPUK_QUANT_NONE) {
         float scale = static_scale;
-        bool fast = scale_in_fast_range(scale) && lane_max <= 0x1p60f;  // (a static scale may meet quotients that overflow)
+        bool fast;
         if constexpr (QUANT == GPUK_QUANT_FP8_DYNAMIC) {
-            float amax[1] = {any_nan ? __builtin_nanf("") : lane_max};
-            block_allreduce<MaxOp, 1>(amax, s_max, num_waves);
-            float ranged;
-            scale = dynamic_scale(amax[0], fp8_max, rcp_fp8_max, &ranged);
+            const float amax = block_allreduce<MaxOp>(lane_max, s_max, num_waves);
+            scale = dynamic_scale(amax, fp8_max, rcp_fp8_max, &fast);
             if (tid == 0) scale_io[row] = scale;
-            fast = scale_in_fast_range(ranged);
+        } else {  // (a static scale may meet quotients that overflow)
+            fast = __builtin_amdgcn_ballot_w64(!(scale_in_fast_range(scale) && lane_max <= 0x1p60f)) == 0;
         }
         // Quotients below the smallest code's half come out 0 with their sign whatever the correction step loses to
         // underflow; the others are the correctly rounded ones.  With the dynamic scale no clamp, as in
         // add_rmsnorm_quant_rows.
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!fast) == 0, 1)) {
+        if (__builtin_expect(fast, 1)) {
             float rcp;
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(mantissa_all_ones(scale)) == 0, 1)) rcp = rcp_rn_mid_range(scale);
             else rcp = 1.0f / scale;
@@ -766,9 +788,8 @@ add_rmsnorm_quant_wide_rows(const wide4<F> *x, const wide4<F> *residual_in,  // 
             ss = __builtin_fmaf(r, r, ss);
         }
     });
-    float sumsq[1] = {ss};
-    block_allreduce<SumOp, 1>(sumsq, s_sum, num_waves);
-    const F rstd = (F)(1.0f / sqrtf(sumsq[0] / hidden_f + eps));
+    const float sumsq = block_allreduce<SumOp>(ss, s_sum, num_waves);
+    const F rstd = (F)(1.0f / sqrtf(sumsq / hidden_f + eps));
 
     // the normed chunk; with CPL = 0 the summed chunk is read back (this lane wrote it above)
     auto normed = [&](int i, int c) {
@@ -789,9 +810,8 @@ add_rmsnorm_quant_wide_rows(const wide4<F> *x, const wide4<F> *residual_in,  // 
 #pragma unroll
                 for (int j = 0; j < 4; ++j) amax = MaxOp::apply(amax, __builtin_fabsf((float)v[j]));
             });
-            float am[1] = {amax};
-            block_allreduce<MaxOp, 1>(am, s_max, num_waves);
-            scale = am[0] == 0.f ? 1.f : am[0] / fp8_max;
+            amax = block_allreduce<MaxOp>(amax, s_max, num_waves);
+            scale = amax == 0.f ? 1.f : amax / fp8_max;
             if (tid == 0) scale_io[blockIdx.x] = scale;
         } else {
             scale = scale_io[0];
@@ -1033,7 +1053,7 @@ RowParameters row_parameters(const void *x, const void *residual_in, const void 
     return {u32x8{low_half(x), high_half(x), low_half(residual_in), high_half(residual_in), (uint32_t)chunks, remap_end, shape, gate},
             u32x4{low_half(gamma), high_half(gamma), low_half(residual_out), high_half(residual_out)},
             u32x2{low_half(norm_out), high_half(norm_out)},
-            RowArgs{scale, hf, 1.0f / hf, (hidden & (hidden - 1)) == 0, eps, fp8_max, reciprocal_of_max(fp8_max)}};
+            RowArgs{scale, hf, 1.0f / hf, eps, eps >= 0.f && eps <= 0x1p60f ? kSumRange : 0u, fp8_max, reciprocal_of_max(fp8_max)}};
 }
 
 template <typename T, int QUANT>

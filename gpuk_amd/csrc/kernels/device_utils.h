@@ -95,15 +95,15 @@ template <> struct Pack16<FP16> {
         asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(b));
         return r;
     }
-    // a * b - lo(w) and a * b - hi(w) in fp32
-    static __device__ __forceinline__ float fma_minus_lo(float a, float b, uint32_t w) {
+    // lo(w) * b + c and hi(w) * b + c in fp32
+    static __device__ __forceinline__ float fma_lo(uint32_t w, float b, float c) {
         float r;
-        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(a), "v"(b), "v"(w));
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(b), "v"(c));
         return r;
     }
-    static __device__ __forceinline__ float fma_minus_hi(float a, float b, uint32_t w) {
+    static __device__ __forceinline__ float fma_hi(uint32_t w, float b, float c) {
         float r;
-        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(a), "v"(b), "v"(w));
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(b), "v"(c));
         return r;
     }
     static __device__ __forceinline__ float add_squares(uint32_t w, float acc) {  // lo(w)^2 first, then hi(w)^2
@@ -191,28 +191,29 @@ __device__ __forceinline__ float wave_allreduce(float v) {
     return Op::apply(Op::apply(r0, r1), Op::apply(r2, r3));
 }
 
-// Workgroup all-reduce of N independent values: wave results meet in LDS (N x 16 floats, at most 16 waves), one
-// barrier, then every wave reads the per-wave results into its lanes (lane l takes wave l mod 16) and folds them with
-// four DPP steps, so the result is the same in every lane of the workgroup.  `slots` must be private to this call
-// site so that two consecutive reductions need only one barrier each.
+// Workgroup all-reduce: wave results meet in LDS (16 floats, at most 16 waves), one barrier, then every wave reads the per-wave
+// results into its lanes (lane l takes wave l mod 16) and folds them with four DPP steps, so the result is the same in every
+// lane of the workgroup.  `slots` must be private to this call site so that two consecutive reductions need only one barrier
+// each.  `meanwhile` is done behind a wave's own part, while it has the others to wait for.
+// (Level or slower: rows combined by two more DPP steps instead of four readlanes, one row of 7168 elements without codes 2.37 /
+// 2.43 us; the slots read by every lane instead of by those with a wave, with codes 2.95 / 2.99; the rows' results through LDS
+// and combined behind the barrier, 216 calls of up to 512 rows 0.975 / 0.978 of the time before the changes of the row kernels.)
 constexpr int kReduceSlots = 16;
-template <typename Op, int N>
-__device__ __forceinline__ void block_allreduce(float (&v)[N], float *slots, int num_waves) {
-#pragma unroll
-    for (int n = 0; n < N; ++n) v[n] = wave_allreduce<Op>(v[n]);
-    if (num_waves == 1) return;
+template <typename Op, typename F>
+__device__ __forceinline__ float block_allreduce(float v, float *slots, int num_waves, F meanwhile) {
+    v = wave_allreduce<Op>(v);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) {
-#pragma unroll
-        for (int n = 0; n < N; ++n) slots[n * kReduceSlots + wave] = v[n];
-    }
+    if (lane == 0) slots[wave] = v;
+    meanwhile();
+    if (__builtin_expect(num_waves == 1, 0)) return v;
     __syncthreads();
     const int src = lane & (kReduceSlots - 1);
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-        const float s = slots[n * kReduceSlots + src];
-        v[n] = group_allreduce<Op, 16>(src < num_waves ? s : Op::identity());
-    }
+    const float s = slots[src];
+    return group_allreduce<Op, 16>(src < num_waves ? s : Op::identity());
+}
+template <typename Op>
+__device__ __forceinline__ float block_allreduce(float v, float *slots, int num_waves) {
+    return block_allreduce<Op>(v, slots, num_waves, [] {});
 }
 
 // Four fp32 -> four OCP e4m3fn codes in one dword (two v_cvt_pk_fp8_f32).  Inputs must already be
@@ -262,6 +263,21 @@ __device__ __forceinline__ float div_by_rcp_finite(float a, float b, float rcp) 
     const float q = a * rcp;
     const float e = __builtin_fmaf(q, b, -a);
     return __builtin_fmaf(-e, rcp, q);
+}
+
+// 1 / s in two parts, hi + lo: lo >= 0, the sum within 2^-40 of it (v_rcp_f32 is within one ULP; three below it, the
+// remainder of the second line is positive and exact to 2^-44).  s in [2^-60, 2^60].
+// a * hi + a * lo in one multiply and one fused multiply-add rounds to the same e4m3fn code as the quotient RN(a / s) for every a of
+// up to 11 significant bits, unless the significand of s is all ones, and keeps the sign of a zero: it differs from the quotient
+// only where that lies within 2^-40 of the middle of two floats, and next to a tie between two codes (five significant bits)
+// no such a exists (tests/test_oracle_norm_quant.py: all significands of s).  One instruction less per element than
+// div_by_rcp_finite, and four and a branch less than the correctly rounded reciprocal that needs.
+struct SplitReciprocal {
+    float hi, lo;
+};
+__device__ __forceinline__ SplitReciprocal split_reciprocal(float s) {
+    const float hi = __builtin_bit_cast(float, __builtin_bit_cast(int32_t, __builtin_amdgcn_rcpf(s)) - 3);
+    return {hi, __builtin_fmaf(-s, hi, 1.0f) * hi};
 }
 
 // ---- Correctly rounded square root and reciprocal by short sequences.  The compiler's expansions of sqrtf() and of

@@ -61,6 +61,8 @@ def lib():
         for name in ("gpuk_oracle_count_short_sqrt_mismatch", "gpuk_oracle_count_short_rcp_mismatch"):
             getattr(L, name).restype = C.c_int64
             getattr(L, name).argtypes = [C.c_uint32, C.c_int64, C.c_int]
+        L.gpuk_oracle_count_split_reciprocal_mismatch.restype = C.c_int64
+        L.gpuk_oracle_count_split_reciprocal_mismatch.argtypes = [C.c_uint32, C.c_uint32, C.c_int, C.c_int]
         _lib = L
     return _lib
 
@@ -139,3 +141,8 @@ def count_short_sqrt_mismatch(first_bits: int, n: int, first_guess_ulp: int) -> 
 def count_short_rcp_mismatch(first_bits: int, n: int, first_guess_ulp: int) -> int:
     """See gpuk_oracle_count_short_rcp_mismatch."""
     return lib().gpuk_oracle_count_short_rcp_mismatch(first_bits, n, first_guess_ulp)
+
+
+def count_split_reciprocal_mismatch(first: int, last: int, below: int, bits: int) -> int:
+    """See gpuk_oracle_count_split_reciprocal_mismatch."""
+    return lib().gpuk_oracle_count_split_reciprocal_mismatch(first, last, below, bits)

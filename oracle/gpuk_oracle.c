@@ -389,3 +389,38 @@ int64_t gpuk_oracle_count_short_rcp_mismatch(uint32_t first_bits, int64_t n, int
     }
     return bad;
 }
+
+/* e4m3fn code of a positive finite value as a number that orders like the codes (unclamped: values beyond the format go on). */
+static int e4m3fn_place(float q) {
+    const uint32_t u = f32_bits(q);
+    if (q < 0x1p-6f) return (int)nearbyintf(q * 512.0f);   /* subnormal codes: multiples of 2^-9, ties to even */
+    return (int)((u + 0x7ffffu + ((u >> 20) & 1u)) >> 20) - ((121 << 3) - 8);
+}
+
+/* Model of the device's quotient by a reciprocal in two parts (hi: `below` ULPs under RN(1/s); lo = RN(RN(1 - s*hi) * hi);
+ * RN(n*hi + RN(n*lo))) against the IEEE quotient, by the e4m3fn code both round to, for the scales with significands
+ * [first, last) and every numerator of `bits` significant bits next to a tie between two codes: elsewhere the two agree
+ * because they differ by less than the distance to the tie.  Also counted: a lo that is negative (zeros would lose their sign). */
+int64_t gpuk_oracle_count_split_reciprocal_mismatch(uint32_t first, uint32_t last, int below, int bits) {
+    float ties[16];
+    int64_t bad = 0;
+    for (int i = 0; i < 8; ++i) {
+        ties[i] = (17 + 2 * i) / 16.0f;           /* normal codes: odd five-bit significands */
+        ties[8 + i] = (i + 0.5f) * 0x1p-9f;       /* subnormal codes */
+    }
+#pragma omp parallel for reduction(+ : bad)
+    for (int64_t m = first; m < (int64_t)last; ++m) {
+        const float s = bits_f32(0x3f800000u | (uint32_t)m), hi = bits_f32(f32_bits(1.0f / s) - (uint32_t)below);
+        const float rest = fmaf(-s, hi, 1.0f), lo = rest * hi;
+        bad += rest < 0.0f;
+        for (int i = 0; i < 16; ++i) {
+            int e;
+            const double near = nearbyint(ldexp(frexp((double)s * ties[i], &e), bits));
+            for (int d = -1; d <= 1; ++d) {
+                const float n = (float)ldexp(near + d, e - bits);
+                bad += e4m3fn_place(n / s) != e4m3fn_place(fmaf(n, hi, n * lo));
+            }
+        }
+    }
+    return bad;
+}

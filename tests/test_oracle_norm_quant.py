@@ -221,3 +221,21 @@ def test_quotients_by_row_length_and_by_fp8_max_are_exact():
     for fp8_max in (448.0, 240.0):
         bad += c_oracle.count_div_rcp_mismatch(amax.contiguous(), torch.full_like(amax, fp8_max))
     assert bad == 0
+
+
+@pytest.mark.parametrize("bits", [8, 11])   # bfloat16 and half precision numerators
+def test_quotients_by_a_split_reciprocal_give_the_same_codes(bits):
+    """The codes of the dynamic scale come from n * hi + n * lo, hi three ULPs below v_rcp_f32 (one ULP): for every
+    significand of the scale but the all-ones one, the same code as the IEEE quotient for every numerator next to a tie
+    between two codes; farther away the two, which differ by 2^-24 of themselves at most, round alike."""
+    for below in (2, 3, 4):
+        assert c_oracle.count_split_reciprocal_mismatch(0, (1 << 23) - 1, below, bits) == 0, below
+    assert c_oracle.count_split_reciprocal_mismatch((1 << 23) - 1, 1 << 23, 3, bits) > 0   # the excluded significand does fail
+
+
+def test_no_scale_of_the_checked_maxima_has_a_significand_of_ones():
+    for fp8_max in (448.0, 240.0):
+        for dtype in (torch.bfloat16, torch.float16):
+            amax = torch.arange(1, 0x7C00, dtype=torch.int32).to(torch.int16).view(dtype).float()
+            scale = amax[amax > 2.0 ** -100] / fp8_max
+            assert not (scale.view(torch.int32) & 0x7FFFFF == 0x7FFFFF).any()
