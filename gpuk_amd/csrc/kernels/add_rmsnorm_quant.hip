@@ -46,14 +46,6 @@ __device__ __forceinline__ bool scale_in_fast_range(float s) {
     return s >= 0x1p-60f && s <= 0x1p60f;
 }
 
-// max(m, |a|, |b|) in one instruction, a NaN beating every number.  Written in assembly: the inputs come out of
-// integer-typed conversions and the compiler turns fabs() of such a value into a separate v_and instead of a source modifier.
-__device__ __forceinline__ float maximum3_abs(float m, float a, float b) {
-    float r;
-    asm("v_maximum3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
-    return r;
-}
-
 // 1 / sqrt(sumsq / H + eps).  The mean as an exact IEEE quotient by multiply and two fused multiply-adds (exact on the guarded
 // range, see div_by_rcp), then the short square root and reciprocal.  Every wave of a row walks this dependent chain before it
 // can go on: one test behind it, and what any of the three is not made for takes the general operations.  A sum in the middle

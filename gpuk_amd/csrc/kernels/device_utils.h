@@ -216,6 +216,14 @@ __device__ __forceinline__ float block_allreduce(float v, float *slots, int num_
     return block_allreduce<Op>(v, slots, num_waves, [] {});
 }
 
+// max(m, |a|, |b|) in one instruction, a NaN beating every number.  Written in assembly: the inputs come out of
+// integer-typed conversions and the compiler turns fabs() of such a value into a separate v_and instead of a source modifier.
+__device__ __forceinline__ float maximum3_abs(float m, float a, float b) {
+    float r;
+    asm("v_maximum3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
+    return r;
+}
+
 // Four fp32 -> four OCP e4m3fn codes in one dword (two v_cvt_pk_fp8_f32).  Inputs must already be
 // clamped to the finite range; rounding is to nearest even.
 __device__ __forceinline__ uint32_t cvt4_e4m3fn(float a, float b, float c, float d) {

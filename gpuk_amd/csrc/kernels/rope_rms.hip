@@ -183,48 +183,49 @@ __device__ __forceinline__ void load_trig_merged(const uint16_t *table, int64_t 
     }
 }
 
-// 8 codes = e4m3fn(clamp(rT(v / scale))) for one chunk; `rcp` is RN(1/scale) and is used when FAST.
-// Then, with bf16 and where no value of the wave comes near what has to be clamped (nor is infinite or a NaN), the quotients
-// are the short ones for finite numerators and the rounded pairs are converted as they are: what the many fp8 rows of a call
-// without shared KV heads wait for.  In us without / with, bf16: 900 tokens of 64+64+64 heads of 128 elements 18.4 / 17.0, of
-// 64 elements (919 tokens) 11.4 / 10.7, 3000 of 32+32+32 27.1 / 24.8, 32 of 64+8+8 2.99 / 2.90, long calls with few KV heads
-// level; with a scale a thousand times too small, so that every wave clamps, 3000 tokens of 32+32+32 27.7 / 28.6.  Short
-// quotients for those too, the rounded pairs clamped as whole numbers, take 25.3 there, but the choice costs the calls that
-// clamp nothing more than it may: decode batches 0.5 to 4 % (8 tokens of 32+32+32 2.93 / 3.03, 64 of 64+8+8 2.75 / 2.81, with
-// the clamped form on a branch of its own 3.00 and 2.80): not done.  fp16 keeps the general form: its own short one was 3 %
-// faster at 2000 tokens of 32+32+32 heads (16.5 / 16.0) and 3 % slower at 4000 (27.95 / 28.7).
+// 8 codes = e4m3fn(clamp(rT(v / scale))) for one chunk.  FAST: scale in [2^-60, 2^60].
+// bf16, FAST: the quotients are the short ones by a reciprocal in two parts, which round to the same bfloat16 (SplitReciprocal;
+// infinities, NaNs and the signs of zeros come through them), and where nothing in the wave has to be clamped (nor is a NaN) the
+// rounded pairs are converted as they are.  These instructions are what the many fp8 rows of a call without shared KV heads
+// wait for.  In us with correctly rounded quotients (three instructions, a reciprocal by division, the largest magnitude taken of the
+// packed values) / so: 500 tokens of 64+64+64 heads of 128 elements 11.2 / 10.5, of 64 elements 7.0 / 6.6, 3000 of 32+32+32 25.7 /
+// 24.3, 6000 of 12+12+12 of 64 14.8 / 13.6, 32 of 64+8+8 2.65 / 2.63, long calls with few KV heads level; where every wave clamps
+// (a scale of 0.004) 3000 of 32+32+32 29.6 / 27.6, 8 tokens 3.49 / 3.27.  fp16, whose ties have a bit more than the short
+// quotient is proven for, keeps the general form.
 template <typename T, bool FAST>
-__device__ __forceinline__ u32x2 quantize_chunk(const u32x4 &v, float scale, float rcp) {
+__device__ __forceinline__ u32x2 quantize_chunk(const u32x4 &v, float scale) {
     using P = Pack16<T>;
+    float q[8];
     if constexpr (FAST && !is_half<T>) {
-        // The largest magnitude by whole-number maxima: those keep a NaN, which a float maximum may drop together with the infinity
-        // it met.  A NaN takes the general form.  (The half below the upper one only makes it larger, by less than a place of bf16.)
-        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-        typedef short i16x2 __attribute__((ext_vector_type(2)));
-        u16x2 most = __builtin_bit_cast(u16x2, v[0] & 0x7fff7fffu);
+        const SplitReciprocal rcp = split_reciprocal(scale);
+        float most = 0.f;
 #pragma unroll
-        for (int j = 1; j < 4; ++j) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, v[j] & 0x7fff7fffu));
-        const uint32_t both = __builtin_bit_cast(uint32_t, most);
-        const bool clamps = __builtin_elementwise_max(both << 16, both) > __builtin_bit_cast(uint32_t, 440.0f * scale);
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(clamps) == 0, 1)) {
+        for (int j = 0; j < 4; ++j) {
+            q[2 * j] = __builtin_fmaf(P::lo(v[j]), rcp.hi, P::lo(v[j]) * rcp.lo);
+            q[2 * j + 1] = __builtin_fmaf(P::hi(v[j]), rcp.hi, P::hi(v[j]) * rcp.lo);
+            most = maximum3_abs(most, q[2 * j], q[2 * j + 1]);
+        }
+        typedef short i16x2 __attribute__((ext_vector_type(2)));
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(most <= kE4M3Max)) == 0, 1)) {
             u32x2 codes;
 #pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-                const auto pair = [&](uint32_t w) {
-                    return __builtin_bit_cast(bf16x2_t, P::pack(div_by_rcp_finite(P::lo(w), scale, rcp), div_by_rcp_finite(P::hi(w), scale, rcp)));
-                };
-                const i16x2 low = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(i16x2{0, 0}, pair(v[j]), 1.0f, false);
-                codes[j / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(low, pair(v[j + 1]), 1.0f, true));
+            for (int j = 0; j < 2; ++j) {
+                const i16x2 low = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(i16x2{0, 0}, __builtin_bit_cast(bf16x2_t, P::pack(q[4 * j], q[4 * j + 1])), 1.0f, false);
+                codes[j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(low, __builtin_bit_cast(bf16x2_t, P::pack(q[4 * j + 2], q[4 * j + 3])), 1.0f, true));
             }
             return codes;
         }
+    } else {
+        const float rcp = 1.0f / scale;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            q[2 * j] = FAST ? div_by_rcp(P::lo(v[j]), scale, rcp) : P::lo(v[j]) / scale;
+            q[2 * j + 1] = FAST ? div_by_rcp(P::hi(v[j]), scale, rcp) : P::hi(v[j]) / scale;
+        }
     }
-    float q[8];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float a = FAST ? div_by_rcp(P::lo(v[j]), scale, rcp) : P::lo(v[j]) / scale;
-        const float b = FAST ? div_by_rcp(P::hi(v[j]), scale, rcp) : P::hi(v[j]) / scale;
-        const uint32_t w = P::pack(a, b);
+        const uint32_t w = P::pack(q[2 * j], q[2 * j + 1]);
         q[2 * j] = P::lo(w);
         q[2 * j + 1] = P::hi(w);
     }
@@ -494,13 +495,13 @@ struct RopeUnit {
                 store_pair<HALF * 2>(dst + c0(sub), oa, ob, a.stream_rows != 0);
             } else if (KVFP8 && !st.is_q) {
                 uint8_t *dst = static_cast<uint8_t *>(a.k_cache) + (st.slot * a.hk + (head - a.hq)) * D;
-                const float s = a.k_scale, rcp = 1.0f / s;
+                const float s = a.k_scale;
                 if (scale_is_fast(s)) {
-                    *reinterpret_cast<u32x2 *>(dst + c0(sub)) = quantize_chunk<T, true>(oa, s, rcp);
-                    *reinterpret_cast<u32x2 *>(dst + c1(sub)) = quantize_chunk<T, true>(ob, s, rcp);
+                    *reinterpret_cast<u32x2 *>(dst + c0(sub)) = quantize_chunk<T, true>(oa, s);
+                    *reinterpret_cast<u32x2 *>(dst + c1(sub)) = quantize_chunk<T, true>(ob, s);
                 } else {
-                    *reinterpret_cast<u32x2 *>(dst + c0(sub)) = quantize_chunk<T, false>(oa, s, rcp);
-                    *reinterpret_cast<u32x2 *>(dst + c1(sub)) = quantize_chunk<T, false>(ob, s, rcp);
+                    *reinterpret_cast<u32x2 *>(dst + c0(sub)) = quantize_chunk<T, false>(oa, s);
+                    *reinterpret_cast<u32x2 *>(dst + c1(sub)) = quantize_chunk<T, false>(ob, s);
                 }
             } else {
                 // q_out row or (16-bit) K cache row of the slot: one store sequence, destination chosen per lane
@@ -514,7 +515,7 @@ struct RopeUnit {
             // V: copied (16-bit cache) or quantised (fp8 cache), chunk by chunk
             const int v_chunks = a.hv * (D / 8), v_first = st.u * 64 + lane;
             const int stride = a.units_per_token * 64;
-            const float s = KVFP8 ? a.v_scale : 1.0f, rcp = 1.0f / s;
+            const float s = KVFP8 ? a.v_scale : 1.0f;
             const bool fast = scale_is_fast(s);
             u32x4 vchunk = st.vchunk;
             for (int c = v_first; slot_ok && c < v_chunks; c += stride) {
@@ -525,7 +526,7 @@ struct RopeUnit {
                     *reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(a.v_cache) + off) = vchunk;
                 } else {
                     *reinterpret_cast<u32x2 *>(static_cast<uint8_t *>(a.v_cache) + off) =
-                        fast ? quantize_chunk<T, true>(vchunk, s, rcp) : quantize_chunk<T, false>(vchunk, s, rcp);
+                        fast ? quantize_chunk<T, true>(vchunk, s) : quantize_chunk<T, false>(vchunk, s);
                 }
             }
         }
@@ -743,13 +744,13 @@ __device__ __forceinline__ void token_store(const RopeArgs &a, uint32_t t, int64
             const int64_t at = (slot * hk + (head - hq)) * D + 8 * sub;
             if constexpr (KVFP8) {
                 uint8_t *dst = static_cast<uint8_t *>(a.k_cache) + at;
-                const float s = a.k_scale, rcp = 1.0f / s;
+                const float s = a.k_scale;
                 if (scale_is_fast(s)) {
-                    *reinterpret_cast<u32x2 *>(dst) = quantize_chunk<T, true>(xa[u], s, rcp);
-                    *reinterpret_cast<u32x2 *>(dst + HALF) = quantize_chunk<T, true>(xb[u], s, rcp);
+                    *reinterpret_cast<u32x2 *>(dst) = quantize_chunk<T, true>(xa[u], s);
+                    *reinterpret_cast<u32x2 *>(dst + HALF) = quantize_chunk<T, true>(xb[u], s);
                 } else {
-                    *reinterpret_cast<u32x2 *>(dst) = quantize_chunk<T, false>(xa[u], s, rcp);
-                    *reinterpret_cast<u32x2 *>(dst + HALF) = quantize_chunk<T, false>(xb[u], s, rcp);
+                    *reinterpret_cast<u32x2 *>(dst) = quantize_chunk<T, false>(xa[u], s);
+                    *reinterpret_cast<u32x2 *>(dst + HALF) = quantize_chunk<T, false>(xb[u], s);
                 }
             } else {
                 store_pair<HALF * 2>(static_cast<uint16_t *>(a.k_cache) + at, xa[u], xb[u], true);
@@ -762,9 +763,9 @@ __device__ __forceinline__ void token_store(const RopeArgs &a, uint32_t t, int64
         if (slot_ok && c < v_chunks) {
             const int64_t off = slot * hv * D + 8 * (int64_t)c;
             if constexpr (KVFP8) {
-                const float s = a.v_scale, rcp = 1.0f / s;
+                const float s = a.v_scale;
                 *reinterpret_cast<u32x2 *>(static_cast<uint8_t *>(a.v_cache) + off) =
-                    scale_is_fast(s) ? quantize_chunk<T, true>(v[j], s, rcp) : quantize_chunk<T, false>(v[j], s, rcp);
+                    scale_is_fast(s) ? quantize_chunk<T, true>(v[j], s) : quantize_chunk<T, false>(v[j], s);
             } else {
                 *reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(a.v_cache) + off) = v[j];
             }

@@ -63,6 +63,8 @@ def lib():
             getattr(L, name).argtypes = [C.c_uint32, C.c_int64, C.c_int]
         L.gpuk_oracle_count_split_reciprocal_mismatch.restype = C.c_int64
         L.gpuk_oracle_count_split_reciprocal_mismatch.argtypes = [C.c_uint32, C.c_uint32, C.c_int, C.c_int]
+        L.gpuk_oracle_count_split_reciprocal_bf16_mismatch.restype = C.c_int64
+        L.gpuk_oracle_count_split_reciprocal_bf16_mismatch.argtypes = [C.c_uint32, C.c_uint32, C.c_int]
         _lib = L
     return _lib
 
@@ -146,3 +148,8 @@ def count_short_rcp_mismatch(first_bits: int, n: int, first_guess_ulp: int) -> i
 def count_split_reciprocal_mismatch(first: int, last: int, below: int, bits: int) -> int:
     """See gpuk_oracle_count_split_reciprocal_mismatch."""
     return lib().gpuk_oracle_count_split_reciprocal_mismatch(first, last, below, bits)
+
+
+def count_split_reciprocal_bf16_mismatch(first: int, last: int, below: int) -> int:
+    """See gpuk_oracle_count_split_reciprocal_bf16_mismatch."""
+    return lib().gpuk_oracle_count_split_reciprocal_bf16_mismatch(first, last, below)

@@ -424,3 +424,21 @@ int64_t gpuk_oracle_count_split_reciprocal_mismatch(uint32_t first, uint32_t las
     }
     return bad;
 }
+
+/* The same quotient rounded to bfloat16, for numerators of bfloat16: the number of (significand of s, tie between two bfloat16)
+ * whose nearest numerator rounds differently from the IEEE quotient. */
+int64_t gpuk_oracle_count_split_reciprocal_bf16_mismatch(uint32_t first, uint32_t last, int below) {
+    int64_t bad = 0;
+#pragma omp parallel for reduction(+ : bad)
+    for (int64_t m = first; m < (int64_t)last; ++m) {
+        const float s = bits_f32(0x3f800000u | (uint32_t)m), hi = bits_f32(f32_bits(1.0f / s) - (uint32_t)below);
+        const float lo = fmaf(-s, hi, 1.0f) * hi;
+        for (int t = 257; t < 512; t += 2) {
+            const float near = s * ((float)t * 0x1p-8f);   /* the numerator of the tie, in [1, 4); its nearest bfloat16: */
+            const float n = bits_f32((f32_bits(near) + 0x7fffu + ((f32_bits(near) >> 16) & 1u)) & 0xffff0000u);
+            const uint32_t q = f32_bits(n / s), r = f32_bits(fmaf(n, hi, n * lo));
+            bad += (q + 0x7fffu + ((q >> 16) & 1u)) >> 16 != (r + 0x7fffu + ((r >> 16) & 1u)) >> 16;
+        }
+    }
+    return bad;
+}

@@ -233,6 +233,12 @@ def test_quotients_by_a_split_reciprocal_give_the_same_codes(bits):
     assert c_oracle.count_split_reciprocal_mismatch((1 << 23) - 1, 1 << 23, 3, bits) > 0   # the excluded significand does fail
 
 
+@pytest.mark.parametrize("below", [2, 3, 4])
+def test_quotients_by_a_split_reciprocal_round_to_the_same_bfloat16(below):
+    """The fp8 cache rows: rT(o / scale) for a bfloat16 o, every significand of the scale, the numerators next to ties."""
+    assert c_oracle.count_split_reciprocal_bf16_mismatch(0, 1 << 23, below) == 0
+
+
 def test_no_scale_of_the_checked_maxima_has_a_significand_of_ones():
     for fp8_max in (448.0, 240.0):
         for dtype in (torch.bfloat16, torch.float16):
