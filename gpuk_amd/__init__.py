@@ -99,6 +99,9 @@ QUANT_NONE = 0
 QUANT_FP8_DYNAMIC = 1
 QUANT_FP8_STATIC = 3   # additive: one per-tensor scale, read from scale_out[0]
 
+_is_compiling = torch.compiler.is_compiling
+_is_current_stream_capturing = _direct.current_stream_is_capturing   # capture_: 0.48 us per call with torch's, 0.21 with this
+
 
 class GPUKDistEnv:
     """Single-GPU counterpart of the reference's GPUKDistEnv (gpuk/__init__.py:54-205).
@@ -157,9 +160,9 @@ class GPUKDistEnv:
     def capture_(self, input: torch.Tensor):
         """Per-call bookkeeping of the reference (gpuk/__init__.py:122-129): remember that a capture happened, and
         after it ended do what consume_capture does."""
-        if torch.compiler.is_compiling():
+        if _is_compiling():
             return
-        if torch.cuda.is_current_stream_capturing():
+        if _is_current_stream_capturing():
             self._IS_CAPTURED = True
         elif self._IS_CAPTURED:
             self.consume_capture()
@@ -193,7 +196,7 @@ class GPUKDistEnv:
         """
         self.capture_(allreduce_in)
         # functional schema, outputs allocated in the operator: the call survives tracing
-        tracing = torch.compiler.is_compiling()
+        tracing = _is_compiling()
         if fp8_out and static_scale is not None:
             op = _add_rms_fused_static if tracing else _add_rms_fused_static_direct
             return op(allreduce_in, residual_in, rms_weight, eps, static_scale)

@@ -4,6 +4,7 @@
 #include <atomic>
 
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPException.h>
 
 #include "ops.h"
 
@@ -17,6 +18,14 @@ namespace {
 std::atomic<double> g_fp8_max{448.0};
 }  // namespace
 
+bool current_stream_is_capturing() {
+    hipStream_t stream = static_cast<hipStream_t>(current_stream());
+    if (!stream) return false;
+    hipStreamCaptureStatus status{};
+    C10_HIP_CHECK(hipStreamIsCapturing(stream, &status));
+    return status != hipStreamCaptureStatusNone;
+}
+
 void set_fp8_max(double value) {
     TORCH_CHECK(value > 0.0 && value <= 448.0, "set_fp8_max: value must be in (0, 448], got ", value);
     g_fp8_max.store(value);
@@ -24,10 +33,9 @@ void set_fp8_max(double value) {
 
 double get_fp8_max() { return g_fp8_max.load(); }
 
-void allreduce_rms(int64_t fptr, Tensor &allreduce_in, Tensor &residual_in, Tensor &rms_gamma, Tensor &residual_out,
-                   Tensor &norm_out, Tensor &scale_out, double eps, int64_t quant_type) {
-    TORCH_CHECK(fptr == 0,
-                "allreduce_rms: this build is the single-GPU share of the op; pass fptr=0 (no all-reduce workspace)");
+namespace {
+void add_rms(const Tensor &allreduce_in, const Tensor &residual_in, const Tensor &rms_gamma, const Tensor &residual_out,
+             const Tensor &norm_out, const Tensor &scale_out, double eps, int64_t quant_type) {
     TORCH_CHECK(allreduce_in.is_contiguous() && residual_in.is_contiguous() && rms_gamma.is_contiguous());
     TORCH_CHECK(residual_out.is_contiguous() && norm_out.is_contiguous() && scale_out.is_contiguous());
     TORCH_CHECK(allreduce_in.dim() >= 1, "allreduce_rms: allreduce_in needs a hidden dimension");
@@ -68,6 +76,14 @@ void allreduce_rms(int64_t fptr, Tensor &allreduce_in, Tensor &residual_in, Tens
                                               current_stream());
     check_status(status, "allreduce_rms");
 }
+}  // namespace
+
+void allreduce_rms(int64_t fptr, Tensor &allreduce_in, Tensor &residual_in, Tensor &rms_gamma, Tensor &residual_out,
+                   Tensor &norm_out, Tensor &scale_out, double eps, int64_t quant_type) {
+    TORCH_CHECK(fptr == 0,
+                "allreduce_rms: this build is the single-GPU share of the op; pass fptr=0 (no all-reduce workspace)");
+    add_rms(allreduce_in, residual_in, rms_gamma, residual_out, norm_out, scale_out, eps, quant_type);
+}
 
 namespace {
 Tensor empty_like_as(const Tensor &t, at::ScalarType dtype) {  // t is contiguous; its strides are kept, as empty_like keeps them
@@ -99,12 +115,12 @@ std::tuple<Tensor, Tensor, Tensor> add_rms_fused(const Tensor &allreduce_in, con
     check_functional_quant_type(quant_type);
     check_inputs(allreduce_in, residual_in);
     const bool fp8 = quant_type != GPUK_QUANT_NONE;
-    Tensor x = allreduce_in, residual = residual_in, gamma = rms_gamma;
-    Tensor residual_out = empty_like_as(residual, residual.scalar_type());
+    const Tensor &x = allreduce_in;
+    Tensor residual_out = empty_like_as(residual_in, residual_in.scalar_type());
     Tensor norm_out = empty_like_as(x, fp8 ? at::kFloat8_e4m3fn : x.scalar_type());
     Tensor scale_out = fp8 ? at::detail::empty_cuda({x.size(0), 1}, at::kFloat, x.device(), std::nullopt)
                            : at::detail::empty_cuda({1}, at::kFloat, x.device(), std::nullopt);
-    allreduce_rms(0, x, residual, gamma, residual_out, norm_out, scale_out, eps, quant_type);
+    add_rms(x, residual_in, rms_gamma, residual_out, norm_out, scale_out, eps, quant_type);
     return {std::move(residual_out), std::move(norm_out), std::move(scale_out)};
 }
 
@@ -112,10 +128,9 @@ std::tuple<Tensor, Tensor> add_rms_fused_static(const Tensor &allreduce_in, cons
                                                 double eps, const Tensor &static_scale) {
     check_static_scale(static_scale, allreduce_in);
     check_inputs(allreduce_in, residual_in);
-    Tensor x = allreduce_in, residual = residual_in, gamma = rms_gamma, scale = static_scale;
-    Tensor residual_out = empty_like_as(residual, residual.scalar_type());
-    Tensor norm_out = empty_like_as(x, at::kFloat8_e4m3fn);
-    allreduce_rms(0, x, residual, gamma, residual_out, norm_out, scale, eps, GPUK_QUANT_FP8_STATIC);
+    Tensor residual_out = empty_like_as(residual_in, residual_in.scalar_type());
+    Tensor norm_out = empty_like_as(allreduce_in, at::kFloat8_e4m3fn);
+    add_rms(allreduce_in, residual_in, rms_gamma, residual_out, norm_out, static_scale, eps, GPUK_QUANT_FP8_STATIC);
     return {std::move(residual_out), std::move(norm_out)};
 }
 

@@ -1,6 +1,8 @@
 // fused_rope_rms / fused_mrope_3d_rms / fused_mrope_3d_rms_set_kv (+ the additive fused_rope_rms_set_kv).
 // Mirrors the host ops at src/ops/fused_rope.cpp:19-166: same argument order, contiguity checks, positions
 // passed by stride, KV-cache dtype decided by comparing it with qkv's dtype (:114).
+#include <ATen/hip/EmptyTensor.h>
+
 #include "ops.h"
 
 namespace gpuk_ops {
@@ -112,15 +114,22 @@ void fused_rope_rms_set_kv(Tensor &qkv, Tensor &qw, Tensor &kw, Tensor &cos_sin,
                num_heads_k, num_heads_v, head_size, is_neox_style, eps, q, k_cache, v_cache, kv_loc, k_scale, v_scale);
 }
 
-// fused_rope_rms_2way: shape inference shared by the Meta and the GPU kernel (src/ops/fused_rope.cpp:168-182).
+namespace {
+void check_contiguous_2way(const Tensor &q0, const Tensor &k0, const Tensor &q1, const Tensor &k1, const Tensor &w_q0, const Tensor &w_k0,
+                           const Tensor &w_q1, const Tensor &w_k1, const Tensor &cos_sin0, const Tensor &cos_sin1) {
+    TORCH_CHECK(q0.is_contiguous() && k0.is_contiguous() && q1.is_contiguous() && k1.is_contiguous());
+    TORCH_CHECK(w_q0.is_contiguous() && w_k0.is_contiguous() && w_q1.is_contiguous() && w_k1.is_contiguous());
+    TORCH_CHECK(cos_sin0.is_contiguous() && cos_sin1.is_contiguous());
+}
+}  // namespace
+
+// fused_rope_rms_2way: shape inference (src/ops/fused_rope.cpp:168-182).
 std::tuple<Tensor, Tensor> fused_rope_rms_2way_meta(Tensor &q0, Tensor &k0, Tensor &q1, Tensor &k1, Tensor &w_q0,
                                                     Tensor &w_k0, Tensor &w_q1, Tensor &w_k1, Tensor &cos_sin0,
                                                     Tensor &cos_sin1, int64_t batch_size, int64_t num_tokens0,
                                                     int64_t num_tokens1, int64_t num_heads_q, int64_t num_heads_k,
                                                     int64_t head_size, bool is_interleaved, double eps) {
-    TORCH_CHECK(q0.is_contiguous() && k0.is_contiguous() && q1.is_contiguous() && k1.is_contiguous());
-    TORCH_CHECK(w_q0.is_contiguous() && w_k0.is_contiguous() && w_q1.is_contiguous() && w_k1.is_contiguous());
-    TORCH_CHECK(cos_sin0.is_contiguous() && cos_sin1.is_contiguous());
+    check_contiguous_2way(q0, k0, q1, k1, w_q0, w_k0, w_q1, w_k1, cos_sin0, cos_sin1);
     Tensor out_q01 = at::empty({batch_size, num_tokens0 + num_tokens1, num_heads_q, head_size}, q0.options());
     Tensor out_k01 = at::empty({batch_size, num_tokens0 + num_tokens1, num_heads_k, head_size}, k0.options());
     return std::make_tuple(std::move(out_q01), std::move(out_k01));
@@ -132,8 +141,7 @@ std::tuple<Tensor, Tensor> fused_rope_rms_2way(Tensor &q0, Tensor &k0, Tensor &q
                                                int64_t num_heads_q, int64_t num_heads_k, int64_t head_size,
                                                bool is_interleaved, double eps) {
     const char *op = "fused_rope_rms_2way";
-    auto outs = fused_rope_rms_2way_meta(q0, k0, q1, k1, w_q0, w_k0, w_q1, w_k1, cos_sin0, cos_sin1, batch_size,
-                                         num_tokens0, num_tokens1, num_heads_q, num_heads_k, head_size, is_interleaved, eps);
+    check_contiguous_2way(q0, k0, q1, k1, w_q0, w_k0, w_q1, w_k1, cos_sin0, cos_sin1);
     TORCH_CHECK(head_size == 64 || head_size == 128 || head_size == 256, op, ": head_size must be 64, 128 or 256");
     TORCH_CHECK(q0.numel() == batch_size * num_tokens0 * num_heads_q * head_size &&
                     k0.numel() == batch_size * num_tokens0 * num_heads_k * head_size &&
@@ -152,13 +160,18 @@ std::tuple<Tensor, Tensor> fused_rope_rms_2way(Tensor &q0, Tensor &k0, Tensor &q
     TORCH_CHECK(q0.is_cuda(), op, ": tensors must live on the GPU");
     const int dtype = activation_dtype(q0, op);
     DeviceGuard guard(q0.device());
+    // (not by at::empty, whose way through the dispatcher costs as much as the allocation)
+    const auto output = [&](int64_t heads) {
+        return at::detail::empty_cuda({batch_size, num_tokens0 + num_tokens1, heads, head_size}, act, q0.device(), std::nullopt);
+    };
+    Tensor out_q01 = output(num_heads_q), out_k01 = output(num_heads_k);
     const int status = gpuk_rope_rms_2way(q0.data_ptr(), k0.data_ptr(), q1.data_ptr(), k1.data_ptr(), w_q0.data_ptr(),
                                           w_k0.data_ptr(), w_q1.data_ptr(), w_k1.data_ptr(), cos_sin0.data_ptr(),
                                           cos_sin1.data_ptr(), batch_size, num_tokens0, num_tokens1, num_heads_q,
                                           num_heads_k, head_size, is_interleaved, (float)eps, dtype,
-                                          std::get<0>(outs).data_ptr(), std::get<1>(outs).data_ptr(), current_stream());
+                                          out_q01.data_ptr(), out_k01.data_ptr(), current_stream());
     check_status(status, op);
-    return outs;
+    return {std::move(out_q01), std::move(out_k01)};
 }
 
 }  // namespace gpuk_ops

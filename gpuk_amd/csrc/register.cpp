@@ -19,6 +19,14 @@ template <typename... A, void (*F)(A...)> struct NoOpLike<F> {
     static void call(A...) {}
 };
 
+// No gradients through the operators that write into tensors of the caller and return nothing: autograd is passed by.  torch's own
+// answer to an operator without a derivative marks returned tensors and so does nothing for these, but collects every argument
+// on a stack and takes it apart again to do so: us per call of allreduce_rms with one row 3.36 / 3.25, of fused_rope_rms_set_kv with 32 tokens
+// 3.51 / 3.25.
+void no_gradients(torch::Library &m, const char *name) {
+    m.impl(name, torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+}
+
 // vmap would run a functional operator slice by slice, each slice its own rows and scales; it is refused here as it is for
 // the in-place operators, which have no batching rule either.
 void no_batching_rule(const c10::OperatorHandle &op, c10::DispatchKeySet, torch::jit::Stack *) {
@@ -33,6 +41,7 @@ TORCH_LIBRARY(gpuk, m) {
     m.def("allreduce_rms(SymInt fptr, Tensor allreduce_in, Tensor residual_in, Tensor rms_gamma, Tensor residual_out, "
           "Tensor norm_out, Tensor scale_out, float eps, SymInt quant_type) -> ()");
     m.impl("allreduce_rms", c10::DispatchKey::CUDA, &allreduce_rms);
+    no_gradients(m, "allreduce_rms");
     m.def("allreduce_rms.mut(SymInt fptr, Tensor allreduce_in, Tensor residual_in, Tensor rms_gamma, "
           "Tensor(a!) residual_out, Tensor(b!) norm_out, Tensor(c!) scale_out, float eps, SymInt quant_type) -> ()");
     m.impl("allreduce_rms.mut", c10::DispatchKey::CUDA, &allreduce_rms);
@@ -44,13 +53,13 @@ TORCH_LIBRARY(gpuk, m) {
           "(Tensor residual_out, Tensor norm_out, Tensor scale_out)");
     m.impl("add_rms_fused", c10::DispatchKey::CUDA, &add_rms_fused);
     m.impl("add_rms_fused", c10::DispatchKey::Meta, &add_rms_fused_meta);
-    m.impl("add_rms_fused", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+    no_gradients(m, "add_rms_fused");
     m.impl("add_rms_fused", torch::dispatch(c10::DispatchKey::FuncTorchBatched, torch::CppFunction::makeFromBoxedFunction<&no_batching_rule>()));
     m.def("add_rms_fused.static(Tensor allreduce_in, Tensor residual_in, Tensor rms_gamma, float eps, Tensor static_scale) -> "
           "(Tensor residual_out, Tensor norm_out)");
     m.impl("add_rms_fused.static", c10::DispatchKey::CUDA, &add_rms_fused_static);
     m.impl("add_rms_fused.static", c10::DispatchKey::Meta, &add_rms_fused_static_meta);
-    m.impl("add_rms_fused.static", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+    no_gradients(m, "add_rms_fused.static");
     m.impl("add_rms_fused.static", torch::dispatch(c10::DispatchKey::FuncTorchBatched, torch::CppFunction::makeFromBoxedFunction<&no_batching_rule>()));
 
     // reference: src/register.cpp:42-45
@@ -58,6 +67,7 @@ TORCH_LIBRARY(gpuk, m) {
           "SymInt num_heads_q, SymInt num_heads_k, SymInt num_heads_v, SymInt head_size, bool is_neox_style, "
           "float eps) -> ()");
     m.impl("fused_rope_rms", c10::DispatchKey::CUDA, &fused_rope_rms);
+    no_gradients(m, "fused_rope_rms");
     m.def("fused_rope_rms.mut(Tensor(a!) qkv, Tensor qw, Tensor kw, Tensor cos_sin, Tensor positions, "
           "SymInt num_tokens, SymInt num_heads_q, SymInt num_heads_k, SymInt num_heads_v, SymInt head_size, "
           "bool is_neox_style, float eps) -> ()");
@@ -69,6 +79,7 @@ TORCH_LIBRARY(gpuk, m) {
           "SymInt num_heads_q, SymInt num_heads_k, SymInt num_heads_v, SymInt head_size, bool is_neox_style, "
           "int[] mrope_section_, bool is_interleaved, float eps) -> ()");
     m.impl("fused_mrope_3d_rms", c10::DispatchKey::CUDA, &fused_mrope_3d_rms);
+    no_gradients(m, "fused_mrope_3d_rms");
     m.def("fused_mrope_3d_rms.mut(Tensor(a!) qkv, Tensor qw, Tensor kw, Tensor cos_sin, Tensor positions, "
           "SymInt num_tokens, SymInt num_heads_q, SymInt num_heads_k, SymInt num_heads_v, SymInt head_size, "
           "bool is_neox_style, int[] mrope_section_, bool is_interleaved, float eps) -> ()");
@@ -81,6 +92,7 @@ TORCH_LIBRARY(gpuk, m) {
           "bool is_neox_style, int[] mrope_section_, bool is_interleaved, float eps, Tensor q, Tensor k_cache, "
           "Tensor v_cache, Tensor kv_loc, float k_scale, float v_scale) -> ()");
     m.impl("fused_mrope_3d_rms_set_kv", c10::DispatchKey::CUDA, &fused_mrope_3d_rms_set_kv);
+    no_gradients(m, "fused_mrope_3d_rms_set_kv");
     m.def("fused_mrope_3d_rms_set_kv.mut(Tensor qkv, Tensor qw, Tensor kw, Tensor cos_sin, Tensor positions, "
           "SymInt num_tokens, SymInt num_heads_q, SymInt num_heads_k, SymInt num_heads_v, SymInt head_size, "
           "bool is_neox_style, int[] mrope_section_, bool is_interleaved, float eps, Tensor(a!) q, "
@@ -94,6 +106,7 @@ TORCH_LIBRARY(gpuk, m) {
           "bool is_neox_style, float eps, Tensor q, Tensor k_cache, Tensor v_cache, Tensor kv_loc, float k_scale, "
           "float v_scale) -> ()");
     m.impl("fused_rope_rms_set_kv", c10::DispatchKey::CUDA, &fused_rope_rms_set_kv);
+    no_gradients(m, "fused_rope_rms_set_kv");
     m.def("fused_rope_rms_set_kv.mut(Tensor qkv, Tensor qw, Tensor kw, Tensor cos_sin, Tensor positions, "
           "SymInt num_tokens, SymInt num_heads_q, SymInt num_heads_k, SymInt num_heads_v, SymInt head_size, "
           "bool is_neox_style, float eps, Tensor(a!) q, Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor kv_loc, "

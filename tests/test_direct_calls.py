@@ -235,3 +235,93 @@ def test_vmap_compile_and_profiler():
     assert any(e.key == "gpuk::fused_rope_rms_2way" for e in prof.key_averages())
     scripted = torch.jit.trace(lambda q0: packet(q0, *args[1:])[0], args[0], check_trace=False)
     assert "gpuk::fused_rope_rms_2way" in str(scripted.graph)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("around", ["plain", "parameter", "parameter, no_grad", "inference", "dispatch mode", "functions mode", "vmap", "grad", "profiler", "fake"])
+def test_two_streams_on_the_gpu_around_autograd(device, around):
+    """The direct call starts below autograd where nothing asks for a gradient and no transform or mode is at work: outputs, their
+    place in a graph and what a mode or a profiler sees are the general call's."""
+    packet = gpuk.fused_rope_rms_2way
+    gen = torch.Generator().manual_seed(3)
+    args = tuple(torch.randn(a.shape, generator=gen).bfloat16().to(device) if torch.is_tensor(a) else a for a in two_way("cpu"))
+    if "parameter" in around:
+        args = (*args[:4], args[4].requires_grad_(), *args[5:])
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    def call(f):
+        seen.clear()
+        if around == "parameter, no_grad":
+            with torch.no_grad():
+                return f(*args)
+        if around == "inference":
+            with torch.inference_mode():
+                return f(*args)
+        if "mode" in around:
+            with Dispatch() if "dispatch" in around else Functions():
+                return f(*args)
+        if around == "vmap":
+            return torch.vmap(lambda q0: f(q0, *args[1:]))(torch.stack([args[0], args[0]]))
+        if around == "grad":
+            return torch.func.grad_and_value(lambda w: f(*args[:4], w, *args[5:])[0].float().sum())(args[4].float().bfloat16())
+        if around == "profiler":
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+                out = f(*args)
+            assert any(e.key == "gpuk::fused_rope_rms_2way" for e in prof.key_averages())
+            return out
+        if around == "fake":
+            with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+                return f(*[mode.from_tensor(a) if torch.is_tensor(a) else a for a in args])
+        return f(*args)
+
+    def result(f):
+        try:
+            out = call(f)
+        except Exception as e:   # noqa: BLE001
+            return type(e), str(e)[:200], list(seen)
+        flat = [t for t in out if torch.is_tensor(t)]
+        return [(t.shape, t.dtype, str(t.device), t.requires_grad, type(t.grad_fn).__name__, t.is_inference(), type(t)) for t in flat], list(seen), flat
+
+    got, want = result(packet), result(general(packet))
+    assert got[:2] == want[:2], (got[:2], want[:2])
+    if around != "fake" and isinstance(got[2], list) and got[2] and torch.is_tensor(got[2][0]):
+        assert all(torch.equal(a, b) for a, b in zip(got[2], want[2]))
+
+
+@pytest.mark.parametrize("name", [n for n in NAMES if "2way" not in n])
+def test_in_place_operators_with_parameters(name):
+    """They return nothing a graph could hold: weights that are parameters change nothing, with gradients asked for or not."""
+    direct, packet = both(name)
+    args = [a.requires_grad_() if torch.is_tensor(a) and a.dim() == 1 and a.is_floating_point() else a for a in arguments(name, "cpu")]
+    with recorded() as calls:
+        for f in (direct, packet):
+            assert f(*args) is None
+            with torch.no_grad():
+                assert f(*args) is None
+    assert len(calls) == 4 and all(c == calls[0] for c in calls)
+    assert all(not torch.is_tensor(a) or a.grad_fn is None for a in args)
+
+
+@pytest.mark.gpu
+def test_capture_status(device):
+    ask, torchs = gpuk._direct.current_stream_is_capturing, torch.cuda.is_current_stream_capturing
+    assert ask() is torchs() is False
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert ask() is torchs() is False
+    buf = torch.zeros(8, device=device)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        assert ask() is torchs() is True
+        buf.add_(1)
+    assert ask() is torchs() is False
