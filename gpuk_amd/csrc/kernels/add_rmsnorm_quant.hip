@@ -203,7 +203,10 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
     // ---- phase 1: res = rT(x + r), stored once; sum of squares of the *rounded* residual.  Waves in this phase
     // are given issue priority over the arithmetic of phases 2-3 so that their residual stores leave early (+0.4 %).
     __builtin_amdgcn_s_setprio(1);
-    float ss0 = 0.f, ss1 = 0.f;
+    // (A partial sum takes the squares of no more than two chunks: a row's sum in four chunks per lane is then as close to that in
+    // 64 bits as in two, over 1536 rows of 8192 bfloat16 elements 3.9e-8 off in the mean square (4.4e-8 with two sums, two chunks 4.0e-8).)
+    constexpr int kSums = NCHUNK >= 4 ? 4 : 2;
+    float ss[kSums] = {};
 #pragma unroll
     for (int i = 0; i < NCHUNK; ++i) {
 #pragma unroll
@@ -212,8 +215,8 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
             if constexpr (is_half<T>) w = P::add(xv[i][j], rv[i][j]);
             else w = P::pack(P::lo(xv[i][j]) + P::lo(rv[i][j]), P::hi(xv[i][j]) + P::hi(rv[i][j]));
             xv[i][j] = w;  // xv now holds the residual
-            if (j & 1) ss1 = P::add_squares(w, ss1);
-            else ss0 = P::add_squares(w, ss0);
+            float &sum = ss[(2 * i + (j & 1)) % kSums];
+            sum = P::add_squares(w, sum);
         }
         if (!GATED && live[i]) store_stream(residual_out + row_base + i * nthreads + tid, xv[i]);
     }
@@ -234,7 +237,9 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
     float res[kUnpacked ? NCHUNK : 1][8], weight[kUnpacked ? NCHUNK : 1][8];
     SplitReciprocal rcp{};  // of the scale; `fast`: quotients take the short form
     bool fast = false;
-    const float sumsq = block_allreduce<SumOp>(ss0 + ss1, s_sum, num_waves, [&] {
+    float lane_sum = ss[0] + ss[1];
+    if constexpr (kSums == 4) lane_sum += ss[2] + ss[3];
+    const float sumsq = block_allreduce<SumOp>(lane_sum, s_sum, num_waves, [&] {
         if constexpr (QUANT == GPUK_QUANT_FP8_STATIC) {
             fast = __builtin_amdgcn_ballot_w64(!(scale_in_fast_range(static_scale) && !mantissa_all_ones(static_scale))) == 0;
             rcp = split_reciprocal(static_scale);
@@ -865,10 +870,19 @@ template <typename T> constexpr RowType row_type = is_half<T> ? RowType::FP16 : 
 // precision, static scale).  From two fifths of a round to eleven twentieths they wait 1.16 times the read time: 460 rows of
 // 8192 elements 6.28 / 5.72 us, 576 of 6144 6.55 / 6.05, 576 of 5120 5.46 / 5.3, level or slower below and above (1228 of 4096
 // 6.6 / 6.8).
+// 16-bit rows of one chunk per lane spread their stores by themselves, each wave as its row is done, and wait from three eighths
+// of a round only (gated / not, us: 2800 of 512 elements 3.71 / 3.45, static 3.33 / 3.32, 400 of 2560 3.63 / 3.36, without codes
+// 3.15 / 2.97, 128 of 5632 3.73 / 3.37, 130 of 7680 4.23 / 3.61; beyond, 580 of 2560 without codes 3.55 / 3.63, half precision 3.54
+// / 3.93), ten waves a row not in the first layer (bfloat16, 200 of 5120 3.73 / 3.55, 256 3.97 / 3.75; 12 to 15 waves level to 6 %
+// behind there).  The shortest of them, half precision without codes on one wave, from a quarter as the others (2800 of 512
+// elements 3.25 / 3.47).
 uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, RowType type, int quant) {
     if (g_gate >= 0) return (uint32_t)g_gate;
     const int64_t resident = resident_rows(threads, nchunk);
     if (tokens > resident || 4 * tokens < resident) return 0;
+    const bool quick = type == RowType::FP16 && quant == GPUK_QUANT_NONE && threads == 64;
+    const bool early = 8 * tokens < 3 * resident || (threads <= 640 && tokens <= kComputeUnits);
+    if (nchunk == 1 && type != RowType::F32 && early && !quick) return 0;
     // (four chunks per lane: the shape pick_shape takes to hold in one round what two chunks per lane cannot)
     const bool short_rows = type == RowType::FP16 && quant == GPUK_QUANT_FP8_STATIC;
     const bool half_filled = short_rows && nchunk == 2 && 5 * tokens >= 2 * resident && 20 * tokens <= 11 * resident;
@@ -881,7 +895,7 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, 
 
 // Lanes per row and chunks per lane.  Two chunks per lane on as many lanes as that needs (up to 1024) stream best or tie
 // for 1024 .. 16384 16-bit elements (1-6 % over one or four chunks per lane; 7168 elements, per call: 3.3 us against 3.5
-// with one chunk at one row, 5.0 against 5.6 at 256 rows); longer rows double the chunks per lane.  Where rounding up to
+// with one chunk at one row, 5.0 against 5.6 at 256 rows), but for the small batches named below; longer rows double the chunks per lane.  Where rounding up to
 // whole waves idles more lanes that way (an odd number of 64 chunks, or a little more than an even one), one chunk per lane
 // serves what the chip holds in one round (1032 elements: 2.2 against 2.45 us at one row, 5.65 against 6.2 at 2048), but
 // larger batches want the loads of two in flight: 12000 rows of 2560 / 3584 / 5632 / 7680 elements 37.0 / 49.6 / 76.6 /
@@ -900,6 +914,35 @@ void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, 
         const int lanes1 = round_up(chunks_per_row, 64), lanes2 = round_up((chunks_per_row + 1) / 2, 64);
         n = (2 * lanes2 > lanes1 && lanes1 <= kMaxThreads) ? 1 : 2;
         while (n < most_chunks && chunks_per_row > kMaxThreads * n) n *= 2;
+        if (n == 2 && !g_force_threads) {
+            // A compute unit that has a row or two is bound by the instructions of its busiest SIMD, chunks per lane times the
+            // waves there: lanes for 5 or 6 waves of two chunks put four chunks on one SIMD, 10 to 12 waves of one chunk three
+            // (us, two / one: 12 rows of 6000 elements 3.44 / 3.20, 64 of 6144 3.45 / 3.10, without codes 3.21 / 2.82, 128 of
+            // 5120 3.63 / 3.35, half precision 3.42 / 3.38; fp32 32 of 3072 3.11 / 2.89, 192 3.48 / 3.32).  As the first layer
+            // fills, the waves share the units' load paths and only the 5 of bfloat16 still gain (256 of 5120 3.96 / 3.75,
+            // without codes level, half precision 3.42 / 3.72, 256 of 5640 4.11 / 4.27); with a second row per unit they gain
+            // again, up to half a layer more (320 of 5640 5.50 / 5.12, 270 of 5120 without codes 4.18 / 3.80), in half precision a
+            // quarter (384 of 5640 without codes 4.88 / 4.98).
+            // 2 waves of two chunks and 4 of one are one wave a SIMD at most, of half the length: 4 rows of 2048 elements 2.48 /
+            // 2.34, 300 3.39 / 2.81, 640 3.65 / 3.57, without codes 3.21 / 2.95, but 768 without codes 3.25 / 3.43 (fp32 gains less,
+            // 2-4 %, and only for a few rows).
+            // Where each of more than half of the units has one row, 3 or 4 full waves of four chunks wait for fewer of each
+            // other (us, two / four: 160 rows of 6144 3.91 / 3.73, 256 4.29 / 4.02, without codes 4.00 / 3.60; 200 of 8192 4.49 /
+            // 4.31, 256 without codes 4.52 / 4.09; 128 rows of 8192 and 7168 elements level, which idle lanes).
+            const int lanes4 = round_up((chunks_per_row + 3) / 4, 64);
+            const bool f32 = type == RowType::F32, f16 = type == RowType::FP16;
+            if (!f32 && 2 * tokens > kComputeUnits && tokens <= kComputeUnits && (lanes4 == 192 || lanes4 == 256) &&
+                15 * lanes4 < 4 * chunks_per_row) {
+                n = 4;
+            } else if (lanes2 == 128) {
+                if (!f32 && 2 * tokens <= 5 * kComputeUnits) n = 1;
+            } else if (lanes2 == 320 || lanes2 == 384) {
+                const bool few = 4 * tokens <= 3 * kComputeUnits;
+                const bool first_layer = tokens <= kComputeUnits && lanes2 == 320 && !f16;
+                const bool second_layer = tokens > kComputeUnits && 4 * tokens <= (f16 ? 5 : 6) * kComputeUnits;
+                if (few || (!f32 && (first_layer || second_layer))) n = 1;
+            }
+        }
         // A batch that two chunks per lane cannot hold in one round but four can (half the lanes per row, so up to
         // 2048 rows of 7168 or 8192 elements instead of 1024) takes four: one round, with the store gate, against two
         // rounds of mixed reads and writes.  7168 elements: 10.8 against 12.8 us at 1100 rows, 10.9 against 14.3 at

@@ -179,6 +179,17 @@ def test_every_chunking_variant(device, nchunk):
         capi.set_tuning("norm_quant_nchunk", 0)
 
 
+# (rows at the edges of their class of lengths, batches at the edges of their shape)
+@pytest.mark.parametrize("tokens,hidden", [(1, 1544), (640, 2048), (641, 2048), (3, 4616), (256, 5120), (257, 5128), (384, 6144), (129, 8192), (256, 6144),
+                                           (256, 8136), (3071, 512)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_shapes_of_small_batches(device, dtype, tokens, hidden):
+    print(f"case small batches {tokens}x{hidden} {dtype}", flush=True)
+    inp = workloads.norm_quant_inputs(tokens, hidden, seed=tokens + hidden, res_sigma=2.0, outlier_frac=0.01, dtype=dtype)
+    for quant in (0, 1):
+        check(inp, quant, run_capi(inp, quant, device), tag=f"[{tokens}x{hidden} {dtype} q{quant}]")
+
+
 @pytest.mark.parametrize("threads,nchunk", [(512, 2), (256, 4), (1024, 2), (128, 8), (448, 2), (1024, 1), (1024, 8)])
 def test_launch_shape_variants(device, threads, nchunk):
     """Workgroup size and chunks per lane are tuning choices only."""
