@@ -1516,63 +1516,71 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     const TokenShape one_item = token_shape(a, D, axes, set_kv, kv_fp8, false), two_items = token_shape(a, D, axes, set_kv, kv_fp8, true);
     const bool two = two_items.units && (g_token_waves == 3 || !one_item.units);
     const TokenShape shape = two ? two_items : one_item;
-    // ... and clearly too large for the kernel above to hold all of its waves at once (from 10240 units, five quarters of what
-    // it holds; below that the kernel above, gated, is ahead or level: 8.3 against 9.7 us at 1536 tokens of 32+8+8 heads, 9.1
-    // against 9.5 at 2100 tokens of 28+4+4; from there on this one is: 32+8+8 heads 10.3 against 11.1 us at 2048 tokens, 13.6
-    // against 14.8 at 3000, 16.6 against 17.3 at 3700, 16.2 against 18.2 at 4096; 28+4+4 heads with three axes 10.0 against
-    // 11.7 us at 3000 tokens, 12.2 against 14.5 at 4096, interleaved sections 10.0 against 11.6 at 2621, 12.7 against 16.2 at
-    // 4096; heads of 256 elements, 28+4+4, two parts of four, from 11264: 10.2 against 12.4 at 1536 tokens, 12.5 against 15.5
-    // at 2048; 64+8+8, two of five, 14.2 against 16.0 at 2048).  With three units per wave from 9216 units: 40+8+8 heads, two
-    // parts, 8.5 against 9.7 us at 1536 tokens, 10.2 against 12.2 at 2048; 16+2+2 7.9 against 8.9 at 3072, 9.4 against 10.6 at
-    // 4096; 12+12+12 10.3 against 12.7, 12.8 against 15.5.
-    // With two items per wave from there to twice that many items: 4096 waves, four on every SIMD, one item each and the others
-    // dealt out evenly.  The SIMD with the most items sets the time (the rotation arithmetic of its waves is two thirds of the
-    // launch), so the time goes up in steps of 1024 items where the kernel above is linear; this one is ahead or level
-    // everywhere (graph replays, 28+4+4 heads, one axis / three: 16.1 / 16.4 against 17.2 / 17.5 us at 4800 tokens, 18.2 / 18.5
-    // against 18.4 / 18.8 at 5200, 19.1 / 19.6 against 21.1 / 21.5 at 6144, 21.7 / 21.7 against 23.5 / 23.7 at 7000, 24.2 /
-    // 24.4 against 24.7 / 25.3 at 7500, 25.3 / 25.3 against 26.8 / 27.3 at 8192, interleaved 19.7 against 22.5 at 6144, 26.0
-    // against 28.5 at 8192; 40+8+8, two parts of three, 12.1 against 13.2 at 2304, 19.9 against 21.5 at 4096; 28+4+4 heads of
-    // 256, two of four, 18.4 against 20.8 at 3000, 25.4 against 27.1 at 4096; level below 4608 items, where the kernel above
-    // stays).  Half as many waves with two items each were behind that: 20.0 at 6144 tokens.
-    // (in place, with no V row and no scatter, the kernel above holds out a little longer: 9.0 against 9.5 us at 2048 tokens of
-    // 32+8 heads, then 11.9 against 11.2 at 3000, 15.4 against 13.7 at 4096; 28+4 heads with three axes 10.7 against 9.5 at
-    // 3000 tokens, 13.2 against 11.5 at 4096, 18.4 against 17.4 at 6144 and 23.2 against 21.6 at 8192 with two items per wave;
-    // 40+8, parts of three, 8.3 against 7.9 at 1536, 10.4 against 9.4 at 2048, 11.2 against 11.4 at 2304 and 13.9 against 13.5
-    // at 3000 with two items per wave)
-    // Half precision, whose arithmetic is packed, from seven eighths of the other kernel's round where nearly all lanes have a
-    // head and two waves are left per SIMD: 40+8+8 heads 6.6 against 7.0 us at 1228 tokens, 6.8 against 7.5 at 1365, 9.6
-    // against 11.7 at 2048 (32+8+8, parts of five, 7.4 against 7.1 at 1471; 48+8+8, an idle unit, 7.2 against 6.8 at 1056).
-    const bool full = 8 * heads >= 7 * places, no_idle_unit = shape.units * shape.parts == (int)a.units_per_token;
-    const int64_t from_units = half && full && no_idle_unit && shape.units <= 4 && shape.items >= 2048 ? 7 * kResidentUnits / 8
-                               : shape.units == 3 ? 9 * kResidentUnits / 8
-                               : !set_kv ? 7 * kResidentUnits / 5 : shape.parts == 1 ? 5 * kResidentUnits / 4 : 11 * kResidentUnits / 8;
-    // (with an fp8 cache the conversions lengthen the wave and the gate hardly matters; one token per wave is still
-    // ahead once the batch is large: 28+4+4 heads 10.8 against 11.9 us at 3000 tokens, 13.3 against 14.2 at 4096; 32+8+8
-    // heads 16.8 against 17.6 at 4096, level at 3000, behind at 2560)
-    const int64_t from_units_fp8 = a.units_per_token == 4 ? 5 * kResidentUnits / 4 : 7 * kResidentUnits / 4;
-    // (two items per wave: level or 1 % behind below, 15.4 against 15.2 us at 4100 tokens)
-    bool large = two ? shape.items >= kTokenWaveCapacity + kTokenWaveCapacity / 8 : a.total_units >= (kv_fp8 ? from_units_fp8 : from_units);
-    // Where the margin is thin it does not cover every fill of the last layer of waves.  Beyond whole tokens of four or five
-    // units of 128-element heads that read one table row, these stay with the kernel above (us, that one / this one).  In
-    // place: pairwise rotation (28+4 heads of 256 in half precision 10.4 / 11.2 at 1611 tokens, 40+8 17.1 / 17.7 at 3802),
-    // parts of five or with idle units (64+8 heads 10.4 / 10.7 at 1370 tokens, 48+8 10.3 / 10.7 at 1739), a layer that has just
-    // begun (64+8 heads 11.5 / 12.6 at 1618 tokens, 3236 items) and two items per wave in bfloat16 (40+8 16.7 / 16.7 at 3749)
-    // or with idle lanes (16+2 in half precision 13.8 / 15.3 at 8186). With a cache: a layer that has just begun where lanes or
-    // units idle (16+2+2 in half precision 7.6 / 8.2 at 3148), two items per wave where lanes idle in bfloat16 but for merged
-    // table rows (16+2+2 16.1 / 16.6 at 7544).  Pairwise with a cache: the latter in every type, seven layers and more (20+4+4
-    // in half precision 21.0 / 21.5 at 7797), a layer that has just begun, and bfloat16 with three V chunks per lane (12+12+12
-    // 14.3 / 14.9 at 3592).
-    // (Over calls drawn afterwards that only one of those with a cache keeps here, the token kernel's time over this one's: two
-    // items per wave with idle lanes 0.81 to 1.03, on average 0.93, pairwise and 0.90 to 1.05, 0.96, in bfloat16 rotated by
-    // halves, a layer that has just begun 0.86 to 1.11, 0.97; the other three level, 0.88 to 1.06.)
-    if (!whole_token(a, D, axes, shape.units, shape.parts)) {
-        const int64_t last = shape.items > 3072 ? shape.items % 1024 : 0;  // items of the last layer, 0: it is full
-        if (!set_kv) large = large && no_idle_unit && (two ? full : last == 0 || last >= 256);  // (and see token_form_in_place)
-        else if (neox) large = large && (!two || full || half || (axes == 3 && !a.merge_rows)) && ((full && no_idle_unit) || last == 0 || last >= 256);
-        else large = large && (!two || (full && shape.items <= 7168)) && (last == 0 || last >= 384) && (half || a.hv * (D / 8) <= 128 * shape.parts);
+    // ... and too large for the kernel above to hold all of its waves at once (8192 units).  Where the two cross was read off
+    // 3000 random calls of 3 to 20 units per token (both kernels in turn, graph replays); over 1100 others, drawn afterwards, the
+    // calls whose kernel the lines change take 0.944 of the time that earlier lines gave them.  us, that kernel / this one:
+    // One item per wave, 16-bit cache.  Half precision, whose arithmetic is packed, from seven eighths of the other kernel's
+    // round where nearly all lanes have a head and no unit idles (40+8+8 heads 6.6 / 7.0 at 1228 tokens, 6.8 / 7.5 at 1365),
+    // with five units from fifteen sixteenths (32+8+8 7.4 / 7.1 at 1471), else and five units rotated pairwise beyond a round
+    // (16+2+2 5.5 / 6.1 at 2415 tokens, 7245 units, but 9.0 / 7.9 at 3031; 48+8+8 13.7 / 11.4 at 2151, two of four).  bfloat16
+    // beyond a round with three units (40+8+8, two parts, 9.7 / 8.5 at 1536 tokens, 12.2 / 10.2 at 2048; 24+8+8 heads of 256
+    // 12.5 / 10.4 at 1288), from seventeen sixteenths where lanes idle
+    // (16+2+2 7.5 / 7.8 at 2739), with four in parts and whole tokens of five from nine eighths of one (32+8+8 11.1 / 10.3 at 2048,
+    // 18.2 / 16.2 at 4096; 28+4+4 heads of 256 pairwise 11.2 / 9.8 at 1286), whole tokens of four and others of five from five
+    // quarters (28+4+4 9.2 / 9.8 at 2244, 11.5 / 10.3 at 2906; 16+2+2 heads of 256 8.8 / 9.3 at 1846).
+    // In place there is no V row and no scatter, and in bfloat16 the kernel above holds out longer with four and five units: 9.0
+    // / 9.5 at 2048 tokens of 32+8 heads, then 11.9 / 11.2 at 3000, 15.4 / 13.7 at 4096; 28+4 heads with three axes 10.7 / 9.5
+    // at 3000; 40+8, parts of three, 8.3 / 7.9 at 1536.
+    // The SIMD with the most items sets the time (the rotation arithmetic of its waves is most of the launch), so it goes up in
+    // steps of 1024 items where the kernel above is linear, and a fourth layer that has just begun (3072 items and `begun`
+    // more) stays there in the forms that it costs more than it gives: 16+2+2 pairwise in half precision 8.8 / 9.5 at 3617
+    // tokens, 12+12+12 pairwise in bfloat16, three V chunks per lane, 14.8 / 15.5 at 3755, 32+8 in place 12.9 / 13.1 at 3150.
+    // Two items per wave, from a full round of items to twice that: 4096 waves, four on every SIMD, one item each and the others
+    // dealt out evenly.  In half precision with a cache at once (28+4+4 15.4 / 12.7 at 4148 tokens, 16+2+2 10.0 / 8.7 at 4367,
+    // pairwise 10.5 / 9.5 at 4545); in bfloat16 with four units from 4352 items, whole
+    // tokens 4608 (28+4+4 15.2 / 15.4 at 4100, 18.4 / 18.2 at 5200, 21.1 / 19.1 at 6144,
+    // 26.8 / 25.3 at 8192; 12+2+2 heads of 256 14.2 / 15.3 at 4123), where lanes idle and one table row is read not in a
+    // layer's first half (16+2+2 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600), pairwise only in its last quarter (13.1 / 13.7 at
+    // 5748, 13.8 / 13.5 at 6135), and pairwise with three units up to 7168 items (64+8+8 heads of 256 19.1 / 20.6 at 7380, in
+    // half precision 18.7 / 19.4 at 7272).  In
+    // place from 4608 items, pairwise 4352, in half precision at once but no further than 7168 items, with idle lanes 6144,
+    // unless whole tokens (16+2 12.7 / 14.9 at 7348, 10.3 / 9.6 at 5526).
+    const int units = shape.units;
+    const int64_t items = shape.items, begun = items > 3072 && items < kTokenWaveCapacity ? items - 3072 : 1024;
+    const int64_t layer = items % 1024 ? items % 1024 : 1024;  // items of the last layer
+    const bool full = 8 * heads >= 7 * places, no_idle_unit = units * shape.parts == (int)a.units_per_token;
+    const bool whole = whole_token(a, D, axes, units, shape.parts);
+    bool large;
+    if (kv_fp8) {
+        // The conversions lengthen the wave, the gate hardly matters, and a layer that has just begun costs more: 28+4+4 heads
+        // 11.9 / 10.8 at 3000 tokens, 14.2 / 13.3 at 4096, 12.5 / 12.9 at 3244; 32+8+8 14.8 / 14.0 at 2990, 14.6 / 15.9 at 3086,
+        // 17.6 / 16.8 at 4096, level at 2500.
+        large = 8 * (int64_t)a.total_units >= (units == 4 ? 10 : 13) * kResidentUnits && layer >= 256;
+    } else if (two) {
+        if (!set_kv) large = half ? whole || (no_idle_unit && items <= (full ? 7168 : 6144)) : items >= (neox ? 4608 : 4352) && (whole || (full && no_idle_unit));
+        else if (half) large = neox || units == 4 || items <= 7168;
+        else if (neox) large = (units == 3 || items >= (whole || !no_idle_unit ? 4608 : 4352)) && (full || layer >= 512 || (axes == 3 && !a.merge_rows));
+        else large = whole ? items >= 4608 : (units == 4 || items <= 7168) && (full || layer >= 768);
+    } else {
+        int64_t from_units = kResidentUnits + 1;
+        if (half) {
+            if (full && no_idle_unit && (units < 5 || (set_kv && neox))) from_units = units == 5 ? 15 * kResidentUnits / 16 : set_kv || units == 3 ? 7 * kResidentUnits / 8 : 59 * kResidentUnits / 64;
+        } else if (set_kv) {
+            if (units > 3) from_units = (units == 4) == whole ? 5 * kResidentUnits / 4 : 9 * kResidentUnits / 8;
+            else if (!full) from_units = 17 * kResidentUnits / 16;
+        } else {
+            if (whole) from_units = 7 * kResidentUnits / 5;
+            else if (units == 4) from_units = 5 * kResidentUnits / 4;
+        }
+        int64_t from_begun;
+        if (!set_kv) from_begun = half ? (!neox ? 640 : !full ? 256 : units == 4 ? 128 : 0) : !neox || units < 5 ? 256 : 384;
+        else if (half) from_begun = !neox ? (units == 3 ? 576 : 384) : full && no_idle_unit ? 0 : 128;
+        else if (neox) from_begun = 0;
+        else from_begun = a.hv * (D / 8) > 128 * shape.parts ? 768 : 256;
+        large = (int64_t)a.total_units >= from_units && begun >= from_begun && (set_kv || whole || no_idle_unit);
     }
     const bool by_rule = g_token_waves == 0 && large;
-    const bool has_form = set_kv || whole_token(a, D, axes, shape.units, shape.parts) || token_form_in_place(neox, half, shape.units, two);
+    const bool has_form = set_kv || whole || token_form_in_place(neox, half, shape.units, two);
     p.token_waves = shape.units && has_form && (g_token_waves >= 2 || by_rule);
     p.two_tokens = p.token_waves && two;
     // (with two items per wave the full read time: 24.4 us at 8192 tokens of 28+4+4 heads with three axes, against 25.4

@@ -460,3 +460,32 @@ def test_rope_launch_shape_report():
     assert L.gpuk_rope_rms_launch_shape(4, 32, 8, 8, 128, 2, 0, 1, 0, *refs) == 1
     assert L.gpuk_rope_rms_launch_shape(4, 32, 8, 8, 128, 1, 0, 1, 0, None, *refs[1:]) == 1
     assert L.gpuk_rope_rms_launch_shape(4, 32, 8, 8, 128, 1, 9, 1, 0, *refs) == 2   # no such dtype
+
+
+def test_rope_kernel_choice():
+    """Which calls the kernel with one wave per token or part of one takes (1: one item per wave, 2: two), from both sides of
+    the lines of its rule, rotation by halves."""
+    from gpuk_amd import capi
+
+    bf16, f16 = torch.bfloat16, torch.float16
+    for heads, D, dtype, cache, changes in (
+            # three units per item: beyond a round of the other kernel's waves, or more where lanes idle; half precision from seven eighths where lanes are full
+            ((16, 2, 2), 128, bf16, True, ((2901, 0), (2902, 1), (4096, 1), (4097, 0), (4607, 0), (4608, 2), (5120, 2), (5300, 0), (8192, 2), (8193, 0))),
+            ((16, 2, 2), 128, f16, True, ((2389, 0), (2730, 0), (2731, 1), (3072, 1), (3073, 0), (3200, 1), (4096, 1), (4097, 2), (8192, 2), (8193, 0))),
+            ((12, 12, 12), 128, f16, True, ((2389, 0), (2390, 1), (3073, 1))),
+            ((24, 8, 8), 256, bf16, True, ((1151, 0), (1152, 1), (2048, 1), (2049, 0))),
+            ((28, 4, 4), 256, bf16, True, ((2048, 1), (2175, 0), (2176, 2))),
+            # four, five: from nine eighths of a round, whole tokens of four from five quarters
+            ((28, 4, 4), 128, bf16, True, ((2559, 0), (2560, 1), (3073, 1), (4607, 0), (4608, 2))),
+            ((28, 4, 4), 128, f16, True, ((1791, 0), (1792, 1), (4096, 1), (4097, 2))),
+            ((32, 8, 8), 128, bf16, True, ((1843, 0), (1844, 1), (3073, 1), (4096, 1), (4097, 0))),
+            ((32, 8, 8), 128, f16, True, ((1535, 0), (1536, 1), (4096, 1), (4097, 0))),
+            # in place
+            ((32, 8, 8), 128, bf16, False, ((2293, 0), (2294, 1), (3455, 0), (3456, 1))),
+            ((16, 2, 2), 128, f16, False, ((2730, 0), (2731, 1), (3327, 0), (3328, 1), (6144, 2), (6145, 0))),
+            ((12, 12, 12), 128, f16, False, ((2389, 0), (2390, 1), (7168, 2), (7169, 0)))):
+        for tokens, expect in changes:
+            assert capi.rope_rms_launch_shape(tokens, *heads, D, 1, dtype, cache, False)[3] == expect, (tokens, heads, D, dtype, cache)
+    # an fp8 cache: whole tokens, not where the last layer of waves has just begun
+    for tokens, heads, expect in ((2560, (28, 4, 4), 1), (3200, (28, 4, 4), 0), (3328, (28, 4, 4), 1), (2662, (32, 8, 8), 0), (2663, (32, 8, 8), 1), (3100, (32, 8, 8), 0)):
+        assert capi.rope_rms_launch_shape(tokens, *heads, 128, 1, bf16, True, True)[3] == expect, (tokens, heads)

@@ -88,3 +88,29 @@ def test_parts_by_rule(device, tokens, heads, D, waves):
         capi.set_tuning("rope_token_waves", 0)
     for name, a, b in zip(("q_out", "k_cache", "v_cache"), got[:3], base[:3]):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"{name}: the two kernels differ"
+
+
+@pytest.mark.parametrize("tokens,heads,D,neox,sections,fp16", [
+    (2731, (16, 2, 2), 128, True, None, False), (2390, (12, 12, 12), 128, False, None, True), (4097, (16, 2, 2), 128, True, [24, 20, 20], True),
+    (1792, (28, 4, 4), 128, False, [16, 24, 24], True), (4097, (28, 4, 4), 128, True, [24, 20, 20], True), (1152, (24, 8, 8), 256, True, None, False),
+    (2179, (14, 2, 2), 256, False, None, False), (1844, (32, 8, 8), 128, False, None, False), (1537, (48, 8, 8), 128, True, [24, 20, 20], False)])
+def test_choice_changes_no_bits(device, tokens, heads, D, neox, sections, fp16):
+    """Calls at the lines of the rule, as it chooses and with one wave per group of heads: the same bits, with a cache and in
+    place, for either rotation, table rows that are merged and tokens without a slot."""
+    print(f"case choice {tokens} {heads} {D} neox={neox} {sections} fp16={fp16}", flush=True)
+    inp = make(tokens, heads[0], D, neox, seed=tokens, mrope=sections is not None, interleaved=sections is not None and sections[0] == 24, hk=heads[1], hv=heads[2])
+    if sections is not None:
+        inp.mrope_section = sections
+        inp.positions[:, ::3] = inp.positions[:1, ::3]
+    if fp16:
+        inp.qkv, inp.qw, inp.kw, inp.cos_sin = (t.to(torch.float16) for t in (inp.qkv, inp.qw, inp.kw, inp.cos_sin))
+        inp.kv_dtype = torch.float16
+    inp.kv_loc[3::13] = -1
+    got = [*run_set_kv(inp, device)[:3], run_inplace(inp, device)]
+    try:
+        capi.set_tuning("rope_token_waves", 1)
+        base = [*run_set_kv(inp, device)[:3], run_inplace(inp, device)]
+    finally:
+        capi.set_tuning("rope_token_waves", 0)
+    for name, a, b in zip(("q_out", "k_cache", "v_cache", "in place"), got, base):
+        assert torch.equal(a.cpu().contiguous().view(torch.uint8), b.cpu().contiguous().view(torch.uint8)), f"{name}: the two kernels differ"
