@@ -130,7 +130,13 @@ __device__ __attribute__((noinline)) u32x2 codes_by_division(f32x8 n, float scal
 // EXACT: lanes x NCHUNK equals the chunks of a row, so every lane owns NCHUNK live chunks and nothing is masked
 // (true for every power-of-two row and for 7168 elements; it removes a sixth of the kernel's instructions, which is
 // what a decode-sized batch waits for: with at most one row per compute unit the run time is the row's arithmetic).
-template <typename T, int NCHUNK, int QUANT, bool EXACT, bool GATED>
+// LANDED: the weights are asked for once the lane's row has landed, and the reduction hides them.  What bounds a row that has a
+// compute unit to itself is that unit's path to the caches, 64 bytes a clock: asked for at once, the weights of its first waves
+// go ahead of the rows of its last, and every wave waits for the last one's squares (one row of 16384 elements: the last wave's
+// loads left 0.79 us after entry, a row's bytes take 0.47).  us, at once / landed, bf16: 40 rows of 7168 elements, dynamic scale,
+// 3.59 / 3.54, 220 4.41 / 4.18, static 4.34 / 3.97, without codes 4.22 / 3.73; 90 of 14336 5.43 / 5.02, 5.27 / 4.77 and 4.79 / 4.29;
+// fp16 40 of 12288 4.26 / 3.98, 4.10 / 3.84 and 3.70 / 3.44.  Which launches take it: see late_weights.
+template <typename T, int NCHUNK, int QUANT, bool EXACT, bool GATED, bool LANDED>
 __global__ void __launch_bounds__(kMaxThreads) __attribute__((amdgpu_waves_per_eu(GATED && NCHUNK <= 4 ? 8 : 4)))
 add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third, const RowArgs rest) {
     Global<const u32x4> *x = global_ptr<const u32x4>(first[0], first[1]), *residual_in = global_ptr<const u32x4>(first[2], first[3]);
@@ -182,11 +188,11 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
             rv[i] = u32x4{0, 0, 0, 0};
         }
     }
+    auto load_weights = [&]() {
 #pragma unroll
-    for (int i = 0; i < NCHUNK; ++i) {
-        const int c = i * nthreads + tid;
-        gv[i] = live[i] ? (gamma - pad)[c] : u32x4{0, 0, 0, 0};
-    }
+        for (int i = 0; i < NCHUNK; ++i) gv[i] = live[i] ? (gamma - pad)[i * nthreads + tid] : u32x4{0, 0, 0, 0};
+    };
+    if constexpr (!LANDED) load_weights();
     // The arguments beyond the preloaded ones are fetched here, behind the row's loads and while those are in flight:
     // left to itself the compiler fetches them where they are first used, after the first barrier, and every wave of
     // the row then waits there for the scalar cache (0.1-0.15 us of a decode-sized call).
@@ -203,6 +209,12 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
     // ---- phase 1: res = rT(x + r), stored once; sum of squares of the *rounded* residual.  Waves in this phase
     // are given issue priority over the arithmetic of phases 2-3 so that their residual stores leave early (+0.4 %).
     __builtin_amdgcn_s_setprio(1);
+    if constexpr (LANDED) {
+#pragma unroll
+        for (int i = 0; i < NCHUNK; ++i) asm volatile("" : "+v"(xv[i]), "+v"(rv[i]));
+        load_weights();
+        __builtin_amdgcn_sched_barrier(0);
+    }
     // (A partial sum takes the squares of no more than two chunks: a row's sum in four chunks per lane is then as close to that in
     // 64 bits as in two, over 1536 rows of 8192 bfloat16 elements 3.9e-8 off in the mean square (4.4e-8 with two sums, two chunks 4.0e-8).)
     constexpr int kSums = NCHUNK >= 4 ? 4 : 2;
@@ -232,9 +244,10 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
     // for, and not in phase 2, where all waves of the row (two on most SIMDs of the only compute unit that a decode row has) issue
     // at once: one row of 16384 elements 4.11 / 4.02 us, 32 of 4096 2.89 / 2.85.  Without codes, whose only chain behind the
     // reduction is a store, it costs as much as it gains (256 rows of 4096 3.10 / 3.16), and four chunks per lane have no registers
-    // for it.
-    constexpr bool kUnpacked = !is_half<T> && NCHUNK <= 2 && QUANT != GPUK_QUANT_NONE;
-    float res[kUnpacked ? NCHUNK : 1][8], weight[kUnpacked ? NCHUNK : 1][8];
+    // for it.  Weights that were asked for late stay packed: a wave that unpacked them there would reach the barrier later (static
+    // scale, 90 rows of 14336 4.85 / 4.77, 133 of 7168 3.64 / 3.62).
+    constexpr bool kUnpacked = !is_half<T> && NCHUNK <= 2 && QUANT != GPUK_QUANT_NONE, kWeightsUnpacked = kUnpacked && !LANDED;
+    float res[kUnpacked ? NCHUNK : 1][8], weight[kWeightsUnpacked ? NCHUNK : 1][8];
     SplitReciprocal rcp{};  // of the scale; `fast`: quotients take the short form
     bool fast = false;
     float lane_sum = ss[0] + ss[1];
@@ -251,14 +264,18 @@ add_rmsnorm_quant_rows(const u32x8 first, const u32x4 second, const u32x2 third,
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     res[i][2 * j] = P::lo(xv[i][j]), res[i][2 * j + 1] = P::hi(xv[i][j]);
-                    weight[i][2 * j] = P::lo(gv[i][j]), weight[i][2 * j + 1] = P::hi(gv[i][j]);
-                    asm volatile("" : "+v"(res[i][2 * j]), "+v"(res[i][2 * j + 1]), "+v"(weight[i][2 * j]), "+v"(weight[i][2 * j + 1]));
+                    asm volatile("" : "+v"(res[i][2 * j]), "+v"(res[i][2 * j + 1]));
+                    if constexpr (kWeightsUnpacked) {
+                        weight[i][2 * j] = P::lo(gv[i][j]), weight[i][2 * j + 1] = P::hi(gv[i][j]);
+                        asm volatile("" : "+v"(weight[i][2 * j]), "+v"(weight[i][2 * j + 1]));
+                    }
                 }
         }
     });
     // element e of the normed chunk i, rT(gamma * rT(res * rstd)), ahead of the last rounding
     const auto unrounded = [&](int i, int e, float rstd) {
-        if constexpr (kUnpacked) return weight[i][e] * P::round(res[i][e] * rstd);
+        if constexpr (kWeightsUnpacked) return weight[i][e] * P::round(res[i][e] * rstd);
+        else if constexpr (kUnpacked) return ((e & 1) ? P::hi(gv[i][e >> 1]) : P::lo(gv[i][e >> 1])) * P::round(res[i][e] * rstd);
         else return 0.f;
     };
     __builtin_amdgcn_s_setprio(0);
@@ -893,6 +910,28 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, 
     return (uint32_t)std::min(ticks, 5000.0);
 }
 
+// Whether a launch of the 16-bit kernel asks for the weights once the row has landed (LANDED, see add_rmsnorm_quant_rows): at most
+// a round of rows, whose waves wait for their own loads and not for other rows', and more of them than short rows have.  us, at
+// once / landed: without a gate, from five waves on, 30 rows of 8192 elements, static, 3.58 / 3.36, 4 of 14336 in half precision 3.62 / 3.29
+// (but not up to 4 rows in bfloat16, whose unpacking then waits with the weights: one of 16384 3.79 / 3.87; static 0.99), 128 of 16384 5.7 / 5.45, 32768 elements (four chunks) 0.98 on average, but not without codes
+// in bfloat16 (14 rows 5.12 / 5.50); four waves and fewer level to 3 % behind, but for
+// 3 and 4 waves of two chunks behind the first layer (361 of 4096 static 3.9 / 3.7, 480 without codes 4.65 / 3.84).  Gated rows
+// have the launch's reads to wait for: nine waves and more of one chunk 0.97, of two chunks in the first layer (131 of 12288
+// 4.87 / 4.61, static 141 4.87 / 4.58, without codes 173 of 14688 5.35 / 5.02) and not behind it (338 of 12288 6.69 / 6.86);
+// without codes, which have the time to be early, three waves and more up to three eighths of a round (379 of 7168 5.44 / 4.75, 597
+// of 4096 4.86 / 4.50, but 537 of 7168 6.27 / 6.36).  Four chunks 1.00 to 1.19 of the time.  More than a round: 1.00 to 1.03 (8192 x
+// 8192 75.6 / 76.7).
+bool late_weights(int64_t tokens, int threads, int nchunk, RowType type, int quant, bool gated) {
+    const int64_t resident = resident_rows(threads, nchunk);
+    if (tokens > resident || nchunk > 4) return false;
+    if (type == RowType::BF16 && quant != GPUK_QUANT_FP8_STATIC && tokens <= 4) return false;
+    const bool wide = threads >= 576;
+    if (nchunk == 4) return !gated && wide && (type == RowType::FP16 || quant != GPUK_QUANT_NONE);
+    if (!gated) return threads >= 320 || (nchunk == 2 && threads >= 192 && 4 * tokens > 5 * kComputeUnits);
+    if (nchunk == 1) return wide;
+    return (wide && tokens <= kComputeUnits) || (quant == GPUK_QUANT_NONE && threads >= 192 && 8 * tokens <= 3 * resident);
+}
+
 // Lanes per row and chunks per lane.  Two chunks per lane on as many lanes as that needs (up to 1024) stream best or tie
 // for 1024 .. 16384 16-bit elements (1-6 % over one or four chunks per lane; 7168 elements, per call: 3.3 us against 3.5
 // with one chunk at one row, 5.0 against 5.6 at 256 rows), but for the small batches named below; longer rows double the chunks per lane.  Where rounding up to
@@ -1108,14 +1147,22 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
     const uint32_t shape = (uint32_t)threads | ((uint32_t)row_group_shift(tokens, hidden * 2) << 16) | (line_mask(threads, nchunk, chunks) << 24);
     const bool exact = (int64_t)threads * nchunk == chunks;
     const RowParameters p = row_parameters(x, residual_in, gamma, residual_out, norm_out, scale, tokens, chunks, shape, gate, hidden, eps, fp8_max);
-#define GPUK_LAUNCH_NQ_AS(N, EXACT, GATED)                                                                              \
-    return launch_kernel(add_rmsnorm_quant_rows<T, N, QUANT, EXACT, GATED>, grid, (uint32_t)threads, 0, stream, p.first, p.second, p.third, p.rest)
+    const bool late = late_weights(tokens, threads, nchunk, row_type<T>, QUANT, gate != 0);
+#define GPUK_LAUNCH_NQ_AS(N, EXACT, GATED, LANDED)                                                                      \
+    return launch_kernel(add_rmsnorm_quant_rows<T, N, QUANT, EXACT, GATED, LANDED>, grid, (uint32_t)threads, 0, stream, p.first, p.second, p.third, p.rest)
+#define GPUK_LAUNCH_NQ_EXACT(N, EXACT)                                                                                 \
+    do {                                                                                                               \
+        if constexpr (N <= 2)                                                                                          \
+            if (gate && late) GPUK_LAUNCH_NQ_AS(N, EXACT, true, true);                                                 \
+        if (gate) GPUK_LAUNCH_NQ_AS(N, EXACT, true, false);                                                            \
+        if constexpr (N <= 4)                                                                                          \
+            if (late) GPUK_LAUNCH_NQ_AS(N, EXACT, false, true);                                                        \
+        GPUK_LAUNCH_NQ_AS(N, EXACT, false, false);                                                                     \
+    } while (0)
 #define GPUK_LAUNCH_NQ(N)                                                                                              \
     do {                                                                                                               \
-        if (exact && gate) GPUK_LAUNCH_NQ_AS(N, true, true);                                                           \
-        else if (exact) GPUK_LAUNCH_NQ_AS(N, true, false);                                                             \
-        else if (gate) GPUK_LAUNCH_NQ_AS(N, false, true);                                                              \
-        else GPUK_LAUNCH_NQ_AS(N, false, false);                                                                       \
+        if (exact) GPUK_LAUNCH_NQ_EXACT(N, true);                                                                      \
+        else GPUK_LAUNCH_NQ_EXACT(N, false);                                                                           \
     } while (0)
     switch (nchunk) {
         case 1: GPUK_LAUNCH_NQ(1); break;
@@ -1125,6 +1172,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
         default: return GPUK_ERR_INTERNAL;
     }
 #undef GPUK_LAUNCH_NQ
+#undef GPUK_LAUNCH_NQ_EXACT
 #undef GPUK_LAUNCH_NQ_AS
 }
 

@@ -190,6 +190,29 @@ def test_shapes_of_small_batches(device, dtype, tokens, hidden):
         check(inp, quant, run_capi(inp, quant, device), tag=f"[{tokens}x{hidden} {dtype} q{quant}]")
 
 
+# (rows that fill their lanes and rows that do not; one, two and four chunks per lane; without a gate, then gated, some only without codes)
+@pytest.mark.parametrize("tokens,hidden", [(1, 5120), (60, 6544), (1, 7168), (40, 7200), (321, 4096), (400, 4000), (9, 32768), (5, 30008),
+                                           (257, 5632), (300, 6000), (130, 12288), (131, 12296), (256, 16384), (379, 7168), (384, 7176)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_weights_asked_for_late(device, dtype, tokens, hidden):
+    """Launches that ask for the weights once the row has landed, at the edges of their rule: the oracle's values, and the same
+    bits where residual_out is one of the inputs (the row is loaded whole before any of it is stored)."""
+    from gpuk_amd import capi
+
+    print(f"case late weights {tokens}x{hidden} {dtype}", flush=True)
+    inp = workloads.norm_quant_inputs(tokens, hidden, seed=tokens + hidden, res_sigma=2.0, outlier_frac=0.01, dtype=dtype)
+    static = torch.tensor([0.03])
+    for quant in (0, 1, 3):
+        got = run_capi(inp, quant, device, static_scale=static)
+        check(inp, quant, got, static_scale=static, tag=f"[{tokens}x{hidden} {dtype} q{quant}]")
+        x, r = inp.x.to(device), inp.residual.to(device)
+        norm = torch.empty_like(got[1])
+        scale = None if quant == 0 else static.to(device) if quant == 3 else torch.empty_like(got[2])
+        capi.add_rmsnorm_quant(x, r, inp.gamma.to(device), x if quant else r, norm, scale, inp.eps, quant, 448.0)
+        for a, b in ((x if quant else r, got[0]), (norm, got[1])):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (tokens, hidden, quant)
+
+
 @pytest.mark.parametrize("threads,nchunk", [(512, 2), (256, 4), (1024, 2), (128, 8), (448, 2), (1024, 1), (1024, 8)])
 def test_launch_shape_variants(device, threads, nchunk):
     """Workgroup size and chunks per lane are tuning choices only."""
