@@ -942,7 +942,8 @@ bool late_weights(int64_t tokens, int threads, int nchunk, RowType type, int qua
 // wave holds with one chunk per lane keep it, a second chunk would be dead in every lane (one / two chunks: 9000 rows of 256
 // elements 5.4 / 6.7 us, 100000 rows 34.8 / 44.6, 20000 of 512 13.5 / 14.3; above 50000 rows of exactly 512 the two-chunk form is
 // 4 % ahead in bfloat16, 150000 rows 90.4 / 86.8, level in half precision).
-void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, int *nchunk) {
+// codes: whether the rows are quantised.
+void pick_shape(int64_t tokens, int chunks_per_row, RowType type, bool codes, int *threads, int *nchunk) {
     const int most_chunks = type == RowType::F32 ? kMaxChunksF32 : kMaxChunks;  // (a forced eight becomes four there)
     auto fits = [&](int n) { return (int64_t)n * kMaxThreads >= chunks_per_row; };
     int n;
@@ -960,11 +961,12 @@ void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, 
             // 5120 3.63 / 3.35, half precision 3.42 / 3.38; fp32 32 of 3072 3.11 / 2.89, 192 3.48 / 3.32).  As the first layer
             // fills, the waves share the units' load paths and only the 5 of bfloat16 still gain (256 of 5120 3.96 / 3.75,
             // without codes level, half precision 3.42 / 3.72, 256 of 5640 4.11 / 4.27); with a second row per unit they gain
-            // again, up to half a layer more (320 of 5640 5.50 / 5.12, 270 of 5120 without codes 4.18 / 3.80), in half precision a
-            // quarter (384 of 5640 without codes 4.88 / 4.98).
+            // again, up to the whole layer (320 of 5640 5.50 / 5.12, 270 of 5120 without codes 4.18 / 3.80, 416 of 6144 static 4.66 /
+            // 4.24, 443 in half precision 5.01 / 4.84, 485 without codes 5.13 / 4.83, 505 of 5120 level).
             // 2 waves of two chunks and 4 of one are one wave a SIMD at most, of half the length: 4 rows of 2048 elements 2.48 /
-            // 2.34, 300 3.39 / 2.81, 640 3.65 / 3.57, without codes 3.21 / 2.95, but 768 without codes 3.25 / 3.43 (fp32 gains less,
-            // 2-4 %, and only for a few rows).
+            // 2.34, 300 3.39 / 2.81, 712 3.81 / 3.66, static 990 3.99 / 3.77, dynamic 1241 5.19 / 5.13; without codes 640 3.21 / 2.95 and,
+            // gated as two chunks are from 1024 on, 932 4.23 / 3.76, but 768 3.25 / 3.43 and 1231 4.26 / 4.34 (fp32 gains less, 2-4 %, and
+            // only for a few rows).
             // Where each of more than half of the units has one row, 3 or 4 full waves of four chunks wait for fewer of each
             // other (us, two / four: 160 rows of 6144 3.91 / 3.73, 256 4.29 / 4.02, without codes 4.00 / 3.60; 200 of 8192 4.49 /
             // 4.31, 256 without codes 4.52 / 4.09; 128 rows of 8192 and 7168 elements level, which idle lanes).
@@ -974,11 +976,12 @@ void pick_shape(int64_t tokens, int chunks_per_row, RowType type, int *threads, 
                 15 * lanes4 < 4 * chunks_per_row) {
                 n = 4;
             } else if (lanes2 == 128) {
-                if (!f32 && 2 * tokens <= 5 * kComputeUnits) n = 1;
+                const bool gated_none = 4 * tokens > 13 * kComputeUnits && tokens <= 4 * kComputeUnits;
+                if (!f32 && (2 * tokens <= 5 * kComputeUnits || (codes ? tokens <= 5 * kComputeUnits : gated_none))) n = 1;
             } else if (lanes2 == 320 || lanes2 == 384) {
                 const bool few = 4 * tokens <= 3 * kComputeUnits;
                 const bool first_layer = tokens <= kComputeUnits && lanes2 == 320 && !f16;
-                const bool second_layer = tokens > kComputeUnits && 4 * tokens <= (f16 ? 5 : 6) * kComputeUnits;
+                const bool second_layer = tokens > kComputeUnits && tokens <= 2 * kComputeUnits;
                 if (few || (!f32 && (first_layer || second_layer))) n = 1;
             }
         }
@@ -1046,7 +1049,7 @@ int launches_for(int64_t tokens, int chunks_per_row, RowType type, bool codes) {
     if (g_pieces == 2) return 2;
     const int64_t piece = tokens - half_of(tokens);  // (the larger one)
     int threads, nchunk;
-    pick_shape(piece, chunks_per_row, type, &threads, &nchunk);
+    pick_shape(piece, chunks_per_row, type, codes, &threads, &nchunk);
     if (nchunk == 1 || piece > resident_rows(threads, nchunk) || chunks_per_row % 8 != 0) return 1;
     const int places = threads * nchunk;
     const bool one_wave = threads == 64, eighth = 8 * chunks_per_row >= 7 * places, fifth = 5 * chunks_per_row >= 4 * places;
@@ -1135,7 +1138,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
                 float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 8);
     int threads, nchunk;
-    pick_shape(tokens, chunks, row_type<T>, &threads, &nchunk);
+    pick_shape(tokens, chunks, row_type<T>, QUANT != GPUK_QUANT_NONE, &threads, &nchunk);
     const dim3 grid((unsigned)tokens);
     if (nchunk == 0) {
         add_rmsnorm_quant_long_rows<T, QUANT><<<grid, kMaxThreads, 0, stream>>>(
@@ -1215,7 +1218,7 @@ int launch_f32_rows(const void *x, const void *residual_in, const void *gamma, v
                     float *scale, int64_t tokens, int64_t hidden, float eps, float fp8_max, hipStream_t stream) {
     const int chunks = (int)(hidden / 4);
     int threads, nchunk;
-    pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
+    pick_shape(tokens, chunks, RowType::F32, QUANT != GPUK_QUANT_NONE, &threads, &nchunk);
     const bool exact = (int64_t)threads * nchunk == chunks;
     const uint32_t gate = f32_store_gate(tokens, hidden, threads, nchunk, QUANT);
     // Weights at once: more than a round, or waves that wait little for each other (see add_rmsnorm_quant_f32_rows).
@@ -1363,7 +1366,7 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
                                                    scale + piece, tokens - piece, hidden, stream);
     }
     int threads, nchunk;
-    pick_shape(tokens, chunks, RowType::BF16, &threads, &nchunk);
+    pick_shape(tokens, chunks, RowType::BF16, true, &threads, &nchunk);
     if (nchunk == 0) return GPUK_ERR_UNSUPPORTED;  // rows that do not stay in registers
     const int group_shift = row_group_shift(tokens, hidden * 2);
     const int remap_end = group_shift > 0 ? (int)((tokens >> (3 + group_shift)) << (3 + group_shift)) : 0;
@@ -1391,7 +1394,7 @@ extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidde
     const bool wide = dtype == GPUK_DTYPE_F32 || dtype == GPUK_DTYPE_F64;
     if (hidden % 8 != 0) return GPUK_ERR_UNSUPPORTED;  // the rule of gpuk_add_rmsnorm_quant, for every dtype
     if (dtype == GPUK_DTYPE_F32 && hidden / 4 <= kMaxChunksF32 * kMaxThreads) {
-        pick_shape(first_piece(tokens, (int)(hidden / 4), RowType::F32), (int)(hidden / 4), RowType::F32, lanes_per_row, chunks_per_lane);
+        pick_shape(first_piece(tokens, (int)(hidden / 4), RowType::F32), (int)(hidden / 4), RowType::F32, true, lanes_per_row, chunks_per_lane);
         return GPUK_OK;
     }
     if (wide) {  // longer fp32 rows and fp64: 4-element chunks, 0 = rows swept three times
@@ -1399,7 +1402,7 @@ extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidde
         return GPUK_OK;
     }
     const RowType type = dtype == GPUK_DTYPE_FP16 ? RowType::FP16 : RowType::BF16;
-    pick_shape(first_piece(tokens, (int)(hidden / 8), type), (int)(hidden / 8), type, lanes_per_row, chunks_per_lane);
+    pick_shape(first_piece(tokens, (int)(hidden / 8), type), (int)(hidden / 8), type, true, lanes_per_row, chunks_per_lane);
     return GPUK_OK;
 }
 
@@ -1415,14 +1418,14 @@ extern "C" int gpuk_add_rmsnorm_quant_store_gate(int64_t tokens, int64_t hidden,
         const int chunks = (int)(hidden / 4);
         if (chunks > kMaxChunksF32 * kMaxThreads) return GPUK_OK;
         tokens = first_piece(tokens, chunks, RowType::F32, quant_mode != GPUK_QUANT_NONE);
-        pick_shape(tokens, chunks, RowType::F32, &threads, &nchunk);
+        pick_shape(tokens, chunks, RowType::F32, quant_mode != GPUK_QUANT_NONE, &threads, &nchunk);
         *ticks = (int)f32_store_gate(tokens, hidden, threads, nchunk, quant_mode);
         return GPUK_OK;
     }
     if (dtype != GPUK_DTYPE_BF16 && dtype != GPUK_DTYPE_FP16) return GPUK_ERR_UNSUPPORTED;
     const RowType type = dtype == GPUK_DTYPE_FP16 ? RowType::FP16 : RowType::BF16;
     tokens = first_piece(tokens, (int)(hidden / 8), type);
-    pick_shape(tokens, (int)(hidden / 8), type, &threads, &nchunk);
+    pick_shape(tokens, (int)(hidden / 8), type, quant_mode != GPUK_QUANT_NONE, &threads, &nchunk);
     if (nchunk) *ticks = (int)store_gate(tokens, hidden * 2, threads, nchunk, type, quant_mode);
     return GPUK_OK;
 }

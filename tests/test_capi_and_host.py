@@ -362,11 +362,11 @@ def test_launch_shape_of_small_batches():
     bf16, f16, f32 = torch.bfloat16, torch.float16, torch.float32
     shape, gate = capi.add_rmsnorm_quant_launch_shape, capi.add_rmsnorm_quant_store_gate
     for hidden, dtype, changes in (
-            (2048, bf16, ((1, 1), (640, 1), (641, 2))), (1544, f16, ((1, 1), (640, 1), (641, 2))), (1536, bf16, ((1, 1), (9, 1))),
+            (2048, bf16, ((1, 1), (1280, 1), (1281, 2))), (1544, f16, ((1, 1), (1280, 1), (1281, 2))), (1536, bf16, ((1, 1), (9, 1))),
             (1024, f32, ((1, 2), (192, 2))), (2056, bf16, ((1, 1), (1200, 1))),
-            (5120, bf16, ((1, 1), (256, 1), (384, 1), (385, 2))), (5120, f16, ((1, 1), (192, 1), (193, 2), (256, 2), (257, 1), (320, 1), (321, 2))),
-            (5640, bf16, ((192, 1), (193, 2), (256, 2), (257, 1), (384, 1), (385, 2))), (2560, f32, ((1, 1), (192, 1), (193, 2), (300, 2))),
-            (6144, f16, ((1, 1), (128, 1), (129, 4), (256, 4), (257, 1), (320, 1), (321, 2))), (6152, bf16, ((1, 1), (200, 1))),
+            (5120, bf16, ((1, 1), (256, 1), (512, 1), (513, 2))), (5120, f16, ((1, 1), (192, 1), (193, 2), (256, 2), (257, 1), (512, 1), (513, 2))),
+            (5640, bf16, ((192, 1), (193, 2), (256, 2), (257, 1), (512, 1), (513, 2))), (2560, f32, ((1, 1), (192, 1), (193, 2), (300, 2))),
+            (6144, f16, ((1, 1), (128, 1), (129, 4), (256, 4), (257, 1), (512, 1), (513, 2))), (6152, bf16, ((1, 1), (200, 1))),
             (8192, bf16, ((1, 2), (128, 2), (129, 4), (256, 4), (257, 2))), (7168, bf16, ((200, 2),)), (7680, bf16, ((200, 1),)), (4096, f32, ((200, 2),))):
         chunks = hidden * (4 if dtype == f32 else 2) // 16
         for tokens, n in changes:
@@ -376,7 +376,8 @@ def test_launch_shape_of_small_batches():
     # precision without codes from a quarter
     for tokens, hidden, dtype, quant, waits in ((3071, 512, bf16, 1, False), (3072, 512, bf16, 1, True), (2048, 512, f16, 0, True), (2047, 512, f16, 0, False),
                                                 (2048, 512, f16, 3, False), (256, 5120, bf16, 1, False), (257, 5120, bf16, 1, True),
-                                                (191, 5632, bf16, 0, False), (192, 5632, bf16, 0, True), (512, 2048, bf16, 1, False)):
+                                                (191, 5632, bf16, 0, False), (192, 5632, bf16, 0, True), (512, 2048, bf16, 1, False), (1280, 2048, bf16, 1, True),
+                                                (832, 2048, bf16, 0, False), (833, 2048, bf16, 0, True), (1024, 2048, bf16, 0, True)):
         assert (gate(tokens, hidden, dtype, quant) > 0) == waits, (tokens, hidden, dtype, quant)
 
 

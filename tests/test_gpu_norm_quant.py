@@ -181,7 +181,7 @@ def test_every_chunking_variant(device, nchunk):
 
 # (rows at the edges of their class of lengths, batches at the edges of their shape)
 @pytest.mark.parametrize("tokens,hidden", [(1, 1544), (640, 2048), (641, 2048), (3, 4616), (256, 5120), (257, 5128), (384, 6144), (129, 8192), (256, 6144),
-                                           (256, 8136), (3071, 512)])
+                                           (256, 8136), (3071, 512), (512, 6144), (1280, 2048), (1024, 2040), (833, 2048)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_shapes_of_small_batches(device, dtype, tokens, hidden):
     print(f"case small batches {tokens}x{hidden} {dtype}", flush=True)
