@@ -1600,29 +1600,63 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // 9.2 / 7.7 at 2048 (5.5 / 5.7 at 1024).  The in-place ops alike: 32+8 heads 5.9 / 5.5 at 1024 tokens, 7.3 / 6.4 at 1400,
     // 8.2 / 7.0 at 1638; 28+4 heads with three axes 6.8 / 6.2 at 1536 tokens, 8.5 / 7.1 at 2048.  Nothing to gain below
     // half a round, 15-35 % slower one unit beyond a round.
-    p.unit_gate = 0;
-    const bool two_thirds = 3 * a.total_units > 2 * kResidentUnits;
-    const bool gated_by_rule = g_unit_gate < 0 && a.total_units <= kResidentUnits &&
-                               (two_thirds || (axes == 1 && !kv_fp8 && a.total_units >= kResidentUnits / 2));
-    const bool fuller = gated_by_rule && two_thirds;
-    if (g_unit_gate > 0) p.unit_gate = (uint32_t)g_unit_gate;
-    else if (gated_by_rule) p.unit_gate = (uint32_t)std::min((fuller ? 1.2 : 1.15) * (double)read_bytes / 70000.0, 5000.0);
+    // Half precision, whose waves are done sooner, gates from three eighths of a round, with an fp8 cache from a half, for any axes,
+    // and opens earlier: at the read time itself below half a round (1.1 times it rotated pairwise) and, rotated by halves with every
+    // lane in use, with an fp8 cache up to two thirds of a round, at 1.1 times it else
+    // (not gated or gated as bfloat16 / so: 690 tokens of 32+8+8 heads 4.77 / 4.4, 981 with interleaved sections 6.23 / 5.3, 247 of
+    // 64+64+64 6.1 / 5.2, in place 995 of 32+8 4.82 / 4.65, an fp8 cache 576 of 64+8+8 5.72 / 5.1; heads of 64,
+    // lanes that idle and many V heads keep 1.2 from two thirds of a round on, 2422 tokens of 16+2+2 5.67 / 6.16, 227 of 64+64+64 heads of
+    // 256 8.4 / 9.3, and pairwise ones 1.15 before it, 340 of
+    // 64+64+64 7.0 / 7.5).  Rotated pairwise in bfloat16 a wave takes longer: 1.3 times from two thirds of a round on (0.96 to 1.00 of the
+    // time over 40 calls, with an fp8 cache level).
+    // Heads of 64 elements in bfloat16 with a 16-bit cache, lanes three quarters full: whole lines (see exchange_lines) behind a
+    // gate, four waves a workgroup, pairwise from 17/32 of a round and by halves from five eighths (1811 tokens of 32+8+8 6.77 /
+    // 5.93, 2550 of 40+8+8 7.84 / 7.45, pairwise 1152 of 64+8+8 7.29 / 6.0; by halves 1590 of 32+8+8 5.41 / 5.70, 16+2+2 5.7 / 5.9,
+    // pairwise 1378 of 32+8+8 5.02 / 5.29).
+    // An fp8 cache with more than a V head for three Q and K heads (but four units a token, 1693 tokens of 16+16+16 8.85 / 9.16) keeps the vector ALUs busy with conversions: a wave that waits
+    // for a gate holds them up, and so do the other waves of its workgroup (gated as above / no gate and single waves from half a
+    // round on: 400 tokens of 64+64+64 in half precision 9.3 / 8.3, 357 pairwise 9.4 / 8.2, 2161 of 12+12+12 9.4 / 8.4, heads of 64 3043
+    // 7.9 / 7.5; bfloat16 369 of 64+64+64 8.4 / 8.0, 303, not gated, 7.2 / 6.8).
     // bytes the call moves: every Q/K/V element in, Q (and K) elements out, the cache rows
     const int64_t elems_qk = (int64_t)a.num_tokens * (a.hq + a.hk) * D, elems_v = (int64_t)a.num_tokens * a.hv * D;
     const int64_t call_bytes = set_kv ? 2 * (elems_qk + elems_v) + 2 * (int64_t)a.num_tokens * a.hq * D +
                                             (kv_fp8 ? 1 : 2) * ((int64_t)a.num_tokens * a.hk * D + elems_v)
                                       : 4 * elems_qk;
     p.stream = g_stream_rows == 2 || (g_stream_rows == 0 && call_bytes >= kStreamFromBytes);
+    p.unit_gate = 0;
+    const int64_t round_8ths = 8 * (int64_t)a.total_units;  // against multiples of kResidentUnits
+    const bool two_thirds = 3 * a.total_units > 2 * kResidentUnits, one_round = a.total_units <= kResidentUnits;
+    const bool gated_lines = D == 64 && set_kv && !kv_fp8 && !half && p.stream && one_round && 4 * heads >= 3 * places &&
+                             4 * round_8ths >= (neox ? 20 : 17) * (int64_t)kResidentUnits;
+    const bool many_v = set_kv && 3 * a.hv > heads, busy = kv_fp8 && many_v && a.units_per_token != 4, no_idle_lane = heads == places;
+    const bool gated_by_rule = g_unit_gate < 0 && one_round && !busy &&
+                               (two_thirds || gated_lines || (half ? !(kv_fp8 && many_v) && round_8ths >= (kv_fp8 ? 4 : 3) * (int64_t)kResidentUnits
+                                                                   : axes == 1 && !kv_fp8 && a.total_units >= kResidentUnits / 2));
+    const bool fuller = gated_by_rule && (two_thirds || gated_lines);
+    double times;  // of the launch's reads at 7 TB/s
+    if (gated_lines) times = neox ? 1.15 : 1.25;
+    else if (two_thirds) times = half && neox && no_idle_lane && !many_v && D != 64 ? 1.1 : !half && !neox && !kv_fp8 ? 1.3 : 1.2;
+    else if (half && 2 * a.total_units < kResidentUnits) times = neox ? 1.0 : 1.1;
+    else times = half && neox && no_idle_lane ? (kv_fp8 ? 1.0 : 1.1) : 1.15;
+    if (g_unit_gate > 0) p.unit_gate = (uint32_t)g_unit_gate;
+    else if (gated_by_rule) p.unit_gate = (uint32_t)std::min(times * (double)read_bytes / 70000.0, 5000.0);
     if (g_stream_rows == 2) p.whole_lines = true;
     else if (half) p.whole_lines = !set_kv || 3 * a.total_units >= kResidentUnits;
     else if (!set_kv) p.whole_lines = 4 * heads >= 3 * places && call_bytes >= (heads == places ? kWholeLinesFromBytes : kWholeLinesFromBytesRagged);
-    else p.whole_lines = (5 * heads >= 4 * places && a.total_units > kResidentUnits) || (4 * heads >= 3 * places && a.total_units > 3 * kResidentUnits);
+    else p.whole_lines = gated_lines || (5 * heads >= 4 * places && a.total_units > kResidentUnits) || (4 * heads >= 3 * places && a.total_units > 3 * kResidentUnits);
     // Workgroup size, swept over 64/128/256/512 lanes and one workgroup per token for 2-9 units per token: four
     // waves where a workgroup then holds whole tokens (its waves share the token's position and table row in the
     // CU's caches: 3-15 % ahead at 28+4 heads) and for large batches (1-3 % ahead from 4096 tokens on), single
     // waves for small batches of other head counts (2-6 % ahead at 64+8 heads with an fp8 cache up to 512 tokens,
-    // within 1-3 % either way for 3, 5 and 6 units per token); 128 lanes is the slowest in most cases.
-    p.threads = g_block_threads ? (uint32_t)g_block_threads : (a.units_per_token % 4 == 0 || a.total_units > 8192 || fuller ? 256u : 64u);
+    // within 1-3 % either way for 3, 5 and 6 units per token); 128 lanes is the slowest in most cases.  In place, without the
+    // scatter, four waves from three eighths of a round (pairwise a half, heads of 64 with idle lanes five eighths): 1028 tokens of
+    // 64+8 heads of 64 6.04 / 5.35 us (but 974 5.01 / 5.27), 2618 of 28+4 pairwise 6.29 / 5.6, 441 of 64+8 heads of 128 4.80 / 4.65,
+    // 995 of 32+8 in half precision 4.82 / 4.56; not pairwise in half precision (1757 of 12+12 5.20 / 5.58) nor
+    // there with idle lanes (905 of 16+2 heads of 256 4.32 / 4.53).
+    const bool four_in_place = !set_kv && (!half || (neox && no_idle_lane)) &&
+                               round_8ths >= (D == 64 && heads != places ? 5 : neox ? 3 : 4) * (int64_t)kResidentUnits;
+    const bool single_waves = busy && one_round && 2 * a.total_units >= kResidentUnits;
+    p.threads = g_block_threads ? (uint32_t)g_block_threads : (!single_waves && (a.units_per_token % 4 == 0 || a.total_units > 8192 || fuller || four_in_place) ? 256u : 64u);
     const uint32_t units_per_block = p.threads / 64;
     p.blocks = (a.total_units + units_per_block - 1) / units_per_block;
     if (p.token_waves) {

@@ -114,3 +114,29 @@ def test_choice_changes_no_bits(device, tokens, heads, D, neox, sections, fp16):
         capi.set_tuning("rope_token_waves", 0)
     for name, a, b in zip(("q_out", "k_cache", "v_cache", "in place"), got, base):
         assert torch.equal(a.cpu().contiguous().view(torch.uint8), b.cpu().contiguous().view(torch.uint8)), f"{name}: the two kernels differ"
+
+
+@pytest.mark.parametrize("tokens,heads,D,neox,fp8,fp16", [
+    (615, (32, 8, 8), 128, True, False, True), (615, (32, 8, 8), 128, False, False, True), (456, (64, 8, 8), 128, True, True, True), (1707, (32, 8, 8), 64, True, False, False),
+    (2177, (28, 4, 4), 64, False, False, False), (257, (64, 64, 64), 128, True, True, False), (1639, (8, 1, 1), 256, True, False, True)])
+def test_gate_and_workgroup_change_no_bits(device, tokens, heads, D, neox, fp8, fp16):
+    """Calls at the lines of the rule for the gate, the lines and the workgroup of the kernel with one wave per group of heads,
+    as it chooses and without a gate in single waves that store through the L2: the same bits, with a cache and in place."""
+    print(f"case gate rule {tokens} {heads} {D} neox={neox} fp8={fp8} fp16={fp16}", flush=True)
+    inp = make(tokens, heads[0], D, neox, seed=tokens + D, fp8=fp8, hk=heads[1], hv=heads[2])
+    if fp16:
+        inp.qkv, inp.qw, inp.kw, inp.cos_sin = (t.to(torch.float16) for t in (inp.qkv, inp.qw, inp.kw, inp.cos_sin))
+        if not fp8:
+            inp.kv_dtype = torch.float16
+    inp.kv_loc[3::13] = -1
+    got = [*run_set_kv(inp, device)[:3], run_inplace(inp, device)]
+    plain = {"rope_token_waves": (1, 0), "rope_unit_gate": (0, -1), "rope_stream_rows": (1, 0), "rope_block_threads": (64, 0)}
+    try:
+        for key, (value, _) in plain.items():
+            capi.set_tuning(key, value)
+        base = [*run_set_kv(inp, device)[:3], run_inplace(inp, device)]
+    finally:
+        for key, (_, rule) in plain.items():
+            capi.set_tuning(key, rule)
+    for name, a, b in zip(("q_out", "k_cache", "v_cache", "in place"), got, base):
+        assert torch.equal(a.cpu().contiguous().view(torch.uint8), b.cpu().contiguous().view(torch.uint8)), f"{name}: the launches differ"
