@@ -338,7 +338,7 @@ __device__ __forceinline__ void store_pair(void *p, const u32x4 &a, const u32x4 
 // With a 16-bit cache: half precision from a third of a round of waves on (28+4+4 3.54 / 3.65 at 907 tokens, 4.6 / 4.2 at 1500;
 // 64+8+8 6.9 / 6.3 at 1500, 17.9 / 15.4 at 4000, 62.3 / 53.1 at 16000, 32+8+8 11.6 / 10.6 and 38.3 / 33.5); bfloat16 beyond one
 // round of waves where units are four fifths full (64+8+8 18.0 / 16.7 and 61.2 / 54.5, 40+8+8 13.4 / 12.9 and 43.3 / 38.5,
-// 32+8+8 12.1 / 11.8 and 37.6 / 34.3, but 5.4 / 6.1 at 1500), beyond three where they are three quarters full (12+12+12 18.2 /
+// 32+8+8 12.1 / 11.8 and 37.6 / 34.3, but 5.4 / 6.1 at 1500; nearer a full round behind a gate, see plan_rope), beyond three where they are three quarters full (12+12+12 18.2 /
 // 18.3 at 9000 tokens, 29.0 / 27.0 at 16000; 16+2+2, of 32 places, 19.2 / 20.8).  An fp8 cache, whose conversions then run on
 // both chunks of every lane, gains 4-6 % with few K heads and loses as much with others (64+8+8 34.8 / 32.8 at 9000 tokens,
 // 32+8+8 36.5 / 37.4 at 16000): not done.
