@@ -1655,7 +1655,11 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // there with idle lanes (905 of 16+2 heads of 256 4.32 / 4.53).
     const bool four_in_place = !set_kv && (!half || (neox && no_idle_lane)) &&
                                round_8ths >= (D == 64 && heads != places ? 5 : neox ? 3 : 4) * (int64_t)kResidentUnits;
-    const bool single_waves = busy && one_round && 2 * a.total_units >= kResidentUnits;
+    // Just beyond a round tokens of three units with a cache, which four waves do not hold whole, are ahead in single waves (20 calls of
+    // 1 to 1.5 rounds 0.90 to 0.995 of the time, level from there: 2966 tokens of 16+2+2 heads, fp8 cache, 8.9 / 8.2, 3166 of 32+8+8 of 64
+    // 10.8 / 9.6, 3481 of 40+8+8 of 64 with a 16-bit cache 12.3 / 11.4; two units 1.05 to 1.1, four 1.06, in place level).
+    const bool three_units = set_kv && a.units_per_token == 3 && !one_round && 2 * (int64_t)a.total_units <= 3 * (int64_t)kResidentUnits;
+    const bool single_waves = three_units || (busy && one_round && 2 * a.total_units >= kResidentUnits);
     p.threads = g_block_threads ? (uint32_t)g_block_threads : (!single_waves && (a.units_per_token % 4 == 0 || a.total_units > 8192 || fuller || four_in_place) ? 256u : 64u);
     const uint32_t units_per_block = p.threads / 64;
     p.blocks = (a.total_units + units_per_block - 1) / units_per_block;

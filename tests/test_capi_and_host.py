@@ -494,7 +494,8 @@ def test_rope_kernel_choice():
 
 def test_rope_workgroups():
     """Lanes per workgroup of the rope kernel with one wave per group of heads: four waves in place from three eighths of a round of
-    waves, in whole lines behind a gate, and single waves where an fp8 cache of many V heads keeps the vector units busy."""
+    waves, in whole lines behind a gate, and single waves where an fp8 cache of many V heads keeps the vector units busy
+    and for tokens of three units just beyond a round."""
     from gpuk_amd import capi
 
     bf16, f16 = torch.bfloat16, torch.float16
@@ -503,5 +504,7 @@ def test_rope_workgroups():
             (1024, (16, 2, 2), 128, f16, False, False, 64), (1023, (64, 8, 8), 64, bf16, False, False, 64), (1024, (64, 8, 8), 64, bf16, False, False, 256),
             (1706, (32, 8, 8), 64, bf16, True, False, 64), (1707, (32, 8, 8), 64, bf16, True, False, 256), (1707, (32, 8, 8), 64, f16, True, False, 64),
             (255, (64, 64, 64), 128, bf16, True, True, 256), (256, (64, 64, 64), 128, bf16, True, True, 64), (512, (64, 64, 64), 128, bf16, True, True, 64),
-            (513, (64, 64, 64), 128, bf16, True, True, 256), (2000, (16, 16, 16), 128, bf16, True, True, 256)):
+            (513, (64, 64, 64), 128, bf16, True, True, 256), (2000, (16, 16, 16), 128, bf16, True, True, 256),
+            (2730, (40, 8, 8), 64, bf16, True, False, 256), (2731, (40, 8, 8), 64, bf16, True, False, 64), (4096, (16, 2, 2), 128, bf16, True, True, 64),
+            (4097, (16, 2, 2), 128, bf16, True, True, 256), (2731, (40, 8, 8), 64, bf16, False, False, 256)):
         assert capi.rope_rms_launch_shape(tokens, *heads, D, 1, dtype, cache, fp8)[1] == lanes, (tokens, heads, D, dtype, cache, fp8)
