@@ -100,7 +100,7 @@ QUANT_FP8_DYNAMIC = 1
 QUANT_FP8_STATIC = 3   # additive: one per-tensor scale, read from scale_out[0]
 
 _is_compiling = torch.compiler.is_compiling
-_is_current_stream_capturing = _direct.current_stream_is_capturing   # capture_: 0.48 us per call with torch's, 0.21 with this
+_is_current_stream_capturing = _direct.current_stream_is_capturing   # (0.30 us by torch's, 0.17 by this)
 
 
 class GPUKDistEnv:

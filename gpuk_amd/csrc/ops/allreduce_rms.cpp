@@ -19,10 +19,8 @@ std::atomic<double> g_fp8_max{448.0};
 }  // namespace
 
 bool current_stream_is_capturing() {
-    hipStream_t stream = static_cast<hipStream_t>(current_stream());
-    if (!stream) return false;
     hipStreamCaptureStatus status{};
-    C10_HIP_CHECK(hipStreamIsCapturing(stream, &status));
+    C10_HIP_CHECK(hipStreamIsCapturing(static_cast<hipStream_t>(current_stream()), &status));
     return status != hipStreamCaptureStatusNone;
 }
 

@@ -26,8 +26,8 @@ using DeviceGuard = c10::hip::HIPGuardMasqueradingAsCUDA;
 // The stream torch would launch on for the device that is current under the caller's guard.
 inline void *current_stream() { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
 
-// Whether that stream is being captured.  The null stream, on which torch works unless told otherwise, cannot be: the runtime, which
-// takes 0.2 us to answer, is asked about others only.
+// Whether that stream is being captured.  The null stream cannot be, but the runtime is asked about it too: while a stream that
+// blocks it is captured the answer is an error, and a caller that synchronises where nothing is captured has to hear that.
 bool current_stream_is_capturing();
 
 inline int activation_dtype(const Tensor &t, const char *op) {

@@ -325,3 +325,34 @@ def test_capture_status(device):
         assert ask() is torchs() is True
         buf.add_(1)
     assert ask() is torchs() is False
+
+
+@pytest.mark.gpu
+def test_capture_status_beside_a_captured_blocking_stream(device):
+    """While a stream that blocks the null stream is captured, the runtime refuses to say that the null stream is not: the query and
+    the env's call, which synchronises the device after a capture, pass that on as torch's query does."""
+    import ctypes
+
+    hip = ctypes.CDLL("libamdhip64.so")
+    env = gpuk.GPUKDistEnv(device_id=torch.cuda.current_device())
+    x = torch.randn(4, 1024, device=device).bfloat16()
+    args = (x, x.clone(), torch.ones(1024, device=device, dtype=x.dtype), 1e-6)
+    want = env.allreduce_add_rms_fused(*args, fp8_out=True)
+    torch.cuda.synchronize()
+    stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 0) == 0
+    try:
+        assert hip.hipStreamBeginCapture(stream, 1) == 0      # thread-local mode
+        try:
+            for ask in (torch.cuda.is_current_stream_capturing, gpuk._direct.current_stream_is_capturing, lambda: env.allreduce_add_rms_fused(*args, fp8_out=True)):
+                with pytest.raises(RuntimeError, match="legacy stream"):
+                    ask()
+        finally:
+            assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+            if graph:
+                hip.hipGraphDestroy(graph)
+    finally:
+        torch.cuda.synchronize()
+        assert hip.hipStreamDestroy(stream) == 0
+    for a, b in zip(env.allreduce_add_rms_fused(*args, fp8_out=True), want):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
