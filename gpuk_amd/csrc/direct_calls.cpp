@@ -13,7 +13,6 @@
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
-#include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 
 #include <optional>
@@ -109,25 +108,8 @@ struct Call<F> {
         if (!handle) handle = c10::Dispatcher::singleton().findSchemaOrThrow(name, overload).template typed<R(A...)>();
     }
 
-    // Whether the call can start below autograd: nothing asks for a gradient, and no transform or mode is at work on the thread or
-    // on a tensor.  For the operator that returns tensors and has no derivative; torch's answer to that would collect the
-    // arguments on a stack and take them apart again to find that out (with the outputs allocated directly, a small call 5.3 / 4.8 us).
     template <size_t... I>
-    static bool starts_below_autograd(const std::tuple<Argument<A>...> &args, std::index_sequence<I...>) {
-        if (!(c10::impl::tls_local_dispatch_key_set().included_ == c10::default_included_set)) return false;
-        const bool grad_mode = c10::GradMode::is_enabled();
-        const auto plain = [&](const auto &argument) {
-            if constexpr (std::is_same_v<std::decay_t<decltype(argument.value)>, at::Tensor>) {
-                const uint64_t keys = c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::ADInplaceOrView}).raw_repr();
-                return (argument.value.key_set().raw_repr() & ~keys) == 0 && !(grad_mode && argument.value.requires_grad());
-            }
-            return true;
-        };
-        return (plain(std::get<I>(args)) && ...);
-    }
-
-    template <size_t... I>
-    static PyObject *run(std::tuple<Argument<A>...> &args, std::index_sequence<I...> each) {
+    static PyObject *run(std::tuple<Argument<A>...> &args, std::index_sequence<I...>) {
         HANDLE_TH_ERRORS
         if constexpr (std::is_void_v<R>) {
             {
@@ -143,10 +125,6 @@ struct Call<F> {
                     // GPUKDistEnv.allreduce_add_rms_fused expect; reshaped from Python it cost as much as an allocation)
                     auto [residual_out, norm_out] = handle->call(std::get<I>(args).pass()...);
                     return std::make_tuple(std::move(residual_out), std::move(norm_out), std::get<4>(args).value.reshape({1}));
-                } else if constexpr (same_function<F, &gpuk_ops::fused_rope_rms_2way>) {
-                    if (!starts_below_autograd(args, each)) return handle->call(std::get<I>(args).pass()...);
-                    at::AutoDispatchBelowAutograd below;
-                    return handle->call(std::get<I>(args).pass()...);
                 } else {
                     return handle->call(std::get<I>(args).pass()...);
                 }

@@ -6,6 +6,7 @@ import types
 import pytest
 import torch
 from torch._subclasses import FakeTensorMode
+from torch.autograd import forward_ad
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
@@ -238,10 +239,10 @@ def test_vmap_compile_and_profiler():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("around", ["plain", "parameter", "parameter, no_grad", "inference", "dispatch mode", "functions mode", "vmap", "grad", "profiler", "fake"])
+@pytest.mark.parametrize("around", ["plain", "parameter", "parameter, no_grad", "inference", "dispatch mode", "functions mode", "vmap", "grad", "profiler", "fake", "dual", "jvp", "hooks", "autocast"])
 def test_two_streams_on_the_gpu_around_autograd(device, around):
-    """The direct call starts below autograd where nothing asks for a gradient and no transform or mode is at work: outputs, their
-    place in a graph and what a mode or a profiler sees are the general call's."""
+    """The operator returns tensors and has no derivative: outputs, their place in a graph, their tangents and what a mode, a
+    profiler or saved-tensor hooks see are the general call's."""
     packet = gpuk.fused_rope_rms_2way
     gen = torch.Generator().manual_seed(3)
     args = tuple(torch.randn(a.shape, generator=gen).bfloat16().to(device) if torch.is_tensor(a) else a for a in two_way("cpu"))
@@ -274,6 +275,19 @@ def test_two_streams_on_the_gpu_around_autograd(device, around):
             return torch.vmap(lambda q0: f(q0, *args[1:]))(torch.stack([args[0], args[0]]))
         if around == "grad":
             return torch.func.grad_and_value(lambda w: f(*args[:4], w, *args[5:])[0].float().sum())(args[4].float().bfloat16())
+        if around == "dual":
+            with forward_ad.dual_level():
+                out = f(forward_ad.make_dual(args[0], torch.ones_like(args[0])), *args[1:])
+                assert all(forward_ad.unpack_dual(t).tangent is None for t in out)
+                return out
+        if around == "jvp":
+            return torch.func.jvp(lambda q0: f(q0, *args[1:]), (args[0],), (torch.ones_like(args[0]),))[0]
+        if around == "hooks":
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append("saved") or t, lambda t: t):
+                return f(*args[:4], args[4].clone().requires_grad_(), *args[5:])
+        if around == "autocast":
+            with torch.autocast("cuda", dtype=torch.float16):
+                return f(*args)
         if around == "profiler":
             with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
                 out = f(*args)
@@ -300,7 +314,7 @@ def test_two_streams_on_the_gpu_around_autograd(device, around):
 
 @pytest.mark.parametrize("name", [n for n in NAMES if "2way" not in n])
 def test_in_place_operators_with_parameters(name):
-    """They return nothing a graph could hold: weights that are parameters change nothing, with gradients asked for or not."""
+    """They return nothing a graph could hold: weights that are parameters or duals change nothing, with gradients asked for or not."""
     direct, packet = both(name)
     args = [a.requires_grad_() if torch.is_tensor(a) and a.dim() == 1 and a.is_floating_point() else a for a in arguments(name, "cpu")]
     with recorded() as calls:
@@ -308,7 +322,11 @@ def test_in_place_operators_with_parameters(name):
             assert f(*args) is None
             with torch.no_grad():
                 assert f(*args) is None
-    assert len(calls) == 4 and all(c == calls[0] for c in calls)
+        with forward_ad.dual_level():
+            duals = [forward_ad.make_dual(a.detach(), torch.ones_like(a)) if torch.is_tensor(a) and a.requires_grad else a for a in args]
+            for f in (direct, packet):
+                assert f(*duals) is None
+    assert len(calls) == 6 and all(c == calls[0] for c in calls[:4]) and calls[4] == calls[5]
     assert all(not torch.is_tensor(a) or a.grad_fn is None for a in args)
 
 
