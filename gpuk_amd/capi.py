@@ -15,7 +15,7 @@ _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "lib
 
 EXPORTS = ("gpuk_status_string", "gpuk_abi_version", "gpuk_add_rmsnorm_quant", "gpuk_rope_rms",
            "gpuk_rope_rms_set_kv", "gpuk_rope_rms_2way", "gpuk_copy_bytes", "gpuk_increment_floats", "gpuk_set_tuning",
-           "gpuk_add_rmsnorm_quant_traffic_only", "gpuk_add_rmsnorm_quant_launch_shape",
+           "gpuk_add_rmsnorm_quant_traffic_only", "gpuk_add_rmsnorm_quant_launch_shape", "gpuk_add_rmsnorm_quant_launch_shape_of",
            "gpuk_add_rmsnorm_quant_store_gate", "gpuk_rope_rms_launch_shape", "gpuk_read_bytes", "gpuk_fill_bytes", "gpuk_empty_grid")
 
 DTYPE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2, torch.float64: 3}
@@ -67,6 +67,8 @@ def lib():
         L.gpuk_add_rmsnorm_quant_traffic_only.argtypes = [C.c_void_p] * 5 + [C.c_int64, C.c_int64, C.c_void_p]
         L.gpuk_add_rmsnorm_quant_launch_shape.restype = C.c_int
         L.gpuk_add_rmsnorm_quant_launch_shape.argtypes = [C.c_int64, C.c_int64, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]
+        L.gpuk_add_rmsnorm_quant_launch_shape_of.restype = C.c_int
+        L.gpuk_add_rmsnorm_quant_launch_shape_of.argtypes = [C.c_int64, C.c_int64, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]
         L.gpuk_add_rmsnorm_quant_store_gate.restype = C.c_int
         L.gpuk_add_rmsnorm_quant_store_gate.argtypes = [C.c_int64, C.c_int64, C.c_int, C.c_int, C.POINTER(C.c_int)]
         L.gpuk_rope_rms_launch_shape.restype = C.c_int
@@ -117,12 +119,12 @@ def add_rmsnorm_quant_traffic_only(x, residual_in, residual_out, codes, scale, s
         raise GpukError(rc, "gpuk_add_rmsnorm_quant_traffic_only")
 
 
-def add_rmsnorm_quant_launch_shape(tokens: int, hidden: int, dtype=torch.bfloat16):
+def add_rmsnorm_quant_launch_shape(tokens: int, hidden: int, dtype=torch.bfloat16, quant: int = QUANT_FP8_DYNAMIC):
     """(lanes per row, 16-byte chunks per lane) of the launch gpuk_add_rmsnorm_quant makes for this batch."""
     lanes, chunks = C.c_int(0), C.c_int(0)
-    rc = lib().gpuk_add_rmsnorm_quant_launch_shape(tokens, hidden, DTYPE[dtype], C.byref(lanes), C.byref(chunks))
+    rc = lib().gpuk_add_rmsnorm_quant_launch_shape_of(tokens, hidden, DTYPE[dtype], quant, C.byref(lanes), C.byref(chunks))
     if rc:
-        raise GpukError(rc, "gpuk_add_rmsnorm_quant_launch_shape")
+        raise GpukError(rc, "gpuk_add_rmsnorm_quant_launch_shape_of")
     return lanes.value, chunks.value
 
 

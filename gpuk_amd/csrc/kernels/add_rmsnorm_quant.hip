@@ -1386,15 +1386,17 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
     return hip_status(hipGetLastError());
 }
 
-extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidden, int dtype, int *lanes_per_row,
-                                                   int *chunks_per_lane) {
+extern "C" int gpuk_add_rmsnorm_quant_launch_shape_of(int64_t tokens, int64_t hidden, int dtype, int quant_mode, int *lanes_per_row,
+                                                      int *chunks_per_lane) {
     using namespace gpuk;
     if (tokens <= 0 || hidden <= 0 || !lanes_per_row || !chunks_per_lane) return GPUK_ERR_INVALID_ARG;
     if (dtype != GPUK_DTYPE_BF16 && dtype != GPUK_DTYPE_FP16 && dtype != GPUK_DTYPE_F32 && dtype != GPUK_DTYPE_F64) return GPUK_ERR_UNSUPPORTED;
-    const bool wide = dtype == GPUK_DTYPE_F32 || dtype == GPUK_DTYPE_F64;
+    if (quant_mode != GPUK_QUANT_NONE && quant_mode != GPUK_QUANT_FP8_DYNAMIC && quant_mode != GPUK_QUANT_FP8_STATIC) return GPUK_ERR_UNSUPPORTED;
+    const bool wide = dtype == GPUK_DTYPE_F32 || dtype == GPUK_DTYPE_F64, codes = quant_mode != GPUK_QUANT_NONE;
     if (hidden % 8 != 0) return GPUK_ERR_UNSUPPORTED;  // the rule of gpuk_add_rmsnorm_quant, for every dtype
     if (dtype == GPUK_DTYPE_F32 && hidden / 4 <= kMaxChunksF32 * kMaxThreads) {
-        pick_shape(first_piece(tokens, (int)(hidden / 4), RowType::F32), (int)(hidden / 4), RowType::F32, true, lanes_per_row, chunks_per_lane);
+        const int chunks = (int)(hidden / 4);
+        pick_shape(first_piece(tokens, chunks, RowType::F32, codes), chunks, RowType::F32, codes, lanes_per_row, chunks_per_lane);
         return GPUK_OK;
     }
     if (wide) {  // longer fp32 rows and fp64: 4-element chunks, 0 = rows swept three times
@@ -1402,8 +1404,12 @@ extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidde
         return GPUK_OK;
     }
     const RowType type = dtype == GPUK_DTYPE_FP16 ? RowType::FP16 : RowType::BF16;
-    pick_shape(first_piece(tokens, (int)(hidden / 8), type), (int)(hidden / 8), type, true, lanes_per_row, chunks_per_lane);
+    pick_shape(first_piece(tokens, (int)(hidden / 8), type), (int)(hidden / 8), type, codes, lanes_per_row, chunks_per_lane);
     return GPUK_OK;
+}
+
+extern "C" int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidden, int dtype, int *lanes_per_row, int *chunks_per_lane) {
+    return gpuk_add_rmsnorm_quant_launch_shape_of(tokens, hidden, dtype, GPUK_QUANT_FP8_DYNAMIC, lanes_per_row, chunks_per_lane);
 }
 
 extern "C" int gpuk_add_rmsnorm_quant_store_gate(int64_t tokens, int64_t hidden, int dtype, int quant_mode, int *ticks) {

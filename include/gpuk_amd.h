@@ -192,11 +192,14 @@ int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *residual_in, 
 /*
  * The launch shape gpuk_add_rmsnorm_quant picks for a batch: lanes per token row (= workgroup size; one workgroup
  * per row) and chunks per lane (8 elements of a 16-bit type, 4 of fp32 / fp64; 0: rows too long for registers, swept
- * three times); of a batch that runs as two launches, the first one's.  A quantised call's: without codes a few
- * batches of short rows are given another.  For reports.
+ * three times); of a batch that runs as two launches, the first one's.  The first form answers for a quantised call,
+ * the second for one of the quantisation mode it is given (without codes a few batches of short rows, and fp32
+ * batches that run as two launches, differ).  For reports.
  */
 int gpuk_add_rmsnorm_quant_launch_shape(int64_t tokens, int64_t hidden, int dtype, int *lanes_per_row,
                                         int *chunks_per_lane);
+int gpuk_add_rmsnorm_quant_launch_shape_of(int64_t tokens, int64_t hidden, int dtype, int quant_mode, int *lanes_per_row,
+                                           int *chunks_per_lane);
 
 /*
  * How long the waves of that launch hold their stores back, in ticks of 10 ns after each wave's entry; 0 where they do not (see

@@ -312,6 +312,30 @@ def test_launch_shape_report():
     assert L.gpuk_add_rmsnorm_quant_launch_shape(4, 1024, 7, C.byref(a), C.byref(b)) == 2
 
 
+def test_launch_shape_report_by_mode():
+    """The shape of a call without codes is its own: rows of two waves of two chunks take one chunk per lane up to 640 of them and
+    from 833 to 1024, where quantised ones do up to 1280; fp32 batches of two launches are cut by the rows' own rule."""
+    from gpuk_amd import capi
+
+    shape, bf16, f16, f32 = capi.add_rmsnorm_quant_launch_shape, torch.bfloat16, torch.float16, torch.float32
+    for dtype in (bf16, f16):
+        for tokens, quantised, plain in ((640, 1, 1), (641, 1, 2), (832, 1, 2), (833, 1, 1), (1024, 1, 1), (1025, 1, 2), (1280, 1, 2), (1281, 2, 2)):
+            lanes = lambda n: (128 * 2 // n, n)
+            for quant, n in ((0, plain), (1, quantised), (3, quantised)):
+                assert shape(tokens, 2048, dtype, quant) == lanes(n), (tokens, quant, dtype)
+    # wide fp32 rows: two launches from 88 to 90 % of the pieces' layers without codes, from 92 to 96 % with them
+    assert shape(1408, 5120, f32, 0) == (320, 4) and shape(1408, 5120, f32, 1) == (640, 2)
+    assert shape(2306, 4096, f32, 0) == (256, 4) and shape(2306, 4096, f32, 1) == (512, 2)
+    assert shape(64, 4096, torch.float64, 0) == shape(64, 4096, torch.float64, 1)
+    L = capi.lib()
+    a, b = ctypes.c_int(0), ctypes.c_int(0)
+    refs = ctypes.byref(a), ctypes.byref(b)
+    assert L.gpuk_add_rmsnorm_quant_launch_shape(700, 2048, 0, *refs) == 0 and (a.value, b.value) == shape(700, 2048)   # a quantised call's
+    assert L.gpuk_add_rmsnorm_quant_launch_shape_of(700, 2048, 0, 2, *refs) == 2    # e4m3fnuz is refused
+    assert L.gpuk_add_rmsnorm_quant_launch_shape_of(700, 2048, 7, 0, *refs) == 2
+    assert L.gpuk_add_rmsnorm_quant_launch_shape_of(0, 2048, 0, 0, *refs) == 1
+
+
 def test_store_gate_report():
     """gpuk_add_rmsnorm_quant_store_gate: a layer of rows, one per compute unit, that has just begun counts for most of a full one,
     but only behind a full one; up to 256 rows wait for their own share of the reads (no GPU needed)."""
