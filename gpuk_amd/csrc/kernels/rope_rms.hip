@@ -1817,6 +1817,21 @@ void build_axis_bitmaps(const int64_t *section, bool interleaved, int half, uint
     }
 }
 
+// The axis maps of a call with three position axes, and whether the sections split at multiples of 8 frequencies, so that a lane's
+// piece of the table comes whole from one row.
+int set_sections(RopeArgs &a, const int64_t *section, int interleaved, int64_t D) {
+    if (!section) return GPUK_ERR_INVALID_ARG;
+    if (section[0] < 0 || section[1] < 0 || section[2] < 0 || section[0] + section[1] + section[2] != D / 2) return GPUK_ERR_INVALID_ARG;
+    build_axis_bitmaps(section, interleaved != 0, (int)(D / 2), a.axis1, a.axis2);
+    a.merge_rows = 1;
+    for (int f = 0; f < D / 2; f += 8) {
+        const uint32_t g1 = (a.axis1[f >> 5] >> (f & 31)) & 0xffu, g2 = (a.axis2[f >> 5] >> (f & 31)) & 0xffu;
+        if ((g1 != 0 && g1 != 0xffu) || (g2 != 0 && g2 != 0xffu)) a.merge_rows = 0;
+    }
+    if (g_merge_rows == 1) a.merge_rows = 0;
+    return GPUK_OK;
+}
+
 // Waves per token of the fp32 / fp64 kernel: 512/D consecutive Q/K heads each, then 128 chunks of the V row each.
 int64_t wide_units_per_token(int64_t hq, int64_t hk, int64_t hv, int64_t D, bool set_kv) {
     const int64_t hpw = 512 / D, v_chunks = set_kv ? hv * (D / 4) : 0;
@@ -1836,16 +1851,8 @@ int rope_common(const void *qkv_in, void *qkv_out, const void *qw, const void *k
     if (hq > 0x7fffff || hk > 0x7fffff || hv > 0x7fffff) return GPUK_ERR_UNSUPPORTED;
     RopeArgs a{};
     if (n_axes == 3) {
-        if (!section) return GPUK_ERR_INVALID_ARG;
-        if (section[0] < 0 || section[1] < 0 || section[2] < 0 || section[0] + section[1] + section[2] != D / 2)
-            return GPUK_ERR_INVALID_ARG;
-        build_axis_bitmaps(section, interleaved != 0, (int)(D / 2), a.axis1, a.axis2);
-        a.merge_rows = 1;
-        for (int f = 0; f < D / 2; f += 8) {
-            const uint32_t g1 = (a.axis1[f >> 5] >> (f & 31)) & 0xffu, g2 = (a.axis2[f >> 5] >> (f & 31)) & 0xffu;
-            if ((g1 != 0 && g1 != 0xffu) || (g2 != 0 && g2 != 0xffu)) a.merge_rows = 0;
-        }
-        if (g_merge_rows == 1) a.merge_rows = 0;
+        const int rc = set_sections(a, section, interleaved, D);
+        if (rc != GPUK_OK) return rc;
     }
     if (T == 0 || hq + hk + (set_kv ? hv : 0) == 0) return GPUK_OK;
     if (!qkv_in || !qw || !kw || !cos_sin || !positions) return GPUK_ERR_INVALID_ARG;
@@ -1894,8 +1901,9 @@ int rope_common(const void *qkv_in, void *qkv_out, const void *qw, const void *k
     return launch_head_size<FP16>(a, D, neox != 0, n_axes, set_kv, kv_fp8, s);
 }
 
+// section: nullptr for sections that split at multiples of 8 frequencies.
 int rope_launch_shape(int64_t T, int64_t hq, int64_t hk, int64_t hv, int64_t D, int n_axes, int dtype, bool set_kv,
-                      int kv_dtype, int *workgroups, int *lanes, int *streamed, int *token_waves) {
+                      int kv_dtype, bool neox, const int64_t *section, int interleaved, int *workgroups, int *lanes, int *streamed, int *token_waves) {
     if (T <= 0 || hq < 0 || hk < 0 || hv < 0 || hq + hk == 0 || (n_axes != 1 && n_axes != 3)) return GPUK_ERR_INVALID_ARG;
     if (D != 64 && D != 128 && D != 256) return GPUK_ERR_UNSUPPORTED;
     if (!workgroups || !lanes || !streamed || !token_waves) return GPUK_ERR_INVALID_ARG;
@@ -1912,14 +1920,18 @@ int rope_launch_shape(int64_t T, int64_t hq, int64_t hk, int64_t hv, int64_t D, 
     a.hq = (int)hq;
     a.hk = (int)hk;
     a.hv = (int)hv;
-    a.merge_rows = g_merge_rows == 1 ? 0u : 1u;  // (three axes: the answer is for sections that split at multiples of 8 frequencies)
+    a.merge_rows = g_merge_rows == 1 ? 0u : 1u;
+    if (n_axes == 3 && section) {
+        const int rc = set_sections(a, section, interleaved, D);
+        if (rc != GPUK_OK) return rc;
+    }
     if (wide) {
         *workgroups = (int)((a.total_units + 3) / 4);
         *lanes = 256;
         *streamed = 1;  // the fp32 / fp64 kernel always stores its rotated rows past the L2
         return GPUK_OK;
     }
-    const RopePlan p = plan_rope(a, (int)D, n_axes, true, set_kv, set_kv && kv_dtype == GPUK_KV_E4M3FN, dtype == GPUK_DTYPE_FP16);
+    const RopePlan p = plan_rope(a, (int)D, n_axes, neox, set_kv, set_kv && kv_dtype == GPUK_KV_E4M3FN, dtype == GPUK_DTYPE_FP16);
     *workgroups = (int)p.blocks;
     *lanes = (int)p.threads;
     *streamed = p.stream ? 1 : 0;
@@ -1944,12 +1956,20 @@ void set_rope_tuning(int key, int value) {
 // profiling build: where the kernels of this file write their phase stamps
 GPUK_STAMPS_SETTER(gpuk_stamps_set_rope)
 
+extern "C" int gpuk_rope_rms_launch_shape_of(int64_t num_tokens, int64_t num_heads_q, int64_t num_heads_k, int64_t num_heads_v,
+                                             int64_t head_size, int n_axes, int dtype, int set_kv, int kv_dtype, int is_neox_style,
+                                             const int64_t *mrope_section, int is_interleaved, int *workgroups,
+                                             int *lanes_per_workgroup, int *streamed, int *token_waves) {
+    return gpuk::rope_launch_shape(num_tokens, num_heads_q, num_heads_k, num_heads_v, head_size, n_axes, dtype, set_kv != 0, kv_dtype,
+                                   is_neox_style != 0, mrope_section, is_interleaved, workgroups, lanes_per_workgroup, streamed, token_waves);
+}
+
 extern "C" int gpuk_rope_rms_launch_shape(int64_t num_tokens, int64_t num_heads_q, int64_t num_heads_k,
                                           int64_t num_heads_v, int64_t head_size, int n_axes, int dtype, int set_kv,
                                           int kv_dtype, int *workgroups, int *lanes_per_workgroup,
                                           int *streamed, int *token_waves) {
-    return gpuk::rope_launch_shape(num_tokens, num_heads_q, num_heads_k, num_heads_v, head_size, n_axes, dtype,
-                                   set_kv != 0, kv_dtype, workgroups, lanes_per_workgroup, streamed, token_waves);
+    return gpuk::rope_launch_shape(num_tokens, num_heads_q, num_heads_k, num_heads_v, head_size, n_axes, dtype, set_kv != 0, kv_dtype,
+                                   true, nullptr, 0, workgroups, lanes_per_workgroup, streamed, token_waves);
 }
 
 extern "C" int gpuk_rope_rms(void *qkv, const void *qw, const void *kw, const void *cos_sin, const int64_t *positions,

@@ -212,14 +212,18 @@ int gpuk_add_rmsnorm_quant_store_gate(int64_t tokens, int64_t hidden, int dtype,
  * workgroups x lanes per workgroup; *streamed = 1 when the rotated rows are stored past the L2; *token_waves = 1 for
  * the kernel in which a wave of 64 lanes takes a whole token or one of several parts of it (batches the chip holds in
  * one round), 2 where it takes two, the second through LDS, 0 for the kernel in which a wave takes a group of heads of a
- * token.  Computed on the host from the sizes and the tuning keys (with three position axes for sections that split at
- * multiples of 8 frequencies, and for NeoX-style rotation: a call of another kind may be launched otherwise); the four
- * outputs are host pointers.  For reports.  Not part of the
- * reference.
+ * token.  Computed on the host from the sizes and the tuning keys; the four outputs are host pointers.  The first form
+ * answers for NeoX-style rotation and, with three position axes, sections that split at multiples of 8 frequencies; the
+ * second for the rotation and the sections (3 host values, NULL as the first form) that it is given.  For reports.  Not
+ * part of the reference.
  */
 int gpuk_rope_rms_launch_shape(int64_t num_tokens, int64_t num_heads_q, int64_t num_heads_k, int64_t num_heads_v,
                                int64_t head_size, int n_axes, int dtype, int set_kv, int kv_dtype, int *workgroups,
                                int *lanes_per_workgroup, int *streamed, int *token_waves);
+int gpuk_rope_rms_launch_shape_of(int64_t num_tokens, int64_t num_heads_q, int64_t num_heads_k, int64_t num_heads_v,
+                                  int64_t head_size, int n_axes, int dtype, int set_kv, int kv_dtype, int is_neox_style,
+                                  const int64_t *mrope_section, int is_interleaved, int *workgroups,
+                                  int *lanes_per_workgroup, int *streamed, int *token_waves);
 
 /*
  * Launch-cost calibration: data[i] += 1 for i in [0, n) (data 16-byte aligned).  With a small n the call costs

@@ -487,6 +487,29 @@ def test_rope_launch_shape_report():
     assert L.gpuk_rope_rms_launch_shape(4, 32, 8, 8, 128, 1, 9, 1, 0, *refs) == 2   # no such dtype
 
 
+def test_rope_launch_shape_report_of_rotation_and_sections():
+    """The report answers for the rotation and the sections it is given: the kernel's choice depends on both."""
+    from gpuk_amd import capi
+
+    shape = lambda T, **kw: capi.rope_rms_launch_shape(T, 28, 4, 4, 128, 3, **kw)
+    assert shape(4608) == shape(4608, mrope_section=[16, 24, 24]) and shape(4608)[3] == 2
+    assert shape(2400, is_neox=False) == shape(2400) and shape(2400)[3] == 0              # whole tokens of four: from five quarters of a round
+    assert shape(2400, mrope_section=[24, 20, 20], is_interleaved=True)[3] == 1           # three table rows: from nine eighths
+    assert capi.rope_rms_launch_shape(1850, 64, 64, 64, 64, is_neox=False)[1] == 256
+    # in place, parts of a token: a form for rotation by halves only
+    assert capi.rope_rms_launch_shape(1536, 40, 8, 8, 128, set_kv=False)[3] == 1
+    assert capi.rope_rms_launch_shape(1536, 40, 8, 8, 128, set_kv=False, is_neox=False)[3] == 0
+    L = capi.lib()
+    outs = [ctypes.c_int(0) for _ in range(4)]
+    refs = [ctypes.byref(o) for o in outs]
+    bad = (ctypes.c_int64 * 3)(16, 24, 23)
+    assert L.gpuk_rope_rms_launch_shape_of(64, 28, 4, 4, 128, 3, 0, 1, 0, 1, bad, 0, *refs) == 1   # sections that do not fill a head
+    assert L.gpuk_rope_rms_launch_shape_of(64, 28, 4, 4, 128, 1, 0, 1, 0, 1, bad, 0, *refs) == 0   # (one axis: not looked at)
+    for T in (64, 1400, 4096, 8192):
+        assert L.gpuk_rope_rms_launch_shape(T, 28, 4, 4, 128, 3, 0, 1, 0, *refs) == 0
+        assert (outs[0].value, outs[1].value, bool(outs[2].value), outs[3].value) == shape(T)
+
+
 def test_rope_kernel_choice():
     """Which calls the kernel with one wave per token or part of one takes (1: one item per wave, 2: two), from both sides of
     the lines of its rule, rotation by halves."""
