@@ -1376,7 +1376,9 @@ extern "C" int gpuk_add_rmsnorm_quant_traffic_only(const void *x, const void *re
     auto co = static_cast<u32x2 *>(codes);
     const dim3 grid((unsigned)tokens);
     const uint32_t gate = store_gate(tokens, hidden * 2, threads, nchunk, RowType::BF16, GPUK_QUANT_FP8_DYNAMIC);
-    const uint32_t shape = (uint32_t)threads | ((uint32_t)group_shift << 16) | (line_mask(threads, nchunk, chunks) << 24);
+    // (one chunk per lane without a gate: the operator's rows start at lane 0)
+    const uint32_t mask = nchunk == 1 && gate == 0 ? 0u : line_mask(threads, nchunk, chunks);
+    const uint32_t shape = (uint32_t)threads | ((uint32_t)group_shift << 16) | (mask << 24);
     switch (nchunk) {
         case 1: add_rmsnorm_quant_traffic_only<1><<<grid, threads, 0, s>>>(xs, rs, chunks, remap_end, shape, gate, ro, co, scale); break;
         case 2: add_rmsnorm_quant_traffic_only<2><<<grid, threads, 0, s>>>(xs, rs, chunks, remap_end, shape, gate, ro, co, scale); break;
