@@ -33,7 +33,7 @@ def check(rows, scale, dtype, device):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("scale", [1.0, 0.02, 0.05, 1.5, 2.0, 1 / 3, 240.0, 1e-4, 3.0 ** 37, 3.0 ** -37, 3.0 ** 40, 2.0 ** -62])
+@pytest.mark.parametrize("scale", [1.0, 0.02, 0.05, 1.5, 2.0, 1 / 3, 1.0 - 2.0 ** -24, 240.0, 1e-4, 3.0 ** 37, 3.0 ** -37, 3.0 ** 40, 2.0 ** -62])
 def test_every_value(device, dtype, scale):
     print(f"case fp8 codes {dtype} scale={scale}", flush=True)
     ordered = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
@@ -42,9 +42,11 @@ def test_every_value(device, dtype, scale):
         check(values.reshape(-1, HV * D), scale, dtype, device)
 
 
-def magnitudes(limit):
-    """All bfloat16 patterns of both signs up to `limit`, in mixed order, zeros filling up the last row."""
-    top = int(torch.tensor(limit, dtype=torch.float32).view(torch.int32)) >> 16     # the largest pattern that is not above it
+def magnitudes(largest_quotient, s):
+    """All bfloat16 patterns of both signs whose quotient by s is at most this, in mixed order, zeros filling up the last row."""
+    patterns = torch.arange(0x7f80, dtype=torch.int32)
+    quotients = patterns.to(torch.int16).view(torch.bfloat16).double() / s.double()
+    top = int((quotients <= largest_quotient).sum()) - 1
     bits = torch.cat([torch.arange(top + 1), torch.arange(top + 1) + 0x8000])
     bits = bits[torch.randperm(len(bits), generator=torch.Generator().manual_seed(5))]
     rows = torch.zeros(-(-len(bits) // (HV * D)) * HV * D, dtype=torch.int64)
@@ -52,17 +54,17 @@ def magnitudes(limit):
     return rows.to(torch.int16).view(torch.bfloat16).reshape(-1, HV * D), top
 
 
-@pytest.mark.parametrize("scale", [1.0, 0.02, 0.05, 1.5, 2.0, 1 / 3, 240.0, 1e-4, 3.0 ** 37, 3.0 ** -37, 2.0 ** -60, 2.0 ** 60])
+@pytest.mark.parametrize("scale", [1.0, 0.02, 0.05, 1.5, 2.0, 1 / 3, 1.0 - 2.0 ** -24, 240.0, 1e-4, 3.0 ** 37, 3.0 ** -37, 2.0 ** -60, 2.0 ** 60])
 def test_every_form_of_the_conversion(device, scale):
     print(f"case fp8 forms scale={scale}", flush=True)
     s = torch.tensor(scale, dtype=torch.float32)
-    unclamped, top = magnitudes(float(440.0 * s))
-    largest = float((unclamped.float().abs().max() / s))
-    assert 432.0 < largest <= 440.0                       # up to the threshold, and rounding up to the top code
+    unclamped, top = magnitudes(448.0, s)
+    largest = float(unclamped.double().abs().max() / s.double())
+    assert 444.0 < largest <= 448.0                       # up to the largest code's value: the next pattern has to be clamped
     check(unclamped, scale, torch.bfloat16, device)
-    finite, finite_top = magnitudes(float(2.0 ** 60 * s))  # quotients of any size, clamped
+    finite, finite_top = magnitudes(2.0 ** 60, s)        # quotients of any size, clamped
     check(finite, scale, torch.bfloat16, device)
-    # passes of values below the threshold but for one, in every lane's first or last place in turn
+    # passes of values up to it but for one, in every lane's first or last place in turn
     bits = unclamped.reshape(-1).view(torch.int16).to(torch.int32)[:PASS] & 0xffff
     above = int((480.0 * s).view(torch.int32)) >> 16       # would not be the top code unless clamped
     offenders = [top, top + 1, top + 0x8001, above, above + 0x8000, finite_top, finite_top + 1, 0x7f7f, 0xff7f, 0x7f80, 0xff80, 0x7f81, 0xffc0, 0x7fff]
