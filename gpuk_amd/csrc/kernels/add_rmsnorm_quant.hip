@@ -921,12 +921,13 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, 
 // without codes, which have the time to be early, three waves and more up to three eighths of a round (379 of 7168 5.44 / 4.75, 597
 // of 4096 4.86 / 4.50, but 537 of 7168 6.27 / 6.36).  Four chunks 1.00 to 1.19 of the time.  More than a round: 1.00 to 1.03 (8192 x
 // 8192 75.6 / 76.7).
+constexpr bool late_in_four_chunks(RowType type, int quant) { return type == RowType::FP16 || quant != GPUK_QUANT_NONE; }
 bool late_weights(int64_t tokens, int threads, int nchunk, RowType type, int quant, bool gated) {
     const int64_t resident = resident_rows(threads, nchunk);
     if (tokens > resident || nchunk > 4) return false;
     if (type == RowType::BF16 && quant != GPUK_QUANT_FP8_STATIC && tokens <= 4) return false;
     const bool wide = threads >= 576;
-    if (nchunk == 4) return !gated && wide && (type == RowType::FP16 || quant != GPUK_QUANT_NONE);
+    if (nchunk == 4) return !gated && wide && late_in_four_chunks(type, quant);
     if (!gated) return threads >= 320 || (nchunk == 2 && threads >= 192 && 4 * tokens > 5 * kComputeUnits);
     if (nchunk == 1) return wide;
     return (wide && tokens <= kComputeUnits) || (quant == GPUK_QUANT_NONE && threads >= 192 && 8 * tokens <= 3 * resident);
@@ -1158,7 +1159,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
         if constexpr (N <= 2)                                                                                          \
             if (gate && late) GPUK_LAUNCH_NQ_AS(N, EXACT, true, true);                                                 \
         if (gate) GPUK_LAUNCH_NQ_AS(N, EXACT, true, false);                                                            \
-        if constexpr (N <= 4)                                                                                          \
+        if constexpr (N <= 2 || (N == 4 && late_in_four_chunks(row_type<T>, QUANT)))                                   \
             if (late) GPUK_LAUNCH_NQ_AS(N, EXACT, false, true);                                                        \
         GPUK_LAUNCH_NQ_AS(N, EXACT, false, false);                                                                     \
     } while (0)
