@@ -1543,21 +1543,24 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // layer's first half (16+2+2 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600), pairwise only in its last quarter (13.1 / 13.7 at
     // 5748, 13.8 / 13.5 at 6135), and pairwise with three units up to 7168 items (64+8+8 heads of 256 19.1 / 20.6 at 7380, in
     // half precision 18.7 / 19.4 at 7272).  In
-    // place from 4608 items, pairwise 4352, in half precision at once but no further than 7168 items, with idle lanes 6144,
-    // unless whole tokens (16+2 12.7 / 14.9 at 7348, 10.3 / 9.6 at 5526).
+    // place bfloat16 (whole tokens, see token_form_in_place) from 4608 items, pairwise 4352, half precision at once but no further
+    // than 7168 items, with idle lanes 6144, unless whole tokens (16+2 12.7 / 14.9 at 7348, 10.3 / 9.6 at 5526).
     const int units = shape.units;
     const int64_t items = shape.items, begun = items > 3072 && items < kTokenWaveCapacity ? items - 3072 : 1024;
     const int64_t layer = items % 1024 ? items % 1024 : 1024;  // items of the last layer
     const bool full = 8 * heads >= 7 * places, no_idle_unit = units * shape.parts == (int)a.units_per_token;
     const bool whole = whole_token(a, D, axes, units, shape.parts);
-    bool large;
-    if (kv_fp8) {
+    const bool has_form = set_kv || whole || token_form_in_place(neox, half, shape.units, two);
+    bool large = false;
+    if (!has_form) {
+        // (the lines below are of forms that there are)
+    } else if (kv_fp8) {
         // The conversions lengthen the wave, the gate hardly matters, and a layer that has just begun costs more: 28+4+4 heads
         // 11.9 / 10.8 at 3000 tokens, 14.2 / 13.3 at 4096, 12.5 / 12.9 at 3244; 32+8+8 14.8 / 14.0 at 2990, 14.6 / 15.9 at 3086,
         // 17.6 / 16.8 at 4096, level at 2500.
         large = 8 * (int64_t)a.total_units >= (units == 4 ? 10 : 13) * kResidentUnits && layer >= 256;
     } else if (two) {
-        if (!set_kv) large = half ? whole || (no_idle_unit && items <= (full ? 7168 : 6144)) : items >= (neox ? 4608 : 4352) && (whole || (full && no_idle_unit));
+        if (!set_kv) large = half ? whole || (no_idle_unit && items <= (full ? 7168 : 6144)) : items >= (neox ? 4608 : 4352);
         else if (half) large = neox || units == 4 || items <= 7168;
         else if (neox) large = (units == 3 || items >= (whole || !no_idle_unit ? 4608 : 4352)) && (full || layer >= 512 || (axes == 3 && !a.merge_rows));
         else large = whole ? items >= 4608 : (units == 4 || items <= 7168) && (full || layer >= 768);
@@ -1580,7 +1583,6 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
         large = (int64_t)a.total_units >= from_units && begun >= from_begun && (set_kv || whole || no_idle_unit);
     }
     const bool by_rule = g_token_waves == 0 && large;
-    const bool has_form = set_kv || whole || token_form_in_place(neox, half, shape.units, two);
     p.token_waves = shape.units && has_form && (g_token_waves >= 2 || by_rule);
     p.two_tokens = p.token_waves && two;
     // (with two items per wave the full read time: 24.4 us at 8192 tokens of 28+4+4 heads with three axes, against 25.4
