@@ -912,22 +912,24 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, 
 
 // Whether a launch of the 16-bit kernel asks for the weights once the row has landed (LANDED, see add_rmsnorm_quant_rows): at most
 // a round of rows, whose waves wait for their own loads and not for other rows', and more of them than short rows have.  us, at
-// once / landed: without a gate, from five waves on, 30 rows of 8192 elements, static, 3.58 / 3.36, 4 of 14336 in half precision 3.62 / 3.29
-// (but not up to 4 rows in bfloat16, whose unpacking then waits with the weights: one of 16384 3.79 / 3.87; static 0.99), 128 of 16384 5.7 / 5.45, 32768 elements (four chunks) 0.98 on average, but not without codes
-// in bfloat16 (14 rows 5.12 / 5.50); four waves and fewer level to 3 % behind, but for
+// once / landed: without a gate, from five waves on, 30 rows of 8192 elements, static, 3.58 / 3.36, 4 of 14336 in half precision 3.62 / 3.29,
+// 128 of 16384 5.7 / 5.45 (but not up to 4 rows of two chunks in bfloat16 without codes, one of 15576 3.35 / 3.46, 88 such calls
+// 1.02; with codes or one chunk 0.98); four waves and fewer level to 3 % behind, but for
 // 3 and 4 waves of two chunks behind the first layer (361 of 4096 static 3.9 / 3.7, 480 without codes 4.65 / 3.84).  Gated rows
 // have the launch's reads to wait for: nine waves and more of one chunk 0.97, of two chunks in the first layer (131 of 12288
 // 4.87 / 4.61, static 141 4.87 / 4.58, without codes 173 of 14688 5.35 / 5.02) and not behind it (338 of 12288 6.69 / 6.86);
 // without codes, which have the time to be early, three waves and more up to three eighths of a round (379 of 7168 5.44 / 4.75, 597
-// of 4096 4.86 / 4.50, but 537 of 7168 6.27 / 6.36).  Four chunks 1.00 to 1.19 of the time.  More than a round: 1.00 to 1.03 (8192 x
-// 8192 75.6 / 76.7).
-constexpr bool late_in_four_chunks(RowType type, int quant) { return type == RowType::FP16 || quant != GPUK_QUANT_NONE; }
+// of 4096 4.86 / 4.50, but 537 of 7168 6.27 / 6.36).  Four chunks have the loads of a whole row in flight per lane and hide the weights'
+// behind them unless the row has most of the lanes: with codes 1.04 of the time at 9 and 10 waves, level at 11 and 12, 0.96 from 13 on (700
+// calls; 60 rows of 32512 elements in bfloat16, static, 9.0 / 8.3, but 40 of 18040 in half precision 5.5 / 5.9), without codes 1.11 and 1.06,
+// 1.01 from 13 on (one row of 17984 3.7 / 4.2), gated 1.00 to 1.19.  More than a round: 1.00 to 1.03 (8192 x 8192 75.6 / 76.7).
+constexpr bool late_in_four_chunks(int quant) { return quant != GPUK_QUANT_NONE; }
 bool late_weights(int64_t tokens, int threads, int nchunk, RowType type, int quant, bool gated) {
     const int64_t resident = resident_rows(threads, nchunk);
     if (tokens > resident || nchunk > 4) return false;
-    if (type == RowType::BF16 && quant != GPUK_QUANT_FP8_STATIC && tokens <= 4) return false;
+    if (type == RowType::BF16 && quant == GPUK_QUANT_NONE && nchunk == 2 && tokens <= 4) return false;
     const bool wide = threads >= 576;
-    if (nchunk == 4) return !gated && wide && late_in_four_chunks(type, quant);
+    if (nchunk == 4) return !gated && threads >= 832 && late_in_four_chunks(quant);
     if (!gated) return threads >= 320 || (nchunk == 2 && threads >= 192 && 4 * tokens > 5 * kComputeUnits);
     if (nchunk == 1) return wide;
     return (wide && tokens <= kComputeUnits) || (quant == GPUK_QUANT_NONE && threads >= 192 && 8 * tokens <= 3 * resident);
@@ -1159,7 +1161,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
         if constexpr (N <= 2)                                                                                          \
             if (gate && late) GPUK_LAUNCH_NQ_AS(N, EXACT, true, true);                                                 \
         if (gate) GPUK_LAUNCH_NQ_AS(N, EXACT, true, false);                                                            \
-        if constexpr (N <= 2 || (N == 4 && late_in_four_chunks(row_type<T>, QUANT)))                                   \
+        if constexpr (N <= 2 || (N == 4 && late_in_four_chunks(QUANT)))                                   \
             if (late) GPUK_LAUNCH_NQ_AS(N, EXACT, false, true);                                                        \
         GPUK_LAUNCH_NQ_AS(N, EXACT, false, false);                                                                     \
     } while (0)
