@@ -1516,40 +1516,37 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     const TokenShape one_item = token_shape(a, D, axes, set_kv, kv_fp8, false), two_items = token_shape(a, D, axes, set_kv, kv_fp8, true);
     const bool two = two_items.units && (g_token_waves == 3 || !one_item.units);
     const TokenShape shape = two ? two_items : one_item;
-    // ... and too large for the kernel above to hold all of its waves at once (8192 units).  Where the two cross was read off
-    // 3000 random calls of 3 to 20 units per token (both kernels in turn, graph replays); over 1100 others, drawn afterwards, the
-    // calls whose kernel the lines change take 0.944 of the time that earlier lines gave them.  us, that kernel / this one:
-    // One item per wave, 16-bit cache.  Half precision, whose arithmetic is packed, from seven eighths of the other kernel's
-    // round where nearly all lanes have a head and no unit idles (40+8+8 heads 6.6 / 7.0 at 1228 tokens, 6.8 / 7.5 at 1365),
-    // with five units from fifteen sixteenths (32+8+8 7.4 / 7.1 at 1471), else and five units rotated pairwise beyond a round
-    // (16+2+2 5.5 / 6.1 at 2415 tokens, 7245 units, but 9.0 / 7.9 at 3031; 48+8+8 13.7 / 11.4 at 2151, two of four).  bfloat16
-    // beyond a round with three units (40+8+8, two parts, 9.7 / 8.5 at 1536 tokens, 12.2 / 10.2 at 2048; 24+8+8 heads of 256
-    // 12.5 / 10.4 at 1288), from seventeen sixteenths where lanes idle
-    // (16+2+2 7.5 / 7.8 at 2739), with four in parts and whole tokens of five from nine eighths of one (32+8+8 11.1 / 10.3 at 2048,
-    // 18.2 / 16.2 at 4096; 28+4+4 heads of 256 pairwise 11.2 / 9.8 at 1286), whole tokens of four and others of five from five
-    // quarters (28+4+4 9.2 / 9.8 at 2244, 11.5 / 10.3 at 2906; 16+2+2 heads of 256 8.8 / 9.3 at 1846).
-    // In place there is no V row and no scatter, and in bfloat16 the kernel above holds out longer with four and five units: 9.0
-    // / 9.5 at 2048 tokens of 32+8 heads, then 11.9 / 11.2 at 3000, 15.4 / 13.7 at 4096; 28+4 heads with three axes 10.7 / 9.5
-    // at 3000; 40+8, parts of three, 8.3 / 7.9 at 1536.
+    // ... and about as large as the kernel above can hold at once (8192 units, a round) or larger.  Where the two cross was read off
+    // 8500 random calls of 3 to 20 units per token (both kernels in turn, graph replays, a call's own runs within 1.4 %); one line
+    // covers all of a kind that cross within a sixteenth of a round.  us, that kernel / this one:
+    // One item per wave.  Half precision, whose arithmetic is packed, from seven eighths of a round (three units with a cache 0.94
+    // of the time up to the round, 0.81 just beyond it; 40+8+8 heads 6.8 / 7.5 at 1365 tokens, 9.6 / 11.7 at 2048), with five units, or
+    // four in place that read one table row, from fifteen sixteenths (32+8+8 7.4 / 7.1 at 1471); five in place, idle units (80+8+8 6.9 / 7.6
+    // at 726, but 48+8+8 13.7 / 11.4 at 2151) and, by halves, idle lanes (16+2+2 5.6 / 6.0 at 2576) beyond the round.  bfloat16 with three
+    // units beyond the round (40+8+8, two parts, 9.7 / 8.5 at 1536 tokens, 12.2 / 10.2 at 2048), with four and five, whose single wave takes
+    // longer, from nine eighths (32+8+8 11.1 / 10.3 at 2048), whole tokens of four and five with idle units from five quarters (28+4+4 8.5 /
+    // 9.4 at 2075, 9.2 / 9.8 at 2244, but 11.5 / 10.3 at 2906; 96+12+12, three parts, 9.6 / 10.8 at 691).  In place there is no V row and no
+    // scatter to share, and the kernel above holds out longer: four units from five quarters, whole tokens of four from eleven eighths, of five from three halves (28+4
+    // heads with three axes 10.7 / 9.5 at 3000 tokens, 32+8 9.0 / 9.5 at 2048, 11.9 / 11.2 at 3000, 15.4 / 13.7 at 4096; 30+6 pairwise 9.6 / 10.6 at
+    // 2288).
     // The SIMD with the most items sets the time (the rotation arithmetic of its waves is most of the launch), so it goes up in
-    // steps of 1024 items where the kernel above is linear, and a fourth layer that has just begun (3072 items and `begun`
-    // more) stays there in the forms that it costs more than it gives: 16+2+2 pairwise in half precision 8.8 / 9.5 at 3617
-    // tokens, 12+12+12 pairwise in bfloat16, three V chunks per lane, 14.8 / 15.5 at 3755, 32+8 in place 12.9 / 13.1 at 3150.
-    // Two items per wave, from a full round of items to twice that: 4096 waves, four on every SIMD, one item each and the others
-    // dealt out evenly.  In half precision with a cache at once (28+4+4 15.4 / 12.7 at 4148 tokens, 16+2+2 10.0 / 8.7 at 4367,
-    // pairwise 10.5 / 9.5 at 4545); in bfloat16 with four units from 4352 items, whole
-    // tokens 4608 (28+4+4 15.2 / 15.4 at 4100, 18.4 / 18.2 at 5200, 21.1 / 19.1 at 6144,
-    // 26.8 / 25.3 at 8192; 12+2+2 heads of 256 14.2 / 15.3 at 4123), where lanes idle and one table row is read not in a
-    // layer's first half (16+2+2 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600), pairwise only in its last quarter (13.1 / 13.7 at
-    // 5748, 13.8 / 13.5 at 6135), and pairwise with three units up to 7168 items (64+8+8 heads of 256 19.1 / 20.6 at 7380, in
-    // half precision 18.7 / 19.4 at 7272).  In
-    // place bfloat16 (whole tokens, see token_form_in_place) from 4608 items, pairwise 4352, half precision at once but no further
-    // than 7168 items, with idle lanes 6144, unless whole tokens (16+2 12.7 / 14.9 at 7348, 10.3 / 9.6 at 5526).
+    // steps of 1024 items where the kernel above is linear: a fourth layer that has just begun (up to 256 items) costs more than
+    // it gives, but for rotation by halves with full lanes, with a cache or in half precision without idle units (274 calls 0.98 of the time, the others
+    // level; 3269 tokens of 18+6+6 10.8 / 10.3, 779 of 48+16+16 heads of 256 13.8 / 12.5).  Pairwise, where a wave's arithmetic is
+    // longest, up to 640 items in half precision in place or with idle lanes (32+4 in place 11.8 / 13.1 at 3293 tokens, 16+2+2 8.5 / 9.3 at
+    // 3457) and in bfloat16 with three V chunks per lane (603 tokens of 64+64+64, six parts, 12.7 / 13.9).
+    // Two items per wave, from 4096 items to twice that: 4096 waves, four on every SIMD, one item each and the others dealt out
+    // evenly.  In half precision at once (28+4+4 15.4 / 12.7 at 4148 tokens, 16+2+2 10.0 / 8.7 at 4367); in bfloat16 where lanes are full,
+    // three table rows are read or, by halves, the last layer is half full (16+2+2 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600), four units that
+    // are whole tokens or some of them idle from 4608 items (28+4+4 15.2 / 15.4 at 4100, 18.4 / 18.2 at 5200, 21.1 / 19.1 at 6144; but 1151
+    // tokens of 112+16+16, four parts, 18.6 / 15.2).  An eighth layer fills them all: in parts of a token in place, and pairwise in place or
+    // with three units, the two are level there or this one is behind (16+2 in place 12.7 / 14.9 at 7348, 64+8+8 heads of 256 pairwise 19.1 / 20.6 at 7380).
     const int units = shape.units;
-    const int64_t items = shape.items, begun = items > 3072 && items < kTokenWaveCapacity ? items - 3072 : 1024;
+    const int64_t items = shape.items;
     const int64_t layer = items % 1024 ? items % 1024 : 1024;  // items of the last layer
     const bool full = 8 * heads >= 7 * places, no_idle_unit = units * shape.parts == (int)a.units_per_token;
     const bool whole = whole_token(a, D, axes, units, shape.parts);
+    const bool three_rows = axes == 3 && !a.merge_rows;
     const bool has_form = set_kv || whole || token_form_in_place(neox, half, shape.units, two);
     bool large = false;
     if (!has_form) {
@@ -1560,27 +1557,22 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
         // 17.6 / 16.8 at 4096, level at 2500.
         large = 8 * (int64_t)a.total_units >= (units == 4 ? 10 : 13) * kResidentUnits && layer >= 256;
     } else if (two) {
-        if (!set_kv) large = half ? whole || (no_idle_unit && items <= (full ? 7168 : 6144)) : items >= (neox ? 4608 : 4352);
-        else if (half) large = neox || units == 4 || items <= 7168;
-        else if (neox) large = (units == 3 || items >= (whole || !no_idle_unit ? 4608 : 4352)) && (full || layer >= 512 || (axes == 3 && !a.merge_rows));
-        else large = whole ? items >= 4608 : (units == 4 || items <= 7168) && (full || layer >= 768);
+        const bool eighth_layer = set_kv ? neox || units == 4 : neox && whole, at_once = units == 3 || (!whole && no_idle_unit);
+        large = (items <= 7168 || eighth_layer) && (half || ((at_once || items >= 4608) && (full || three_rows || (neox && layer >= 512))));
     } else {
-        int64_t from_units = kResidentUnits + 1;
+        int64_t sixteenths = 16;  // of a round, 16: beyond one
         if (half) {
-            if (full && no_idle_unit && (units < 5 || (set_kv && neox))) from_units = units == 5 ? 15 * kResidentUnits / 16 : set_kv || units == 3 ? 7 * kResidentUnits / 8 : 59 * kResidentUnits / 64;
-        } else if (set_kv) {
-            if (units > 3) from_units = (units == 4) == whole ? 5 * kResidentUnits / 4 : 9 * kResidentUnits / 8;
-            else if (!full) from_units = 17 * kResidentUnits / 16;
-        } else {
-            if (whole) from_units = 7 * kResidentUnits / 5;
-            else if (units == 4) from_units = 5 * kResidentUnits / 4;
+            if (no_idle_unit && (full || !neox)) sixteenths = units != 5 && (units == 3 || set_kv || !neox || three_rows) ? 14 : units == 4 || set_kv ? 15 : 16;
+        } else if (units > 3) {
+            if (set_kv) sixteenths = (whole && units == 4) || (units == 5 && !no_idle_unit) ? 20 : 18;
+            else sixteenths = units == 5 ? 24 : whole ? 22 : 20;
         }
-        int64_t from_begun;
-        if (!set_kv) from_begun = half ? (!neox ? 640 : !full ? 256 : units == 4 ? 128 : 0) : !neox || units < 5 ? 256 : 384;
-        else if (half) from_begun = !neox ? (units == 3 ? 576 : 384) : full && no_idle_unit ? 0 : 128;
-        else if (neox) from_begun = 0;
-        else from_begun = a.hv * (D / 8) > 128 * shape.parts ? 768 : 256;
-        large = (int64_t)a.total_units >= from_units && begun >= from_begun && (set_kv || whole || no_idle_unit);
+        int64_t from_begun = 256;
+        if (neox) from_begun = full && (half ? no_idle_unit : set_kv) ? 0 : 256;
+        else if (half ? !(set_kv && full) : set_kv && a.hv * (D / 8) > 128 * shape.parts) from_begun = 640;
+        const int64_t begun = items > 3072 && items < kTokenWaveCapacity ? items - 3072 : 1024;
+        large = 16 * (int64_t)a.total_units >= sixteenths * kResidentUnits + (sixteenths == 16 ? 1 : 0) && begun >= from_begun &&
+                (set_kv || whole || no_idle_unit);
     }
     const bool by_rule = g_token_waves == 0 && large;
     p.token_waves = shape.units && has_form && (g_token_waves >= 2 || by_rule);

@@ -495,6 +495,9 @@ def test_rope_launch_shape_report_of_rotation_and_sections():
     assert shape(4608) == shape(4608, mrope_section=[16, 24, 24]) and shape(4608)[3] == 2
     assert shape(2400, is_neox=False) == shape(2400) and shape(2400)[3] == 0              # whole tokens of four: from five quarters of a round
     assert shape(2400, mrope_section=[24, 20, 20], is_interleaved=True)[3] == 1           # three table rows: from nine eighths
+    assert shape(3100)[3] == 1 and shape(3100, is_neox=False)[3] == 0                     # a layer of waves that has just begun
+    assert shape(4200)[3] == 0                                                            # two whole tokens of four: from 4608
+    assert shape(4200, mrope_section=[24, 20, 20], is_interleaved=True)[3] == 2           # three table rows: at once
     assert capi.rope_rms_launch_shape(1850, 64, 64, 64, 64, is_neox=False)[1] == 256
     # in place, parts of a token: a form for rotation by halves only
     assert capi.rope_rms_launch_shape(1536, 40, 8, 8, 128, set_kv=False)[3] == 1
@@ -512,28 +515,40 @@ def test_rope_launch_shape_report_of_rotation_and_sections():
 
 def test_rope_kernel_choice():
     """Which calls the kernel with one wave per token or part of one takes (1: one item per wave, 2: two), from both sides of
-    the lines of its rule, rotation by halves."""
+    the lines of its rule: rotation by halves, then pairwise."""
     from gpuk_amd import capi
 
     bf16, f16 = torch.bfloat16, torch.float16
-    for heads, D, dtype, cache, changes in (
-            # three units per item: beyond a round of the other kernel's waves, or more where lanes idle; half precision from seven eighths where lanes are full
-            ((16, 2, 2), 128, bf16, True, ((2901, 0), (2902, 1), (4096, 1), (4097, 0), (4607, 0), (4608, 2), (5120, 2), (5300, 0), (8192, 2), (8193, 0))),
-            ((16, 2, 2), 128, f16, True, ((2389, 0), (2730, 0), (2731, 1), (3072, 1), (3073, 0), (3200, 1), (4096, 1), (4097, 2), (8192, 2), (8193, 0))),
-            ((12, 12, 12), 128, f16, True, ((2389, 0), (2390, 1), (3073, 1))),
-            ((24, 8, 8), 256, bf16, True, ((1151, 0), (1152, 1), (2048, 1), (2049, 0))),
-            ((28, 4, 4), 256, bf16, True, ((2048, 1), (2175, 0), (2176, 2))),
-            # four, five: from nine eighths of a round, whole tokens of four from five quarters
-            ((28, 4, 4), 128, bf16, True, ((2559, 0), (2560, 1), (3073, 1), (4607, 0), (4608, 2))),
-            ((28, 4, 4), 128, f16, True, ((1791, 0), (1792, 1), (4096, 1), (4097, 2))),
-            ((32, 8, 8), 128, bf16, True, ((1843, 0), (1844, 1), (3073, 1), (4096, 1), (4097, 0))),
-            ((32, 8, 8), 128, f16, True, ((1535, 0), (1536, 1), (4096, 1), (4097, 0))),
-            # in place
-            ((32, 8, 8), 128, bf16, False, ((2293, 0), (2294, 1), (3455, 0), (3456, 1))),
-            ((16, 2, 2), 128, f16, False, ((2730, 0), (2731, 1), (3327, 0), (3328, 1), (6144, 2), (6145, 0))),
-            ((12, 12, 12), 128, f16, False, ((2389, 0), (2390, 1), (7168, 2), (7169, 0)))):
-        for tokens, expect in changes:
-            assert capi.rope_rms_launch_shape(tokens, *heads, D, 1, dtype, cache, False)[3] == expect, (tokens, heads, D, dtype, cache)
+    for heads, D, dtype, cache, halves, pairwise in (
+            # (tokens, which kernel from there on, at every change up to 8400)
+            # three units per item: beyond a round of the other kernel's waves; half precision from seven eighths, by halves where lanes are full
+            ((16, 2, 2), 128, bf16, True, ((2731, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (5121, 0), (5632, 2), (6145, 0), (6656, 2), (7169, 0), (7680, 2), (8193, 0)),
+             ((2731, 1), (3073, 0), (3328, 1), (4097, 0))),
+            ((16, 2, 2), 128, f16, True, ((2731, 1), (3073, 0), (3328, 1), (4097, 2), (8193, 0)), ((2390, 1), (3073, 0), (3712, 1), (4097, 2), (7169, 0))),
+            ((12, 12, 12), 128, bf16, True, ((2731, 1), (4097, 0)), ((2731, 1), (3073, 0), (3712, 1), (4097, 0))),
+            ((12, 12, 12), 128, f16, True, ((2390, 1), (4097, 0)), ((2390, 1), (3073, 0), (3328, 1), (4097, 0))),
+            ((24, 8, 8), 256, bf16, True, ((1152, 1), (2049, 0)), ((1152, 1), (1537, 0), (1664, 1), (2049, 0))),
+            # four, five: bfloat16 from nine eighths of a round, whole tokens of four and five with idle units from five quarters
+            ((28, 4, 4), 256, bf16, True, ((1152, 1), (2049, 2), (4097, 0)), ((1152, 1), (1537, 0), (1664, 1), (2049, 2), (4097, 0))),
+            ((28, 4, 4), 128, bf16, True, ((2560, 1), (4097, 0), (4608, 2), (8193, 0)), ((2560, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (8193, 0))),
+            ((28, 4, 4), 128, f16, True, ((1792, 1), (4097, 2), (8193, 0)), ((1792, 1), (3073, 0), (3328, 1), (4097, 2), (8193, 0))),
+            ((32, 8, 8), 128, bf16, True, ((1844, 1), (4097, 0)), ((1844, 1), (3073, 0), (3328, 1), (4097, 0))),
+            ((32, 8, 8), 128, f16, True, ((1536, 1), (4097, 0)), ((1536, 1), (3073, 0), (3328, 1), (4097, 0))),
+            ((96, 12, 12), 128, bf16, True, ((732, 1), (1366, 2), (2049, 0)), ((732, 1), (1025, 0), (1110, 1), (1366, 2), (1434, 0), (1639, 2), (2049, 0))),
+            # in place; pairwise whole tokens only
+            ((32, 8, 8), 128, bf16, False, ((2458, 1), (3073, 0), (3328, 1), (4097, 0)), ((2458, 1), (3073, 0), (3328, 1), (4097, 0))),
+            ((28, 4, 4), 128, bf16, False, ((2816, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (8193, 0)), ((2816, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (7169, 0))),
+            ((28, 4, 4), 128, f16, False, ((1920, 1), (4097, 2), (8193, 0)), ((1792, 1), (3073, 0), (3712, 1), (4097, 2), (7169, 0))),
+            ((16, 2, 2), 128, f16, False, ((2731, 1), (3073, 0), (3328, 1), (4097, 2), (7169, 0)), ()),
+            ((12, 12, 12), 128, f16, False, ((2390, 1), (4097, 2), (7169, 0)), ())):
+        for changes, neox in ((halves, True), (pairwise, False)):
+            kernel = lambda T: capi.rope_rms_launch_shape(T, *heads, D, 1, dtype, cache, False, neox)[3]
+            was = 0
+            for tokens, expect in changes:
+                assert (kernel(tokens - 1), kernel(tokens)) == (was, expect), (tokens, heads, D, dtype, cache, neox)
+                was = expect
+            last = changes[-1][0] if changes else 300
+            assert all(kernel(T) == was for T in range(last, 8400, 101)), (heads, D, dtype, cache, neox)
     # an fp8 cache: whole tokens, not where the last layer of waves has just begun
     for tokens, heads, expect in ((2560, (28, 4, 4), 1), (3200, (28, 4, 4), 0), (3328, (28, 4, 4), 1), (2662, (32, 8, 8), 0), (2663, (32, 8, 8), 1), (3100, (32, 8, 8), 0)):
         assert capi.rope_rms_launch_shape(tokens, *heads, 128, 1, bf16, True, True)[3] == expect, (tokens, heads)
