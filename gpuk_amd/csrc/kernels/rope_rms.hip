@@ -1537,8 +1537,9 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // 3457) and in bfloat16 with three V chunks per lane (603 tokens of 64+64+64, six parts, 12.7 / 13.9).
     // Two items per wave, from 4096 items to twice that: 4096 waves, four on every SIMD, one item each and the others dealt out
     // evenly.  In half precision at once (28+4+4 15.4 / 12.7 at 4148 tokens, 16+2+2 10.0 / 8.7 at 4367); in bfloat16 where lanes are full,
-    // three table rows are read or, by halves, the last layer is half full (16+2+2 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600), four units that
-    // are whole tokens or some of them idle from 4608 items (28+4+4 15.2 / 15.4 at 4100, 18.4 / 18.2 at 5200, 21.1 / 19.1 at 6144; but 1151
+    // three table rows are read or the last layer is half full (145 calls with idle lanes 0.97 of the time, 44 of a layer less full 1.03; 16+2+2
+    // 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600, pairwise 16+4+4 14.6 / 12.9 at 5031), four units that
+    // are whole tokens or some of them idle, but for three rows, from 4608 items (28+4+4 15.2 / 15.4 at 4100, 18.4 / 18.2 at 5200, 21.1 / 19.1 at 6144; but 1151
     // tokens of 112+16+16, four parts, 18.6 / 15.2).  An eighth layer fills them all: in parts of a token in place, and pairwise in place or
     // with three units, the two are level there or this one is behind (16+2 in place 12.7 / 14.9 at 7348, 64+8+8 heads of 256 pairwise 19.1 / 20.6 at 7380).
     const int units = shape.units;
@@ -1557,8 +1558,8 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
         // 17.6 / 16.8 at 4096, level at 2500.
         large = 8 * (int64_t)a.total_units >= (units == 4 ? 10 : 13) * kResidentUnits && layer >= 256;
     } else if (two) {
-        const bool eighth_layer = set_kv ? neox || units == 4 : neox && whole, at_once = units == 3 || (!whole && no_idle_unit);
-        large = (items <= 7168 || eighth_layer) && (half || ((at_once || items >= 4608) && (full || three_rows || (neox && layer >= 512))));
+        const bool eighth_layer = set_kv ? neox || units == 4 : neox && whole, at_once = units == 3 || three_rows || (!whole && no_idle_unit);
+        large = (items <= 7168 || eighth_layer) && (half || ((at_once || items >= 4608) && (full || three_rows || layer >= 512)));
     } else {
         int64_t sixteenths = 16;  // of a round, 16: beyond one
         if (half) {

@@ -523,7 +523,7 @@ def test_rope_kernel_choice():
             # (tokens, which kernel from there on, at every change up to 8400)
             # three units per item: beyond a round of the other kernel's waves; half precision from seven eighths, by halves where lanes are full
             ((16, 2, 2), 128, bf16, True, ((2731, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (5121, 0), (5632, 2), (6145, 0), (6656, 2), (7169, 0), (7680, 2), (8193, 0)),
-             ((2731, 1), (3073, 0), (3328, 1), (4097, 0))),
+             ((2731, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (5121, 0), (5632, 2), (6145, 0), (6656, 2), (7169, 0))),
             ((16, 2, 2), 128, f16, True, ((2731, 1), (3073, 0), (3328, 1), (4097, 2), (8193, 0)), ((2390, 1), (3073, 0), (3712, 1), (4097, 2), (7169, 0))),
             ((12, 12, 12), 128, bf16, True, ((2731, 1), (4097, 0)), ((2731, 1), (3073, 0), (3712, 1), (4097, 0))),
             ((12, 12, 12), 128, f16, True, ((2390, 1), (4097, 0)), ((2390, 1), (3073, 0), (3328, 1), (4097, 0))),
