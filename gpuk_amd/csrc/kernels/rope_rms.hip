@@ -1596,8 +1596,9 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // 8.2 / 7.0 at 1638; 28+4 heads with three axes 6.8 / 6.2 at 1536 tokens, 8.5 / 7.1 at 2048.  Nothing to gain below
     // half a round, 15-35 % slower one unit beyond a round.
     // Half precision, whose waves are done sooner, gates from three eighths of a round, with an fp8 cache from a half, for any axes,
-    // and opens earlier: at the read time itself below half a round (1.1 times it rotated pairwise) and, rotated by halves with every
-    // lane in use, with an fp8 cache up to two thirds of a round, at 1.1 times it else
+    // and opens earlier: at the read time itself below half a round (1.1 times it rotated pairwise) and, with a cache, rotated by halves
+    // with every lane in use, at 1.1 times it (0.99 of the time over 190 calls; in place 1.02, 2863 tokens of 14+2 heads 5.0 / 5.3), with an fp8
+    // cache at the read time up to two thirds of a round and at 1.2 times it, where the two are level, from there
     // (not gated or gated as bfloat16 / so: 690 tokens of 32+8+8 heads 4.77 / 4.4, 981 with interleaved sections 6.23 / 5.3, 247 of
     // 64+64+64 6.1 / 5.2, in place 995 of 32+8 4.82 / 4.65, an fp8 cache 576 of 64+8+8 5.72 / 5.1; heads of 64,
     // lanes that idle and many V heads keep 1.2 from two thirds of a round on, 2422 tokens of 16+2+2 5.67 / 6.16, 227 of 64+64+64 heads of
@@ -1630,9 +1631,9 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     const bool fuller = gated_by_rule && (two_thirds || gated_lines);
     double times;  // of the launch's reads at 7 TB/s
     if (gated_lines) times = neox ? 1.15 : 1.25;
-    else if (two_thirds) times = half && neox && no_idle_lane && !many_v && D != 64 ? 1.1 : !half && !neox && !kv_fp8 ? 1.3 : 1.2;
+    else if (two_thirds) times = half && neox && no_idle_lane && set_kv && !kv_fp8 && !many_v && D != 64 ? 1.1 : !half && !neox && !kv_fp8 ? 1.3 : 1.2;
     else if (half && 2 * a.total_units < kResidentUnits) times = neox ? 1.0 : 1.1;
-    else times = half && neox && no_idle_lane ? (kv_fp8 ? 1.0 : 1.1) : 1.15;
+    else times = half && neox && no_idle_lane && set_kv ? (kv_fp8 ? 1.0 : 1.1) : 1.15;
     if (g_unit_gate > 0) p.unit_gate = (uint32_t)g_unit_gate;
     else if (gated_by_rule) p.unit_gate = (uint32_t)std::min(times * (double)read_bytes / 70000.0, 5000.0);
     if (g_stream_rows == 2) p.whole_lines = true;
@@ -1644,12 +1645,11 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // CU's caches: 3-15 % ahead at 28+4 heads) and for large batches (1-3 % ahead from 4096 tokens on), single
     // waves for small batches of other head counts (2-6 % ahead at 64+8 heads with an fp8 cache up to 512 tokens,
     // within 1-3 % either way for 3, 5 and 6 units per token); 128 lanes is the slowest in most cases.  In place, without the
-    // scatter, four waves from three eighths of a round (pairwise a half, heads of 64 with idle lanes five eighths): 1028 tokens of
-    // 64+8 heads of 64 6.04 / 5.35 us (but 974 5.01 / 5.27), 2618 of 28+4 pairwise 6.29 / 5.6, 441 of 64+8 heads of 128 4.80 / 4.65,
-    // 995 of 32+8 in half precision 4.82 / 4.56; not pairwise in half precision (1757 of 12+12 5.20 / 5.58) nor
-    // there with idle lanes (905 of 16+2 heads of 256 4.32 / 4.53).
-    const bool four_in_place = !set_kv && (!half || (neox && no_idle_lane)) &&
-                               round_8ths >= (D == 64 && heads != places ? 5 : neox ? 3 : 4) * (int64_t)kResidentUnits;
+    // scatter, four waves in bfloat16 rotated by halves from five eighths of a round (141 calls 0.96 of the time of single waves) and
+    // wherever heads of 64 elements that fill their lanes are gated (61 calls 0.93, with idle lanes 99 calls level); not before (860 calls level), pairwise (480 calls 1.03, 1609 tokens of 16+8
+    // heads 5.1 / 5.9) or in half precision (620 calls 1.06, 503 of 64+8 4.4 / 4.9), which take four from two thirds of a round on, as all
+    // gated launches do (see above).
+    const bool four_in_place = !set_kv && !half && ((neox && round_8ths >= 5 * (int64_t)kResidentUnits) || (D == 64 && no_idle_lane && gated_by_rule));
     // Just beyond a round tokens of three units with a cache, which four waves do not hold whole, are ahead in single waves (20 calls of
     // 1 to 1.5 rounds 0.90 to 0.995 of the time, level from there: 2966 tokens of 16+2+2 heads, fp8 cache, 8.9 / 8.2, 3166 of 32+8+8 of 64
     // 10.8 / 9.6, 3481 of 40+8+8 of 64 with a 16-bit cache 12.3 / 11.4; two units 1.05 to 1.1, four 1.06, in place level).

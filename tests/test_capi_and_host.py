@@ -555,15 +555,19 @@ def test_rope_kernel_choice():
 
 
 def test_rope_workgroups():
-    """Lanes per workgroup of the rope kernel with one wave per group of heads: four waves in place from three eighths of a round of
-    waves, in whole lines behind a gate, and single waves where an fp8 cache of many V heads keeps the vector units busy
-    and for tokens of three units just beyond a round."""
+    """Lanes per workgroup of the rope kernel with one wave per group of heads: four waves in place in bfloat16 by halves from five eighths of
+    a round of waves and behind the gate of heads of 64 that fill their lanes, in other forms from two thirds, in whole lines behind a gate, and single waves
+    where an fp8 cache of many V heads keeps the vector units busy and for tokens of three units just beyond a round."""
     from gpuk_amd import capi
 
     bf16, f16 = torch.bfloat16, torch.float16
+    for tokens, heads, dtype, neox, lanes in ((1023, (32, 8, 8), bf16, True, 64), (1024, (32, 8, 8), bf16, True, 256), (1092, (32, 8, 8), bf16, False, 64), (1093, (32, 8, 8), bf16, False, 256),
+                                              (1092, (32, 8, 8), f16, True, 64), (1093, (32, 8, 8), f16, True, 256), (1820, (16, 2, 2), f16, False, 64), (1821, (16, 2, 2), f16, False, 256)):
+        assert capi.rope_rms_launch_shape(tokens, *heads, 128, 1, dtype, False, False, neox)[1] == lanes, (tokens, heads, dtype, neox)
+    for heads, changes in (((72, 8, 8), 820), ((64, 8, 8), 1093)):   # (lanes that idle: from two thirds)
+        assert [capi.rope_rms_launch_shape(T, *heads, 64, 1, bf16, False, False, False)[1] for T in (changes - 1, changes)] == [64, 256]
     for tokens, heads, D, dtype, cache, fp8, lanes in (
-            (614, (32, 8, 8), 128, bf16, False, False, 64), (615, (32, 8, 8), 128, bf16, False, False, 256), (615, (32, 8, 8), 128, f16, False, False, 256),
-            (1024, (16, 2, 2), 128, f16, False, False, 64), (1023, (64, 8, 8), 64, bf16, False, False, 64), (1024, (64, 8, 8), 64, bf16, False, False, 256),
+            (1023, (64, 8, 8), 64, bf16, False, False, 64), (1024, (64, 8, 8), 64, bf16, False, False, 256), (1092, (64, 8, 8), 64, f16, False, False, 64),
             (1706, (32, 8, 8), 64, bf16, True, False, 64), (1707, (32, 8, 8), 64, bf16, True, False, 256), (1707, (32, 8, 8), 64, f16, True, False, 64),
             (255, (64, 64, 64), 128, bf16, True, True, 256), (256, (64, 64, 64), 128, bf16, True, True, 64), (512, (64, 64, 64), 128, bf16, True, True, 64),
             (513, (64, 64, 64), 128, bf16, True, True, 256), (2000, (16, 16, 16), 128, bf16, True, True, 256),
