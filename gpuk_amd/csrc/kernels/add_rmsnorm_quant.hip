@@ -921,15 +921,16 @@ uint32_t store_gate(int64_t tokens, int64_t row_bytes, int threads, int nchunk, 
 // without codes, which have the time to be early, three waves and more up to three eighths of a round (379 of 7168 5.44 / 4.75, 597
 // of 4096 4.86 / 4.50, but 537 of 7168 6.27 / 6.36).  Four chunks have the loads of a whole row in flight per lane and hide the weights'
 // behind them unless the row has most of the lanes: with codes 1.04 of the time at 9 and 10 waves, level at 11 and 12, 0.96 from 13 on (700
-// calls; 60 rows of 32512 elements in bfloat16, static, 9.0 / 8.3, but 40 of 18040 in half precision 5.5 / 5.9), without codes 1.11 and 1.06,
-// 1.01 from 13 on (one row of 17984 3.7 / 4.2), gated 1.00 to 1.19.  More than a round: 1.00 to 1.03 (8192 x 8192 75.6 / 76.7).
-constexpr bool late_in_four_chunks(int quant) { return quant != GPUK_QUANT_NONE; }
+// calls; 57 rows of 32512 elements in bfloat16, static, 9.0 / 8.3, but 40 of 18040 in half precision 5.5 / 5.9), without codes 1.11 and
+// 1.06, and from 13 on 1.02 up to 32 rows (one of 17984 3.7 / 4.2) and 0.97 beyond (118 of 27112 8.2 / 7.5), in half precision; not in
+// bfloat16 (14 rows of 32768 5.12 / 5.50), gated 1.00 to 1.19.  More than a round: 1.00 to 1.03 (8192 x 8192 75.6 / 76.7).
+constexpr bool late_in_four_chunks(RowType type, int quant) { return type == RowType::FP16 || quant != GPUK_QUANT_NONE; }
 bool late_weights(int64_t tokens, int threads, int nchunk, RowType type, int quant, bool gated) {
     const int64_t resident = resident_rows(threads, nchunk);
     if (tokens > resident || nchunk > 4) return false;
     if (type == RowType::BF16 && quant == GPUK_QUANT_NONE && nchunk == 2 && tokens <= 4) return false;
     const bool wide = threads >= 576;
-    if (nchunk == 4) return !gated && threads >= 832 && late_in_four_chunks(quant);
+    if (nchunk == 4) return !gated && threads >= 832 && late_in_four_chunks(type, quant) && (quant != GPUK_QUANT_NONE || tokens > 32);
     if (!gated) return threads >= 320 || (nchunk == 2 && threads >= 192 && 4 * tokens > 5 * kComputeUnits);
     if (nchunk == 1) return wide;
     return (wide && tokens <= kComputeUnits) || (quant == GPUK_QUANT_NONE && threads >= 192 && 8 * tokens <= 3 * resident);
@@ -1161,7 +1162,7 @@ int launch_rows(const void *x, const void *residual_in, const void *gamma, void 
         if constexpr (N <= 2)                                                                                          \
             if (gate && late) GPUK_LAUNCH_NQ_AS(N, EXACT, true, true);                                                 \
         if (gate) GPUK_LAUNCH_NQ_AS(N, EXACT, true, false);                                                            \
-        if constexpr (N <= 2 || (N == 4 && late_in_four_chunks(QUANT)))                                   \
+        if constexpr (N <= 2 || (N == 4 && late_in_four_chunks(row_type<T>, QUANT)))                                  \
             if (late) GPUK_LAUNCH_NQ_AS(N, EXACT, false, true);                                                        \
         GPUK_LAUNCH_NQ_AS(N, EXACT, false, false);                                                                     \
     } while (0)

@@ -191,7 +191,7 @@ def test_shapes_of_small_batches(device, dtype, tokens, hidden):
 
 
 # (rows that fill their lanes and rows that do not; one, two and four chunks per lane; without a gate, then gated, some only without codes)
-@pytest.mark.parametrize("tokens,hidden", [(1, 5120), (60, 6544), (1, 7168), (40, 7200), (321, 4096), (400, 4000), (9, 32768), (5, 30008), (3, 24576), (4, 24584),
+@pytest.mark.parametrize("tokens,hidden", [(1, 5120), (60, 6544), (1, 7168), (40, 7200), (321, 4096), (400, 4000), (9, 32768), (5, 30008), (3, 24576), (4, 24584), (32, 24584), (33, 24584),
                                            (257, 5632), (300, 6000), (130, 12288), (131, 12296), (256, 16384), (379, 7168), (384, 7176)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_weights_asked_for_late(device, dtype, tokens, hidden):
