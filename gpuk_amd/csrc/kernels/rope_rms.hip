@@ -1584,7 +1584,7 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     p.gate = (uint32_t)std::min(gate, 5000.0);
     // The kernel with one wave per unit gates its stores in the same way where its waves are all resident at once
     // (8192 of them, eight per SIMD) and fill at least half of that round.
-    // The gate is 1.15 to 1.2 times the read time at 7 TB/s (its waves enter over a few microseconds, and the gate
+    // The gate is 1.2 times the read time at 7 TB/s (its waves enter over a few microseconds, and the gate
     // counts from each wave's own entry); from two thirds of a round on the launch is made of four-wave workgroups
     // whatever the head count, because 8192 single-wave workgroups take so long to place that the last waves' reads
     // fall into the first waves' writes.  Measured (us, ungated single-wave workgroups / gated as chosen here): 32+8+8
@@ -1595,16 +1595,13 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // 9.2 / 7.7 at 2048 (5.5 / 5.7 at 1024).  The in-place ops alike: 32+8 heads 5.9 / 5.5 at 1024 tokens, 7.3 / 6.4 at 1400,
     // 8.2 / 7.0 at 1638; 28+4 heads with three axes 6.8 / 6.2 at 1536 tokens, 8.5 / 7.1 at 2048.  Nothing to gain below
     // half a round, 15-35 % slower one unit beyond a round.
-    // Half precision, whose waves are done sooner, gates from three eighths of a round, with an fp8 cache from a half, for any axes,
-    // and opens earlier: at the read time itself below half a round (1.1 times it rotated pairwise) and, with a cache, rotated by halves
-    // with every lane in use, at 1.1 times it (0.99 of the time over 190 calls; in place 1.02, 2863 tokens of 14+2 heads 5.0 / 5.3), with an fp8
-    // cache at the read time up to two thirds of a round and at 1.2 times it, where the two are level, from there
-    // (not gated or gated as bfloat16 / so: 690 tokens of 32+8+8 heads 4.77 / 4.4, 981 with interleaved sections 6.23 / 5.3, 247 of
-    // 64+64+64 6.1 / 5.2, in place 995 of 32+8 4.82 / 4.65, an fp8 cache 576 of 64+8+8 5.72 / 5.1; heads of 64,
-    // lanes that idle and many V heads keep 1.2 from two thirds of a round on, 2422 tokens of 16+2+2 5.67 / 6.16, 227 of 64+64+64 heads of
-    // 256 8.4 / 9.3, and pairwise ones 1.15 before it, 340 of
-    // 64+64+64 7.0 / 7.5).  Rotated pairwise in bfloat16 a wave takes longer: 1.3 times from two thirds of a round on (0.96 to 1.00 of the
-    // time over 40 calls, with an fp8 cache level).
+    // Half precision, whose waves are done sooner, gates from three eighths of a round, with an fp8 cache from a half, for any axes
+    // (not gated / so: 690 tokens of 32+8+8 heads 4.77 / 4.4, 981 with interleaved sections 6.23 / 5.3, 247 of 64+64+64 6.1 / 5.2, in place
+    // 995 of 32+8 4.82 / 4.65, an fp8 cache 576 of 64+8+8 5.72 / 5.1).
+    // 1.2 times serves all forms within 1 % (over 7000 random calls of shorter and longer gates) but two: bfloat16 rotated pairwise, whose waves
+    // take longer, waits 1.3 times from two thirds of a round on (0.98 of the time over 640 calls, with an fp8 cache level), and half
+    // precision by halves with every lane in use and a 16-bit cache 1.1 times (0.99 over 190 calls; in place 1.02, 2863 tokens of 14+2 heads
+    // 5.0 / 5.3, with many V heads 1.02).
     // Heads of 64 elements in bfloat16 with a 16-bit cache, lanes three quarters full: whole lines (see exchange_lines) behind a
     // gate, four waves a workgroup, pairwise from 17/32 of a round and by halves from five eighths (1811 tokens of 32+8+8 6.77 /
     // 5.93, 2550 of 40+8+8 7.84 / 7.45, pairwise 1152 of 64+8+8 7.29 / 6.0; by halves 1590 of 32+8+8 5.41 / 5.70, 16+2+2 5.7 / 5.9,
@@ -1629,11 +1626,8 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
                                (two_thirds || gated_lines || (half ? !(kv_fp8 && many_v) && round_8ths >= (kv_fp8 ? 4 : 3) * (int64_t)kResidentUnits
                                                                    : axes == 1 && !kv_fp8 && a.total_units >= kResidentUnits / 2));
     const bool fuller = gated_by_rule && (two_thirds || gated_lines);
-    double times;  // of the launch's reads at 7 TB/s
-    if (gated_lines) times = neox ? 1.15 : 1.25;
-    else if (two_thirds) times = half && neox && no_idle_lane && set_kv && !kv_fp8 && !many_v && D != 64 ? 1.1 : !half && !neox && !kv_fp8 ? 1.3 : 1.2;
-    else if (half && 2 * a.total_units < kResidentUnits) times = neox ? 1.0 : 1.1;
-    else times = half && neox && no_idle_lane && set_kv ? (kv_fp8 ? 1.0 : 1.1) : 1.15;
+    // times the launch's reads at 7 TB/s
+    const double times = !half && !neox && !kv_fp8 && two_thirds ? 1.3 : half && neox && no_idle_lane && set_kv && !kv_fp8 && !many_v ? 1.1 : 1.2;
     if (g_unit_gate > 0) p.unit_gate = (uint32_t)g_unit_gate;
     else if (gated_by_rule) p.unit_gate = (uint32_t)std::min(times * (double)read_bytes / 70000.0, 5000.0);
     if (g_stream_rows == 2) p.whole_lines = true;
