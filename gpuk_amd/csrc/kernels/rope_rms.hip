@@ -1538,10 +1538,12 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // Two items per wave, from 4096 items to twice that: 4096 waves, four on every SIMD, one item each and the others dealt out
     // evenly.  In half precision at once (28+4+4 15.4 / 12.7 at 4148 tokens, 16+2+2 10.0 / 8.7 at 4367); in bfloat16 where lanes are full,
     // three table rows are read or the last layer is half full (145 calls with idle lanes 0.97 of the time, 44 of a layer less full 1.03; 16+2+2
-    // 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600, pairwise 16+4+4 14.6 / 12.9 at 5031), four units that
-    // are whole tokens or some of them idle, but for three rows, from 4608 items (28+4+4 15.2 / 15.4 at 4100, 18.4 / 18.2 at 5200, 21.1 / 19.1 at 6144; but 1151
-    // tokens of 112+16+16, four parts, 18.6 / 15.2).  An eighth layer fills them all: in parts of a token in place, and pairwise in place or
-    // with three units, the two are level there or this one is behind (16+2 in place 12.7 / 14.9 at 7348, 64+8+8 heads of 256 pairwise 19.1 / 20.6 at 7380).
+    // 12.2 / 13.0 at 5237, 17.1 / 16.9 at 7600, pairwise 16+4+4 14.6 / 12.9 at 5031), four units from
+    // 4608 items (281 calls before that 1.04, whole tokens 28+4+4 15.2 / 15.4 at 4100, 18.4 / 18.2 at 5200, 21.1 / 19.1 at 6144), but at once
+    // pairwise with three rows (50 calls 0.92) and in two or four full parts, of which the first items are whole tokens (45 calls
+    // 0.94, 1151 tokens of 112+16+16 18.6 / 15.2).  An eighth layer fills them all: rotated pairwise and, in place, in parts of a token
+    // the two are level there or this one is behind (16+2 in place 12.7 / 14.9 at 7348, 64+8+8 heads of 256 pairwise 19.1 / 20.6 at 7380, 2566
+    // tokens of 80+8+8 pairwise 22.6 / 23.8) unless three rows are read or a token has 16 units (112+16+16, 1805 tokens, 27.7 / 24.9).
     const int units = shape.units;
     const int64_t items = shape.items;
     const int64_t layer = items % 1024 ? items % 1024 : 1024;  // items of the last layer
@@ -1558,7 +1560,8 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
         // 17.6 / 16.8 at 4096, level at 2500.
         large = 8 * (int64_t)a.total_units >= (units == 4 ? 10 : 13) * kResidentUnits && layer >= 256;
     } else if (two) {
-        const bool eighth_layer = set_kv ? neox || units == 4 : neox && whole, at_once = units == 3 || three_rows || (!whole && no_idle_unit);
+        const bool eighth_layer = set_kv ? neox || three_rows || a.units_per_token == 16 : neox && whole;
+        const bool at_once = units == 3 || (three_rows && !neox) || (no_idle_unit && shape.parts % 2 == 0);
         large = (items <= 7168 || eighth_layer) && (half || ((at_once || items >= 4608) && (full || three_rows || layer >= 512)));
     } else {
         int64_t sixteenths = 16;  // of a round, 16: beyond one
@@ -1601,7 +1604,7 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // 1.2 times serves all forms within 1 % (over 7000 random calls of shorter and longer gates) but two: bfloat16 rotated pairwise, whose waves
     // take longer, waits 1.3 times from two thirds of a round on (0.98 of the time over 640 calls, with an fp8 cache level), and half
     // precision by halves with every lane in use and a 16-bit cache 1.1 times (0.99 over 190 calls; in place 1.02, 2863 tokens of 14+2 heads
-    // 5.0 / 5.3, with many V heads 1.02).
+    // 5.0 / 5.3, with many V heads 1.02, heads of 64 level, 2523 tokens of 32+16+16 8.0 / 8.9).
     // Heads of 64 elements in bfloat16 with a 16-bit cache, lanes three quarters full: whole lines (see exchange_lines) behind a
     // gate, four waves a workgroup, pairwise from 17/32 of a round and by halves from five eighths (1811 tokens of 32+8+8 6.77 /
     // 5.93, 2550 of 40+8+8 7.84 / 7.45, pairwise 1152 of 64+8+8 7.29 / 6.0; by halves 1590 of 32+8+8 5.41 / 5.70, 16+2+2 5.7 / 5.9,
@@ -1627,7 +1630,7 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
                                                                    : axes == 1 && !kv_fp8 && a.total_units >= kResidentUnits / 2));
     const bool fuller = gated_by_rule && (two_thirds || gated_lines);
     // times the launch's reads at 7 TB/s
-    const double times = !half && !neox && !kv_fp8 && two_thirds ? 1.3 : half && neox && no_idle_lane && set_kv && !kv_fp8 && !many_v ? 1.1 : 1.2;
+    const double times = !half && !neox && !kv_fp8 && two_thirds ? 1.3 : half && neox && no_idle_lane && set_kv && !kv_fp8 && !many_v && D != 64 ? 1.1 : 1.2;
     if (g_unit_gate > 0) p.unit_gate = (uint32_t)g_unit_gate;
     else if (gated_by_rule) p.unit_gate = (uint32_t)std::min(times * (double)read_bytes / 70000.0, 5000.0);
     if (g_stream_rows == 2) p.whole_lines = true;
@@ -1640,10 +1643,13 @@ RopePlan plan_rope(const RopeArgs &a, int D, int axes, bool neox, bool set_kv, b
     // waves for small batches of other head counts (2-6 % ahead at 64+8 heads with an fp8 cache up to 512 tokens,
     // within 1-3 % either way for 3, 5 and 6 units per token); 128 lanes is the slowest in most cases.  In place, without the
     // scatter, four waves in bfloat16 rotated by halves from five eighths of a round (141 calls 0.96 of the time of single waves) and
-    // wherever heads of 64 elements that fill their lanes are gated (61 calls 0.93, with idle lanes 99 calls level); not before (860 calls level), pairwise (480 calls 1.03, 1609 tokens of 16+8
+    // wherever heads of 64 elements that fill their lanes are gated (61 calls 0.93, with idle lanes 99 calls level), and from three
+    // eighths, pairwise a half, where two fifths of the lanes idle (334 calls 0.97, 1724 tokens of 8+1 4.44 / 3.93); not before (860 calls level), pairwise (480 calls 1.03, 1609 tokens of 16+8
     // heads 5.1 / 5.9) or in half precision (620 calls 1.06, 503 of 64+8 4.4 / 4.9), which take four from two thirds of a round on, as all
     // gated launches do (see above).
-    const bool four_in_place = !set_kv && !half && ((neox && round_8ths >= 5 * (int64_t)kResidentUnits) || (D == 64 && no_idle_lane && gated_by_rule));
+    const bool two_fifths_idle = 5 * heads < 3 * places && round_8ths >= (neox ? 3 : 4) * (int64_t)kResidentUnits;
+    const bool four_in_place = !set_kv && !half &&
+                               (two_fifths_idle || (neox && round_8ths >= 5 * (int64_t)kResidentUnits) || (D == 64 && no_idle_lane && gated_by_rule));
     // Just beyond a round tokens of three units with a cache, which four waves do not hold whole, are ahead in single waves (20 calls of
     // 1 to 1.5 rounds 0.90 to 0.995 of the time, level from there: 2966 tokens of 16+2+2 heads, fp8 cache, 8.9 / 8.2, 3166 of 32+8+8 of 64
     // 10.8 / 9.6, 3481 of 40+8+8 of 64 with a 16-bit cache 12.3 / 11.4; two units 1.05 to 1.1, four 1.06, in place level).

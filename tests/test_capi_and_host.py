@@ -497,7 +497,7 @@ def test_rope_launch_shape_report_of_rotation_and_sections():
     assert shape(2400, mrope_section=[24, 20, 20], is_interleaved=True)[3] == 1           # three table rows: from nine eighths
     assert shape(3100)[3] == 1 and shape(3100, is_neox=False)[3] == 0                     # a layer of waves that has just begun
     assert shape(4200)[3] == 0                                                            # two whole tokens of four: from 4608
-    assert shape(4200, mrope_section=[24, 20, 20], is_interleaved=True)[3] == 2           # three table rows: at once
+    assert shape(4200, is_neox=False, mrope_section=[24, 20, 20], is_interleaved=True)[3] == 2   # three table rows pairwise: at once
     assert capi.rope_rms_launch_shape(1850, 64, 64, 64, 64, is_neox=False)[1] == 256
     # in place, parts of a token: a form for rotation by halves only
     assert capi.rope_rms_launch_shape(1536, 40, 8, 8, 128, set_kv=False)[3] == 1
@@ -529,12 +529,12 @@ def test_rope_kernel_choice():
             ((12, 12, 12), 128, f16, True, ((2390, 1), (4097, 0)), ((2390, 1), (3073, 0), (3328, 1), (4097, 0))),
             ((24, 8, 8), 256, bf16, True, ((1152, 1), (2049, 0)), ((1152, 1), (1537, 0), (1664, 1), (2049, 0))),
             # four, five: bfloat16 from nine eighths of a round, whole tokens of four and five with idle units from five quarters
-            ((28, 4, 4), 256, bf16, True, ((1152, 1), (2049, 2), (4097, 0)), ((1152, 1), (1537, 0), (1664, 1), (2049, 2), (4097, 0))),
-            ((28, 4, 4), 128, bf16, True, ((2560, 1), (4097, 0), (4608, 2), (8193, 0)), ((2560, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (8193, 0))),
-            ((28, 4, 4), 128, f16, True, ((1792, 1), (4097, 2), (8193, 0)), ((1792, 1), (3073, 0), (3328, 1), (4097, 2), (8193, 0))),
+            ((28, 4, 4), 256, bf16, True, ((1152, 1), (2049, 2), (4097, 0)), ((1152, 1), (1537, 0), (1664, 1), (2049, 2), (3585, 0))),
+            ((28, 4, 4), 128, bf16, True, ((2560, 1), (4097, 0), (4608, 2), (8193, 0)), ((2560, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (7169, 0))),
+            ((28, 4, 4), 128, f16, True, ((1792, 1), (4097, 2), (8193, 0)), ((1792, 1), (3073, 0), (3328, 1), (4097, 2), (7169, 0))),
             ((32, 8, 8), 128, bf16, True, ((1844, 1), (4097, 0)), ((1844, 1), (3073, 0), (3328, 1), (4097, 0))),
             ((32, 8, 8), 128, f16, True, ((1536, 1), (4097, 0)), ((1536, 1), (3073, 0), (3328, 1), (4097, 0))),
-            ((96, 12, 12), 128, bf16, True, ((732, 1), (1366, 2), (2049, 0)), ((732, 1), (1025, 0), (1110, 1), (1366, 2), (1434, 0), (1639, 2), (2049, 0))),
+            ((96, 12, 12), 128, bf16, True, ((732, 1), (1366, 2), (2049, 0)), ((732, 1), (1025, 0), (1110, 1), (1366, 2), (1434, 0), (1639, 2), (1793, 0))),
             # in place; pairwise whole tokens only
             ((32, 8, 8), 128, bf16, False, ((2458, 1), (3073, 0), (3328, 1), (4097, 0)), ((2458, 1), (3073, 0), (3328, 1), (4097, 0))),
             ((28, 4, 4), 128, bf16, False, ((2816, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (8193, 0)), ((2816, 1), (3073, 0), (3328, 1), (4097, 0), (4608, 2), (7169, 0))),
@@ -564,6 +564,8 @@ def test_rope_workgroups():
     for tokens, heads, dtype, neox, lanes in ((1023, (32, 8, 8), bf16, True, 64), (1024, (32, 8, 8), bf16, True, 256), (1092, (32, 8, 8), bf16, False, 64), (1093, (32, 8, 8), bf16, False, 256),
                                               (1092, (32, 8, 8), f16, True, 64), (1093, (32, 8, 8), f16, True, 256), (1820, (16, 2, 2), f16, False, 64), (1821, (16, 2, 2), f16, False, 256)):
         assert capi.rope_rms_launch_shape(tokens, *heads, 128, 1, dtype, False, False, neox)[1] == lanes, (tokens, heads, dtype, neox)
+    for T, neox, lanes in ((1535, True, 64), (1536, True, 256), (2047, False, 64), (2048, False, 256)):   # two fifths of the lanes idle
+        assert capi.rope_rms_launch_shape(T, 8, 1, 1, 128, 1, bf16, False, False, neox)[1] == lanes, (T, neox)
     for heads, changes in (((72, 8, 8), 820), ((64, 8, 8), 1093)):   # (lanes that idle: from two thirds)
         assert [capi.rope_rms_launch_shape(T, *heads, 64, 1, bf16, False, False, False)[1] for T in (changes - 1, changes)] == [64, 256]
     for tokens, heads, D, dtype, cache, fp8, lanes in (
